@@ -17,8 +17,8 @@ Fourier case. The forms timed on the same steps, each with the same
 iteration cap (3000), each run the way the caller runs its time steps: every
 solve is handed the form's own solution of the step before, its
 volume-weighted mean removed (PressureProjection.cpp:325-431):
-  * fp64: the FP64 drop-in (the reference algorithm, FP64 MFMA block-Jacobi
-    GEMM); its steps that do not reach the tolerance are counted;
+  * fp64: the FP64 drop-in (the reference algorithm, the block-Jacobi inverse
+    by sine transforms); its steps that do not reach the tolerance are counted;
   * prev_guess: the chosen form — FP16 split-precision MFMA GEMM with FP32
     accumulation, FP32 Krylov vectors, FP64 iterative refinement — from the
     previous pressure;
@@ -77,7 +77,6 @@ sys.path.insert(0, ROOT)
 
 METRIC = "Poisson solves/sec at rel. residual 1e-7 (mixed+learned vs FP64); HBM GB/s"
 HBM_PEAK = 8000.0       # GB/s, MI355X
-FP64_MFMA_PEAK = 78.6   # TFLOP/s, dense FP64 matrix
 F16_MFMA_PEAK = 2500.0  # TFLOP/s, dense FP16/BF16 matrix
 MAX_ITER = 3000         # iteration cap of every timed form
 REF_TOL = 1e-10         # true relative residual of the untimed reference solves
@@ -845,14 +844,13 @@ def main():
                                                           for r in res64])), 4),
                  "solves_per_s_converged_steps": (round(1e3 / float(np.mean(fp64_conv_ms)), 4)
                                                   if fp64_conv_ms else None),
-                 "gemm_TFLOP/s": round(g64["TFLOP/s"], 2),
-                 "gemm_mfma_frac": round(g64["TFLOP/s"] / FP64_MFMA_PEAK, 4),
+                 "precond_GB/s": round(g64["GB/s"], 1),
                  "kernels_us": {KERNELS[k]: round(v["avg_us"], 2) for k, v in k64.items()}},
         "fp64_dst": ({**summary(res64_dst, tol),
                       "ms_per_iteration": round(float(np.mean([r[0] / r[1]["iterations"]
                                                                for r in res64_dst])), 4),
-                      "note": "FP64 drop-in with precond = DST: the same exact block inverse "
-                              "by sine transforms instead of the P_inv GEMM"}
+                      "note": "FP64 drop-in with precond = DST (in FP64 the same kernels as "
+                              "the default)"}
                      if res64_dst else None),
         "precond_dst": ({**summary(res_dst, tol),
                          "speedup_vs_gemm_form": round(ms / float(np.mean([r[0] for r in res_dst])),

@@ -17,8 +17,6 @@ void launch_getvec64(hipStream_t s, long long n, long long zero_row, const doubl
                      double tol_b);
 void launch_spmv64(hipStream_t s, int mode, const DevGrid<double>& g, const double* x, double* y,
                    const double* a, double* c, double* c2, SolverState* st, double* part);
-void launch_precond64(hipStream_t s, int mode, int nb, const double* Ppk, const double* invh,
-                      const KrylovVectors<double>& v, SolverState* st);
 void launch_update64(hipStream_t s, long long n, const KrylovVectors<double>& v, SolverState* st,
                      double* part);
 void launch_copy_opt64(hipStream_t s, long long n, const KrylovVectors<double>& v,

@@ -9,15 +9,14 @@
 // partials, then the last workgroup adds them in workgroup order) and the
 // scalar recurrences run on the device, so the host only polls a status word
 // every few iterations:
-//   K1 k_precond<P>   p = r + beta (p - omega nu)  [p = r after a restart,
+//   K1 k_precond_dst<P> p = r + beta (p - omega nu)  [p = r after a restart,
 //                     rhat = r]; z1 = M^-1 p
 //   K2 k_spmv<DOT1>   nu = A z1; alpha = rho / ((rhat, nu) + eps)
-//   K3 k_precond<S>   s = r - alpha nu (in r); z2 = M^-1 s
+//   K3 k_precond_dst<S> s = r - alpha nu (in r); z2 = M^-1 s
 //   K4 k_spmv<DOT2>   t = A z2; omega = (t, s) / ((t, t) + eps)
 //   K5 k_update       x' = x + alpha z1 + omega z2; r = s - omega t;
 //                     rho' = (rhat, r), |r|; x_opt / convergence / restart
-// M^-1 = blockdiag(h_b^-1 P_inv) is one GEMM over all blocks on the FP64
-// matrix cores (v_mfma_f64_16x16x4f64).
+// M^-1 = blockdiag(h_b^-1 P_inv), applied by sine transforms (diffusion.hip).
 
 #include <hip/hip_runtime.h>
 
@@ -27,153 +26,9 @@
 
 namespace cup3d {
 
-typedef double double4_t __attribute__((ext_vector_type(4)));
-
-// ---------------------------------------------------------------------------
-// K1 / K3: fused vector update + block-Jacobi GEMM on the FP64 matrix cores.
-//
-// A workgroup of 8 wavefronts owns 32 blocks (one workgroup per CU at 8192
-// blocks). Their updated vectors (p or s) are written to HBM and staged in
-// LDS as 32 rows of 512 doubles (row stride 514, which keeps the fragment
-// reads free of bank conflicts). Each wavefront computes 64 output cells x
-// 32 blocks as 4 x 2 tiles of v_mfma_f64_16x16x4f64:
-//   D[j][i] += sum_k V[j][k] * P[k][i]     (j: block, i: output cell)
-// with the A operand (V) read from LDS and the B operand (P_inv) streamed
-// from L2 in a fragment-packed layout: fragment (it, kt) holds
-// P[4 kt + l/16][16 it + l%16] in lane l, 64 consecutive doubles. P_inv
-// (2 MiB) is streamed once per 32 blocks.
-// The reference computes z_b = invh_b * P_inv p_b with cublasDgemm(OP_T, OP_N)
-// + blockDscal (BiCGSTAB.cu:526-528,553-555); P_inv is symmetric.
-// ---------------------------------------------------------------------------
-constexpr int PC_W = 8;          // wavefronts per workgroup
-constexpr int PC_T = PC_W * 64;  // threads per workgroup
-constexpr int PC_LD = BLEN + 2;  // LDS row stride (doubles)
-
-typedef double double2_t __attribute__((ext_vector_type(2)));
-
-template <int MODE, int PC_NB>
-__global__ __launch_bounds__(PC_T) void k_precond_f64(int nb, const double* __restrict__ Ppk,
-                                                      const double* __restrict__ invh,
-                                                      KrylovVectors<double> v, SolverState* st) {
-  constexpr int JT = PC_NB / 16;  // block tiles
-  __shared__ double Vs[PC_NB * PC_LD];
-  if (MODE != PREC_PLAIN && st->status != ST_RUNNING) return;
-  const int j0 = (int)blockIdx.x * PC_NB;
-  const double beta = MODE == PREC_P ? st->beta : 0.0;
-  const double omega = MODE == PREC_P ? st->omega : 0.0;
-  const double alpha = MODE == PREC_S ? st->alpha : 0.0;
-  const int pzero = MODE == PREC_P ? st->p_zero : 0;
-  const int restart = MODE == PREC_P ? st->restart_pending : 0;
-  double* __restrict__ out = MODE == PREC_S ? v.z2 : v.z1;
-  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-  // phase 1: wave w owns blocks [NPB w, NPB w + NPB), two at a time; element
-  // u of a lane covers cells 128 (u % 4) + 2 l, +1 of block 2 h + u / 4. All
-  // loads of a pair are issued before the first use.
-  constexpr int NPB = PC_NB / PC_W;  // 4 or 2
-#pragma unroll
-  for (int hh = 0; hh < NPB / 2; ++hh) {
-    double2_t ra[8], rb[8], rc[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int b = j0 + NPB * w + 2 * hh + u / 4;
-      const size_t i2 = ((size_t)b * BLEN + 128 * (u & 3) + 2 * l) / 2;
-      if (b < nb) {
-        if (MODE == PREC_P) {
-          ra[u] = reinterpret_cast<const double2_t*>(v.r)[i2];
-          rb[u] = reinterpret_cast<const double2_t*>(v.nu)[i2];
-          rc[u] = reinterpret_cast<const double2_t*>(v.p)[i2];
-        } else if (MODE == PREC_S) {
-          ra[u] = reinterpret_cast<const double2_t*>(v.r)[i2];
-          rb[u] = reinterpret_cast<const double2_t*>(v.nu)[i2];
-        } else {
-          ra[u] = reinterpret_cast<const double2_t*>(v.p)[i2];
-        }
-      } else {
-        ra[u] = rb[u] = rc[u] = (double2_t){0.0, 0.0};
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int jj = NPB * w + 2 * hh + u / 4;
-      const int b = j0 + jj;
-      const size_t i2 = ((size_t)b * BLEN + 128 * (u & 3) + 2 * l) / 2;
-      double2_t val = ra[u];
-      if (MODE == PREC_P) {
-        // p = r + beta (p - omega nu)   (BiCGSTAB.cu:518-522)
-        if (!pzero) {
-          val.x = fma(beta, fma(-omega, rb[u].x, rc[u].x), ra[u].x);
-          val.y = fma(beta, fma(-omega, rb[u].y, rc[u].y), ra[u].y);
-        }
-        if (b < nb) {
-          reinterpret_cast<double2_t*>(v.p)[i2] = val;
-          if (restart) reinterpret_cast<double2_t*>(v.rhat)[i2] = ra[u];
-        }
-      } else if (MODE == PREC_S) {
-        // s = r - alpha nu   (BiCGSTAB.cu:546-549)
-        val.x = fma(-alpha, rb[u].x, ra[u].x);
-        val.y = fma(-alpha, rb[u].y, ra[u].y);
-        if (b < nb) reinterpret_cast<double2_t*>(v.r)[i2] = val;
-      }
-      const int k = 128 * (u & 3) + 2 * l;
-      Vs[jj * PC_LD + k] = val.x;
-      Vs[jj * PC_LD + k + 1] = val.y;
-    }
-  }
-  __syncthreads();
-  // phase 2: wave w owns output cells [64 w, 64 w + 64) of all PC_NB blocks
-  const int lr = l & 15, lk = l >> 4;
-  double4_t acc[4][JT];
-#pragma unroll
-  for (int t = 0; t < 4; ++t)
-#pragma unroll
-    for (int jt = 0; jt < JT; ++jt) acc[t][jt] = (double4_t){0.0, 0.0, 0.0, 0.0};
-  const double* __restrict__ pb = Ppk + (size_t)(4 * w) * 128 * 64 + l;
-  // P fragments stream from L2 through a 4-stage register ring: the loads for
-  // k-step kt+4 are issued while the MFMAs of kt run, hiding L2 latency.
-  constexpr int NST = 4;
-  double bq[NST][4];
-#pragma unroll
-  for (int s_ = 0; s_ < NST; ++s_)
-#pragma unroll
-    for (int t = 0; t < 4; ++t) bq[s_][t] = pb[((size_t)t * 128 + s_) * 64];
-  for (int k0 = 0; k0 < 128; k0 += NST) {
-#pragma unroll
-    for (int s_ = 0; s_ < NST; ++s_) {
-      const int kt = k0 + s_;
-      double a[JT];
-#pragma unroll
-      for (int jt = 0; jt < JT; ++jt) a[jt] = Vs[(16 * jt + lr) * PC_LD + 4 * kt + lk];
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int jt = 0; jt < JT; ++jt)
-          acc[t][jt] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[jt], bq[s_][t], acc[t][jt], 0, 0, 0);
-      const int kn = kt + NST < 128 ? kt + NST : kt;
-#pragma unroll
-      for (int t = 0; t < 4; ++t) bq[s_][t] = pb[((size_t)t * 128 + kn) * 64];
-    }
-  }
-  // D layout of v_mfma_f64_16x16x4f64: register q of lane l holds
-  // D[l/16 + 4q][l%16]
-#pragma unroll
-  for (int jt = 0; jt < JT; ++jt)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int b = j0 + jt * 16 + lk + 4 * q;
-      if (b < nb) {
-        const double s = invh[b];
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-          out[(size_t)b * BLEN + (4 * w + t) * 16 + lr] = acc[t][jt][q] * s;
-      }
-    }
-}
-
 // ---------------------------------------------------------------------------
 // Host launchers
 // ---------------------------------------------------------------------------
-static inline int wg_for_blocks(int nb, int per) { return (nb + per - 1) / per; }
-
 void launch_getvec64(hipStream_t s, long long n, long long zero_row, const double* rhs,
                      const double* x0, double* b, double* x, SolverState* st, double* part,
                      double tol_b) {
@@ -191,28 +46,6 @@ void launch_spmv64(hipStream_t s, int mode, const DevGrid<double>& g, const doub
     case SPMV_DOT2: spmv_launch<double, SPMV_DOT2>(s, g, x, y, a, c, c2, st, part); break;
     case SPMV_RESID: spmv_launch<double, SPMV_RESID>(s, g, x, y, a, c, c2, st, part); break;
   }
-}
-
-// Blocks per workgroup: 32 halves the L2 stream of P_inv but needs 8192
-// blocks to give every CU a workgroup; smaller grids use 16.
-static inline int precond64_width(int nb) { return nb >= 32 * 256 ? 32 : 16; }
-
-template <int NB>
-static void launch_precond64_w(hipStream_t s, int mode, int nb, const double* Ppk,
-                               const double* invh, const KrylovVectors<double>& v,
-                               SolverState* st) {
-  const int nwg = wg_for_blocks(nb, NB);
-  switch (mode) {
-    case PREC_P: k_precond_f64<PREC_P, NB><<<nwg, PC_T, 0, s>>>(nb, Ppk, invh, v, st); break;
-    case PREC_S: k_precond_f64<PREC_S, NB><<<nwg, PC_T, 0, s>>>(nb, Ppk, invh, v, st); break;
-    default: k_precond_f64<PREC_PLAIN, NB><<<nwg, PC_T, 0, s>>>(nb, Ppk, invh, v, st); break;
-  }
-}
-
-void launch_precond64(hipStream_t s, int mode, int nb, const double* Ppk, const double* invh,
-                      const KrylovVectors<double>& v, SolverState* st) {
-  if (precond64_width(nb) == 32) launch_precond64_w<32>(s, mode, nb, Ppk, invh, v, st);
-  else launch_precond64_w<16>(s, mode, nb, Ppk, invh, v, st);
 }
 
 void launch_update64(hipStream_t s, long long n, const KrylovVectors<double>& v, SolverState* st,
@@ -415,15 +248,6 @@ void launch_guess_blend(hipStream_t s, long long n, const double* x0, const Gues
   const int nwg = (int)std::min<long long>((n + WG_THREADS - 1) / WG_THREADS, 8192);
   k_guess_blend<<<nwg, WG_THREADS, 0, s>>>(n, x0, h, g, m < HIST_MAX ? m : HIST_MAX, pred, gnet,
                                            row, x);
-}
-
-// Fragment-packed P for the B operand: Ppk[(it*128 + kt)*64 + l] = P[4kt + l/16][16it + l%16].
-void pack_pinv_f64(const std::vector<double>& P, std::vector<double>& pk) {
-  pk.assign((size_t)BLEN * BLEN, 0.0);
-  for (int it = 0; it < 32; ++it)
-    for (int kt = 0; kt < 128; ++kt)
-      for (int l = 0; l < 64; ++l)
-        pk[((size_t)it * 128 + kt) * 64 + l] = P[(size_t)(4 * kt + l / 16) * BLEN + 16 * it + l % 16];
 }
 
 }  // namespace cup3d

@@ -135,7 +135,4 @@ void set_global_error(const std::string& m);
 bool build_topology(const TopologyInput& in, HostTopology& out, std::string& err);
 void build_pinv_dst(std::vector<double>& P);  // 512x512 row-major, = A_loc^-1 with sign of the reference
 
-// Precond GEMM operand packing (kernels_precond.hip)
-void pack_pinv_f64(const std::vector<double>& P, std::vector<double>& packed);
-
 }  // namespace cup3d

@@ -105,9 +105,8 @@ struct cup3d_poisson {
 
   // preconditioner
   std::vector<double> P;
-  DevBuf d_P64;
-  DevBuf d_dst;    // DST block-inverse table (DST_TABLE doubles), for cfg.precond = DST
-  DevBuf d_dst32;  // its FP32 rounding (the mixed forms' inner solve) and implicit diffusion
+  DevBuf d_dst;    // DST block-inverse table (DST_TABLE doubles): FP64 forms, implicit diffusion
+  DevBuf d_dst32;  // its FP32 rounding (the mixed forms' inner solve with cfg.precond = DST)
 
   // FP64 Krylov workspace
   DevBuf d_vec64;  // 11 vectors of n doubles
@@ -188,22 +187,24 @@ int upload(cup3d_poisson* H, DevBuf& d, const void* src, size_t bytes) {
   return 0;
 }
 
-// M^-1 of the FP64 form: the P_inv GEMM on the FP64 matrix cores, or (Helmholtz
-// grids, or cfg.precond = DST) the exact block inverse by sine transforms.
+// M^-1 in FP64: the exact block inverse in factored form, three sine transforms,
+// the eigenvalues and three more (96 flops a cell), for both settings of
+// cfg.precond and for Helmholtz grids. The dense 512 x 512 product it replaces
+// is the same matrix at 1024 flops a cell, bound by the FP64 matrix cores:
+// fused with the p update, K1 took 98.9 us that way and takes 34.2 us now on
+// 4.19 M cells (168 MB of vectors, 4.9 TB/s), 43 us (four workgroups) and
+// 5 us on 32 k cells.
 void launch_precond_fp64(cup3d_poisson* H, const DevGrid<double>& g, int mode,
                          const KrylovVectors<double>& v) {
   SolverState* st = H->d_state.as<SolverState>();
-  if (g.helm || H->cfg.precond == CUP3D_PRECOND_DST)
-    launch_precond_dst(H->stream, mode, H->nb, H->d_dst.as<double>(), g.h,
-                       g.helm ? g.helm_sigma : 0.0, v, st);
-  else
-    launch_precond64(H->stream, mode, H->nb, H->d_P64.as<double>(), g.invh, v, st);
+  launch_precond_dst(H->stream, mode, H->nb, H->d_dst.as<double>(), g.h,
+                     g.helm ? g.helm_sigma : 0.0, v, st);
 }
 
 // Run the FP64 classical BiCGSTAB on the device. b64/x64 must already hold
 // getVec's b and x0 (in v64.b and v64.x[0]); the state must be initialised.
 // With a Helmholtz grid (g.helm, implicit diffusion) the preconditioner is
-// the DST block inverse of each block's level instead of the P_inv GEMM.
+// the block inverse of each block's level.
 int run_bicgstab64(cup3d_poisson* H, const DevGrid<double>& g) {
   hipStream_t s = H->stream;
   SolverState* st = H->d_state.as<SolverState>();
@@ -305,15 +306,13 @@ int cup3d_poisson_create(const cup3d_poisson_config* cfg, cup3d_poisson_t* out) 
     g_create_error = "HIP stream/event/pinned allocation failed";
     return -1;
   }
-  // block-Jacobi inverse (PoissonSolverExp ctor) and its MFMA packing
+  // block-Jacobi inverse (PoissonSolverExp ctor): the dense matrix for the
+  // half-precision GEMM, the sine-transform table for the rest
   build_pinv_dst(H->P);
-  std::vector<double> pk;
-  pack_pinv_f64(H->P, pk);
   double dtab[DST_TABLE];
   float dtab32[DST_TABLE];
   dst_tables(dtab, dtab32);
-  if (upload(H.get(), H->d_P64, pk.data(), pk.size() * sizeof(double)) != 0 ||
-      upload(H.get(), H->d_dst, dtab, sizeof(dtab)) != 0 ||
+  if (upload(H.get(), H->d_dst, dtab, sizeof(dtab)) != 0 ||
       upload(H.get(), H->d_dst32, dtab32, sizeof(dtab32)) != 0 ||
       mixed_init_pinv(H->mixed, H->P, H->err) != 0 || cnn_init(H->cnn, H->err) != 0) {
     g_create_error = H->err;
@@ -1262,8 +1261,7 @@ int cup3d_debug_time_kernel(cup3d_poisson_t H, int which, int reps, double* avg_
     HIPCHECK(hipEventElapsedTime(&ms, H->ev0, H->ev1));
     *avg_ms = ms / reps;
     const double words[5] = {2, 2, 8, 5, 3};
-    const bool dst = H->cfg.precond == CUP3D_PRECOND_DST;
-    const double fpc[5] = {8, dst ? 96.0 : 1024.0, 8, dst ? 96.0 + 4 : 1024.0 + 4, 10};
+    const double fpc[5] = {8, 96, 8, 96 + 4, 10};
     by = 8.0 * words[which] * N;
     fl = fpc[which] * N;
   }

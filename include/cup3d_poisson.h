@@ -121,12 +121,13 @@ typedef struct {
   int extrapolate;   /* 0 = off (the reference contract); K = 1..8 = also extrapolate
                         the guess in time from the last K solves' (see above) */
   int precond;       /* how M^-1 = blockdiag(h_b^-1 P_inv) is applied.
-                        CUP3D_PRECOND_GEMM (0): P_inv x block matrix on the matrix cores
-                        (FP64, as the reference, BiCGSTAB.cu:526-528; the mixed forms:
-                        FP16/BF16 with FP32 accumulate); CUP3D_PRECOND_DST (1): the same
-                        exact inverse by 8-point sine transforms (P_inv is diagonalised
-                        by the 3-D DST) in the form's own precision (FP64, or FP32 in the
-                        mixed forms' inner solve), bound by HBM, not the matrix cores. */
+                        CUP3D_PRECOND_GEMM (0): in the mixed forms the dense P_inv x block
+                        matrix on the FP16/BF16 matrix cores with FP32 accumulate (P_inv
+                        rounded once); in FP64 the same product (BiCGSTAB.cu:526-528) in
+                        factored form, by 8-point sine transforms (P_inv is diagonalised
+                        by the 3-D DST), exact to rounding;
+                        CUP3D_PRECOND_DST (1): the factored form in every precision (FP32
+                        in the mixed forms' inner solve, its P_inv not rounded to 16 bits). */
 } cup3d_poisson_config;
 
 enum { CUP3D_PRECOND_GEMM = 0, CUP3D_PRECOND_DST = 1 };

@@ -36,8 +36,8 @@ int cup3d_debug_apply_operator32(cup3d_poisson_t h, const double* d_x, double* d
 /* Kernel timing for roofline reports: runs one kernel class `reps` times on
  * the handle's stream between two HIP events, on the data of the last solve,
  * and returns the average duration in ms. which: 0 = operator (SpMV),
- * 1 = block-Jacobi GEMM, 2 = fused x/r update (K5), 3 = fused p update +
- * GEMM (K1), 4 = SpMV + dot (K2), in the handle's precision. Also returns
+ * 1 = block-Jacobi inverse, 2 = fused x/r update (K5), 3 = fused p update +
+ * block-Jacobi inverse (K1), 4 = SpMV + dot (K2), in the handle's precision. Also returns
  * the algorithmic bytes (vectors read + written) and flops of one launch
  * (GEMM flops count the MFMA passes actually issued).
  * Must follow a solve on the current topology. Returns 0 or < 0. */
