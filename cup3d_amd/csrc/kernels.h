@@ -15,6 +15,8 @@ enum PrecMode { PREC_PLAIN = 0, PREC_P = 1, PREC_S = 2 };
 void launch_getvec64(hipStream_t s, long long n, long long zero_row, const double* rhs,
                      const double* x0, double* b, double* x, SolverState* st, double* part,
                      double tol_b);
+// part null (SPMV_PLAIN and SPMV_RESID on a grid with bMean 0 or 3): no sums are
+// taken and st is not used.
 void launch_spmv64(hipStream_t s, int mode, const DevGrid<double>& g, const double* x, double* y,
                    const double* a, double* c, double* c2, SolverState* st, double* part);
 void launch_update64(hipStream_t s, long long n, const KrylovVectors<double>& v, SolverState* st,

@@ -307,6 +307,9 @@ constexpr size_t STREAM_MIN_BYTES = size_t(64) << 20;
 // three; the workgroup barrier is the partial-sum reduction at the end.
 // ---------------------------------------------------------------------------
 //
+// a and c may be the same vector (SPMV_RESID in place): a lane reads its cells
+// of a before it writes the same cells of c, and no other lane reads them.
+//
 // HELM (FP64, bMean 0): the implicit-diffusion operator of one velocity
 // component, KernelLHSDiffusion (AdvectionDiffusionImplicit.h:40-56): the
 // same stencil and coarse-fine faces, plus -h^3 sigma x and the Dirichlet
@@ -314,8 +317,7 @@ constexpr size_t STREAM_MIN_BYTES = size_t(64) << 20;
 // selected by g.dmask, both folded into the diagonal of the cell.
 template <typename T, int MODE, int BM, bool IFACE, bool HELM = false, bool NT = false>
 __global__ __launch_bounds__(WG_THREADS) void k_spmv(DevGrid<T> g, const T* __restrict__ x,
-                                                     T* __restrict__ y, const T* __restrict__ a,
-                                                     T* __restrict__ c, T* __restrict__ c2,
+                                                     T* __restrict__ y, const T* a, T* c, T* c2,
                                                      SolverState* st, double* part) {
   constexpr bool NEED_A = MODE != SPMV_PLAIN;
   // sum_b h_b^3 sum x feeds the bMean = 1 row and the bMean = 2 term only
@@ -496,6 +498,7 @@ __global__ __launch_bounds__(WG_THREADS) void k_spmv(DevGrid<T> g, const T* __re
       }
     }
   }
+  if ((MODE == SPMV_PLAIN || MODE == SPMV_RESID) && !part) return;  // no sums wanted
   grid_store_partial<3>(v, part);
 }
 
@@ -657,6 +660,9 @@ inline void spmv_launch_iface(hipStream_t s, const DevGrid<T>& g, const T* x, T*
   }
   if (!launched) spmv_kernel<T, MODE, BM, HELM, false>(s, nwg, g, x, y, a, c, c2, st, part);
   if (mid) (void)hipEventRecord(mid, s);
+  // SPMV_PLAIN and SPMV_RESID without sums (part null; bMean 0 and 3 only): the
+  // vectors are complete, and the finalize kernel is 4 us of a 20-60 us call
+  if (!part) return;
   if (BM == 2) {
     k_bmean2_sum<MODE><<<1, WG_THREADS, 0, s>>>(st, part, nwg);
     // nb * 64 threads of 8 cells: (nb + 3) / 4 workgroups again, so the

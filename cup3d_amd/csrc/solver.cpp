@@ -92,10 +92,11 @@ struct cup3d_poisson {
 
   // topology: the tables live on the device (built there by the topology
   // kernels, two generations so that a rejected block list leaves the
-  // current one in place); the host keeps the block list, h^3 per block,
-  // the origin block and the face counts
+  // current one in place); the host keeps the block list, the volume, the
+  // origin block and the face counts
   HostTopology topo;
   std::vector<int> blocks;  // nb x 4
+  double volume = 0.0;      // sum of 512 h_b^3 in block order (0: not summed yet)
   int nb = 0;
   long long n = 0;
   DevTopo tp[2];
@@ -394,15 +395,11 @@ int cup3d_poisson_set_topology(cup3d_poisson_t H, int64_t nblocks, const cup3d_b
   Tn.origin_block = info[TI_ORIGIN];
   Tn.n_coarse_faces = info[TI_N_COARSE];
   Tn.n_fine_faces = info[TI_N_FINE];
-  Tn.h3.resize(nb);
-  for (size_t b = 0; b < nb; ++b) {
-    const double h = H->cfg.h0 / double(1 << bl[4 * b]);
-    Tn.h3[b] = h * h * h;
-  }
   if (H->cfg.bmean == 1 && Tn.origin_block >= 0) Tn.bmean_row = (long long)Tn.origin_block * BLEN;
   H->tcur = 1 - H->tcur;
   H->blocks.swap(bl);
   H->topo = std::move(Tn);
+  H->volume = 0.0;
   // from here on a failure (device allocation) leaves the handle without a
   // topology: solves are refused until set_topology succeeds
   struct Commit {
@@ -790,9 +787,13 @@ int cup3d_poisson_remove_mean(cup3d_poisson_t H, double* d_x, double* mean) {
   if (H->nb <= 0) return fail(H, "set_topology must be called first");
   if (check_vectors(H, {d_x}) != 0) return -1;
   HIPCHECK(hipSetDevice(H->device));
-  double vol = 0.0;
-  for (double h3 : H->topo.h3) vol += 512.0 * h3;
-  const double inv_vol = 1.0 / vol;
+  if (H->volume == 0.0) {
+    for (int b = 0; b < H->nb; ++b) {
+      const double h = H->cfg.h0 / double(1 << H->blocks[4 * b]);
+      H->volume += 512.0 * (h * h * h);
+    }
+  }
+  const double inv_vol = 1.0 / H->volume;
   launch_remove_mean(H->stream, H->n, d_x, H->tp[H->tcur].h3.as<double>(), inv_vol,
                      H->d_part.as<double>(), H->d_gdots.as<double>());
   HIPCHECK(hipGetLastError());
@@ -856,12 +857,11 @@ int cup3d_poisson_apply_operator(cup3d_poisson_t H, const double* d_x, double* d
   if (H->nb <= 0) return fail(H, "set_topology must be called first");
   if (check_vectors(H, {d_x, d_y}) != 0) return -1;
   HIPCHECK(hipSetDevice(H->device));
-  SolverState init = make_state(H->cfg);
-  *H->h_state = init;
-  HIPCHECK(hipMemcpyAsync(H->d_state.p, H->h_state, sizeof(SolverState), hipMemcpyHostToDevice,
-                          H->stream));
+  // only the bMean = 1 and 2 terms need the sums (the plain modes do not read
+  // the solver state, so it is not initialised)
+  const bool sums = H->cfg.bmean == 1 || H->cfg.bmean == 2;
   launch_spmv64(H->stream, SPMV_PLAIN, H->g64, d_x, d_y, nullptr, nullptr, nullptr,
-                H->d_state.as<SolverState>(), H->d_part.as<double>());
+                H->d_state.as<SolverState>(), sums ? H->d_part.as<double>() : nullptr);
   HIPCHECK(hipGetLastError());
   HIPCHECK(hipStreamSynchronize(H->stream));
   return 0;
@@ -913,15 +913,16 @@ int cup3d_projection_increment(cup3d_poisson_t H, double* d_rhs, const double* d
   DevGrid<double> g = H->g64;
   g.bmean = 0;
   g.bmean_row = -1;
-  SolverState init = make_state(H->cfg);
-  *H->h_state = init;
-  HIPCHECK(hipMemcpyAsync(H->d_state.p, H->h_state, sizeof(SolverState), hipMemcpyHostToDevice,
-                          H->stream));
-  double* tmp = H->v64.nu;
-  launch_spmv64(H->stream, SPMV_RESID, g, d_p_old, nullptr, d_rhs, tmp, nullptr,
-                H->d_state.as<SolverState>(), H->d_part.as<double>());
-  HIPCHECK(hipMemcpyAsync(d_rhs, tmp, (size_t)H->n * sizeof(double), hipMemcpyDeviceToDevice,
-                          H->stream));
+  // in place; through a Krylov vector when p_old overlaps rhs, whose cells the
+  // neighbours of a written block may still read
+  const uintptr_t pr = (uintptr_t)d_rhs, pp = (uintptr_t)d_p_old, len = H->n * sizeof(double);
+  const bool overlap = pr < pp + len && pp < pr + len;
+  double* out = overlap ? H->v64.nu : d_rhs;
+  launch_spmv64(H->stream, SPMV_RESID, g, d_p_old, nullptr, d_rhs, out, nullptr,
+                nullptr, nullptr);
+  if (overlap)
+    HIPCHECK(hipMemcpyAsync(d_rhs, out, (size_t)H->n * sizeof(double), hipMemcpyDeviceToDevice,
+                            H->stream));
   HIPCHECK(hipGetLastError());
   HIPCHECK(hipStreamSynchronize(H->stream));
   return 0;
@@ -1083,11 +1084,7 @@ int cup3d_diffusion_apply_operator(cup3d_poisson_t H, int comp, double nu, doubl
   DevGrid<double> g;
   if (diffusion_grid(H, comp, nu, dt, g) != 0) return -1;
   HIPCHECK(hipSetDevice(H->device));
-  *H->h_state = make_state(H->cfg);
-  HIPCHECK(hipMemcpyAsync(H->d_state.p, H->h_state, sizeof(SolverState), hipMemcpyHostToDevice,
-                          H->stream));
-  launch_spmv64(H->stream, SPMV_PLAIN, g, d_x, d_y, nullptr, nullptr, nullptr,
-                H->d_state.as<SolverState>(), H->d_part.as<double>());
+  launch_spmv64(H->stream, SPMV_PLAIN, g, d_x, d_y, nullptr, nullptr, nullptr, nullptr, nullptr);
   HIPCHECK(hipGetLastError());
   HIPCHECK(hipStreamSynchronize(H->stream));
   return 0;
