@@ -22,6 +22,8 @@ constexpr int CNN_NW = CNN_OB3 + 1;                         // 8241
 // FP16 fragment-packed weights: layer 1 7 k-steps, layers 2 and 3 14 each
 constexpr int CNN_KT1 = 7, CNN_KT2 = 14, CNN_KT3 = 14;
 constexpr int CNN_PK = (CNN_KT1 + CNN_KT2 + CNN_KT3) * 64 * 8;
+// FP32 fragments of the training kernels (cnn.hip)
+constexpr int CNN_FRAG = (14 + 108 + 108 + 8 + 7) * 64;
 
 struct CnnSample {
   float* res_h = nullptr;   // (b - A p_prev) / h_b  [n]
@@ -35,12 +37,15 @@ struct CnnState {
   float* d_w = nullptr;      // FP32 master weights [CNN_NW]
   float* d_adam = nullptr;   // m, v [2 * CNN_NW]
   void* d_wpk = nullptr;     // FP16 packed weights for inference
+  float* d_frag = nullptr;   // FP32 weight fragments for training
   double* d_scal = nullptr;  // device scalars: [0] = s_r, [1] = s_p of the last predict
   double* d_part = nullptr;
-  float* d_scratch = nullptr;  // training activations / gradients
+  float* d_scratch = nullptr;  // per-item gradients and losses
   long long scratch_cap = 0;
   int* d_items = nullptr;
   int items_cap = 0;
+  void* d_refs = nullptr;  // the samples' device pointers and scales
+  size_t refs_cap = 0;
   double* d_pred = nullptr;   // prediction buffer for the warm start
   int cap_nb = 0;             // blocks d_part and d_pred hold
   int nb = 0;

@@ -22,9 +22,9 @@
 // K = 27 offsets x input channels; the 8 consecutive K of a lane are 8
 // channels of one offset: one 16-byte LDS read), FP32 accumulation, bias and
 // GELU in FP32.
-// Training (k_cnn_train_item + k_cnn_adam): FP32, one workgroup per
-// (sample, block) item, forward and backward with activations in global
-// scratch, per-item gradients summed in item order (deterministic), Adam.
+// Training (k_cnn_train_item + k_cnn_adam): FP32 on v_mfma_f32_16x16x4_f32, one
+// workgroup per (sample, block) item, forward and backward in LDS, per-item
+// gradients summed in a fixed order (deterministic), Adam.
 
 #include <hip/hip_runtime.h>
 
@@ -42,9 +42,6 @@ typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float gelu(float x) { return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f)); }
-__device__ __forceinline__ float gelu_grad(float x) {
-  return 0.5f * (1.0f + erff(x * 0.70710678118654752f)) + x * expf(-0.5f * x * x) * 0.3989422804014327f;
-}
 
 // Index into a field of the cell that padded position (pz, py, px) in 0..9
 // of block b takes its value from (the halo rule above).
@@ -68,13 +65,6 @@ __device__ __forceinline__ size_t halo_index(const int* __restrict__ nbr, int b,
   }
   for (int d = 0; d < 3; ++d) c[d] = c[d] < 0 ? 0 : (c[d] > 7 ? 7 : c[d]);
   return (size_t)blk * BLEN + c[2] * 64 + c[1] * 8 + c[0];
-}
-
-// Value of field f at padded position (pz, py, px) in 0..9 of block b.
-template <typename T>
-__device__ __forceinline__ float halo_value(const T* __restrict__ f, const int* __restrict__ nbr,
-                                            int b, int pz, int py, int px) {
-  return (float)f[halo_index(nbr, b, pz, py, px)];
 }
 
 // ---------------------------------------------------------------------------
@@ -291,226 +281,452 @@ struct SampleRef {
   float s_p;
 };
 
-// per-item scratch layout (floats)
-constexpr int TS_X = 0;                        // [2][1000]
-constexpr int TS_Z1 = TS_X + 2 * PADC;         // [16][512]
-constexpr int TS_H1 = TS_Z1 + CNN_C * BLEN;    // [16][1000] padded
-constexpr int TS_Z2 = TS_H1 + CNN_C * PADC;    // [16][512]
-constexpr int TS_H2 = TS_Z2 + CNN_C * BLEN;    // [16][1000] padded
-constexpr int TS_D = TS_H2 + CNN_C * PADC;     // [512] dout
-constexpr int TS_DZ2 = TS_D + BLEN;            // [16][512]
-constexpr int TS_DZ1 = TS_DZ2 + CNN_C * BLEN;  // [16][512]
-constexpr int TS_SIZE = TS_DZ1 + CNN_C * BLEN;
+// ---------------------------------------------------------------------------
+// One (sample, block) item per workgroup of 8 wavefronts, forward and backward
+// with everything in LDS and registers: every contraction is an implicit GEMM
+// on v_mfma_f32_16x16x4_f32 (FP32 inputs and accumulation). Wavefront w owns
+// the z plane w of the block: four tiles of 16 cells (two x rows), so the 16
+// channels x 16 cells accumulators of the forward layers, of their
+// pre-activations and of the backward layers are the same registers.
+//   layer 1, 2      M = 16 cells, N = 16 channels, K = (offset, channel)
+//   layer 3         M = 16 cells, N = offset, K = channel: the products of
+//                   every cell with the 27 taps, then 27 shifted adds
+//   dZ2, dZ1        the same convolutions with the taps mirrored
+//   dW              M, N = channels (or N = taps), K = the 512 cells: offsets
+//                   or tap tiles are split over the wavefronts
+// Bound by the FP32 matrix cores: 12 064 MFMAs of 32 cycles an item over 4
+// SIMDs, 40 us at 2.4 GHz; a batch of 256 items gives every CU one. With
+// scalar FP32 loops through a global scratch buffer (200 KB an item) a step of
+// 256 items took 2156 us; now 80 us.
+//
+// LDS (floats): the input patch, act1 on the zero-padded 10^3 patch, then act2
+// and the tap products (later dZ2 on its padded patch), dL/dout padded, the
+// prediction with the target's halo, the local residual. A channel stride of
+// 1010 (18 mod 32 banks) keeps the 16 channels x 2 cells a half-wave reads for
+// the weight gradients in different banks.
+// ---------------------------------------------------------------------------
+constexpr int TR_T = 512;               // threads per item
+constexpr int TR_CS = PADC + 10;        // channel stride of the padded patches
+constexpr int TR_HS = BLEN + 20;        // of the unpadded ones (16-byte rows)
+constexpr int TR_X = 0;                 // [2][1000]
+constexpr int TR_H1 = TR_X + 2 * PADC;  // [16][TR_CS]; later dZ1 [16][TR_HS]
+constexpr int TR_H2 = TR_H1 + CNN_C * TR_CS;   // [16][TR_HS]; later dZ2 [16][TR_CS]
+constexpr int TR_P = TR_H2 + CNN_C * TR_HS;    // [16][TR_HS] tap products, reductions
+constexpr int TR_D = TR_P + CNN_C * TR_HS;     // [1000]
+constexpr int TR_OP = TR_D + PADC;             // [1000]
+constexpr int TR_RHO = TR_OP + PADC;           // [512]
+constexpr int TR_RED = TR_RHO + BLEN;          // [8][16] per-wavefront sums
+constexpr int TR_LDS = TR_RED + 8 * 16;
+static_assert(TR_X % 4 == 0 && TR_H1 % 4 == 0 && TR_H2 % 4 == 0 && TR_P % 4 == 0 && TR_HS % 4 == 0,
+              "16-byte rows");
+static_assert(TR_P + CNN_C * TR_HS - TR_H2 >= CNN_C * TR_CS, "dZ2 fits over act2 and the products");
+static_assert(TR_LDS * 4 <= 160 * 1024, "LDS of one CU");
+
+// offset of tap off (dz, dy, dx) in the padded 10^3 patch
+__device__ __forceinline__ constexpr int tap(int off) {
+  return (off / 9) * 100 + ((off / 3) % 3) * 10 + off % 3;
+}
+
+// FP32 weight fragments (B operands), 64 values each: value of lane l = k 16 + n
+// of k-step s. Mirrored taps (26 - off) turn the transposed convolutions of the
+// backward pass into the forward ones.
+//   F1  (14): off = 2 s + k / 2, c = k % 2, n = output channel
+//   F2 (108): off = s / 4, c = 4 (s % 4) + k, n = output channel
+//   T2 (108): off = 26 - s / 4, k = output channel 4 (s % 4) + k, n = input channel
+//   F3   (8): tile s / 4 of taps n, c = 4 (s % 4) + k
+//   T3   (7): off = 26 - (4 s + k), n = channel
+constexpr int FR_F1 = 0, FR_F2 = 14, FR_T2 = FR_F2 + 108, FR_F3 = FR_T2 + 108, FR_T3 = FR_F3 + 8;
+static_assert((FR_T3 + 7) * 64 == CNN_FRAG, "fragment buffer");
+
+// Weight j into the fragments that hold it (the missing taps stay zero).
+__device__ __forceinline__ void frag_store(float* __restrict__ fr, int j, float v) {
+  if (j < CNN_NW1) {
+    const int o = j / 54, c = (j / 27) % 2, off = j % 27;
+    fr[(FR_F1 + off / 2) * 64 + ((off % 2) * 2 + c) * 16 + o] = v;
+  } else if (j >= CNN_OW2 && j < CNN_OW2 + CNN_NW2) {
+    const int i = j - CNN_OW2, o = i / (CNN_C * 27), c = (i / 27) % CNN_C, off = i % 27;
+    fr[(FR_F2 + off * 4 + c / 4) * 64 + (c % 4) * 16 + o] = v;
+    fr[(FR_T2 + (26 - off) * 4 + o / 4) * 64 + (o % 4) * 16 + c] = v;
+  } else if (j >= CNN_OW3 && j < CNN_OW3 + CNN_NW3) {
+    const int i = j - CNN_OW3, c = i / 27, off = i % 27, r = 26 - off;
+    fr[(FR_F3 + (off / 16) * 4 + c / 4) * 64 + (c % 4) * 16 + off % 16] = v;
+    fr[(FR_T3 + r / 4) * 64 + (r % 4) * 16 + c] = v;
+  }
+}
+
+__global__ void k_cnn_frag(const float* __restrict__ w, float* __restrict__ fr) {
+  const int j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j < CNN_NW) frag_store(fr, j, w[j]);
+}
+
+// Position of weight j's gradient in an item's gradient: W2 as [off][o][c], the
+// order its accumulators are stored in; everything else as the weights.
+__device__ __forceinline__ int grad_index(int j) {
+  if (j < CNN_OW2 || j >= CNN_OW2 + CNN_NW2) return j;
+  const int i = j - CNN_OW2, o = i / (CNN_C * 27), c = (i / 27) % CNN_C, off = i % 27;
+  return CNN_OW2 + off * (CNN_C * CNN_C) + o * CNN_C + c;
+}
+__device__ __forceinline__ int weight_index(int e) {  // its inverse
+  if (e < CNN_OW2 || e >= CNN_OW2 + CNN_NW2) return e;
+  const int i = e - CNN_OW2, off = i / (CNN_C * CNN_C), o = (i / CNN_C) % CNN_C, c = i % CNN_C;
+  return CNN_OW2 + (o * CNN_C + c) * 27 + off;
+}
+
+__device__ __forceinline__ float4_t mfma32(float a, float b, float4_t c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// acc[t] += the 16 -> 16 channel convolution of the padded patches `in` at the
+// four cell tiles of this wavefront; base = k TR_CS + the lane's cell of tile 0.
+// The fragments of the next three taps are loaded while these are multiplied.
+__device__ __forceinline__ void conv16(const float* in, const float* __restrict__ fr, int base,
+                                       int l, float4_t (&acc)[4]) {
+  float bq[12], bn[12];
+#pragma unroll
+  for (int s = 0; s < 12; ++s) bq[s] = fr[s * 64 + l];
+#pragma unroll 1
+  for (int r = 0; r < 9; ++r) {
+    const float* nf = fr + (r < 8 ? r + 1 : r) * 12 * 64;
+#pragma unroll
+    for (int s = 0; s < 12; ++s) bn[s] = nf[s * 64 + l];
+    const float* row = in + base + (r / 3) * 100 + (r % 3) * 10;
+#pragma unroll
+    for (int dx = 0; dx < 3; ++dx)
+#pragma unroll
+      for (int cg = 0; cg < 4; ++cg)
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          acc[t] = mfma32(row[4 * cg * TR_CS + 20 * t + dx], bq[dx * 4 + cg], acc[t]);
+#pragma unroll
+    for (int s = 0; s < 12; ++s) bq[s] = bn[s];
+  }
+}
+
+// Sum over the 16 lanes-groups of a channel (lane l % 16) within the wavefront.
+__device__ __forceinline__ float channel_sum(const float4_t (&v)[4]) {
+  float s = 0.f;
+#pragma unroll
+  for (int t = 0; t < 4; ++t) s += (v[t][0] + v[t][1]) + (v[t][2] + v[t][3]);
+  s += __shfl_xor(s, 16, 64);
+  s += __shfl_xor(s, 32, 64);
+  return s;
+}
+
+__device__ __forceinline__ float wave_sum32(float v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  return v;
+}
 
 // Forward (and, unless EVAL, backward) of one (sample, block) item.
 template <bool EVAL>
-__global__ __launch_bounds__(WG_THREADS) void k_cnn_train_item(
+__global__ __launch_bounds__(TR_T) void k_cnn_train_item(
     int nitems, const int* __restrict__ items, const SampleRef* __restrict__ samples,
-    const int* __restrict__ nbr, const float* __restrict__ wg, float* __restrict__ scratch,
+    const int* __restrict__ nbr, const float* __restrict__ wg, const float* __restrict__ fr,
     float* __restrict__ gbuf, float* __restrict__ lossbuf, float inv_ntot, float lam) {
-  __shared__ float W[CNN_NW];
-  __shared__ float OP[PADC];   // target halo, then the prediction inside it
-  __shared__ float RHO[BLEN];  // local residual
+  __shared__ __attribute__((aligned(16))) float S[TR_LDS];
   const int it = blockIdx.x;
   if (it >= nitems) return;
-  const int tid = threadIdx.x;
-  const int k = items[2 * it], b = items[2 * it + 1];
-  const SampleRef S = samples[k];
-  float* __restrict__ sc = scratch + (size_t)it * TS_SIZE;
-  float* X = sc + TS_X;
-  float* Z1 = sc + TS_Z1;
-  float* H1 = sc + TS_H1;
-  float* Z2 = sc + TS_Z2;
-  float* H2 = sc + TS_H2;
-  float* D = sc + TS_D;
-  float* DZ2 = sc + TS_DZ2;
-  float* DZ1 = sc + TS_DZ1;
-  for (int j = tid; j < CNN_NW; j += WG_THREADS) W[j] = wg[j];
-  const float inv_sr = 1.0f / S.s_r, inv_sp = 1.0f / S.s_p;
-  for (int p = tid; p < PADC; p += WG_THREADS) {
-    const int pz = p / 100, py = (p / 10) % 10, px = p % 10;
-    X[p] = halo_value(S.res_h, nbr, b, pz, py, px) * inv_sr;
-    X[PADC + p] = halo_value(S.prev, nbr, b, pz, py, px) * inv_sp;
-    OP[p] = halo_value(S.target, nbr, b, pz, py, px);
-    const bool ring = pz == 0 || pz == 9 || py == 0 || py == 9 || px == 0 || px == 9;
-    if (ring)
-      for (int c = 0; c < CNN_C; ++c) {
-        H1[c * PADC + p] = 0.f;
-        H2[c * PADC + p] = 0.f;
+  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
+  const int li = l & 15, k = l >> 4;  // MFMA row or column, and k of the A and B operands
+  const int b = items[2 * it + 1];
+  const SampleRef smp = samples[items[2 * it]];
+  float *X = S + TR_X, *H1 = S + TR_H1, *H2 = S + TR_H2, *P = S + TR_P, *D = S + TR_D,
+        *OP = S + TR_OP, *RHO = S + TR_RHO, *RED = S + TR_RED;
+  const float4_t zero4 = {0.f, 0.f, 0.f, 0.f};
+  // the input patches and the target with its halo; zero rings
+  {
+    const float inv_sr = 1.0f / smp.s_r, inv_sp = 1.0f / smp.s_p;
+    float v[2][3];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int p = tid + j * TR_T;
+      const size_t gi =
+          p < PADC ? halo_index(nbr, b, p / 100, (p / 10) % 10, p % 10) : (size_t)b * BLEN;
+      v[j][0] = smp.res_h[gi];
+      v[j][1] = smp.prev[gi];
+      v[j][2] = smp.target[gi];
+    }
+    for (int i = tid; i < CNN_C * TR_CS / 4; i += TR_T) reinterpret_cast<float4_t*>(H1)[i] = zero4;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int p = tid + j * TR_T;
+      if (p < PADC) {
+        X[p] = v[j][0] * inv_sr;
+        X[PADC + p] = v[j][1] * inv_sp;
+        OP[p] = v[j][2];
+        D[p] = 0.f;
       }
+    }
   }
   __syncthreads();
+  const int cell0 = w * 100 + (li >> 3) * 10 + (li & 7);  // tile 0, padded origin
+  // the accumulator rows of this lane: cells 4 k + q of a tile (q consecutive in x)
+  const int out0 = (w + 1) * 100 + ((k >> 1) + 1) * 10 + 4 * (k & 1) + 1;  // padded, tile 0
+  const int m0 = 64 * w + 4 * k;                                           // unpadded, tile 0
+  float4_t z1[4], c1[4], z2[4], c2[4];  // pre-activations and their normal CDF
   // layer 1 (valid)
-  for (int m = tid; m < BLEN; m += WG_THREADS) {
-    const int z = m >> 6, y = (m >> 3) & 7, x = m & 7;
-    for (int o = 0; o < CNN_C; ++o) {
-      float a = W[CNN_OB1 + o];
-      for (int c = 0; c < 2; ++c)
-        for (int off = 0; off < 27; ++off) {
-          const int dz = off / 9, dy = (off / 3) % 3, dx = off % 3;
-          a += W[(o * 2 + c) * 27 + off] * X[c * PADC + ((z + dz) * 10 + y + dy) * 10 + x + dx];
-        }
-      Z1[o * BLEN + m] = a;
-      H1[o * PADC + padded(m)] = gelu(a);
+  {
+    const float bias = wg[CNN_OB1 + li];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) z1[t] = (float4_t){bias, bias, bias, bias};
+    const float* x = X + (k & 1) * PADC + cell0;
+#pragma unroll
+    for (int s = 0; s < 14; ++s) {
+      const float bf = fr[(FR_F1 + s) * 64 + l];
+      const int o = k >> 1 ? (2 * s + 1 < 27 ? tap(2 * s + 1) : 0) : tap(2 * s);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) z1[t] = mfma32(x[o + 20 * t], bf, z1[t]);
     }
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        c1[t][q] = 0.5f * (1.0f + erff(z1[t][q] * 0.70710678118654752f));
+        H1[li * TR_CS + out0 + 20 * t + q] = z1[t][q] * c1[t][q];
+      }
   }
   __syncthreads();
   // layer 2 (same)
-  for (int m = tid; m < BLEN; m += WG_THREADS) {
-    const int z = m >> 6, y = (m >> 3) & 7, x = m & 7;
-    for (int o = 0; o < CNN_C; ++o) {
-      float a = W[CNN_OB2 + o];
-      for (int c = 0; c < CNN_C; ++c)
-        for (int off = 0; off < 27; ++off) {
-          const int dz = off / 9, dy = (off / 3) % 3, dx = off % 3;
-          a += W[CNN_OW2 + (o * CNN_C + c) * 27 + off] *
-               H1[c * PADC + ((z + dz) * 10 + y + dy) * 10 + x + dx];
-        }
-      Z2[o * BLEN + m] = a;
-      H2[o * PADC + padded(m)] = gelu(a);
+  {
+    const float bias = wg[CNN_OB2 + li];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) z2[t] = (float4_t){bias, bias, bias, bias};
+    conv16(H1, fr + FR_F2 * 64, k * TR_CS + cell0, l, z2);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      float4_t h;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        c2[t][q] = 0.5f * (1.0f + erff(z2[t][q] * 0.70710678118654752f));
+        h[q] = z2[t][q] * c2[t][q];
+      }
+      *reinterpret_cast<float4_t*>(&H2[li * TR_HS + m0 + 16 * t]) = h;
     }
   }
   __syncthreads();
-  // layer 3 (same) and the loss gradient
-  __shared__ float lred[WG_THREADS];
-  float lsum = 0.f;
-  const float* T = S.target + (size_t)b * BLEN;
-  for (int m = tid; m < BLEN; m += WG_THREADS) {
-    const int z = m >> 6, y = (m >> 3) & 7, x = m & 7;
-    float a = W[CNN_OB3];
-    for (int c = 0; c < CNN_C; ++c)
-      for (int off = 0; off < 27; ++off) {
-        const int dz = off / 9, dy = (off / 3) % 3, dx = off % 3;
-        a += W[CNN_OW3 + c * 27 + off] * H2[c * PADC + ((z + dz) * 10 + y + dy) * 10 + x + dx];
-      }
-    const float d = a - T[m];
-    lsum += d * d;
-    D[m] = d * inv_ntot;
-    OP[padded(m)] = a;
+  // layer 3 (same): tap products, 16 taps at a time, then the shifted sum
+  const int z = tid >> 6, y = (tid >> 3) & 7, x = tid & 7, pm = padded(tid);
+  float out = wg[CNN_OB3];
+#pragma unroll 1
+  for (int n2 = 0; n2 < 2; ++n2) {
+    float4_t acc[4] = {zero4, zero4, zero4, zero4};
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const float bf = fr[(FR_F3 + n2 * 4 + s) * 64 + l];
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        acc[t] = mfma32(H2[(4 * s + k) * TR_HS + 64 * w + 16 * t + li], bf, acc[t]);
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      *reinterpret_cast<float4_t*>(&P[li * TR_HS + m0 + 16 * t]) = acc[t];
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < 16; ++n) {
+      const int off = 16 * n2 + n;
+      if (off >= 27) break;
+      const int zz = z + off / 9 - 1, yy = y + (off / 3) % 3 - 1, xx = x + off % 3 - 1;
+      if ((unsigned)zz < 8u && (unsigned)yy < 8u && (unsigned)xx < 8u)
+        out += P[n * TR_HS + (zz * 8 + yy) * 8 + xx];
+    }
+    __syncthreads();
   }
+  // the loss and its gradient
+  const float d = out - OP[pm];
+  float lsum = d * d;
+  float dout = d * inv_ntot;
+  OP[pm] = out;
   __syncthreads();
   if (lam != 0.f) {
     // rho = lap7(out) - q, the stencil closed by the target halo outside
     // the block; its gradient adds lam * (in-block L^T rho) / N to dL/dout
-    for (int m = tid; m < BLEN; m += WG_THREADS) {
-      const int P = padded(m);
-      const float r = ((OP[P - 1] + OP[P + 1]) + (OP[P - 10] + OP[P + 10]) +
-                       (OP[P - 100] + OP[P + 100])) - 6.f * OP[P] - X[P];
-      RHO[m] = r;
-      lsum += lam * r * r;
-    }
+    const float r = ((OP[pm - 1] + OP[pm + 1]) + (OP[pm - 10] + OP[pm + 10]) +
+                     (OP[pm - 100] + OP[pm + 100])) - 6.f * OP[pm] - X[pm];
+    RHO[tid] = r;
+    lsum += lam * r * r;
     __syncthreads();
-    for (int m = tid; m < BLEN; m += WG_THREADS) {
-      const int z = m >> 6, y = (m >> 3) & 7, x = m & 7;
-      float gsum = -6.f * RHO[m];
-      if (x > 0) gsum += RHO[m - 1];
-      if (x < 7) gsum += RHO[m + 1];
-      if (y > 0) gsum += RHO[m - 8];
-      if (y < 7) gsum += RHO[m + 8];
-      if (z > 0) gsum += RHO[m - 64];
-      if (z < 7) gsum += RHO[m + 64];
-      D[m] += lam * gsum * inv_ntot;
+    float gsum = -6.f * r;
+    if (x > 0) gsum += RHO[tid - 1];
+    if (x < 7) gsum += RHO[tid + 1];
+    if (y > 0) gsum += RHO[tid - 8];
+    if (y < 7) gsum += RHO[tid + 8];
+    if (z > 0) gsum += RHO[tid - 64];
+    if (z < 7) gsum += RHO[tid + 64];
+    dout += lam * gsum * inv_ntot;
+  }
+  D[pm] = dout;
+  {
+    const float ls = wave_sum32(lsum), ds = wave_sum32(dout);
+    if (l == 0) {
+      RED[w] = ls;
+      RED[16 + w] = ds;
     }
   }
-  lred[tid] = lsum;
-  __syncthreads();  // lred and D complete before the sum and the backward pass
-  if (tid == 0) {
+  __syncthreads();  // D and RED complete
+  float* G = gbuf + (size_t)it * CNN_NW;
+  if (tid < 2 && !(EVAL && tid == 1)) {
     float s = 0.f;
-    for (int i = 0; i < WG_THREADS; ++i) s += lred[i];
-    lossbuf[it] = s;
+    for (int i = 0; i < 8; ++i) s += RED[16 * tid + i];
+    if (tid == 0) lossbuf[it] = s;
+    else G[CNN_OB3] = s;
   }
   if (EVAL) return;
-  float* G = gbuf + (size_t)it * CNN_NW;
-  // dW3, db3
-  for (int j = tid; j < CNN_NW3; j += WG_THREADS) {
-    const int c = j / 27, off = j % 27, dz = off / 9, dy = (off / 3) % 3, dx = off % 3;
-    float a = 0.f;
-    for (int m = 0; m < BLEN; ++m) {
-      const int z = m >> 6, y = (m >> 3) & 7, x = m & 7;
-      a += H2[c * PADC + ((z + dz) * 10 + y + dy) * 10 + x + dx] * D[m];
+  // dW3: taps n of tile w % 2 over the cells of z planes 2 (w / 2), + 1
+  float4_t a3 = zero4;
+  {
+    const int off = 16 * (w & 1) + li;
+    const float* dp = D + (off < 27 ? tap(26 - off) : 0) + k;
+    const float* hp = H2 + li * TR_HS + k;
+#pragma unroll 4
+    for (int s = 0; s < 32; ++s) {  // four cells of a row
+      const int row = 16 * (w >> 1) + (s >> 1), xh = 4 * (s & 1);
+      a3 = mfma32(hp[row * 8 + xh], dp[(row >> 3) * 100 + (row & 7) * 10 + xh], a3);
     }
-    G[CNN_OW3 + j] = a;
-  }
-  if (tid == 0) {
-    float a = 0.f;
-    for (int m = 0; m < BLEN; ++m) a += D[m];
-    G[CNN_OB3] = a;
+    *reinterpret_cast<float4_t*>(&P[w * 256 + 4 * l]) = a3;
   }
   // dZ2 = (W3^T * D) . gelu'(Z2)
-  for (int i = tid; i < CNN_C * BLEN; i += WG_THREADS) {
-    const int c = i / BLEN, m = i % BLEN, z = m >> 6, y = (m >> 3) & 7, x = m & 7;
-    float a = 0.f;
-    for (int off = 0; off < 27; ++off) {
-      const int dz = off / 9, dy = (off / 3) % 3, dx = off % 3;
-      const int zz = z + 1 - dz, yy = y + 1 - dy, xx = x + 1 - dx;
-      if (zz >= 0 && zz < 8 && yy >= 0 && yy < 8 && xx >= 0 && xx < 8)
-        a += W[CNN_OW3 + c * 27 + off] * D[(zz * 8 + yy) * 8 + xx];
+  float4_t g2[4] = {zero4, zero4, zero4, zero4};
+#pragma unroll
+  for (int s = 0; s < 7; ++s) {
+    const int off = 4 * s + k;
+    const float bf = fr[(FR_T3 + s) * 64 + l];
+    const float* dp = D + cell0 + (off < 27 ? tap(off) : 0);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) g2[t] = mfma32(dp[20 * t], bf, g2[t]);
+  }
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float v = z2[t][q];
+      g2[t][q] *= c2[t][q] + v * expf(-0.5f * v * v) * 0.3989422804014327f;
     }
-    DZ2[i] = a * gelu_grad(Z2[i]);
+  const float s2 = channel_sum(g2);
+  __syncthreads();  // the dW3 partials; H2 and RED read by all
+  {
+    // partial sums of dW3 in the order of the z planes
+    const int n2 = tid >> 8, e = tid & 255, c = 4 * (e >> 6) + (e & 3), off = 16 * n2 + ((e >> 2) & 15);
+    const float v = ((P[n2 * 256 + e] + P[(n2 + 2) * 256 + e]) + P[(n2 + 4) * 256 + e]) +
+                    P[(n2 + 6) * 256 + e];
+    if (off < 27) G[CNN_OW3 + c * 27 + off] = v;
+    if (l < 16) RED[w * 16 + l] = s2;
+  }
+  __syncthreads();  // P and H2 free
+  float* Z = H2;  // dZ2 on the padded patch
+  for (int i = tid; i < CNN_C * TR_CS / 4; i += TR_T) reinterpret_cast<float4_t*>(Z)[i] = zero4;
+  if (tid < CNN_C) {
+    float s = 0.f;
+    for (int i = 0; i < 8; ++i) s += RED[i * 16 + tid];
+    G[CNN_OB2 + tid] = s;
   }
   __syncthreads();
-  // dW2, db2
-  for (int j = tid; j < CNN_NW2; j += WG_THREADS) {
-    const int o = j / (CNN_C * 27), c = (j / 27) % CNN_C, off = j % 27;
-    const int dz = off / 9, dy = (off / 3) % 3, dx = off % 3;
-    float a = 0.f;
-    for (int m = 0; m < BLEN; ++m) {
-      const int z = m >> 6, y = (m >> 3) & 7, x = m & 7;
-      a += H1[c * PADC + ((z + dz) * 10 + y + dy) * 10 + x + dx] * DZ2[o * BLEN + m];
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) Z[li * TR_CS + out0 + 20 * t + q] = g2[t][q];
+  __syncthreads();
+  // dW2: taps w, w + 8, w + 16 (and 24 + w for w < 3), all cells
+  {
+    float4_t acc[4] = {zero4, zero4, zero4, zero4};
+    const float* zp = Z + li * TR_CS + 111 + k;
+    const float* hp = H1 + li * TR_CS + k;
+    const int o0 = tap(w), o1 = tap(w + 8), o2 = tap(w + 16), o3 = tap(w < 3 ? w + 24 : w);
+#pragma unroll 2
+    for (int row = 0; row < 64; ++row) {
+      const int r = (row >> 3) * 100 + (row & 7) * 10;
+#pragma unroll
+      for (int xh = 0; xh < 8; xh += 4) {
+        const float a = zp[r + xh];
+        acc[0] = mfma32(a, hp[r + xh + o0], acc[0]);
+        acc[1] = mfma32(a, hp[r + xh + o1], acc[1]);
+        acc[2] = mfma32(a, hp[r + xh + o2], acc[2]);
+        if (w < 3) acc[3] = mfma32(a, hp[r + xh + o3], acc[3]);
+      }
     }
-    G[CNN_OW2 + j] = a;
-  }
-  for (int o = tid; o < CNN_C; o += WG_THREADS) {
-    float a = 0.f;
-    for (int m = 0; m < BLEN; ++m) a += DZ2[o * BLEN + m];
-    G[CNN_OB2 + o] = a;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (j < 3 || w < 3)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          G[CNN_OW2 + (w + 8 * j) * 256 + (4 * k + q) * 16 + li] = acc[j][q];
   }
   // dZ1 = (W2^T * dZ2) . gelu'(Z1)
-  for (int i = tid; i < CNN_C * BLEN; i += WG_THREADS) {
-    const int c = i / BLEN, m = i % BLEN, z = m >> 6, y = (m >> 3) & 7, x = m & 7;
-    float a = 0.f;
-    for (int o = 0; o < CNN_C; ++o)
-      for (int off = 0; off < 27; ++off) {
-        const int dz = off / 9, dy = (off / 3) % 3, dx = off % 3;
-        const int zz = z + 1 - dz, yy = y + 1 - dy, xx = x + 1 - dx;
-        if (zz >= 0 && zz < 8 && yy >= 0 && yy < 8 && xx >= 0 && xx < 8)
-          a += W[CNN_OW2 + (o * CNN_C + c) * 27 + off] * DZ2[o * BLEN + (zz * 8 + yy) * 8 + xx];
-      }
-    DZ1[i] = a * gelu_grad(Z1[i]);
+  float4_t g1[4] = {zero4, zero4, zero4, zero4};
+  conv16(Z, fr + FR_T2 * 64, k * TR_CS + cell0, l, g1);
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float v = z1[t][q];
+      g1[t][q] *= c1[t][q] + v * expf(-0.5f * v * v) * 0.3989422804014327f;
+    }
+  const float s1 = channel_sum(g1);
+  __syncthreads();  // H1, Z and RED read by all
+#pragma unroll
+  for (int t = 0; t < 4; ++t) *reinterpret_cast<float4_t*>(&H1[li * TR_HS + m0 + 16 * t]) = g1[t];
+  if (l < 16) RED[w * 16 + l] = s1;
+  __syncthreads();
+  if (tid < CNN_C) {
+    float s = 0.f;
+    for (int i = 0; i < 8; ++i) s += RED[i * 16 + tid];
+    G[CNN_OB1 + tid] = s;
+  }
+  // dW1: (channel, tap) pairs n of tile w % 4 over z planes 4 (w / 4) .. + 3
+  {
+    const int pr = 16 * (w & 3) + li;
+    const float* xp = X + (pr < 54 ? (pr / 27) * PADC + tap(pr % 27) : 0) + k;
+    const float* hp = H1 + li * TR_HS + k;
+    float4_t acc = zero4;
+#pragma unroll 4
+    for (int s = 0; s < 64; ++s) {
+      const int row = 32 * (w >> 2) + (s >> 1), xh = 4 * (s & 1);
+      acc = mfma32(hp[row * 8 + xh], xp[(row >> 3) * 100 + (row & 7) * 10 + xh], acc);
+    }
+    *reinterpret_cast<float4_t*>(&Z[w * 256 + 4 * l]) = acc;
   }
   __syncthreads();
-  // dW1, db1
-  for (int j = tid; j < CNN_NW1; j += WG_THREADS) {
-    const int o = j / 54, c = (j / 27) % 2, off = j % 27;
-    const int dz = off / 9, dy = (off / 3) % 3, dx = off % 3;
-    float a = 0.f;
-    for (int m = 0; m < BLEN; ++m) {
-      const int z = m >> 6, y = (m >> 3) & 7, x = m & 7;
-      a += X[c * PADC + ((z + dz) * 10 + y + dy) * 10 + x + dx] * DZ1[o * BLEN + m];
-    }
-    G[j] = a;
-  }
-  for (int o = tid; o < CNN_C; o += WG_THREADS) {
-    float a = 0.f;
-    for (int m = 0; m < BLEN; ++m) a += DZ1[o * BLEN + m];
-    G[CNN_OB1 + o] = a;
+  for (int i = tid; i < 1024; i += TR_T) {
+    const int n4 = i >> 8, e = i & 255, o = 4 * (e >> 6) + (e & 3), pr = 16 * n4 + ((e >> 2) & 15);
+    if (pr < 54) G[o * 54 + pr] = Z[n4 * 256 + e] + Z[(n4 + 4) * 256 + e];
   }
 }
 
-// Sum the per-item gradients in item order and take one Adam step
-// (Kingma & Ba 2015; beta1 = 0.9, beta2 = 0.999, eps = 1e-8).
-__global__ void k_cnn_adam(int nitems, const float* __restrict__ gbuf, float* __restrict__ w,
-                           float* __restrict__ mv, float lr, float bc1, float bc2) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= CNN_NW) return;
+// Sum the per-item gradients and take one Adam step (Kingma & Ba 2015; beta1 =
+// 0.9, beta2 = 0.999, eps = 1e-8). 64 weights a workgroup, the items split in
+// AD_G contiguous groups that are added in order: the sum reads nitems x 33 KB
+// once, with enough loads in flight (256 items: 4.8 us against 64 us for one
+// thread per weight over all items).
+constexpr int AD_G = 16;
+__global__ __launch_bounds__(64 * AD_G) void k_cnn_adam(int nitems, const float* __restrict__ gbuf,
+                                                        float* __restrict__ w,
+                                                        float* __restrict__ fr,
+                                                        float* __restrict__ mv, float lr,
+                                                        float bc1, float bc2) {
+  __shared__ float part[AD_G][64];
+  const int e = blockIdx.x * 64 + (threadIdx.x & 63), grp = threadIdx.x >> 6;
+  const int per = (nitems + AD_G - 1) / AD_G;
+  const int i0 = grp * per, i1 = min(nitems, i0 + per);
+  float s = 0.f;
+  if (e < CNN_NW) {
+#pragma unroll 8
+    for (int i = i0; i < i1; ++i) s += gbuf[(size_t)i * CNN_NW + e];
+  }
+  part[grp][threadIdx.x & 63] = s;
+  __syncthreads();
+  if (grp != 0 || e >= CNN_NW) return;
   float g = 0.f;
-  for (int i = 0; i < nitems; ++i) g += gbuf[(size_t)i * CNN_NW + j];
+#pragma unroll
+  for (int i = 0; i < AD_G; ++i) g += part[i][threadIdx.x];
+  const int j = weight_index(e);
   float m = mv[j], v = mv[CNN_NW + j];
   m = 0.9f * m + 0.1f * g;
   v = 0.999f * v + 0.001f * g * g;
   mv[j] = m;
   mv[CNN_NW + j] = v;
-  w[j] -= lr * (m / bc1) / (sqrtf(v / bc2) + 1e-8f);
+  const float wj = w[j] - lr * (m / bc1) / (sqrtf(v / bc2) + 1e-8f);
+  w[j] = wj;
+  frag_store(fr, j, wj);
 }
 
 // Training-set entry: res / h_b, p_prev and (p - p_prev - m) / s_r in FP32,
@@ -549,9 +765,11 @@ int cnn_init(CnnState& C, std::string& err) {
   CCHECK(hipMalloc(&C.d_w, CNN_NW * sizeof(float)));
   CCHECK(hipMalloc(&C.d_adam, 2 * CNN_NW * sizeof(float)));
   CCHECK(hipMalloc(&C.d_wpk, CNN_PK * sizeof(_Float16)));
+  CCHECK(hipMalloc(&C.d_frag, CNN_FRAG * sizeof(float)));
   CCHECK(hipMalloc(&C.d_scal, 8 * sizeof(double)));
   CCHECK(hipMemset(C.d_w, 0, CNN_NW * sizeof(float)));
   CCHECK(hipMemset(C.d_adam, 0, 2 * CNN_NW * sizeof(float)));
+  CCHECK(hipMemset(C.d_frag, 0, CNN_FRAG * sizeof(float)));  // the missing taps stay zero
   return 0;
 }
 
@@ -589,6 +807,8 @@ int cnn_set_weights(CnnState& C, const float* w, int nw, std::string& err) {
   CCHECK(hipMemset(C.d_adam, 0, 2 * CNN_NW * sizeof(float)));
   C.adam_t = 0;
   if (repack(C, nullptr, err)) return -1;
+  k_cnn_frag<<<(CNN_NW + 255) / 256, 256>>>(C.d_w, C.d_frag);
+  CCHECK(hipGetLastError());
   CCHECK(hipDeviceSynchronize());
   C.have_weights = true;
   return 0;
@@ -661,31 +881,40 @@ void cnn_clear_samples(CnnState& C) {
   C.samples.clear();
 }
 
-static int ensure_train_buffers(CnnState& C, int nitems, std::string& err) {
-  const long long need = (long long)nitems * (TS_SIZE + CNN_NW + 1);
+// Gradients and losses of nitems items (losses twice: a call's first and its
+// latest step), and nlist entries of the item list; the buffers grow only.
+static int ensure_train_buffers(CnnState& C, int nitems, int nlist, std::string& err) {
+  const long long need = (long long)nitems * (CNN_NW + 2);
   if (need > C.scratch_cap) {
     if (C.d_scratch) (void)hipFree(C.d_scratch);
     C.d_scratch = nullptr;
+    C.scratch_cap = 0;
     CCHECK(hipMalloc(&C.d_scratch, need * sizeof(float)));
     C.scratch_cap = need;
   }
-  if (nitems > C.items_cap) {
+  if (nlist > C.items_cap) {
     if (C.d_items) (void)hipFree(C.d_items);
     C.d_items = nullptr;
-    CCHECK(hipMalloc(&C.d_items, 2 * nitems * sizeof(int)));
-    C.items_cap = nitems;
+    C.items_cap = 0;
+    CCHECK(hipMalloc(&C.d_items, 2 * (size_t)nlist * sizeof(int)));
+    C.items_cap = nlist;
   }
   return 0;
 }
 
-static int upload_samples(CnnState& C, std::vector<SampleRef>& refs, SampleRef** d_refs,
-                          std::string& err) {
-  refs.resize(C.samples.size());
+static int upload_samples(CnnState& C, std::string& err) {
+  std::vector<SampleRef> refs(C.samples.size());
   for (size_t k = 0; k < C.samples.size(); ++k)
     refs[k] = {C.samples[k].res_h, C.samples[k].prev, C.samples[k].target, C.samples[k].s_r,
                C.samples[k].s_p};
-  CCHECK(hipMalloc(d_refs, refs.size() * sizeof(SampleRef)));
-  CCHECK(hipMemcpy(*d_refs, refs.data(), refs.size() * sizeof(SampleRef), hipMemcpyHostToDevice));
+  if (refs.size() > C.refs_cap) {
+    if (C.d_refs) (void)hipFree(C.d_refs);
+    C.d_refs = nullptr;
+    C.refs_cap = 0;
+    CCHECK(hipMalloc(&C.d_refs, refs.size() * sizeof(SampleRef)));
+    C.refs_cap = refs.size();
+  }
+  CCHECK(hipMemcpy(C.d_refs, refs.data(), refs.size() * sizeof(SampleRef), hipMemcpyHostToDevice));
   return 0;
 }
 
@@ -717,46 +946,51 @@ int cnn_train(CnnState& C, hipStream_t s, int steps, int batch, float lr, float 
     for (int i = CNN_OW3; i < CNN_OW3 + CNN_NW3; ++i) w[i] *= 0.1f;  // start near p_prev
     if (cnn_set_weights(C, w.data(), CNN_NW, err)) return -1;
   }
-  if (ensure_train_buffers(C, batch, err)) return -1;
-  std::vector<SampleRef> refs;
-  SampleRef* d_refs = nullptr;
-  if (upload_samples(C, refs, &d_refs, err)) return -1;
-  float* scratch = C.d_scratch;
-  float* gbuf = scratch + (size_t)batch * TS_SIZE;
-  float* lbuf = gbuf + (size_t)batch * CNN_NW;
-  std::vector<int> items(2 * batch);
-  std::vector<float> lh(batch);
+  // the items of up to TRAIN_LIST / batch steps are drawn and uploaded at a time
+  constexpr int TRAIN_LIST = 1 << 14;
+  const int chunk = std::min(steps, std::max(1, TRAIN_LIST / batch));
+  if (ensure_train_buffers(C, batch, chunk * batch, err)) return -1;
+  if (upload_samples(C, err)) return -1;
+  const SampleRef* refs = static_cast<const SampleRef*>(C.d_refs);
+  float* gbuf = C.d_scratch;
+  float* lbuf = gbuf + (size_t)batch * CNN_NW;  // [0, batch): first step, then the others
+  std::vector<int> items(2 * (size_t)chunk * batch);
   std::mt19937_64 R(seed);
   const int ns = (int)C.samples.size();
   const float inv_ntot = 1.0f / (float)((double)batch * BLEN);
   for (int step = 0; step < steps; ++step) {
-    for (int i = 0; i < batch; ++i) {
-      items[2 * i] = (int)(R() % (uint64_t)ns);
-      items[2 * i + 1] = (int)(R() % (uint64_t)C.nb);
+    if (step % chunk == 0) {
+      if (step > 0) CCHECK(hipStreamSynchronize(s));  // the list's last upload is done
+      const int m = std::min(chunk, steps - step) * batch;
+      for (int i = 0; i < m; ++i) {
+        items[2 * i] = (int)(R() % (uint64_t)ns);
+        items[2 * i + 1] = (int)(R() % (uint64_t)C.nb);
+      }
+      CCHECK(hipMemcpyAsync(C.d_items, items.data(), 2 * (size_t)m * sizeof(int),
+                            hipMemcpyHostToDevice, s));
     }
-    CCHECK(hipMemcpyAsync(C.d_items, items.data(), items.size() * sizeof(int),
-                          hipMemcpyHostToDevice, s));
-    k_cnn_train_item<false><<<batch, WG_THREADS, 0, s>>>(batch, C.d_items, d_refs, C.d_nbr, C.d_w,
-                                                         scratch, gbuf, lbuf, inv_ntot,
-                                                         C.res_weight);
+    k_cnn_train_item<false><<<batch, TR_T, 0, s>>>(
+        batch, C.d_items + 2 * (size_t)(step % chunk) * batch, refs, C.d_nbr, C.d_w, C.d_frag,
+        gbuf, lbuf + (step > 0 ? batch : 0), inv_ntot, C.res_weight);
     C.adam_t += 1;
     const float bc1 = 1.0f - std::pow(0.9f, (float)C.adam_t);
     const float bc2 = 1.0f - std::pow(0.999f, (float)C.adam_t);
-    k_cnn_adam<<<(CNN_NW + 255) / 256, 256, 0, s>>>(batch, gbuf, C.d_w, C.d_adam, lr, bc1, bc2);
-    if (step == 0 || step == steps - 1) {
-      CCHECK(hipMemcpyAsync(lh.data(), lbuf, batch * sizeof(float), hipMemcpyDeviceToHost, s));
-      CCHECK(hipStreamSynchronize(s));
-      double L = 0;
-      for (float v : lh) L += v;
-      L *= 0.5 / ((double)batch * BLEN);
-      if (loss) loss[step == 0 ? 0 : 1] = L;
-      if (loss && steps == 1) loss[1] = L;
-    }
+    k_cnn_adam<<<(CNN_NW + 63) / 64, 64 * AD_G, 0, s>>>(batch, gbuf, C.d_w, C.d_frag, C.d_adam, lr,
+                                                        bc1, bc2);
   }
   CCHECK(hipGetLastError());
   if (repack(C, s, err)) return -1;
+  std::vector<float> lh(2 * (size_t)batch);
+  CCHECK(hipMemcpyAsync(lh.data(), lbuf, lh.size() * sizeof(float), hipMemcpyDeviceToHost, s));
   CCHECK(hipStreamSynchronize(s));
-  (void)hipFree(d_refs);
+  if (loss) {
+    for (int k = 0; k < 2; ++k) {
+      const float* f = lh.data() + (k && steps > 1 ? batch : 0);
+      double L = 0;
+      for (int i = 0; i < batch; ++i) L += f[i];
+      loss[k] = L * (0.5 / ((double)batch * BLEN));
+    }
+  }
   return 0;
 }
 
@@ -766,12 +1000,10 @@ int cnn_eval(CnnState& C, hipStream_t s, int k, double* loss, std::string& err) 
     return -1;
   }
   const int chunk = std::min(C.nb, 2048);
-  if (ensure_train_buffers(C, chunk, err)) return -1;
-  std::vector<SampleRef> refs;
-  SampleRef* d_refs = nullptr;
-  if (upload_samples(C, refs, &d_refs, err)) return -1;
-  float* scratch = C.d_scratch;
-  float* gbuf = scratch + (size_t)chunk * TS_SIZE;
+  if (ensure_train_buffers(C, chunk, chunk, err)) return -1;
+  if (upload_samples(C, err)) return -1;
+  const SampleRef* refs = static_cast<const SampleRef*>(C.d_refs);
+  float* gbuf = C.d_scratch;
   float* lbuf = gbuf + (size_t)chunk * CNN_NW;
   std::vector<int> items(2 * chunk);
   std::vector<float> lh(chunk);
@@ -783,13 +1015,13 @@ int cnn_eval(CnnState& C, hipStream_t s, int k, double* loss, std::string& err) 
       items[2 * i + 1] = b0 + i;
     }
     CCHECK(hipMemcpyAsync(C.d_items, items.data(), 2 * m * sizeof(int), hipMemcpyHostToDevice, s));
-    k_cnn_train_item<true><<<m, WG_THREADS, 0, s>>>(m, C.d_items, d_refs, C.d_nbr, C.d_w,
-                                                    scratch, gbuf, lbuf, 0.f, C.res_weight);
+    k_cnn_train_item<true><<<m, TR_T, 0, s>>>(m, C.d_items, refs, C.d_nbr, C.d_w, C.d_frag, gbuf,
+                                              lbuf, 0.f, C.res_weight);
+    CCHECK(hipGetLastError());
     CCHECK(hipMemcpyAsync(lh.data(), lbuf, m * sizeof(float), hipMemcpyDeviceToHost, s));
     CCHECK(hipStreamSynchronize(s));
     for (int i = 0; i < m; ++i) L += lh[i];
   }
-  (void)hipFree(d_refs);
   *loss = 0.5 * L / ((double)C.nb * BLEN);
   return 0;
 }
@@ -798,7 +1030,7 @@ __global__ void k_cnn_sum_grads(int nitems, const float* __restrict__ gbuf, floa
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= CNN_NW) return;
   float a = 0.f;
-  for (int i = 0; i < nitems; ++i) a += gbuf[(size_t)i * CNN_NW + j];
+  for (int i = 0; i < nitems; ++i) a += gbuf[(size_t)i * CNN_NW + grad_index(j)];
   g[j] = a;
 }
 
@@ -817,32 +1049,30 @@ int cnn_gradient(CnnState& C, hipStream_t s, int k, float res_weight, float* gra
     return -1;
   }
   const int m = C.nb;
-  if (ensure_train_buffers(C, m + 1, err)) return -1;
-  std::vector<SampleRef> refs;
-  SampleRef* d_refs = nullptr;
-  if (upload_samples(C, refs, &d_refs, err)) return -1;
-  float* scratch = C.d_scratch;
-  float* gbuf = scratch + (size_t)(m + 1) * TS_SIZE;
-  float* lbuf = gbuf + (size_t)(m + 1) * CNN_NW;
+  if (ensure_train_buffers(C, m + 1, m, err)) return -1;
+  if (upload_samples(C, err)) return -1;
+  float* gbuf = C.d_scratch;
   float* gsum = gbuf + (size_t)m * CNN_NW;
+  float* lbuf = gsum + CNN_NW;
   std::vector<int> items(2 * m);
   for (int i = 0; i < m; ++i) {
     items[2 * i] = k;
     items[2 * i + 1] = i;
   }
   CCHECK(hipMemcpyAsync(C.d_items, items.data(), 2 * m * sizeof(int), hipMemcpyHostToDevice, s));
-  k_cnn_train_item<false><<<m, WG_THREADS, 0, s>>>(m, C.d_items, d_refs, C.d_nbr, C.d_w, scratch,
-                                                   gbuf, lbuf, 1.0f / ((float)m * BLEN),
-                                                   res_weight);
+  k_cnn_train_item<false><<<m, TR_T, 0, s>>>(m, C.d_items,
+                                             static_cast<const SampleRef*>(C.d_refs), C.d_nbr,
+                                             C.d_w, C.d_frag, gbuf, lbuf,
+                                             1.0f / ((float)m * BLEN), res_weight);
   k_cnn_sum_grads<<<(CNN_NW + 255) / 256, 256, 0, s>>>(m, gbuf, gsum);
   std::vector<float> lh(m);
   CCHECK(hipMemcpyAsync(grad, gsum, CNN_NW * sizeof(float), hipMemcpyDeviceToHost, s));
   CCHECK(hipMemcpyAsync(lh.data(), lbuf, m * sizeof(float), hipMemcpyDeviceToHost, s));
+  CCHECK(hipGetLastError());
   CCHECK(hipStreamSynchronize(s));
   double L = 0;
   for (float v : lh) L += v;
   *loss = 0.5 * L / ((double)m * BLEN);
-  (void)hipFree(d_refs);
   return 0;
 }
 
@@ -856,6 +1086,8 @@ void cnn_free(CnnState& C) {
   if (C.d_pred) (void)hipFree(C.d_pred);
   if (C.d_scratch) (void)hipFree(C.d_scratch);
   if (C.d_items) (void)hipFree(C.d_items);
+  if (C.d_refs) (void)hipFree(C.d_refs);
+  (void)hipFree(C.d_frag);
   C = CnnState();
 }
 

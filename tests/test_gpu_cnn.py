@@ -119,3 +119,27 @@ def test_training_reduces_loss_and_fallback(gpu):
     assert rep["guess_used"] == 2 and rep["guess_resid"] < 0.9 * rep2["err_init"]
     print("guess used", rep["guess_used"], "resid net/prev", rep["guess_resid"] / rep2["err_init"],
           "iters", rep["iterations"], "vs", rep2["iterations"])
+
+
+@pytest.mark.parametrize("batch", [1, 17, 9000])
+def test_training_is_the_same_for_every_batch_of_one_item(gpu, batch):
+    """On a grid of one block with one sample every item of every minibatch is
+    the same one, so the mean gradient and the Adam steps do not depend on the
+    batch size: 1 (empty groups of the gradient sum), 17 (a ragged one) and
+    9000 (one step per uploaded item list) against 16. Adding n equal terms in
+    FP32 is off by at most n / 16 + 16 roundings, 3.5e-5 relative, and an Adam
+    step by about twice that; the bar is 1e-3 of the length of three steps."""
+    blocks = np.zeros((1, 4), np.int32)
+    S = PoissonSolver((1, 1, 1), 0.125, (2, 2, 2), bmean=0).set_topology(blocks)
+    rhs, prev, _ = smooth_fields(blocks, 0.125, 3)
+    S.cnn_add_sample(dev(rhs), dev(prev), dev(1.1 * prev))
+    w0 = C.init_weights(6).astype(np.float32)
+    out = []
+    for n in (16, batch):
+        S.cnn_set_weights(w0)
+        loss = S.cnn_train(3, batch=n, lr=1e-3, seed=4, res_weight=0.5)
+        out.append((S.cnn_get_weights(), loss))
+    moved = np.linalg.norm(out[0][0] - w0)
+    assert moved > 0.5 * 1e-3 * np.sqrt(len(w0))
+    assert np.linalg.norm(out[1][0] - out[0][0]) <= 1e-3 * 3e-3 * np.sqrt(len(w0))
+    assert np.allclose(out[1][1], out[0][1], rtol=1e-4)
