@@ -18,14 +18,16 @@ namespace cup3d {
 constexpr int DST_TABLE = BS * BS + BS;
 void dst_tables(double* tab, float* tab32);  // FP64 table and its FP32 rounding
 
-// mode PREC_P / PREC_S / PREC_PLAIN as launch_precond64; h per block,
-// sigma = 1 / (nu dt).
+// mode PREC_P / PREC_S / PREC_PLAIN; h per block, sigma = 1 / (nu dt); fin and
+// f: whether and from where the kernel takes its scalars' sums.
 void launch_precond_dst(hipStream_t s, int mode, int nb, const double* tab, const double* h,
-                        double sigma, const KrylovVectors<double>& v, SolverState* st);
+                        double sigma, const KrylovVectors<double>& v, SolverState* st,
+                        int fin = FIN_KERNEL, const FinArgs& f = FinArgs());
 // The same in FP32 for the mixed forms' inner solve (sigma = 0: the pressure
 // equation's block inverse h^-1 P_inv).
 void launch_precond_dst32(hipStream_t s, int mode, int nb, const float* tab, const float* h,
-                          const KrylovVectors<float>& v, SolverState* st);
+                          const KrylovVectors<float>& v, SolverState* st,
+                          int fin = FIN_KERNEL, const FinArgs& f = FinArgs());
 // u = vel[:, comp], a = -h^3 sigma vel_old[:, comp] (vel, vel_old: [n][3]).
 void launch_diffusion_gather(hipStream_t s, long long n, int comp, const double* h3, double sigma,
                              const double* vel, const double* vel_old, double* u, double* a);

@@ -117,37 +117,51 @@ __device__ __forceinline__ void dst_apply(const T* __restrict__ tab, T* L, int l
 //           z1 = M^-1 p
 //   PREC_S  s = r - alpha nu (into r); z2 = M^-1 s
 //   PREC_PLAIN  z1 = M^-1 p
-template <typename T, int MODE>
+template <typename T, int MODE, int FIN>
 __global__ __launch_bounds__(WG_THREADS) void k_precond_dst(int nb, const T* __restrict__ tab,
                                                             const T* __restrict__ hb, T sigma,
-                                                            KrylovVectors<T> v,
-                                                            SolverState* st) {
+                                                            KrylovVectors<T> v, SolverState* st,
+                                                            FinArgs f) {
   __shared__ T Ls[WG_THREADS / 64][DL_WAVE];
-  if (MODE != PREC_PLAIN && st->status != ST_RUNNING) return;
+  __shared__ SolverState S;
+  if (!FIN && MODE != PREC_PLAIN && st->status != ST_RUNNING) return;
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int b = blockIdx.x * (WG_THREADS / 64) + w;
-  if (b >= nb) return;  // no workgroup barrier below: only this wavefront's slice
-  const T beta = MODE == PREC_P ? (T)st->beta : (T)0;
-  const T omega = MODE == PREC_P ? (T)st->omega : (T)0;
-  const T alpha = MODE == PREC_S ? (T)st->alpha : (T)0;
-  const int pzero = MODE == PREC_P ? st->p_zero : 0;
-  const int restart = MODE == PREC_P ? st->restart_pending : 0;
   const size_t off = (size_t)b * BLEN + lane;
   T c[BS], ra[BS], rb[BS];
+  if (b < nb) {
 #pragma unroll
-  for (int iz = 0; iz < BS; ++iz) {
-    const size_t i = off + iz * 64;
-    if (MODE == PREC_P) {
-      ra[iz] = v.r[i];
-      rb[iz] = v.nu[i];
-      c[iz] = v.p[i];
-    } else if (MODE == PREC_S) {
-      ra[iz] = v.r[i];
-      rb[iz] = v.nu[i];
-    } else {
-      c[iz] = v.p[i];
+    for (int iz = 0; iz < BS; ++iz) {
+      const size_t i = off + iz * 64;
+      if (MODE == PREC_P) {
+        ra[iz] = v.r[i];
+        rb[iz] = v.nu[i];
+        c[iz] = v.p[i];
+      } else if (MODE == PREC_S) {
+        ra[iz] = v.r[i];
+        rb[iz] = v.nu[i];
+      } else {
+        c[iz] = v.p[i];
+      }
     }
   }
+  const SolverState* sp = st;
+  if constexpr (FIN != FIN_KERNEL) {
+    T yr = 0;
+    consumer_state<MODE == PREC_P ? USE_P : USE_S, FIN, T>(st, f, S, yr);
+    if (S.status != ST_RUNNING) return;
+    sp = &S;
+    if (FIN == FIN_ROW && MODE == PREC_S && b < nb && (long long)off == f.row) {
+      rb[0] = yr;  // the mean-constraint row of nu, which the SpMV left out
+      v.nu[off] = yr;
+    }
+  }
+  if (b >= nb) return;  // no workgroup barrier below: only this wavefront's slice
+  const T beta = MODE == PREC_P ? (T)sp->beta : (T)0;
+  const T omega = MODE == PREC_P ? (T)sp->omega : (T)0;
+  const T alpha = MODE == PREC_S ? (T)sp->alpha : (T)0;
+  const int pzero = MODE == PREC_P ? sp->p_zero : 0;
+  const int restart = MODE == PREC_P ? sp->restart_pending : 0;
 #pragma unroll
   for (int iz = 0; iz < BS; ++iz) {
     const size_t i = off + iz * 64;
@@ -167,15 +181,28 @@ __global__ __launch_bounds__(WG_THREADS) void k_precond_dst(int nb, const T* __r
   for (int iz = 0; iz < BS; ++iz) out[off + iz * 64] = c[iz];
 }
 
+template <typename T, int MODE, int FIN>
+void launch_precond_dst_m(hipStream_t s, int nb, const T* tab, const T* h, T sigma,
+                          const KrylovVectors<T>& v, SolverState* st, const FinArgs& f) {
+  const int nwg = (nb + WG_THREADS / 64 - 1) / (WG_THREADS / 64);
+  k_precond_dst<T, MODE, FIN><<<nwg, WG_THREADS, 0, s>>>(nb, tab, h, sigma, v, st, f);
+}
+
 template <typename T>
 void launch_precond_dst_t(hipStream_t s, int mode, int nb, const T* tab, const T* h, T sigma,
-                          const KrylovVectors<T>& v, SolverState* st) {
-  const int nwg = (nb + WG_THREADS / 64 - 1) / (WG_THREADS / 64);
-  switch (mode) {
-    case PREC_P: k_precond_dst<T, PREC_P><<<nwg, WG_THREADS, 0, s>>>(nb, tab, h, sigma, v, st); break;
-    case PREC_S: k_precond_dst<T, PREC_S><<<nwg, WG_THREADS, 0, s>>>(nb, tab, h, sigma, v, st); break;
-    default: k_precond_dst<T, PREC_PLAIN><<<nwg, WG_THREADS, 0, s>>>(nb, tab, h, sigma, v, st); break;
-  }
+                          const KrylovVectors<T>& v, SolverState* st, int fin, const FinArgs& f) {
+  if (mode == PREC_P && fin)
+    launch_precond_dst_m<T, PREC_P, FIN_SUMS>(s, nb, tab, h, sigma, v, st, f);
+  else if (mode == PREC_P)
+    launch_precond_dst_m<T, PREC_P, FIN_KERNEL>(s, nb, tab, h, sigma, v, st, f);
+  else if (mode == PREC_S && fin == FIN_ROW)
+    launch_precond_dst_m<T, PREC_S, FIN_ROW>(s, nb, tab, h, sigma, v, st, f);
+  else if (mode == PREC_S && fin)
+    launch_precond_dst_m<T, PREC_S, FIN_SUMS>(s, nb, tab, h, sigma, v, st, f);
+  else if (mode == PREC_S)
+    launch_precond_dst_m<T, PREC_S, FIN_KERNEL>(s, nb, tab, h, sigma, v, st, f);
+  else
+    launch_precond_dst_m<T, PREC_PLAIN, FIN_KERNEL>(s, nb, tab, h, sigma, v, st, f);
 }
 
 // Component c of the velocity into the solver's vectors: u = u*_c and
@@ -216,13 +243,15 @@ void dst_tables(double* tab, float* tab32) {
 }
 
 void launch_precond_dst(hipStream_t s, int mode, int nb, const double* tab, const double* h,
-                        double sigma, const KrylovVectors<double>& v, SolverState* st) {
-  launch_precond_dst_t<double>(s, mode, nb, tab, h, sigma, v, st);
+                        double sigma, const KrylovVectors<double>& v, SolverState* st, int fin,
+                        const FinArgs& f) {
+  launch_precond_dst_t<double>(s, mode, nb, tab, h, sigma, v, st, fin, f);
 }
 
 void launch_precond_dst32(hipStream_t s, int mode, int nb, const float* tab, const float* h,
-                          const KrylovVectors<float>& v, SolverState* st) {
-  launch_precond_dst_t<float>(s, mode, nb, tab, h, 0.0f, v, st);
+                          const KrylovVectors<float>& v, SolverState* st, int fin,
+                          const FinArgs& f) {
+  launch_precond_dst_t<float>(s, mode, nb, tab, h, 0.0f, v, st, fin, f);
 }
 
 void launch_diffusion_gather(hipStream_t s, long long n, int comp, const double* h3, double sigma,

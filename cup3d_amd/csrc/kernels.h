@@ -12,15 +12,38 @@ namespace cup3d {
 enum SpmvMode { SPMV_PLAIN = 0, SPMV_INIT = 1, SPMV_DOT1 = 2, SPMV_DOT2 = 3, SPMV_RESID = 4 };
 enum PrecMode { PREC_PLAIN = 0, PREC_P = 1, PREC_S = 2 };
 
+// Where the scalars of an iteration are computed: by finalize kernels, or by
+// the kernels that use them (krylov.h), with the bMean = 1 row or without.
+enum Fin { FIN_KERNEL = 0, FIN_SUMS = 1, FIN_ROW = 2 };
+struct FinArgs {
+  const double* part = nullptr;
+  int nparts = 0;
+  long long row = -1;
+};
+constexpr int FIN_MAX_BLOCKS = 8192;
+
+// The way a grid's iterations take (bMean = 2 needs its sum before the
+// epilogue of the SpMV, so it keeps the kernels).
+inline int fin_mode(int nb, int bmean, long long row) {
+  if (nb > FIN_MAX_BLOCKS || bmean == 2) return FIN_KERNEL;
+  return bmean == 1 && row >= 0 ? FIN_ROW : FIN_SUMS;
+}
+// The sums of K5 lie behind those of the SpMVs, which K5 still reads.
+inline double* k5_part(double* part, int nb) { return part + 4 * (size_t)((nb + 3) / 4 + 8); }
+// Copies of the solver state (krylov.h): st[0] is the one the host reads.
+constexpr int STATE_COPIES = 3;
+
 void launch_getvec64(hipStream_t s, long long n, long long zero_row, const double* rhs,
                      const double* x0, double* b, double* x, SolverState* st, double* part,
                      double tol_b);
 // part null (SPMV_PLAIN and SPMV_RESID on a grid with bMean 0 or 3): no sums are
 // taken and st is not used.
 void launch_spmv64(hipStream_t s, int mode, const DevGrid<double>& g, const double* x, double* y,
-                   const double* a, double* c, double* c2, SolverState* st, double* part);
-void launch_update64(hipStream_t s, long long n, const KrylovVectors<double>& v, SolverState* st,
-                     double* part);
+                   const double* a, double* c, double* c2, SolverState* st, double* part,
+                   bool fin = true);
+// K5; returns its number of partials. last: with its finalize kernel.
+int launch_update64(hipStream_t s, const DevGrid<double>& g, const KrylovVectors<double>& v,
+                    SolverState* st, double* part, int fin = FIN_KERNEL, bool last = true);
 void launch_copy_opt64(hipStream_t s, long long n, const KrylovVectors<double>& v,
                        const SolverState* st, double* out);
 

@@ -38,19 +38,20 @@ void launch_getvec64(hipStream_t s, long long n, long long zero_row, const doubl
 }
 
 void launch_spmv64(hipStream_t s, int mode, const DevGrid<double>& g, const double* x, double* y,
-                   const double* a, double* c, double* c2, SolverState* st, double* part) {
+                   const double* a, double* c, double* c2, SolverState* st, double* part,
+                   bool fin) {
   switch (mode) {
-    case SPMV_PLAIN: spmv_launch<double, SPMV_PLAIN>(s, g, x, y, a, c, c2, st, part); break;
-    case SPMV_INIT: spmv_launch<double, SPMV_INIT>(s, g, x, y, a, c, c2, st, part); break;
-    case SPMV_DOT1: spmv_launch<double, SPMV_DOT1>(s, g, x, y, a, c, c2, st, part); break;
-    case SPMV_DOT2: spmv_launch<double, SPMV_DOT2>(s, g, x, y, a, c, c2, st, part); break;
-    case SPMV_RESID: spmv_launch<double, SPMV_RESID>(s, g, x, y, a, c, c2, st, part); break;
+    case SPMV_PLAIN: spmv_launch<double, SPMV_PLAIN>(s, g, x, y, a, c, c2, st, part, fin); break;
+    case SPMV_INIT: spmv_launch<double, SPMV_INIT>(s, g, x, y, a, c, c2, st, part, fin); break;
+    case SPMV_DOT1: spmv_launch<double, SPMV_DOT1>(s, g, x, y, a, c, c2, st, part, fin); break;
+    case SPMV_DOT2: spmv_launch<double, SPMV_DOT2>(s, g, x, y, a, c, c2, st, part, fin); break;
+    case SPMV_RESID: spmv_launch<double, SPMV_RESID>(s, g, x, y, a, c, c2, st, part, fin); break;
   }
 }
 
-void launch_update64(hipStream_t s, long long n, const KrylovVectors<double>& v, SolverState* st,
-                     double* part) {
-  launch_k5<double>(s, n, v, st, part);
+int launch_update64(hipStream_t s, const DevGrid<double>& g, const KrylovVectors<double>& v,
+                    SolverState* st, double* part, int fin, bool last) {
+  return launch_k5<double>(s, g, v, st, part, fin, last);
 }
 
 void launch_copy_opt64(hipStream_t s, long long n, const KrylovVectors<double>& v,

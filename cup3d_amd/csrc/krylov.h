@@ -66,6 +66,90 @@ __device__ __forceinline__ void fin_store(SolverState* st, const SolverState& S)
         reinterpret_cast<const unsigned*>(&S)[threadIdx.x];
 }
 
+// ---------------------------------------------------------------------------
+// Scalars in the consumer (FIN_SUMS, FIN_ROW): on grids of up to
+// FIN_MAX_BLOCKS blocks the kernel that needs a sum adds the producer's
+// partials itself, every workgroup all of them while its first vector loads
+// are in flight, instead of a one-workgroup finalize kernel in between:
+//   K1 (USE_P)  the sums of K5: |r|, x_opt, convergence, restart, beta
+//   K3 (USE_S)  the sum of K2: alpha
+//   K5 (USE_X)  the sums of K4: omega
+// The state passes through three copies, st[0] -> K3 -> st[1] -> K5 -> st[2]
+// -> K1 -> st[0], each written by the first workgroup of the kernel that
+// computes it and read by later kernels only. The partials are added by 256
+// threads in the finalize kernels' order, so both ways give the same bits.
+// FIN_ROW also carries the bMean = 1 row (A x)[row] = sum h^3 x to the lane that
+// owns the row.
+// A finalize kernel costs about 5.5 us with its launch gap, three of them an
+// iteration; adding n / 2048 partials in each of the consumer's workgroups
+// grows with their product. Measured per capped solve with finalize kernels
+// and without: 819 blocks (BF16, 32 iterations) 1880 -> 1548 us, 8192 blocks
+// (FP16, 32) 3299 -> 3051 us, (FP64, 8) 1500 -> 1483 us; 12 320 blocks (FP16)
+// 4430 -> 4491 us, (FP64) 2073 -> 2137 us. Hence the limit of 8192.
+// ---------------------------------------------------------------------------
+enum Consumer { USE_P = 0, USE_S = 1, USE_X = 2 };
+
+__device__ inline void set_alpha(SolverState& S, double dot) {
+  S.dot_a = dot;
+  S.alpha = S.rho_curr / (dot + S.eps);  // set_alpha (BiCGSTAB.cu:276-279)
+  S.p_zero = 0;
+  S.restart_pending = 0;
+}
+__device__ inline void set_omega(SolverState& S, double ts, double tt) {
+  S.dot_ts = ts;
+  S.dot_tt = tt;
+  S.omega = ts / (tt + S.eps);  // set_omega (:281-284)
+}
+__device__ inline void update_scalars(SolverState& S, double rho, double rr);
+
+// The state a consumer works with, in S (LDS); every thread of a workgroup of
+// at least 256 must call it. yr: the bMean = 1 row of the producer's product
+// (FIN_ROW).
+template <int USE, int FIN, typename T>
+__device__ __forceinline__ void consumer_state(SolverState* st, const FinArgs& f, SolverState& S,
+                                               T& yr) {
+  constexpr int K = USE == USE_P ? 2 : (USE == USE_S ? 1 : 2) + (FIN == FIN_ROW ? 1 : 0);
+  __shared__ double red[K][4];
+  const SolverState* src = st + (USE == USE_P ? 2 : (USE == USE_S ? 0 : 1));
+  SolverState* dst = st + (USE == USE_P ? 0 : (USE == USE_S ? 1 : 2));
+  const int tid = threadIdx.x;
+  if (tid < STATE_WORDS)
+    reinterpret_cast<unsigned*>(&S)[tid] = reinterpret_cast<const unsigned*>(src)[tid];
+  double aux = 0.0;
+  if (USE != USE_P && FIN == FIN_ROW) aux = f.part[(size_t)K * f.nparts];
+  if (tid < WG_THREADS) {
+    double acc[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) acc[k] = 0.0;
+#pragma unroll 4
+    for (int i = tid; i < f.nparts; i += WG_THREADS)
+#pragma unroll
+      for (int k = 0; k < K; ++k) acc[k] += f.part[(size_t)i * K + k];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const double s = wave_sum(acc[k]);
+      if ((tid & 63) == 0) red[k][tid >> 6] = s;
+    }
+  }
+  __syncthreads();
+  double tot[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) tot[k] = ((red[k][0] + red[k][1]) + red[k][2]) + red[k][3];
+  if (USE != USE_P && FIN == FIN_ROW) {
+    yr = (T)tot[0];
+    tot[1] += aux * (double)yr;
+    if (USE == USE_X) tot[K - 1] += (double)yr * (double)yr;
+  }
+  if (tid == 0 && S.status == ST_RUNNING) {
+    if (USE == USE_P) update_scalars(S, tot[0], tot[K - 1]);
+    else if (USE == USE_S) set_alpha(S, tot[K - 1]);
+    else set_omega(S, tot[K - 2], tot[K - 1]);
+  }
+  __syncthreads();
+  if (blockIdx.x == 0 && tid < STATE_WORDS)
+    reinterpret_cast<unsigned*>(dst)[tid] = reinterpret_cast<const unsigned*>(&S)[tid];
+}
+
 // Contiguous 8-element vector access (16-byte loads/stores).
 template <typename T>
 __device__ __forceinline__ void load8(const T* __restrict__ p, T (&v)[8]) {
@@ -315,13 +399,23 @@ constexpr size_t STREAM_MIN_BYTES = size_t(64) << 20;
 // same stencil and coarse-fine faces, plus -h^3 sigma x and the Dirichlet
 // ghosts of BlockLabBC (Definitions.h:58-122,287-330) on the boundary faces
 // selected by g.dmask, both folded into the diagonal of the cell.
+// Sums a product takes: sum h^3 x (bMean 1 and 2), then the mode's dots.
+template <int MODE, int BM>
+struct SpmvSums {
+  static constexpr int MEAN = BM == 1 || BM == 2 ? 1 : 0;
+  static constexpr int DOTS =
+      MODE == SPMV_PLAIN ? 0 : (MODE == SPMV_DOT1 || MODE == SPMV_RESID ? 1 : 2);
+  static constexpr int N = MEAN + DOTS;
+};
+
 template <typename T, int MODE, int BM, bool IFACE, bool HELM = false, bool NT = false>
 __global__ __launch_bounds__(WG_THREADS) void k_spmv(DevGrid<T> g, const T* __restrict__ x,
                                                      T* __restrict__ y, const T* a, T* c, T* c2,
                                                      SolverState* st, double* part) {
   constexpr bool NEED_A = MODE != SPMV_PLAIN;
   // sum_b h_b^3 sum x feeds the bMean = 1 row and the bMean = 2 term only
-  constexpr bool NEED_SUM = BM == 1 || BM == 2;
+  using Sums = SpmvSums<MODE, BM>;
+  constexpr bool NEED_SUM = Sums::MEAN == 1;
   __shared__ T xs[4][BLEN];
   __shared__ T ys[IFACE ? 4 : 1][IFACE ? BLEN : 1];
   __shared__ T pl[IFACE ? 4 : 1][IFACE ? 64 : 1];
@@ -464,9 +558,12 @@ __global__ __launch_bounds__(WG_THREADS) void k_spmv(DevGrid<T> g, const T* __re
   const bool origin = valid && row == (long long)off;
   if (BM == 3 && origin && lane == 0) yv[0] = h * col[0];  // row h*I (.cpp:311-318)
   // epilogue: stores and partial sums
-  double v[3] = {0.0, 0.0, 0.0};
+  double v[3] = {0.0, 0.0, 0.0};  // sum h^3 x, then the dots
   if (valid) {
     if (NEED_SUM) v[0] = (double)h * (double)h * (double)h * msum;
+    // the row's other factor, for the kernel that completes the dot (FIN_ROW)
+    if (BM == 1 && (MODE == SPMV_DOT1 || MODE == SPMV_DOT2) && origin && lane == 0)
+      part[(size_t)Sums::N * gridDim.x] = (double)(A_LDS ? as[w][0] : av[0]);
 #pragma unroll
     for (int iz = 0; iz < BS; ++iz) {
       const size_t i = off + iz * 64 + lane;
@@ -499,7 +596,12 @@ __global__ __launch_bounds__(WG_THREADS) void k_spmv(DevGrid<T> g, const T* __re
     }
   }
   if ((MODE == SPMV_PLAIN || MODE == SPMV_RESID) && !part) return;  // no sums wanted
-  grid_store_partial<3>(v, part);
+  if constexpr (Sums::N > 0) {
+    double p[Sums::N];
+#pragma unroll
+    for (int k = 0; k < Sums::N; ++k) p[k] = v[k + 1 - Sums::MEAN];
+    grid_store_partial<Sums::N>(p, part);
+  }
 }
 
 // Finalize of k_spmv (one workgroup): totals, the bMean = 1 row
@@ -510,9 +612,12 @@ __global__ __launch_bounds__(WG_THREADS) void k_spmv_fin(long long row, T* __res
                                                          T* __restrict__ c, T* __restrict__ c2,
                                                          SolverState* st, const double* part,
                                                          int nparts) {
+  using Sums = SpmvSums<MODE, BM>;
   __shared__ SolverState S;
-  double tot[3];
-  fin_load<3>(st, S, part, nparts, tot);
+  double sums[Sums::N], tot[3] = {0.0, 0.0, 0.0};
+  fin_load<Sums::N>(st, S, part, nparts, sums);
+#pragma unroll
+  for (int k = 0; k < Sums::N; ++k) tot[k + 1 - Sums::MEAN] = sums[k];
   if (MODE != SPMV_PLAIN && MODE != SPMV_RESID && S.status != ST_RUNNING) return;
   if (threadIdx.x == 0) {
     // bMean = 1: y[row] = sum_b h_b^3 sum x  (BiCGSTAB.cu:406-407)
@@ -550,14 +655,9 @@ __global__ __launch_bounds__(WG_THREADS) void k_spmv_fin(long long row, T* __res
       S.rhrh = tot[2];
       begin_iteration(&S, tot[2], tot[2]);
     } else if (MODE == SPMV_DOT1) {
-      S.dot_a = tot[1];
-      S.alpha = S.rho_curr / (tot[1] + S.eps);  // set_alpha (:276-279)
-      S.p_zero = 0;
-      S.restart_pending = 0;
+      set_alpha(S, tot[1]);
     } else if (MODE == SPMV_DOT2) {
-      S.dot_ts = tot[1];
-      S.dot_tt = tot[2];
-      S.omega = tot[1] / (tot[2] + S.eps);  // set_omega (:281-284)
+      set_omega(S, tot[1], tot[2]);
     } else if (MODE == SPMV_RESID) {
       S.true_rr = tot[1];
     }
@@ -574,9 +674,10 @@ __global__ __launch_bounds__(WG_THREADS) void k_spmv_fin(long long row, T* __res
 template <int MODE>
 __global__ __launch_bounds__(WG_THREADS) void k_bmean2_sum(SolverState* st, const double* part,
                                                            int nparts) {
+  constexpr int N = SpmvSums<MODE, 2>::N;
   __shared__ SolverState S;
-  double tot[3];
-  fin_load<3>(st, S, part, nparts, tot);
+  double tot[N];
+  fin_load<N>(st, S, part, nparts, tot);
   if (MODE != SPMV_PLAIN && MODE != SPMV_RESID && S.status != ST_RUNNING) return;
   if (threadIdx.x == 0) S.mean_sum = tot[0];
   fin_store(st, S);
@@ -633,7 +734,11 @@ __global__ __launch_bounds__(WG_THREADS) void k_bmean2_apply(DevGrid<T> g, T* __
     }
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) v[0] = red;  // k_spmv_fin keeps it as mean_sum
-  grid_store_partial<3>(v, part);
+  constexpr int N = SpmvSums<MODE, 2>::N;
+  double p[N];
+#pragma unroll
+  for (int k = 0; k < N; ++k) p[k] = v[k];
+  grid_store_partial<N>(p, part);
 }
 
 // Launch for a grid: picks the bMean and interface variants.
@@ -648,7 +753,7 @@ inline void spmv_kernel(hipStream_t s, int nwg, const DevGrid<T>& g, const T* x,
 }
 template <typename T, int MODE, int BM, bool HELM = false>
 inline void spmv_launch_iface(hipStream_t s, const DevGrid<T>& g, const T* x, T* y, const T* a,
-                              T* c, T* c2, SolverState* st, double* part,
+                              T* c, T* c2, SolverState* st, double* part, bool fin,
                               hipEvent_t mid = nullptr) {
   int nwg = (g.nb + 3) / 4;
   bool launched = false;
@@ -662,7 +767,7 @@ inline void spmv_launch_iface(hipStream_t s, const DevGrid<T>& g, const T* x, T*
   if (mid) (void)hipEventRecord(mid, s);
   // SPMV_PLAIN and SPMV_RESID without sums (part null; bMean 0 and 3 only): the
   // vectors are complete, and the finalize kernel is 4 us of a 20-60 us call
-  if (!part) return;
+  if (!part || !fin) return;  // or the sums are left to the consumer (fin false)
   if (BM == 2) {
     k_bmean2_sum<MODE><<<1, WG_THREADS, 0, s>>>(st, part, nwg);
     // nb * 64 threads of 8 cells: (nb + 3) / 4 workgroups again, so the
@@ -670,21 +775,23 @@ inline void spmv_launch_iface(hipStream_t s, const DevGrid<T>& g, const T* x, T*
     nwg = (int)(((long long)g.nb * (BLEN / 8) + WG_THREADS - 1) / WG_THREADS);
     k_bmean2_apply<T, MODE><<<nwg, WG_THREADS, 0, s>>>(g, y, a, c, c2, st, part);
   }
-  k_spmv_fin<T, MODE, BM><<<1, WG_THREADS, 0, s>>>(g.bmean_row, y, a, c, c2, st, part, nwg);
+  if constexpr (SpmvSums<MODE, BM>::N > 0)
+    k_spmv_fin<T, MODE, BM><<<1, WG_THREADS, 0, s>>>(g.bmean_row, y, a, c, c2, st, part, nwg);
 }
 template <typename T, int MODE>
 inline void spmv_launch(hipStream_t s, const DevGrid<T>& g, const T* x, T* y, const T* a, T* c,
-                        T* c2, SolverState* st, double* part, hipEvent_t mid = nullptr) {
+                        T* c2, SolverState* st, double* part, bool fin = true,
+                        hipEvent_t mid = nullptr) {
   if constexpr (sizeof(T) == 8) {
     if (g.helm) {  // implicit diffusion: no bMean row
-      spmv_launch_iface<T, MODE, 0, true>(s, g, x, y, a, c, c2, st, part, mid);
+      spmv_launch_iface<T, MODE, 0, true>(s, g, x, y, a, c, c2, st, part, fin, mid);
       return;
     }
   }
-  if (g.bmean == 1) spmv_launch_iface<T, MODE, 1>(s, g, x, y, a, c, c2, st, part, mid);
-  else if (g.bmean == 2) spmv_launch_iface<T, MODE, 2>(s, g, x, y, a, c, c2, st, part, mid);
-  else if (g.bmean == 3) spmv_launch_iface<T, MODE, 3>(s, g, x, y, a, c, c2, st, part, mid);
-  else spmv_launch_iface<T, MODE, 0>(s, g, x, y, a, c, c2, st, part, mid);
+  if (g.bmean == 1) spmv_launch_iface<T, MODE, 1>(s, g, x, y, a, c, c2, st, part, fin, mid);
+  else if (g.bmean == 2) spmv_launch_iface<T, MODE, 2>(s, g, x, y, a, c, c2, st, part, fin, mid);
+  else if (g.bmean == 3) spmv_launch_iface<T, MODE, 3>(s, g, x, y, a, c, c2, st, part, fin, mid);
+  else spmv_launch_iface<T, MODE, 0>(s, g, x, y, a, c, c2, st, part, fin, mid);
 }
 
 // ---------------------------------------------------------------------------
@@ -702,35 +809,47 @@ __device__ __forceinline__ int third_buffer(int a, int b) {
 // runs CH = 2 halves the partial sums the finalize kernel reads (30 M cells:
 // 185 us against 191 us with it); smaller grids keep every CU busy with
 // CH = 1 (4.2 M cells, FP64: 48.7 us against 54.6 us).
-template <typename T, int CH>
+template <typename T, int CH, int FIN>
 __global__ __launch_bounds__(WG_THREADS) void k_update(long long n, KrylovVectors<T> v,
-                                                       SolverState* st, double* part) {
-  if (st->status != ST_RUNNING) return;
-  const int xc = st->xcur, xo = st->xopt, xn = third_buffer(xc, xo);
-  const T alpha = (T)st->alpha, omega = (T)st->omega;
+                                                       SolverState* st, FinArgs f, double* part) {
+  static_assert(FIN == FIN_KERNEL || CH == 1, "the first run's loads overlap the sums");
+  __shared__ SolverState S;
+  if (!FIN && st->status != ST_RUNNING) return;
   double s[2] = {0.0, 0.0};
   // each thread owns 8 consecutive elements of each of this workgroup's runs
 #pragma unroll
   for (int c = 0; c < CH; ++c) {
-  const long long i0 = ((long long)blockIdx.x * CH + c) * (4 * BLEN) + 8 * threadIdx.x;
-  if (i0 < n) {
+    const long long i0 = ((long long)blockIdx.x * CH + c) * (4 * BLEN) + 8 * threadIdx.x;
     T xv[8], z1[8], z2[8], t[8], r[8], rh[8];
-    load8(v.x[xc] + i0, xv);
-    load8(v.z1 + i0, z1);
-    load8(v.z2 + i0, z2);
-    load8(v.t + i0, t);
-    load8(v.r + i0, r);
-    load8(v.rhat + i0, rh);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      xv[e] = fma(omega, z2[e], fma(alpha, z1[e], xv[e]));
-      r[e] = fma(-omega, t[e], r[e]);
-      s[0] += (double)rh[e] * (double)r[e];
-      s[1] += (double)r[e] * (double)r[e];
+    if (i0 < n) {
+      load8(v.z1 + i0, z1);
+      load8(v.z2 + i0, z2);
+      load8(v.t + i0, t);
+      load8(v.r + i0, r);
+      load8(v.rhat + i0, rh);
     }
-    store8(v.x[xn] + i0, xv);
-    store8(v.r + i0, r);
-  }
+    T yr = 0;
+    const SolverState* sp = st;
+    if constexpr (FIN != FIN_KERNEL) {
+      consumer_state<USE_X, FIN, T>(st, f, S, yr);
+      if (S.status != ST_RUNNING) return;
+      sp = &S;
+      if (FIN == FIN_ROW && i0 == f.row) t[0] = yr;
+    }
+    if (i0 < n) {
+      const int xc = sp->xcur, xn = third_buffer(xc, sp->xopt);
+      const T alpha = (T)sp->alpha, omega = (T)sp->omega;
+      load8(v.x[xc] + i0, xv);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        xv[e] = fma(omega, z2[e], fma(alpha, z1[e], xv[e]));
+        r[e] = fma(-omega, t[e], r[e]);
+        s[0] += (double)rh[e] * (double)r[e];
+        s[1] += (double)r[e] * (double)r[e];
+      }
+      store8(v.x[xn] + i0, xv);
+      store8(v.r + i0, r);
+    }
   }
   grid_store_partial<2>(s, part);
 }
@@ -761,27 +880,35 @@ __device__ inline void update_scalars(SolverState& S, double rho, double rr) {
   begin_iteration(&S, rho, rr);
 }
 
-static __global__ __launch_bounds__(WG_THREADS) void k_update_fin(SolverState* st, const double* part,
+// src: the state before K5 (st, or the consumers' last copy), dst: after it.
+static __global__ __launch_bounds__(WG_THREADS) void k_update_fin(const SolverState* src,
+                                                           SolverState* dst, const double* part,
                                                            int nparts) {
   __shared__ SolverState S;
   double tot[2];
-  fin_load<2>(st, S, part, nparts, tot);
-  if (S.status != ST_RUNNING) return;
-  if (threadIdx.x == 0) update_scalars(S, tot[0], tot[1]);
-  fin_store(st, S);
+  fin_load<2>(src, S, part, nparts, tot);
+  if (threadIdx.x == 0 && S.status == ST_RUNNING) update_scalars(S, tot[0], tot[1]);
+  fin_store(dst, S);
 }
 
-// K5 and its finalize kernel (an event, if given, is recorded between them).
+// K5 and, unless the next K1 takes its sums, the finalize kernel (an event, if
+// given, is recorded between them). Returns the number of partials.
 template <typename T>
-inline void launch_k5(hipStream_t s, long long n, const KrylovVectors<T>& v, SolverState* st,
-                      double* part, hipEvent_t mid = nullptr) {
-  const long long runs = (n + 4 * BLEN - 1) / (4 * BLEN);
+inline int launch_k5(hipStream_t s, const DevGrid<T>& g, const KrylovVectors<T>& v,
+                     SolverState* st, double* part, int fin = FIN_KERNEL, bool last = true,
+                     hipEvent_t mid = nullptr) {
+  const long long n = g.n, runs = (n + 4 * BLEN - 1) / (4 * BLEN);
   const int ch = runs >= 8192 ? 2 : 1;
   const int nwg = (int)((runs + ch - 1) / ch);
-  if (ch == 2) k_update<T, 2><<<nwg, WG_THREADS, 0, s>>>(n, v, st, part);
-  else k_update<T, 1><<<nwg, WG_THREADS, 0, s>>>(n, v, st, part);
+  const FinArgs f{part, (g.nb + 3) / 4, g.bmean_row};
+  double* p5 = k5_part(part, g.nb);
+  if (fin == FIN_SUMS) k_update<T, 1, FIN_SUMS><<<nwg, WG_THREADS, 0, s>>>(n, v, st, f, p5);
+  else if (fin == FIN_ROW) k_update<T, 1, FIN_ROW><<<nwg, WG_THREADS, 0, s>>>(n, v, st, f, p5);
+  else if (ch == 2) k_update<T, 2, FIN_KERNEL><<<nwg, WG_THREADS, 0, s>>>(n, v, st, f, p5);
+  else k_update<T, 1, FIN_KERNEL><<<nwg, WG_THREADS, 0, s>>>(n, v, st, f, p5);
   if (mid) (void)hipEventRecord(mid, s);
-  k_update_fin<<<1, WG_THREADS, 0, s>>>(st, part, nwg);
+  if (last) k_update_fin<<<1, WG_THREADS, 0, s>>>(fin ? st + 2 : st, st, p5, nwg);
+  return nwg;
 }
 
 // Copy the best iterate out: x_user = X[xopt] (PoissonSolverExp.cpp:452-472

@@ -116,7 +116,7 @@ struct PrecScalars {
 };
 
 template <int MODE>
-__device__ __forceinline__ PrecScalars prec_scalars(const SolverState* st) {
+__device__ __forceinline__ PrecScalars prec_scalars(const SolverState* st) {  // global or LDS
   PrecScalars c;
   c.beta = MODE == PREC_P ? (float)st->beta : 0.f;
   c.omega = MODE == PREC_P ? (float)st->omega : 0.f;
@@ -297,23 +297,42 @@ __device__ __forceinline__ void precond_gemm(int nb, int j0, int w, int l,
 
 // One workgroup applies M^-1 to NBW consecutive blocks: every wave fills
 // (phase 1), then every wave multiplies (phases 2 and 3).
-template <int MODE, typename H, int NBW, bool SPLIT, bool NT = false>
+template <int MODE, typename H, int NBW, bool SPLIT, bool NT = false, int FIN = FIN_KERNEL>
 __global__ __launch_bounds__(GT) void k_precond_h(int nb, const H* __restrict__ Ppk,
                                                   float p_unscale,
                                                   const float* __restrict__ invh,
                                                   KrylovVectors<float> v,
                                                   const float* __restrict__ pin,
-                                                  float* __restrict__ pout, SolverState* st) {
+                                                  float* __restrict__ pout, SolverState* st,
+                                                  FinArgs f) {
   constexpr int NS = SPLIT ? 2 : 1;
   __shared__ __attribute__((aligned(16))) H As[NS][NBW * HLD];
   __shared__ float sc[NBW];
-  if (MODE != PREC_PLAIN && st->status != ST_RUNNING) return;
-  const PrecScalars c = prec_scalars<MODE>(st);
+  __shared__ SolverState S;
+  if (!FIN && MODE != PREC_PLAIN && st->status != ST_RUNNING) return;
   const int j0 = (int)blockIdx.x * NBW;
   float* __restrict__ out = MODE == PREC_PLAIN ? pout : (MODE == PREC_S ? v.z2 : v.z1);
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
   FillRegs<NBW, GW> R;
   precond_load<MODE, NBW, GW, NT>(nb, j0, w, l, v, pin, R);
+  const SolverState* sp = st;
+  if constexpr (FIN != FIN_KERNEL) {
+    float yr = 0.f;
+    consumer_state<MODE == PREC_P ? USE_P : USE_S, FIN, float>(st, f, S, yr);
+    if (S.status != ST_RUNNING) return;
+    sp = &S;
+    if (FIN == FIN_ROW && MODE == PREC_S && l == 0) {
+#pragma unroll
+      for (int u = 0; u < FillRegs<NBW, GW>::F4; u += 2) {
+        const int b = j0 + w * FillRegs<NBW, GW>::NPB + u / 2;
+        if (b < nb && (long long)b * BLEN == f.row) {
+          R.rb[u].x = yr;  // the mean-constraint row of nu, which the SpMV left out
+          v.nu[f.row] = yr;
+        }
+      }
+    }
+  }
+  const PrecScalars c = prec_scalars<MODE>(sp);
   precond_convert<MODE, H, NBW, SPLIT, GW, NT>(nb, j0, w, l, p_unscale, invh, v, c, R, As[0],
                                            As[NS - 1], sc);
   __syncthreads();
@@ -455,69 +474,66 @@ namespace {
 // per workgroup, so 32 blocks halve that traffic against 16; 32 is also the
 // faster choice on grids too small to give every CU a workgroup (4440 blocks:
 // 14.4 us against 15.9 us for K1).
-static inline int gemm_width(int) { return 32; }
+constexpr int GEMM_NB = 32;
 
 template <typename H, bool SPLIT, int NBW>
 void launch_precond_hw(hipStream_t s, int mode, int nb, const H* P, float unscale,
                        const float* invh, const KrylovVectors<float>& v, const float* pin,
-                       float* pout, SolverState* st) {
+                       float* pout, SolverState* st, int fin, const FinArgs& f) {
   const int nwg = (nb + NBW - 1) / NBW;
   // K1 and K3 stream their vectors nontemporally when they are large
+  // (larger than any grid whose scalars are computed in the consumer)
   const bool nt = (size_t)nb * BLEN * sizeof(float) >= STREAM_MIN_BYTES;
-  if (mode == PREC_P && nt)
-    k_precond_h<PREC_P, H, NBW, SPLIT, true><<<nwg, GT, 0, s>>>(nb, P, unscale, invh, v, pin, pout, st);
-  else if (mode == PREC_P)
-    k_precond_h<PREC_P, H, NBW, SPLIT><<<nwg, GT, 0, s>>>(nb, P, unscale, invh, v, pin, pout, st);
-  else if (mode == PREC_S && nt)
-    k_precond_h<PREC_S, H, NBW, SPLIT, true><<<nwg, GT, 0, s>>>(nb, P, unscale, invh, v, pin, pout, st);
-  else if (mode == PREC_S)
-    k_precond_h<PREC_S, H, NBW, SPLIT><<<nwg, GT, 0, s>>>(nb, P, unscale, invh, v, pin, pout, st);
-  else
-    k_precond_h<PREC_PLAIN, H, NBW, SPLIT><<<nwg, GT, 0, s>>>(nb, P, unscale, invh, v, pin, pout, st);
-}
-
-template <typename H, bool SPLIT>
-void launch_precond_hh(hipStream_t s, int mode, int nb, const H* P, float unscale,
-                       const float* invh, const KrylovVectors<float>& v, const float* pin,
-                       float* pout, SolverState* st) {
-  if (gemm_width(nb) == 32)
-    launch_precond_hw<H, SPLIT, 32>(s, mode, nb, P, unscale, invh, v, pin, pout, st);
-  else
-    launch_precond_hw<H, SPLIT, 16>(s, mode, nb, P, unscale, invh, v, pin, pout, st);
+  static_assert((size_t)FIN_MAX_BLOCKS * BLEN * sizeof(float) < STREAM_MIN_BYTES, "no NT with FIN");
+#define CUP3D_PREC_LAUNCH(MODE, NT, FIN)                                                     \
+  k_precond_h<MODE, H, NBW, SPLIT, NT, FIN>                                                  \
+      <<<nwg, GT, 0, s>>>(nb, P, unscale, invh, v, pin, pout, st, f)
+  if (mode == PREC_P && fin) CUP3D_PREC_LAUNCH(PREC_P, false, FIN_SUMS);
+  else if (mode == PREC_P && nt) CUP3D_PREC_LAUNCH(PREC_P, true, FIN_KERNEL);
+  else if (mode == PREC_P) CUP3D_PREC_LAUNCH(PREC_P, false, FIN_KERNEL);
+  else if (mode == PREC_S && fin == FIN_ROW) CUP3D_PREC_LAUNCH(PREC_S, false, FIN_ROW);
+  else if (mode == PREC_S && fin) CUP3D_PREC_LAUNCH(PREC_S, false, FIN_SUMS);
+  else if (mode == PREC_S && nt) CUP3D_PREC_LAUNCH(PREC_S, true, FIN_KERNEL);
+  else if (mode == PREC_S) CUP3D_PREC_LAUNCH(PREC_S, false, FIN_KERNEL);
+  else CUP3D_PREC_LAUNCH(PREC_PLAIN, false, FIN_KERNEL);
+#undef CUP3D_PREC_LAUNCH
 }
 
 template <typename H>
 void launch_precond_h(hipStream_t s, int mode, int nb, const void* Ppk, float unscale,
                       bool split, const float* invh, const KrylovVectors<float>& v,
-                      const float* pin, float* pout, SolverState* st) {
+                      const float* pin, float* pout, SolverState* st, int fin, const FinArgs& f) {
   const H* P = static_cast<const H*>(Ppk);
-  if (split) launch_precond_hh<H, true>(s, mode, nb, P, unscale, invh, v, pin, pout, st);
-  else launch_precond_hh<H, false>(s, mode, nb, P, unscale, invh, v, pin, pout, st);
+  if (split)
+    launch_precond_hw<H, true, GEMM_NB>(s, mode, nb, P, unscale, invh, v, pin, pout, st, fin, f);
+  else
+    launch_precond_hw<H, false, GEMM_NB>(s, mode, nb, P, unscale, invh, v, pin, pout, st, fin, f);
 }
 
 void launch_precond_mixed(const MixedWorkspace& M, hipStream_t s, int precision, int mode,
-                          const DevGrid<float>& g, const float* pin, float* pout, SolverState* st) {
+                          const DevGrid<float>& g, const float* pin, float* pout, SolverState* st,
+                          int fin = FIN_KERNEL, const FinArgs& f = FinArgs()) {
   if (M.use_dst) {
     KrylovVectors<float> v = M.v32;
     if (mode == PREC_PLAIN) {
       v.p = const_cast<float*>(pin);
       v.z1 = pout;
     }
-    launch_precond_dst32(s, mode, g.nb, M.dst32, g.h, v, st);
+    launch_precond_dst32(s, mode, g.nb, M.dst32, g.h, v, st, fin, f);
     return;
   }
   if (precision == CUP3D_PREC_MIXED_FP16)
     launch_precond_h<_Float16>(s, mode, g.nb, M.d_P16, 1.0f / P16_SCALE, M.split, g.invh, M.v32,
-                               pin, pout, st);
+                               pin, pout, st, fin, f);
   else
     launch_precond_h<__bf16>(s, mode, g.nb, M.d_Pbf, 1.0f, M.split, g.invh, M.v32, pin, pout,
-                             st);
+                             st, fin, f);
 }
 
 template <int MODE>
 void spmv32(hipStream_t s, const DevGrid<float>& g, const float* x, float* y, const float* a,
-            SolverState* st, double* part, hipEvent_t mid = nullptr) {
-  spmv_launch<float, MODE>(s, g, x, y, a, nullptr, nullptr, st, part, mid);
+            SolverState* st, double* part, bool fin = true, hipEvent_t mid = nullptr) {
+  spmv_launch<float, MODE>(s, g, x, y, a, nullptr, nullptr, st, part, fin, mid);
 }
 
 int grid_1d(long long n) { return (int)std::min<long long>((n + WG_THREADS - 1) / WG_THREADS, 8192); }
@@ -661,6 +677,9 @@ int mixed_solve(MixedWorkspace& M, hipStream_t s, const cup3d_poisson_config& cf
   // halving (BiCGSTAB's residual often rises before it falls) would otherwise
   // repeat the same unproductive restart until max_refine is spent.
   int stall_iters = CUP3D_STALL_ITERS;
+  const int fin = fin_mode(g32.nb, g32.bmean, g32.bmean_row);
+  const FinArgs fs{part, (g32.nb + 3) / 4, g32.bmean_row};  // K2's sums, for K3
+  FinArgs fp{k5_part(part, g32.nb), 0, -1};                 // K5's, for the next K1
   while (!done && steps <= cfg.max_refine) {
     const double scale = rnorm;
     const double inner_rel = std::max(cfg.inner_tol, 0.5 * tol / scale);
@@ -679,21 +698,25 @@ int mixed_solve(MixedWorkspace& M, hipStream_t s, const cup3d_poisson_config& cf
       // kernels of iterations after convergence exit at once)
       const int tm_it = poll / 2;
       const int iter0 = h_st->iter;
-      for (int it = 0; it < poll; ++it) {
+      // no more than the iterations the cap leaves
+      const int batch = std::min(poll, std::max(1, cfg.max_iter - h_st->iters_done));
+      for (int it = 0; it < batch; ++it) {
         // event pairs (2k, 2k+1) bracket the main kernel of K(k+1)
         const bool tm = M.prof && it == tm_it;
         if (tm) MCHECK(hipEventRecord(M.pev[0], s));
-        launch_precond_mixed(M, s, cfg.precision, PREC_P, g32, nullptr, nullptr, st);
+        launch_precond_mixed(M, s, cfg.precision, PREC_P, g32, nullptr, nullptr, st,
+                             it > 0 ? fin : FIN_KERNEL, fp);
         if (tm) MCHECK(hipEventRecord(M.pev[1], s));
         if (tm) MCHECK(hipEventRecord(M.pev[2], s));
-        spmv32<SPMV_DOT1>(s, g32, v.z1, v.nu, v.rhat, st, part, tm ? M.pev[3] : nullptr);
+        spmv32<SPMV_DOT1>(s, g32, v.z1, v.nu, v.rhat, st, part, !fin, tm ? M.pev[3] : nullptr);
         if (tm) MCHECK(hipEventRecord(M.pev[4], s));
-        launch_precond_mixed(M, s, cfg.precision, PREC_S, g32, nullptr, nullptr, st);
+        launch_precond_mixed(M, s, cfg.precision, PREC_S, g32, nullptr, nullptr, st, fin, fs);
         if (tm) MCHECK(hipEventRecord(M.pev[5], s));
         if (tm) MCHECK(hipEventRecord(M.pev[6], s));
-        spmv32<SPMV_DOT2>(s, g32, v.z2, v.t, v.r, st, part, tm ? M.pev[7] : nullptr);
+        spmv32<SPMV_DOT2>(s, g32, v.z2, v.t, v.r, st, part, !fin, tm ? M.pev[7] : nullptr);
         if (tm) MCHECK(hipEventRecord(M.pev[8], s));
-        launch_k5<float>(s, n, v, st, part, tm ? M.pev[9] : nullptr);
+        fp.nparts = launch_k5<float>(s, g32, v, st, part, fin, !fin || it == batch - 1,
+                                     tm ? M.pev[9] : nullptr);
       }
       MCHECK(hipGetLastError());
       MCHECK(hipMemcpyAsync(h_st, st, sizeof(SolverState), hipMemcpyDeviceToHost, s));
@@ -817,7 +840,7 @@ int mixed_time_kernel(MixedWorkspace& M, hipStream_t s, int which, int reps,
       case 0: spmv32<SPMV_PLAIN>(s, g32, v.z1, v.nu, nullptr, st, part); break;
       case 1: launch_precond_mixed(M, s, precision, PREC_PLAIN, g32, v.p, v.z1, st); break;
       case 2:
-        launch_k5<float>(s, M.n, v, st, part);
+        launch_k5<float>(s, g32, v, st, part);
         break;
       case 3: launch_precond_mixed(M, s, precision, PREC_P, g32, nullptr, nullptr, st); break;
       default: spmv32<SPMV_DOT1>(s, g32, v.z1, v.nu, v.rhat, st, part); break;

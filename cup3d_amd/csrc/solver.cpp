@@ -196,10 +196,11 @@ int upload(cup3d_poisson* H, DevBuf& d, const void* src, size_t bytes) {
 // 4.19 M cells (168 MB of vectors, 4.9 TB/s), 43 us (four workgroups) and
 // 5 us on 32 k cells.
 void launch_precond_fp64(cup3d_poisson* H, const DevGrid<double>& g, int mode,
-                         const KrylovVectors<double>& v) {
+                         const KrylovVectors<double>& v, int fin = FIN_KERNEL,
+                         const FinArgs& f = FinArgs()) {
   SolverState* st = H->d_state.as<SolverState>();
   launch_precond_dst(H->stream, mode, H->nb, H->d_dst.as<double>(), g.h,
-                     g.helm ? g.helm_sigma : 0.0, v, st);
+                     g.helm ? g.helm_sigma : 0.0, v, st, fin, f);
 }
 
 // Run the FP64 classical BiCGSTAB on the device. b64/x64 must already hold
@@ -211,7 +212,6 @@ int run_bicgstab64(cup3d_poisson* H, const DevGrid<double>& g) {
   SolverState* st = H->d_state.as<SolverState>();
   double* part = H->d_part.as<double>();
   const KrylovVectors<double>& v = H->v64;
-  auto precond = [&](int mode) { launch_precond_fp64(H, g, mode, v); };
   // r = b - A x0; rhat = r (BiCGSTAB.cu:435-467)
   launch_spmv64(s, SPMV_INIT, g, v.x[0], v.nu, v.b, v.r, v.rhat, st, part);
   const int poll = H->cfg.poll_every > 0 ? H->cfg.poll_every : 8;
@@ -219,15 +219,21 @@ int run_bicgstab64(cup3d_poisson* H, const DevGrid<double>& g) {
   // short solve (the implicit-diffusion solves take a few iterations) is not
   // held up by the host enqueueing the rest of a full batch, whose kernels
   // would only find the state converged; a long solve polls a few more times.
+  // No more than the iterations the cap leaves are launched.
+  const int fin = fin_mode(g.nb, g.bmean, g.bmean_row);
+  const FinArgs fs{part, (g.nb + 3) / 4, g.bmean_row};  // K2's sums, for K3
+  FinArgs fp{k5_part(part, g.nb), 0, -1};               // K5's, for the next K1
   int batch = 1;
   long long launched = 0;
   while (true) {
+    const int left = (int)std::max(1LL, H->cfg.max_iter - launched);
+    batch = std::min(batch, left);
     for (int k = 0; k < batch; ++k) {
-      precond(PREC_P);
-      launch_spmv64(s, SPMV_DOT1, g, v.z1, v.nu, v.rhat, nullptr, nullptr, st, part);
-      precond(PREC_S);
-      launch_spmv64(s, SPMV_DOT2, g, v.z2, v.t, v.r, nullptr, nullptr, st, part);
-      launch_update64(s, H->n, v, st, part);
+      launch_precond_fp64(H, g, PREC_P, v, k > 0 ? fin : FIN_KERNEL, fp);
+      launch_spmv64(s, SPMV_DOT1, g, v.z1, v.nu, v.rhat, nullptr, nullptr, st, part, !fin);
+      launch_precond_fp64(H, g, PREC_S, v, fin, fs);
+      launch_spmv64(s, SPMV_DOT2, g, v.z2, v.t, v.r, nullptr, nullptr, st, part, !fin);
+      fp.nparts = launch_update64(s, g, v, st, part, fin, !fin || k == batch - 1);
     }
     launched += batch;
     HIPCHECK(hipGetLastError());
@@ -320,7 +326,7 @@ int cup3d_poisson_create(const cup3d_poisson_config* cfg, cup3d_poisson_t* out) 
     return -1;
   }
   H->mixed.dst32 = H->d_dst32.as<float>();
-  if (H->d_state.alloc(sizeof(SolverState)) != hipSuccess) {
+  if (H->d_state.alloc(STATE_COPIES * sizeof(SolverState)) != hipSuccess) {
     g_create_error = "hipMalloc(state) failed";
     return -1;
   }
@@ -465,7 +471,7 @@ int cup3d_poisson_set_topology(cup3d_poisson_t H, int64_t nblocks, const cup3d_b
   if (!H->d_gdots.p &&
       H->d_gdots.alloc(GUESS_MAXV * (GUESS_MAXV + 1) / 2 * sizeof(double)) != hipSuccess)
     return fail(H, "hipMalloc(guess dots) failed");
-  HIPCHECK(hipMemset(H->d_state.p, 0, sizeof(SolverState)));
+  HIPCHECK(hipMemset(H->d_state.p, 0, STATE_COPIES * sizeof(SolverState)));
   if (mixed_set_topology(H->mixed, H->nb, H->n, H->err) != 0) return -1;
   if (cnn_set_topology(H->cnn, H->nb, C.nbr.as<int>(), C.h.as<double>(), H->err) != 0)
     return -1;
@@ -1244,7 +1250,7 @@ int cup3d_debug_time_kernel(cup3d_poisson_t H, int which, int reps, double* avg_
       switch (which) {
         case 0: launch_spmv64(s, SPMV_PLAIN, H->g64, v.z1, v.nu, nullptr, nullptr, nullptr, st, part); break;
         case 1: launch_precond_fp64(H, H->g64, PREC_PLAIN, v); break;
-        case 2: launch_update64(s, H->n, v, st, part); break;
+        case 2: launch_update64(s, H->g64, v, st, part); break;
         case 3: launch_precond_fp64(H, H->g64, PREC_P, v); break;
         default: launch_spmv64(s, SPMV_DOT1, H->g64, v.z1, v.nu, v.rhat, nullptr, nullptr, st, part); break;
       }

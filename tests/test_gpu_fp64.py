@@ -475,3 +475,26 @@ def test_c5_full_size_first_iterations_match_oracle(gpu):
             want = np.asarray(fx["x10_values"])
             assert np.abs(got - want).max() <= 1e-8 * np.abs(want).max()
         del S, x
+
+
+@pytest.mark.parametrize("bmean", [0, 1, 3])
+@pytest.mark.parametrize("bpd", [(1, 1, 1), (3, 1, 1), (5, 1, 1), (7, 5, 8), (32, 16, 17)])
+def test_capped_solve_across_block_counts(gpu, bpd, bmean):
+    """Three iterations of the FP64 form from a zero guess at block counts where
+    the sums of an iteration change hands: one workgroup, a partly filled one,
+    two, 280, and 8704 blocks (finalize kernels instead of sums in the
+    consumers), with and without the mean-constraint row. The oracle's iterate
+    after the same iterations to 1e-10, as in the first-iterations tests; two
+    runs agree bitwise."""
+    blocks, bpd, h0, bc = uniform(bpd, (WALL,) * 3)
+    n = len(blocks) * 512
+    S = PoissonSolver(bpd, h0, bc, bmean=bmean, tol_rel=0.0, max_iter=3).set_topology(blocks)
+    b = compatible_rhs(blocks, h0, 5)
+    x = torch.zeros(n, dtype=torch.float64, device=gpu)
+    rep = S.solve_device(dev(b), x)
+    x2 = torch.zeros_like(x)
+    S.solve_device(dev(b), x2)
+    assert rep["iterations"] == 3 and rep["status"] == 1
+    assert torch.equal(x, x2)
+    xo, info = pyoracle.Oracle(blocks, bpd, h0, bc, bmean).bicgstab(b, tol_rel=0.0, max_iter=3)
+    assert np.linalg.norm(x.cpu().numpy() - xo) <= 1e-10 * np.linalg.norm(xo)
