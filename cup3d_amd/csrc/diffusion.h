@@ -11,21 +11,14 @@
 
 namespace cup3d {
 
-// Table of the DST block inverse (DST_TABLE doubles, device-resident for the
-// kernels): S1[k][i] = sqrt(2/9) sin(pi (k+1)(i+1) / 9) row-major, then the
-// eigenvalues l_k = 2 cos(pi (k+1) / 9) - 2 of the zero-padded 1-D second
-// difference.
-constexpr int DST_TABLE = BS * BS + BS;
-void dst_tables(double* tab, float* tab32);  // FP64 table and its FP32 rounding
-
 // mode PREC_P / PREC_S / PREC_PLAIN; h per block, sigma = 1 / (nu dt); fin and
 // f: whether and from where the kernel takes its scalars' sums.
-void launch_precond_dst(hipStream_t s, int mode, int nb, const double* tab, const double* h,
+void launch_precond_dst(hipStream_t s, int mode, int nb, const double* h,
                         double sigma, const KrylovVectors<double>& v, SolverState* st,
                         int fin = FIN_KERNEL, const FinArgs& f = FinArgs());
 // The same in FP32 for the mixed forms' inner solve (sigma = 0: the pressure
 // equation's block inverse h^-1 P_inv).
-void launch_precond_dst32(hipStream_t s, int mode, int nb, const float* tab, const float* h,
+void launch_precond_dst32(hipStream_t s, int mode, int nb, const float* h,
                           const KrylovVectors<float>& v, SolverState* st,
                           int fin = FIN_KERNEL, const FinArgs& f = FinArgs());
 // u = vel[:, comp], a = -h^3 sigma vel_old[:, comp] (vel, vel_old: [n][3]).

@@ -18,11 +18,17 @@
 // matrices, and the kernel is bound by HBM like the vector updates it is
 // fused with.
 //
-// One wavefront per block, lane = (ix, iy), each lane holding its z column:
-// the z transform runs in registers, the y and x transforms through this
-// wavefront's own LDS slice (rows padded to 9 doubles so the x-transform
-// reads of the eight rows fall in distinct banks), so the wavefront
-// synchronises only with itself.
+// One wavefront per block. Every 1-D transform runs on eight values in one
+// lane's registers: the z transforms on the column of lane (ix, iy), the y and
+// x transforms after a transposition through the wavefront's own LDS slice
+// (eight writes and eight reads a lane; rows padded to 9 values and planes to
+// 72, so that the reads along x and along y fall in distinct banks), and the
+// wavefront synchronises only with itself. S1 has four distinct magnitudes and
+// S1[k][7-i] = (-1)^k S1[k][i], so a transform is 8 additions and 32
+// multiplications by literals, and no table is read.
+// Transforming y and x with one LDS read per product, S1 in scalar registers
+// (64 of them spilled) and eight divisions a lane instead, K1 on 64 blocks, one
+// wavefront's latency, took 9.2 us; now 6.4 us (8192 blocks: 34.2 -> 31.7 us).
 
 #include <hip/hip_runtime.h>
 
@@ -37,78 +43,100 @@ constexpr int DL_ROW = 9;               // padded row (ix) stride, values
 constexpr int DL_PLANE = BS * DL_ROW;   // one z plane (or z mode)
 constexpr int DL_WAVE = BS * DL_PLANE;  // one wavefront's slice
 
-// out[k] = sum_i S[k][i] in[i] (S symmetric: also the inverse transform);
-// the table index is the same in every lane (scalar loads)
+// sqrt(2/9) sin(pi m / 9), m = 1..4, and the eigenvalues 2 cos(pi (k+1) / 9) - 2
+constexpr double DST_C[4] = {0.1612298417653168423518581, 0.3030129851146957862456487,
+                             0.4082482904638630163662140, 0.4642428268800126285975068};
+__device__ constexpr double DST_L[BS] = {
+    -0.1206147584281832318917814, -0.4679111137620439295952147, -1.0,
+    -1.652703644666139302296567,  -2.347296355333860697703433,  -3.0,
+    -3.532088886237956070404785,  -3.879385241571816768108219};
+
+__device__ constexpr double dst_entry(int k, int i) {  // S1[k][i]
+  int m = (k + 1) * (i + 1) % 18;
+  double sign = 1.0;
+  if (m > 9) {
+    m = 18 - m;
+    sign = -1.0;
+  }
+  if (m > 4) m = 9 - m;
+  return m == 0 ? 0.0 : sign * DST_C[m - 1];
+}
+
+// v = S1 v (S1 symmetric and orthogonal: also the inverse transform)
 template <typename T>
-__device__ __forceinline__ void dst8(const T* __restrict__ S, const T (&in)[BS], T (&out)[BS]) {
+__device__ __forceinline__ void dst8(T (&v)[BS]) {
+  T e[2][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    e[0][i] = v[i] + v[7 - i];
+    e[1][i] = v[i] - v[7 - i];
+  }
 #pragma unroll
   for (int k = 0; k < BS; ++k) {
-    T acc = 0;
+    T acc = (T)dst_entry(k, 0) * e[k & 1][0];
 #pragma unroll
-    for (int i = 0; i < BS; ++i) acc = fma(S[k * BS + i], in[i], acc);
-    out[k] = acc;
+    for (int i = 1; i < 4; ++i)
+      if (dst_entry(k, i) != 0.0) acc = fma((T)dst_entry(k, i), e[k & 1][i], acc);
+    v[k] = acc;
   }
 }
 
-// Transform along y (AXIS 1) or x (AXIS 0) of the eight planes held in the
-// slice L: this lane (a, c) = (lane & 7, lane >> 3) produces, for every z
-// plane k, the value at output index c (y) or a (x); row holds S[c][*] or
-// S[a][*] in registers.
-template <int AXIS, typename T>
-__device__ __forceinline__ void dst_lds(const T (&row)[BS], const T* L, int lane, T (&out)[BS]) {
-  const int a = lane & 7, c = lane >> 3;
+// The lane's values to and from the slice, strides in values: index j of the
+// lane's axis at base + j * stride.
+template <int STRIDE, typename T>
+__device__ __forceinline__ void put8(T* L, int base, const T (&v)[BS]) {
 #pragma unroll
-  for (int k = 0; k < BS; ++k) {
-    T acc = 0;
+  for (int j = 0; j < BS; ++j) L[base + j * STRIDE] = v[j];
+  wave_sync();
+}
+template <int STRIDE, typename T>
+__device__ __forceinline__ void get8(const T* L, int base, T (&v)[BS]) {
 #pragma unroll
-    for (int j = 0; j < BS; ++j) {
-      const T v = AXIS == 1 ? L[k * DL_PLANE + j * DL_ROW + a] : L[k * DL_PLANE + c * DL_ROW + j];
-      acc = fma(row[j], v, acc);
-    }
-    out[k] = acc;
-  }
+  for (int j = 0; j < BS; ++j) v[j] = L[base + j * STRIDE];
+  wave_sync();
 }
 
-template <typename T>
-__device__ __forceinline__ void to_lds(T* L, int lane, const T (&v)[BS]) {
-  const int a = lane & 7, c = lane >> 3;
-#pragma unroll
-  for (int k = 0; k < BS; ++k) L[k * DL_PLANE + c * DL_ROW + a] = v[k];
+// 1 / x to the last bit or two: the hardware's estimate and two Newton steps
+// (one in FP32)
+__device__ __forceinline__ double recip(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = fma(fma(-x, r, 1.0), r, r);
+  return fma(fma(-x, r, 1.0), r, r);
+}
+__device__ __forceinline__ float recip(float x) {
+  const float r = __builtin_amdgcn_rcpf(x);
+  return fmaf(fmaf(-x, r, 1.0f), r, r);
 }
 
 // z = h^-1 A_loc(sigma_b)^-1 v for the column v of this lane (in place).
-// tab: S1 (64 values, row-major) then l_0..l_7.
 template <typename T>
-__device__ __forceinline__ void dst_apply(const T* __restrict__ tab, T* L, int lane, T h,
-                                          T sigma, T (&v)[BS]) {
-  const int kx = lane & 7, ky = lane >> 3;
-  T rx[BS], ry[BS];
+__device__ __forceinline__ void dst_apply(T* L, int lane, T h, T sigma, T (&v)[BS]) {
+  const int a = lane & 7, c = lane >> 3;
+  const int zcol = c * DL_ROW + a, ycol = c * DL_PLANE + a, xrow = c * DL_PLANE + a * DL_ROW;
+  const T shift = h * h * sigma;
+  const T base = (T)DST_L[a] + (T)DST_L[c] - shift;  // of (ky, kz) = (a, c)
+  dst8(v);  // z, lane (ix, iy)
+  put8<DL_PLANE>(L, zcol, v);
+  get8<DL_ROW>(L, ycol, v);
+  dst8(v);  // y, lane (ix, kz)
+  put8<DL_ROW>(L, ycol, v);
+  get8<1>(L, xrow, v);
+  dst8(v);  // x, lane (ky, kz)
+  const T ih = (T)1 / h;
+  if (shift < (T)1e18) {  // the estimate's range; a shift beyond it divides
 #pragma unroll
-  for (int j = 0; j < BS; ++j) {
-    rx[j] = tab[kx * BS + j];
-    ry[j] = tab[ky * BS + j];
+    for (int k = 0; k < BS; ++k) v[k] *= recip(base + (T)DST_L[k]) * ih;
+  } else {
+#pragma unroll
+    for (int k = 0; k < BS; ++k) v[k] = v[k] / (h * (base + (T)DST_L[k]));
   }
-  const T base = tab[BS * BS + kx] + tab[BS * BS + ky] - h * h * sigma;
-  T w[BS];
-  dst8(tab, v, w);  // z transform: w[kz] at (ix, iy)
-  to_lds(L, lane, w);
-  wave_sync();
-  dst_lds<1>(ry, L, lane, v);  // y: v[kz] at (ix, ky)
-  wave_sync();
-  to_lds(L, lane, v);
-  wave_sync();
-  dst_lds<0>(rx, L, lane, w);  // x: w[kz] at (kx, ky)
-#pragma unroll
-  for (int k = 0; k < BS; ++k) w[k] = w[k] / (h * (base + tab[BS * BS + k]));
-  wave_sync();
-  to_lds(L, lane, w);
-  wave_sync();
-  dst_lds<0>(rx, L, lane, v);  // inverse x: v[kz] at (ix, ky)
-  wave_sync();
-  to_lds(L, lane, v);
-  wave_sync();
-  dst_lds<1>(ry, L, lane, w);  // inverse y: w[kz] at (ix, iy)
-  dst8(tab, w, v);             // inverse z: v[iz]
+  dst8(v);  // inverse x
+  put8<1>(L, xrow, v);
+  get8<DL_ROW>(L, ycol, v);
+  dst8(v);  // inverse y
+  put8<DL_ROW>(L, ycol, v);
+  get8<DL_PLANE>(L, zcol, v);
+  dst8(v);  // inverse z
 }
 
 // K1 / K3 of the classical iteration (kernels.hip) with this preconditioner,
@@ -118,10 +146,9 @@ __device__ __forceinline__ void dst_apply(const T* __restrict__ tab, T* L, int l
 //   PREC_S  s = r - alpha nu (into r); z2 = M^-1 s
 //   PREC_PLAIN  z1 = M^-1 p
 template <typename T, int MODE, int FIN>
-__global__ __launch_bounds__(WG_THREADS) void k_precond_dst(int nb, const T* __restrict__ tab,
-                                                            const T* __restrict__ hb, T sigma,
-                                                            KrylovVectors<T> v, SolverState* st,
-                                                            FinArgs f) {
+__global__ __launch_bounds__(WG_THREADS) void k_precond_dst(int nb, const T* __restrict__ hb,
+                                                            T sigma, KrylovVectors<T> v,
+                                                            SolverState* st, FinArgs f) {
   __shared__ T Ls[WG_THREADS / 64][DL_WAVE];
   __shared__ SolverState S;
   if (!FIN && MODE != PREC_PLAIN && st->status != ST_RUNNING) return;
@@ -129,14 +156,18 @@ __global__ __launch_bounds__(WG_THREADS) void k_precond_dst(int nb, const T* __r
   const int b = blockIdx.x * (WG_THREADS / 64) + w;
   const size_t off = (size_t)b * BLEN + lane;
   T c[BS], ra[BS], rb[BS];
+  // after a restart (and in the first iteration) p = r: nu and p are not read
+  const bool fresh = !FIN && MODE == PREC_P && st->p_zero;
   if (b < nb) {
 #pragma unroll
     for (int iz = 0; iz < BS; ++iz) {
       const size_t i = off + iz * 64;
       if (MODE == PREC_P) {
         ra[iz] = v.r[i];
-        rb[iz] = v.nu[i];
-        c[iz] = v.p[i];
+        if (!fresh) {
+          rb[iz] = v.nu[i];
+          c[iz] = v.p[i];
+        }
       } else if (MODE == PREC_S) {
         ra[iz] = v.r[i];
         rb[iz] = v.nu[i];
@@ -175,34 +206,34 @@ __global__ __launch_bounds__(WG_THREADS) void k_precond_dst(int nb, const T* __r
       v.r[i] = c[iz];
     }
   }
-  dst_apply<T>(tab, Ls[w], lane, hb[b], sigma, c);
+  dst_apply<T>(Ls[w], lane, hb[b], sigma, c);
   T* __restrict__ out = MODE == PREC_S ? v.z2 : v.z1;
 #pragma unroll
   for (int iz = 0; iz < BS; ++iz) out[off + iz * 64] = c[iz];
 }
 
 template <typename T, int MODE, int FIN>
-void launch_precond_dst_m(hipStream_t s, int nb, const T* tab, const T* h, T sigma,
+void launch_precond_dst_m(hipStream_t s, int nb, const T* h, T sigma,
                           const KrylovVectors<T>& v, SolverState* st, const FinArgs& f) {
   const int nwg = (nb + WG_THREADS / 64 - 1) / (WG_THREADS / 64);
-  k_precond_dst<T, MODE, FIN><<<nwg, WG_THREADS, 0, s>>>(nb, tab, h, sigma, v, st, f);
+  k_precond_dst<T, MODE, FIN><<<nwg, WG_THREADS, 0, s>>>(nb, h, sigma, v, st, f);
 }
 
 template <typename T>
-void launch_precond_dst_t(hipStream_t s, int mode, int nb, const T* tab, const T* h, T sigma,
+void launch_precond_dst_t(hipStream_t s, int mode, int nb, const T* h, T sigma,
                           const KrylovVectors<T>& v, SolverState* st, int fin, const FinArgs& f) {
   if (mode == PREC_P && fin)
-    launch_precond_dst_m<T, PREC_P, FIN_SUMS>(s, nb, tab, h, sigma, v, st, f);
+    launch_precond_dst_m<T, PREC_P, FIN_SUMS>(s, nb, h, sigma, v, st, f);
   else if (mode == PREC_P)
-    launch_precond_dst_m<T, PREC_P, FIN_KERNEL>(s, nb, tab, h, sigma, v, st, f);
+    launch_precond_dst_m<T, PREC_P, FIN_KERNEL>(s, nb, h, sigma, v, st, f);
   else if (mode == PREC_S && fin == FIN_ROW)
-    launch_precond_dst_m<T, PREC_S, FIN_ROW>(s, nb, tab, h, sigma, v, st, f);
+    launch_precond_dst_m<T, PREC_S, FIN_ROW>(s, nb, h, sigma, v, st, f);
   else if (mode == PREC_S && fin)
-    launch_precond_dst_m<T, PREC_S, FIN_SUMS>(s, nb, tab, h, sigma, v, st, f);
+    launch_precond_dst_m<T, PREC_S, FIN_SUMS>(s, nb, h, sigma, v, st, f);
   else if (mode == PREC_S)
-    launch_precond_dst_m<T, PREC_S, FIN_KERNEL>(s, nb, tab, h, sigma, v, st, f);
+    launch_precond_dst_m<T, PREC_S, FIN_KERNEL>(s, nb, h, sigma, v, st, f);
   else
-    launch_precond_dst_m<T, PREC_PLAIN, FIN_KERNEL>(s, nb, tab, h, sigma, v, st, f);
+    launch_precond_dst_m<T, PREC_PLAIN, FIN_KERNEL>(s, nb, h, sigma, v, st, f);
 }
 
 // Component c of the velocity into the solver's vectors: u = u*_c and
@@ -232,26 +263,16 @@ __global__ __launch_bounds__(WG_THREADS) void k_diff_scatter(long long n, int co
 
 }  // namespace
 
-void dst_tables(double* tab, float* tab32) {
-  const double pi = 3.14159265358979323846;
-  for (int k = 0; k < BS; ++k) {
-    tab[BS * BS + k] = 2.0 * std::cos(pi * (k + 1) / 9.0) - 2.0;
-    for (int i = 0; i < BS; ++i)
-      tab[k * BS + i] = std::sqrt(2.0 / 9.0) * std::sin(pi * (k + 1) * (i + 1) / 9.0);
-  }
-  for (int i = 0; i < DST_TABLE; ++i) tab32[i] = (float)tab[i];
-}
-
-void launch_precond_dst(hipStream_t s, int mode, int nb, const double* tab, const double* h,
+void launch_precond_dst(hipStream_t s, int mode, int nb, const double* h,
                         double sigma, const KrylovVectors<double>& v, SolverState* st, int fin,
                         const FinArgs& f) {
-  launch_precond_dst_t<double>(s, mode, nb, tab, h, sigma, v, st, fin, f);
+  launch_precond_dst_t<double>(s, mode, nb, h, sigma, v, st, fin, f);
 }
 
-void launch_precond_dst32(hipStream_t s, int mode, int nb, const float* tab, const float* h,
+void launch_precond_dst32(hipStream_t s, int mode, int nb, const float* h,
                           const KrylovVectors<float>& v, SolverState* st, int fin,
                           const FinArgs& f) {
-  launch_precond_dst_t<float>(s, mode, nb, tab, h, 0.0f, v, st, fin, f);
+  launch_precond_dst_t<float>(s, mode, nb, h, 0.0f, v, st, fin, f);
 }
 
 void launch_diffusion_gather(hipStream_t s, long long n, int comp, const double* h3, double sigma,

@@ -519,7 +519,7 @@ void launch_precond_mixed(const MixedWorkspace& M, hipStream_t s, int precision,
       v.p = const_cast<float*>(pin);
       v.z1 = pout;
     }
-    launch_precond_dst32(s, mode, g.nb, M.dst32, g.h, v, st, fin, f);
+    launch_precond_dst32(s, mode, g.nb, g.h, v, st, fin, f);
     return;
   }
   if (precision == CUP3D_PREC_MIXED_FP16)

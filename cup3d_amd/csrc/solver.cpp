@@ -106,8 +106,6 @@ struct cup3d_poisson {
 
   // preconditioner
   std::vector<double> P;
-  DevBuf d_dst;    // DST block-inverse table (DST_TABLE doubles): FP64 forms, implicit diffusion
-  DevBuf d_dst32;  // its FP32 rounding (the mixed forms' inner solve with cfg.precond = DST)
 
   // FP64 Krylov workspace
   DevBuf d_vec64;  // 11 vectors of n doubles
@@ -181,25 +179,18 @@ SolverState make_state(const cup3d_poisson_config& c) {
   return s;
 }
 
-int upload(cup3d_poisson* H, DevBuf& d, const void* src, size_t bytes) {
-  if (d.alloc(bytes) != hipSuccess) return fail(H, "hipMalloc failed (" + std::to_string(bytes) + " bytes)");
-  if (bytes && hipMemcpy(d.p, src, bytes, hipMemcpyHostToDevice) != hipSuccess)
-    return fail(H, "hipMemcpy H2D failed");
-  return 0;
-}
-
 // M^-1 in FP64: the exact block inverse in factored form, three sine transforms,
 // the eigenvalues and three more (96 flops a cell), for both settings of
 // cfg.precond and for Helmholtz grids. The dense 512 x 512 product it replaces
 // is the same matrix at 1024 flops a cell, bound by the FP64 matrix cores:
-// fused with the p update, K1 took 98.9 us that way and takes 34.2 us now on
-// 4.19 M cells (168 MB of vectors, 4.9 TB/s), 43 us (four workgroups) and
-// 5 us on 32 k cells.
+// fused with the p update, K1 took 98.9 us that way and takes 31.7 us now on
+// 4.19 M cells (168 MB of vectors, 5.3 TB/s), 43 us (four workgroups) and
+// 6.4 us on 32 k cells.
 void launch_precond_fp64(cup3d_poisson* H, const DevGrid<double>& g, int mode,
                          const KrylovVectors<double>& v, int fin = FIN_KERNEL,
                          const FinArgs& f = FinArgs()) {
   SolverState* st = H->d_state.as<SolverState>();
-  launch_precond_dst(H->stream, mode, H->nb, H->d_dst.as<double>(), g.h,
+  launch_precond_dst(H->stream, mode, H->nb, g.h,
                      g.helm ? g.helm_sigma : 0.0, v, st, fin, f);
 }
 
@@ -313,19 +304,13 @@ int cup3d_poisson_create(const cup3d_poisson_config* cfg, cup3d_poisson_t* out) 
     g_create_error = "HIP stream/event/pinned allocation failed";
     return -1;
   }
-  // block-Jacobi inverse (PoissonSolverExp ctor): the dense matrix for the
-  // half-precision GEMM, the sine-transform table for the rest
+  // block-Jacobi inverse (PoissonSolverExp ctor): the dense matrix of the
+  // half-precision GEMM
   build_pinv_dst(H->P);
-  double dtab[DST_TABLE];
-  float dtab32[DST_TABLE];
-  dst_tables(dtab, dtab32);
-  if (upload(H.get(), H->d_dst, dtab, sizeof(dtab)) != 0 ||
-      upload(H.get(), H->d_dst32, dtab32, sizeof(dtab32)) != 0 ||
-      mixed_init_pinv(H->mixed, H->P, H->err) != 0 || cnn_init(H->cnn, H->err) != 0) {
+  if (mixed_init_pinv(H->mixed, H->P, H->err) != 0 || cnn_init(H->cnn, H->err) != 0) {
     g_create_error = H->err;
     return -1;
   }
-  H->mixed.dst32 = H->d_dst32.as<float>();
   if (H->d_state.alloc(STATE_COPIES * sizeof(SolverState)) != hipSuccess) {
     g_create_error = "hipMalloc(state) failed";
     return -1;
@@ -1107,7 +1092,7 @@ int cup3d_diffusion_apply_preconditioner(cup3d_poisson_t H, double nu, double dt
   KrylovVectors<double> v = H->v64;
   v.p = const_cast<double*>(d_p);
   v.z1 = d_z;
-  launch_precond_dst(H->stream, PREC_PLAIN, H->nb, H->d_dst.as<double>(), g.h, g.helm_sigma, v,
+  launch_precond_dst(H->stream, PREC_PLAIN, H->nb, g.h, g.helm_sigma, v,
                      H->d_state.as<SolverState>());
   HIPCHECK(hipGetLastError());
   HIPCHECK(hipStreamSynchronize(H->stream));
@@ -1298,7 +1283,7 @@ int cup3d_debug_time_diffusion_kernel(cup3d_poisson_t H, int which, double nu, d
     if (which == 0)
       launch_spmv64(s, SPMV_PLAIN, g, v.z1, v.nu, nullptr, nullptr, nullptr, st, part);
     else
-      launch_precond_dst(s, which == 1 ? PREC_P : PREC_PLAIN, H->nb, H->d_dst.as<double>(), g.h,
+      launch_precond_dst(s, which == 1 ? PREC_P : PREC_PLAIN, H->nb, g.h,
                          g.helm_sigma, v, st);
   };
   launch();  // warm
