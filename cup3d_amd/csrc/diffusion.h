@@ -1,5 +1,5 @@
 // Implicit diffusion kernels (diffusion.hip): the DST block preconditioner
-// and the velocity gather/scatter of a diffusion step.
+// and the velocity update of a diffusion step.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -21,11 +21,7 @@ void launch_precond_dst(hipStream_t s, int mode, int nb, const double* h,
 void launch_precond_dst32(hipStream_t s, int mode, int nb, const float* h,
                           const KrylovVectors<float>& v, SolverState* st,
                           int fin = FIN_KERNEL, const FinArgs& f = FinArgs());
-// u = vel[:, comp], a = -h^3 sigma vel_old[:, comp] (vel, vel_old: [n][3]).
-void launch_diffusion_gather(hipStream_t s, long long n, int comp, const double* h3, double sigma,
-                             const double* vel, const double* vel_old, double* u, double* a);
-// vel[:, comp] += x.
-void launch_diffusion_scatter(hipStream_t s, long long n, int comp, const double* x,
-                              double* vel);
+// vel[:, c] += x[c] (null: 0) for the three components of an [n][3] field.
+void launch_diffusion_add(hipStream_t s, long long n, const double* const x[3], double* vel);
 
 }  // namespace cup3d

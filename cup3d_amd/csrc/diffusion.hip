@@ -236,29 +236,23 @@ void launch_precond_dst_t(hipStream_t s, int mode, int nb, const T* h, T sigma,
     launch_precond_dst_m<T, PREC_PLAIN, FIN_KERNEL>(s, nb, h, sigma, v, st, f);
 }
 
-// Component c of the velocity into the solver's vectors: u = u*_c and
-// a = -h^3 sigma u^n_c (the operator's residual a - A u is then the step's
-// rhs, see launch_diffusion_gather).
-__global__ __launch_bounds__(WG_THREADS) void k_diff_gather(long long n, int comp,
-                                                            const double* __restrict__ h3,
-                                                            double sigma,
-                                                            const double* __restrict__ vel,
-                                                            const double* __restrict__ vel_old,
-                                                            double* __restrict__ u,
-                                                            double* __restrict__ a) {
+// u* += the three solutions (AdvectionDiffusionImplicit.cpp:407-418), two
+// cells (three 16-byte accesses) per thread; a null solution is 0.
+__global__ __launch_bounds__(WG_THREADS) void k_diff_add(long long n, const double* __restrict__ x,
+                                                         const double* __restrict__ y,
+                                                         const double* __restrict__ z,
+                                                         double* __restrict__ vel) {
+  typedef double double2_t __attribute__((ext_vector_type(2)));
   const long long i = (long long)blockIdx.x * WG_THREADS + threadIdx.x;
-  if (i >= n) return;
-  u[i] = vel[3 * i + comp];
-  a[i] = -h3[i / BLEN] * sigma * vel_old[3 * i + comp];
-}
-
-// u*_c += x (AdvectionDiffusionImplicit.cpp:407-418).
-__global__ __launch_bounds__(WG_THREADS) void k_diff_scatter(long long n, int comp,
-                                                             const double* __restrict__ x,
-                                                             double* __restrict__ vel) {
-  const long long i = (long long)blockIdx.x * WG_THREADS + threadIdx.x;
-  if (i >= n) return;
-  vel[3 * i + comp] += x[i];
+  if (2 * i >= n) return;
+  const double2_t zero = {0.0, 0.0};
+  const double2_t a = x ? reinterpret_cast<const double2_t*>(x)[i] : zero;
+  const double2_t b = y ? reinterpret_cast<const double2_t*>(y)[i] : zero;
+  const double2_t c = z ? reinterpret_cast<const double2_t*>(z)[i] : zero;
+  double2_t* __restrict__ v = reinterpret_cast<double2_t*>(vel) + 3 * i;
+  v[0] += (double2_t){a.x, b.x};
+  v[1] += (double2_t){c.x, a.y};
+  v[2] += (double2_t){b.y, c.y};
 }
 
 }  // namespace
@@ -275,16 +269,9 @@ void launch_precond_dst32(hipStream_t s, int mode, int nb, const float* h,
   launch_precond_dst_t<float>(s, mode, nb, h, 0.0f, v, st, fin, f);
 }
 
-void launch_diffusion_gather(hipStream_t s, long long n, int comp, const double* h3, double sigma,
-                             const double* vel, const double* vel_old, double* u, double* a) {
-  const int nwg = (int)((n + WG_THREADS - 1) / WG_THREADS);
-  k_diff_gather<<<nwg, WG_THREADS, 0, s>>>(n, comp, h3, sigma, vel, vel_old, u, a);
-}
-
-void launch_diffusion_scatter(hipStream_t s, long long n, int comp, const double* x,
-                              double* vel) {
-  const int nwg = (int)((n + WG_THREADS - 1) / WG_THREADS);
-  k_diff_scatter<<<nwg, WG_THREADS, 0, s>>>(n, comp, x, vel);
+void launch_diffusion_add(hipStream_t s, long long n, const double* const x[3], double* vel) {
+  const int nwg = (int)((n / 2 + WG_THREADS - 1) / WG_THREADS);
+  k_diff_add<<<nwg, WG_THREADS, 0, s>>>(n, x[0], x[1], x[2], vel);
 }
 
 }  // namespace cup3d

@@ -9,7 +9,16 @@
 
 namespace cup3d {
 
-enum SpmvMode { SPMV_PLAIN = 0, SPMV_INIT = 1, SPMV_DOT1 = 2, SPMV_DOT2 = 3, SPMV_RESID = 4 };
+// PLAIN  y = A x                       INIT   y = A x, c = c2 = a - y, |y|^2, |c|^2
+// DOT1   y = A x, (a, y)               DOT2   y = A x, (a, y), (y, y)
+// RESID  c = a - A x, |c|^2
+// START  y = c = c2 = -h^3 sigma a - A x, its norm (Helmholtz grids; x and a are
+//        one component of an [n][3] field)
+// FINAL  |a - A x|^2 of the best iterate x (g.xo, the state), copied to y (may be null)
+enum SpmvMode {
+  SPMV_PLAIN = 0, SPMV_INIT = 1, SPMV_DOT1 = 2, SPMV_DOT2 = 3, SPMV_RESID = 4, SPMV_START = 5,
+  SPMV_FINAL = 6
+};
 enum PrecMode { PREC_PLAIN = 0, PREC_P = 1, PREC_S = 2 };
 
 // Where the scalars of an iteration are computed: by finalize kernels, or by
@@ -33,19 +42,27 @@ inline double* k5_part(double* part, int nb) { return part + 4 * (size_t)((nb + 
 // Copies of the solver state (krylov.h): st[0] is the one the host reads.
 constexpr int STATE_COPIES = 3;
 
+// The state starts as `init`, with ||b|| and the absolute tolerance.
 void launch_getvec64(hipStream_t s, long long n, long long zero_row, const double* rhs,
-                     const double* x0, double* b, double* x, SolverState* st, double* part,
-                     double tol_b);
-// part null (SPMV_PLAIN and SPMV_RESID on a grid with bMean 0 or 3): no sums are
-// taken and st is not used.
+                     const double* x0, double* b, double* x, const SolverState& init,
+                     SolverState* st, double* part, double tol_b);
+// The same and the initial residual for x0 = 0: b = r = rhat = rhs (zero in the
+// bMean cell; rhat may be null), x = 0 unless null, and the first iteration's
+// scalars.
+void launch_start_zero64(hipStream_t s, int nb, long long zero_row, const double* rhs, double* b,
+                         double* r, double* rhat, double* x, const SolverState& init,
+                         SolverState* st, double* part, double tol_b);
+// The scalars of SPMV_START (nb blocks).
+void launch_start_fin(hipStream_t s, int nb, const SolverState& init, SolverState* st,
+                      const double* part, double tol_b);
+// part null (SPMV_PLAIN and SPMV_RESID on a grid with bMean 0 or 3, SPMV_FINAL for
+// its copy): no sums are taken.
 void launch_spmv64(hipStream_t s, int mode, const DevGrid<double>& g, const double* x, double* y,
                    const double* a, double* c, double* c2, SolverState* st, double* part,
                    bool fin = true);
 // K5; returns its number of partials. last: with its finalize kernel.
 int launch_update64(hipStream_t s, const DevGrid<double>& g, const KrylovVectors<double>& v,
                     SolverState* st, double* part, int fin = FIN_KERNEL, bool last = true);
-void launch_copy_opt64(hipStream_t s, long long n, const KrylovVectors<double>& v,
-                       const SolverState* st, double* out);
 
 // The caller around the solve (projection.hip): the rhs of the pressure
 // equation from the velocity (and an obstacle's udef / chi, both or neither

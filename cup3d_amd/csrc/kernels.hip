@@ -30,11 +30,23 @@ namespace cup3d {
 // Host launchers
 // ---------------------------------------------------------------------------
 void launch_getvec64(hipStream_t s, long long n, long long zero_row, const double* rhs,
-                     const double* x0, double* b, double* x, SolverState* st, double* part,
-                     double tol_b) {
+                     const double* x0, double* b, double* x, const SolverState& init,
+                     SolverState* st, double* part, double tol_b) {
   const int nwg = (int)((n + 4 * BLEN - 1) / (4 * BLEN));
-  k_getvec<double><<<nwg, WG_THREADS, 0, s>>>(n, zero_row, rhs, x0, b, x, st, part, tol_b);
-  k_getvec_fin<<<1, WG_THREADS, 0, s>>>(st, part, nwg, tol_b);
+  k_getvec<<<nwg, WG_THREADS, 0, s>>>(n, zero_row, rhs, x0, b, x, part);
+  k_getvec_fin<<<1, WG_THREADS, 0, s>>>(init, st, part, nwg, tol_b);
+}
+
+void launch_start_zero64(hipStream_t s, int nb, long long zero_row, const double* rhs, double* b,
+                         double* r, double* rhat, double* x, const SolverState& init,
+                         SolverState* st, double* part, double tol_b) {
+  k_start_zero<<<(nb + 3) / 4, WG_THREADS, 0, s>>>(nb, zero_row, rhs, b, r, rhat, x, part);
+  launch_start_fin(s, nb, init, st, part, tol_b);
+}
+
+void launch_start_fin(hipStream_t s, int nb, const SolverState& init, SolverState* st,
+                      const double* part, double tol_b) {
+  k_start_fin<<<1, WG_THREADS, 0, s>>>(init, st, part, (nb + 3) / 4, tol_b);
 }
 
 void launch_spmv64(hipStream_t s, int mode, const DevGrid<double>& g, const double* x, double* y,
@@ -46,18 +58,14 @@ void launch_spmv64(hipStream_t s, int mode, const DevGrid<double>& g, const doub
     case SPMV_DOT1: spmv_launch<double, SPMV_DOT1>(s, g, x, y, a, c, c2, st, part, fin); break;
     case SPMV_DOT2: spmv_launch<double, SPMV_DOT2>(s, g, x, y, a, c, c2, st, part, fin); break;
     case SPMV_RESID: spmv_launch<double, SPMV_RESID>(s, g, x, y, a, c, c2, st, part, fin); break;
+    case SPMV_START: spmv_launch<double, SPMV_START>(s, g, x, y, a, c, c2, st, part, false); break;
+    case SPMV_FINAL: spmv_launch<double, SPMV_FINAL>(s, g, x, y, a, c, c2, st, part, fin); break;
   }
 }
 
 int launch_update64(hipStream_t s, const DevGrid<double>& g, const KrylovVectors<double>& v,
                     SolverState* st, double* part, int fin, bool last) {
   return launch_k5<double>(s, g, v, st, part, fin, last);
-}
-
-void launch_copy_opt64(hipStream_t s, long long n, const KrylovVectors<double>& v,
-                       const SolverState* st, double* out) {
-  const int nwg = (int)std::min<long long>((n + WG_THREADS - 1) / WG_THREADS, 4096);
-  k_copy_opt<double><<<nwg, WG_THREADS, 0, s>>>(n, v, st, out);
 }
 
 // ---------------------------------------------------------------------------

@@ -176,46 +176,87 @@ __device__ __forceinline__ void store8(T* __restrict__ p, const T (&v)[8]) {
 }
 
 // ---------------------------------------------------------------------------
-// getVec (PoissonSolverExp.cpp:375-418): b = rhs, x = x0, both zeroed at the
-// bMean cell for bMeanConstraint 1 and 3; also ||b||^2.
+// getVec (PoissonSolverExp.cpp:375-418): b = rhs, x = x0 (may be the same
+// vector), both zeroed at the bMean cell for bMeanConstraint 1 and 3; also
+// ||b||^2.
 // ---------------------------------------------------------------------------
-template <typename T>
-__global__ __launch_bounds__(WG_THREADS) void k_getvec(long long n, long long zero_row,
-                                                       const double* __restrict__ rhs,
-                                                       const double* __restrict__ x0,
-                                                       T* __restrict__ b, T* __restrict__ x,
-                                                       SolverState* st, double* part,
-                                                       double tol_b) {
+[[maybe_unused]] static __global__ __launch_bounds__(WG_THREADS) void k_getvec(
+    long long n, long long zero_row, const double* __restrict__ rhs, const double* x0,
+    double* __restrict__ b, double* x, double* part) {
   double v[1] = {0.0};
   const long long i0 = (long long)blockIdx.x * (4 * BLEN) + 8 * threadIdx.x;
   if (i0 < n) {
     double bv[8], xv[8];
     load8(rhs + i0, bv);
-    if (x0) load8(x0 + i0, xv);
-    T bo[8], xo[8];
+    const bool copy = x != x0 || (zero_row >= i0 && zero_row < i0 + 8);
+    if (x0 && copy) load8(x0 + i0, xv);
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       if (!x0) xv[e] = 0.0;
       if (i0 + e == zero_row) bv[e] = xv[e] = 0.0;
-      bo[e] = (T)bv[e];
-      xo[e] = (T)xv[e];
       v[0] += bv[e] * bv[e];
     }
-    store8(b + i0, bo);
-    store8(x + i0, xo);
+    store8(b + i0, bv);
+    if (copy) store8(x + i0, xv);
   }
   grid_store_partial<1>(v, part);
 }
 
+// ||b|| and the absolute tolerance it sets, into a fresh state.
 [[maybe_unused]] static __global__ __launch_bounds__(WG_THREADS) void k_getvec_fin(
-    SolverState* st, const double* part, int nparts, double tol_b) {
+    SolverState init, SolverState* st, const double* part, int nparts, double tol_b) {
   __shared__ SolverState S;
   double tot[1];
-  fin_load<1>(st, S, part, nparts, tot);
+  grid_sum_partials<1>(part, nparts, tot);
   if (threadIdx.x == 0) {
+    S = init;
     S.bnorm2 = tot[0];
-    const double tb = tol_b * sqrt(tot[0]);
-    if (tb > S.tol_abs) S.tol_abs = tb;
+    S.tol_abs = fmax(S.tol_abs, tol_b * sqrt(tot[0]));
+  }
+  fin_store(st, S);
+}
+
+// Start from x0 = 0: b = r = rhat = rhs without an operator application. The
+// sum is taken as the SpMV's residual mode takes it (a column of eight cells
+// per lane), so |r| has the same bits as through A x0.
+[[maybe_unused]] static __global__ __launch_bounds__(WG_THREADS) void k_start_zero(
+    int nb, long long zero_row, const double* __restrict__ rhs, double* __restrict__ b,
+    double* __restrict__ r, double* __restrict__ rhat, double* __restrict__ x, double* part) {
+  double v[1] = {0.0};
+  const int blk = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (blk < nb) {
+    const long long off = (long long)blk * BLEN + (threadIdx.x & 63);
+    double q[BS];
+#pragma unroll
+    for (int iz = 0; iz < BS; ++iz) q[iz] = rhs[off + iz * 64];
+#pragma unroll
+    for (int iz = 0; iz < BS; ++iz) {
+      const long long i = off + iz * 64;
+      if (i == zero_row) q[iz] = 0.0;
+      b[i] = q[iz];
+      r[i] = q[iz];
+      if (rhat) rhat[i] = q[iz];
+      if (x) x[i] = 0.0;
+      v[0] += q[iz] * q[iz];
+    }
+  }
+  grid_store_partial<1>(v, part);
+}
+
+// The first iteration's scalars for a zero guess, |b|^2 = |r|^2 = the sum.
+[[maybe_unused]] static __global__ __launch_bounds__(WG_THREADS) void k_start_fin(
+    SolverState init, SolverState* st, const double* part, int nparts, double tol_b) {
+  __shared__ SolverState S;
+  double tot[1];
+  grid_sum_partials<1>(part, nparts, tot);
+  if (threadIdx.x == 0) {
+    S = init;
+    S.bnorm2 = S.true_rr = S.rhrh = tot[0];
+    S.tol_abs = fmax(S.tol_abs, tol_b * sqrt(tot[0]));
+    S.nu2 = 0.0;
+    S.err = S.err_init = S.err_opt = sqrt(tot[0]);
+    S.x_zero = S.opt_zero = 1;
+    begin_iteration(&S, tot[0], tot[0]);
   }
   fin_store(st, S);
 }
@@ -288,7 +329,7 @@ __device__ __forceinline__ size_t coarse_plane_index(int f, int cb, int lane) {
   return (size_t)cb * BLEN + (minus ? 7 : 0) * sd + (lane & 7) * st1 + (lane >> 3) * st2;
 }
 
-template <typename T>
+template <typename T, int XS>
 __device__ __forceinline__ void iface_face(const DevGrid<T>& g, const T* __restrict__ x,
                                            const T* xs, T* pl, T* ys, int b, int f, int fk,
                                            int par, int lane, int nb0, int nbq, bool have_plane,
@@ -307,7 +348,7 @@ __device__ __forceinline__ void iface_face(const DevGrid<T>& g, const T* __restr
   if (fk == FACE_COARSE) {
     // stage the coarse block's face layer, [t2][t1] (prefetched by the
     // caller for the first two such faces)
-    pl[lane] = have_plane ? plane : x[coarse_plane_index(f, nb0, lane)];
+    pl[lane] = have_plane ? plane : x[coarse_plane_index(f, nb0, lane) * XS];
     wave_sync();
     const T h = g.h[b];
     const int c1 = (u >> 1) + (((par >> t1) & 1) ? BS / 2 : 0);
@@ -330,8 +371,8 @@ __device__ __forceinline__ void iface_face(const DevGrid<T>& g, const T* __restr
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int f1 = (u & 3) * 2 + (q & 1), f2 = (v & 3) * 2 + (q >> 1);
-      xfc[q] = x[fo + lc * sd + f1 * st1 + f2 * st2];
-      xff[q] = x[fo + lf * sd + f1 * st1 + f2 * st2];
+      xfc[q] = x[(fo + lc * sd + f1 * st1 + f2 * st2) * XS];
+      xff[q] = x[(fo + lf * sd + f1 * st1 + f2 * st2) * XS];
     }
     // The four fine ghosts share this cell's Taylor expansion and differ in
     // the signs s1, s2 = +-1 of the first-derivative and mixed terms, which
@@ -404,15 +445,16 @@ template <int MODE, int BM>
 struct SpmvSums {
   static constexpr int MEAN = BM == 1 || BM == 2 ? 1 : 0;
   static constexpr int DOTS =
-      MODE == SPMV_PLAIN ? 0 : (MODE == SPMV_DOT1 || MODE == SPMV_RESID ? 1 : 2);
+      MODE == SPMV_PLAIN ? 0 : (MODE == SPMV_INIT || MODE == SPMV_DOT2 ? 2 : 1);
   static constexpr int N = MEAN + DOTS;
 };
 
 template <typename T, int MODE, int BM, bool IFACE, bool HELM = false, bool NT = false>
-__global__ __launch_bounds__(WG_THREADS) void k_spmv(DevGrid<T> g, const T* __restrict__ x,
+__global__ __launch_bounds__(WG_THREADS) void k_spmv(DevGrid<T> g, const T* __restrict__ xin,
                                                      T* __restrict__ y, const T* a, T* c, T* c2,
                                                      SolverState* st, double* part) {
   constexpr bool NEED_A = MODE != SPMV_PLAIN;
+  constexpr int XS = MODE == SPMV_START ? 3 : 1;  // stride of x and a
   // sum_b h_b^3 sum x feeds the bMean = 1 row and the bMean = 2 term only
   using Sums = SpmvSums<MODE, BM>;
   constexpr bool NEED_SUM = Sums::MEAN == 1;
@@ -425,7 +467,10 @@ __global__ __launch_bounds__(WG_THREADS) void k_spmv(DevGrid<T> g, const T* __re
   // with coarse-fine faces the epilogue operand waits in LDS, not registers
   constexpr bool A_LDS = IFACE && NEED_A;
   __shared__ T as[A_LDS ? 4 : 1][A_LDS ? BLEN : 1];
-  if (MODE != SPMV_PLAIN && MODE != SPMV_RESID && st->status != ST_RUNNING) return;
+  if ((MODE == SPMV_DOT1 || MODE == SPMV_DOT2) && st->status != ST_RUNNING) return;
+  // FINAL: the best iterate; while that is still 0, its buffer holds nothing
+  const T* __restrict__ x = MODE == SPMV_FINAL ? g.xo[st->xopt] : xin;
+  const bool zero = MODE == SPMV_FINAL && st->opt_zero;
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int ix = lane & 7, iy = lane >> 3;
   const int b = xcd_remap(blockIdx.x, gridDim.x) * 4 + w;
@@ -443,10 +488,10 @@ __global__ __launch_bounds__(WG_THREADS) void k_spmv(DevGrid<T> g, const T* __re
     const int nxm = nb6[0], nxp = nb6[1], nym = nb6[2], nyp = nb6[3], nzm = nb6[4], nzp = nb6[5];
     h = g.h[b];
 #pragma unroll
-    for (int iz = 0; iz < BS; ++iz) col[iz] = x[off + iz * 64 + lane];
+    for (int iz = 0; iz < BS; ++iz) col[iz] = x[(off + iz * 64 + lane) * XS];
     if (NEED_A) {
 #pragma unroll
-      for (int iz = 0; iz < BS; ++iz) av[iz] = ld_stream<NT>(&a[off + iz * 64 + lane]);
+      for (int iz = 0; iz < BS; ++iz) av[iz] = ld_stream<NT>(&a[(off + iz * 64 + lane) * XS]);
     }
     // face halos: a lane is on at most one x face and one y face. A lane on
     // a face with a same-level neighbour reads the neighbour's face cell;
@@ -457,15 +502,15 @@ __global__ __launch_bounds__(WG_THREADS) void k_spmv(DevGrid<T> g, const T* __re
     const int sx = ix == 0 ? 7 : 0;
     const int ny = iy == 0 ? nym : (iy == 7 ? nyp : -1);
     const int sy = iy == 0 ? 7 : 0;
-    const T* px = x + (nx >= 0 ? (size_t)nx * BLEN + iy * 8 + sx : off + lane);
-    const T* py = x + (ny >= 0 ? (size_t)ny * BLEN + sy * 8 + ix : off + lane);
+    const T* px = x + (nx >= 0 ? (size_t)nx * BLEN + iy * 8 + sx : off + lane) * XS;
+    const T* py = x + (ny >= 0 ? (size_t)ny * BLEN + sy * 8 + ix : off + lane) * XS;
 #pragma unroll
     for (int iz = 0; iz < BS; ++iz) {
-      hx[iz] = px[iz * 64];
-      hy[iz] = py[iz * 64];
+      hx[iz] = px[iz * 64 * XS];
+      hy[iz] = py[iz * 64 * XS];
     }
-    zlo = x[nzm >= 0 ? (size_t)nzm * BLEN + 7 * 64 + lane : off + lane];
-    zhi = x[nzp >= 0 ? (size_t)nzp * BLEN + lane : off + 7 * 64 + lane];
+    zlo = x[(nzm >= 0 ? (size_t)nzm * BLEN + 7 * 64 + lane : off + lane) * XS];
+    zhi = x[(nzp >= 0 ? (size_t)nzp * BLEN + lane : off + 7 * 64 + lane) * XS];
     if (IFACE) {
       // the face layers of the coarser neighbours of the first two faces
       // that have one, loaded now so that their latency overlaps the stencil
@@ -476,8 +521,8 @@ __global__ __launch_bounds__(WG_THREADS) void k_spmv(DevGrid<T> g, const T* __re
           else if (cf1 < 0) cf1 = f;
         }
       }
-      if (cf0 >= 0) pre0 = x[coarse_plane_index(cf0, __builtin_amdgcn_readlane(meta, 4 * cf0), lane)];
-      if (cf1 >= 0) pre1 = x[coarse_plane_index(cf1, __builtin_amdgcn_readlane(meta, 4 * cf1), lane)];
+      if (cf0 >= 0) pre0 = x[coarse_plane_index(cf0, __builtin_amdgcn_readlane(meta, 4 * cf0), lane) * XS];
+      if (cf1 >= 0) pre1 = x[coarse_plane_index(cf1, __builtin_amdgcn_readlane(meta, 4 * cf1), lane) * XS];
     }
 #pragma unroll
     for (int iz = 0; iz < BS; ++iz) xs[w][iz * 64 + lane] = col[iz];
@@ -544,7 +589,7 @@ __global__ __launch_bounds__(WG_THREADS) void k_spmv(DevGrid<T> g, const T* __re
       for (int f = 0; f < 6; ++f) {
         const int fk = __builtin_amdgcn_readfirstlane(fmeta[w][24 + f]);
         if (fk >= FACE_COARSE)
-          iface_face<T>(g, x, xs[w], pl[w], ys[w], b, f, fk, par, lane, fmeta[w][4 * f],
+          iface_face<T, XS>(g, x, xs[w], pl[w], ys[w], b, f, fk, par, lane, fmeta[w][4 * f],
                         fmeta[w][4 * f + fq], f == cf0 || f == cf1, f == cf0 ? pre0 : pre1);
       }
     }
@@ -569,7 +614,10 @@ __global__ __launch_bounds__(WG_THREADS) void k_spmv(DevGrid<T> g, const T* __re
       const size_t i = off + iz * 64 + lane;
       // the bMean row is written by the last workgroup only, so no two
       // workgroups (possibly on different XCDs) ever store the same address
-      if ((BM == 1) && origin && lane == 0 && iz == 0) continue;
+      if ((BM == 1) && origin && lane == 0 && iz == 0) {
+        if (MODE == SPMV_FINAL && y) y[i] = zero ? (T)0 : col[iz];
+        continue;
+      }
       const T yy = yv[iz];
       if (A_LDS) av[iz] = as[w][iz * 64 + lane];
       if (MODE == SPMV_PLAIN) {
@@ -592,10 +640,20 @@ __global__ __launch_bounds__(WG_THREADS) void k_spmv(DevGrid<T> g, const T* __re
         const T rr = av[iz] - yy;
         c[i] = rr;
         v[1] += (double)rr * (double)rr;
+      } else if (MODE == SPMV_START) {
+        const T rr = -(h * h * h) * (T)g.helm_sigma * av[iz] - yy;
+        y[i] = rr;
+        c[i] = rr;
+        c2[i] = rr;
+        v[1] += (double)rr * (double)rr;
+      } else if (MODE == SPMV_FINAL) {
+        const T rr = zero ? av[iz] : av[iz] - yy;
+        v[1] += (double)rr * (double)rr;
+        if (y) y[i] = zero ? (T)0 : col[iz];
       }
     }
   }
-  if ((MODE == SPMV_PLAIN || MODE == SPMV_RESID) && !part) return;  // no sums wanted
+  if ((MODE == SPMV_PLAIN || MODE == SPMV_RESID || MODE == SPMV_FINAL) && !part) return;
   if constexpr (Sums::N > 0) {
     double p[Sums::N];
 #pragma unroll
@@ -618,7 +676,7 @@ __global__ __launch_bounds__(WG_THREADS) void k_spmv_fin(long long row, T* __res
   fin_load<Sums::N>(st, S, part, nparts, sums);
 #pragma unroll
   for (int k = 0; k < Sums::N; ++k) tot[k + 1 - Sums::MEAN] = sums[k];
-  if (MODE != SPMV_PLAIN && MODE != SPMV_RESID && S.status != ST_RUNNING) return;
+  if ((MODE == SPMV_DOT1 || MODE == SPMV_DOT2) && S.status != ST_RUNNING) return;
   if (threadIdx.x == 0) {
     // bMean = 1: y[row] = sum_b h_b^3 sum x  (BiCGSTAB.cu:406-407)
     if (BM == 1 && row >= 0) {
@@ -643,6 +701,9 @@ __global__ __launch_bounds__(WG_THREADS) void k_spmv_fin(long long row, T* __res
         const T rr = a[row] - yr;
         c[row] = rr;
         tot[1] += (double)rr * (double)rr;
+      } else if (MODE == SPMV_FINAL) {
+        const T rr = S.opt_zero ? a[row] : a[row] - yr;
+        tot[1] += (double)rr * (double)rr;
       }
     }
     S.mean_sum = tot[0];
@@ -658,7 +719,7 @@ __global__ __launch_bounds__(WG_THREADS) void k_spmv_fin(long long row, T* __res
       set_alpha(S, tot[1]);
     } else if (MODE == SPMV_DOT2) {
       set_omega(S, tot[1], tot[2]);
-    } else if (MODE == SPMV_RESID) {
+    } else if (MODE == SPMV_RESID || MODE == SPMV_FINAL) {
       S.true_rr = tot[1];
     }
   }
@@ -678,7 +739,7 @@ __global__ __launch_bounds__(WG_THREADS) void k_bmean2_sum(SolverState* st, cons
   __shared__ SolverState S;
   double tot[N];
   fin_load<N>(st, S, part, nparts, tot);
-  if (MODE != SPMV_PLAIN && MODE != SPMV_RESID && S.status != ST_RUNNING) return;
+  if ((MODE == SPMV_DOT1 || MODE == SPMV_DOT2) && S.status != ST_RUNNING) return;
   if (threadIdx.x == 0) S.mean_sum = tot[0];
   fin_store(st, S);
 }
@@ -689,7 +750,7 @@ __global__ __launch_bounds__(WG_THREADS) void k_bmean2_apply(DevGrid<T> g, T* __
                                                              T* __restrict__ c,
                                                              T* __restrict__ c2,
                                                              SolverState* st, double* part) {
-  if (MODE != SPMV_PLAIN && MODE != SPMV_RESID && st->status != ST_RUNNING) return;
+  if ((MODE == SPMV_DOT1 || MODE == SPMV_DOT2) && st->status != ST_RUNNING) return;
   const double red = st->mean_sum;
   // one thread per 8 consecutive cells (never across a block)
   const long long j = (long long)blockIdx.x * WG_THREADS + threadIdx.x;
@@ -765,10 +826,10 @@ inline void spmv_launch_iface(hipStream_t s, const DevGrid<T>& g, const T* x, T*
   }
   if (!launched) spmv_kernel<T, MODE, BM, HELM, false>(s, nwg, g, x, y, a, c, c2, st, part);
   if (mid) (void)hipEventRecord(mid, s);
-  // SPMV_PLAIN and SPMV_RESID without sums (part null; bMean 0 and 3 only): the
-  // vectors are complete, and the finalize kernel is 4 us of a 20-60 us call
-  if (!part || !fin) return;  // or the sums are left to the consumer (fin false)
-  if (BM == 2) {
+  // without sums (part null) the vectors are complete, and the finalize kernel
+  // is 4 us of a 20-60 us call; with fin false the sums are left to the consumer
+  if (!part || !fin) return;
+  if constexpr (BM == 2 && MODE != SPMV_FINAL) {
     k_bmean2_sum<MODE><<<1, WG_THREADS, 0, s>>>(st, part, nwg);
     // nb * 64 threads of 8 cells: (nb + 3) / 4 workgroups again, so the
     // partial buffer sized for k_spmv holds them
@@ -788,6 +849,8 @@ inline void spmv_launch(hipStream_t s, const DevGrid<T>& g, const T* x, T* y, co
       return;
     }
   }
+  if constexpr (MODE == SPMV_START) return;  // Helmholtz grids only
+  else
   if (g.bmean == 1) spmv_launch_iface<T, MODE, 1>(s, g, x, y, a, c, c2, st, part, fin, mid);
   else if (g.bmean == 2) spmv_launch_iface<T, MODE, 2>(s, g, x, y, a, c, c2, st, part, fin, mid);
   else if (g.bmean == 3) spmv_launch_iface<T, MODE, 3>(s, g, x, y, a, c, c2, st, part, fin, mid);
@@ -839,7 +902,12 @@ __global__ __launch_bounds__(WG_THREADS) void k_update(long long n, KrylovVector
     if (i0 < n) {
       const int xc = sp->xcur, xn = third_buffer(xc, sp->xopt);
       const T alpha = (T)sp->alpha, omega = (T)sp->omega;
-      load8(v.x[xc] + i0, xv);
+      if (sp->x_zero) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) xv[e] = 0;
+      } else {
+        load8(v.x[xc] + i0, xv);
+      }
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         xv[e] = fma(omega, z2[e], fma(alpha, z1[e], xv[e]));
@@ -864,6 +932,7 @@ __device__ inline void update_scalars(SolverState& S, double rho, double rr) {
   S.err = err;
   S.iters_done = S.iter;
   S.xcur = xn;
+  S.x_zero = 0;
   if (!(err == err) || err > 1.7e308) {
     S.status = ST_NONFINITE;
     return;
@@ -871,6 +940,7 @@ __device__ inline void update_scalars(SolverState& S, double rho, double rr) {
   if (err < S.err_opt) {
     S.err_opt = err;
     S.xopt = xn;
+    S.opt_zero = 0;
     if (err <= S.tol_abs || err / S.err_init <= S.tol_rel) {
       S.status = ST_CONVERGED;
       return;
@@ -909,18 +979,6 @@ inline int launch_k5(hipStream_t s, const DevGrid<T>& g, const KrylovVectors<T>&
   if (mid) (void)hipEventRecord(mid, s);
   if (last) k_update_fin<<<1, WG_THREADS, 0, s>>>(fin ? st + 2 : st, st, p5, nwg);
   return nwg;
-}
-
-// Copy the best iterate out: x_user = X[xopt] (PoissonSolverExp.cpp:452-472
-// scatter; BiCGSTAB.cu:625 copies x_opt).
-template <typename T>
-__global__ __launch_bounds__(WG_THREADS) void k_copy_opt(long long n, KrylovVectors<T> v,
-                                                         const SolverState* st,
-                                                         double* __restrict__ out) {
-  const T* __restrict__ src = v.x[st->xopt];
-  for (long long i = (long long)blockIdx.x * WG_THREADS + threadIdx.x; i < n;
-       i += (long long)gridDim.x * WG_THREADS)
-    out[i] = (double)src[i];
 }
 
 }  // namespace cup3d

@@ -343,55 +343,54 @@ __global__ __launch_bounds__(GT) void k_precond_h(int nb, const H* __restrict__ 
 // iteration-0 scalars (BiCGSTAB.cu:435-471 with x0 = 0).
 __global__ __launch_bounds__(WG_THREADS) void k_inner_init(long long n, const double* __restrict__ r64,
                                                            double scale, KrylovVectors<float> v,
-                                                           SolverState* st, double* part) {
+                                                           double* part) {
   double s[1] = {0.0};
   const long long i0 = (long long)blockIdx.x * (4 * BLEN) + 8 * threadIdx.x;
   if (i0 < n) {
     double rd[8];
-    float r[8], z[8];
+    float r[8];
     load8(r64 + i0, rd);
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       r[e] = (float)(rd[e] * scale);
-      z[e] = 0.f;
       s[0] += (double)r[e] * (double)r[e];
     }
     store8(v.r + i0, r);
     store8(v.rhat + i0, r);
-    store8(v.x[0] + i0, z);
   }
   grid_store_partial<1>(s, part);
 }
 
-__global__ __launch_bounds__(WG_THREADS) void k_inner_init_fin(SolverState* st, const double* part,
-                                                               int nparts) {
+__global__ __launch_bounds__(WG_THREADS) void k_inner_init_fin(SolverState init, SolverState* st,
+                                                               const double* part, int nparts) {
   __shared__ SolverState S;
   double tot[1];
-  fin_load<1>(st, S, part, nparts, tot);
+  grid_sum_partials<1>(part, nparts, tot);
   if (threadIdx.x == 0) {
+    S = init;
     S.nu2 = 0.0;
     S.err = sqrt(tot[0]);
     S.err_init = S.err;
     S.err_opt = S.err;
     S.rhrh = tot[0];
+    S.x_zero = S.opt_zero = 1;
     begin_iteration(&S, tot[0], tot[0]);
   }
   fin_store(st, S);
 }
 
-// Fold the FP32 increment into the FP64 iterate: x64 += scale * x32[k];
-// x32[k] = 0, with k = xcur (zero = 1: the recurrence continues from this
-// iterate) or xopt (zero = 0: the process ends here).
+// Fold the FP32 increment into the FP64 iterate: x64 += scale * x32[k], with
+// k = xcur (cur = 1: the recurrence continues from this iterate, its increment
+// then 0, see k_replace_fin) or xopt (cur = 0: the process ends here).
 __global__ __launch_bounds__(WG_THREADS) void k_fold(long long n, double* __restrict__ x64,
                                                      KrylovVectors<float> v,
                                                      const SolverState* st, double scale,
-                                                     int zero) {
-  float* __restrict__ d = v.x[zero ? st->xcur : st->xopt];
+                                                     int cur) {
+  if (cur ? st->x_zero : st->opt_zero) return;
+  const float* __restrict__ d = v.x[cur ? st->xcur : st->xopt];
   for (long long i = (long long)blockIdx.x * WG_THREADS + threadIdx.x; i < n;
-       i += (long long)gridDim.x * WG_THREADS) {
+       i += (long long)gridDim.x * WG_THREADS)
     x64[i] = fma(scale, (double)d[i], x64[i]);
-    if (zero) d[i] = 0.f;
-  }
 }
 
 // Residual replacement: r32 = r64 * inv_scale (the true FP64 residual of
@@ -430,6 +429,7 @@ __global__ __launch_bounds__(WG_THREADS) void k_replace_fin(SolverState* st, con
     S.err = sqrt(tot[1]);
     S.err_opt = S.err;
     S.xopt = S.xcur;
+    S.x_zero = S.opt_zero = 1;  // folded into the FP64 iterate
     if (S.status == ST_CONVERGED) {
       S.status = ST_RUNNING;
       S.rho_prev = S.rho_curr;
@@ -446,12 +446,6 @@ __global__ __launch_bounds__(WG_THREADS) void k_replace_fin(SolverState* st, con
     }
   }
   fin_store(st, S);
-}
-
-__global__ void k_copy64(long long n, const double* __restrict__ a, double* __restrict__ b) {
-  for (long long i = (long long)blockIdx.x * WG_THREADS + threadIdx.x; i < n;
-       i += (long long)gridDim.x * WG_THREADS)
-    b[i] = a[i];
 }
 
 __global__ void k_cast64to32(long long n, const double* __restrict__ a, float* __restrict__ b) {
@@ -622,21 +616,14 @@ int mixed_solve(MixedWorkspace& M, hipStream_t s, const cup3d_poisson_config& cf
                 const double* d_x0, cup3d_solve_report* rep, std::string& err) {
   const long long n = M.n;
   const KrylovVectors<float>& v = M.v32;
-  double* x64 = v64.x[0];
+  double* x64 = d_x;
   double* b64 = v64.b;
   double* r64 = v64.r;
-  // getVec + ||b|| (FP64)
+  // getVec + ||b|| (FP64); the iterate is d_x itself
   SolverState init = inner_state(cfg, 0.0);
   init.tol_abs = cfg.tol_abs;
-  *h_st = init;
-  MCHECK(hipMemcpyAsync(st, h_st, sizeof(SolverState), hipMemcpyHostToDevice, s));
   const long long zero_row =
       (cfg.bmean == 1 || cfg.bmean == 3) && origin_block >= 0 ? (long long)origin_block * BLEN : -1;
-  launch_getvec64(s, n, zero_row, d_rhs, d_x0, b64, x64, st, part, cfg.tol_rhs);
-  MCHECK(hipMemcpyAsync(h_st, st, sizeof(SolverState), hipMemcpyDeviceToHost, s));
-  MCHECK(hipStreamSynchronize(s));
-  const double bnorm2 = h_st->bnorm2;
-  const double tol_abs = h_st->tol_abs;
   int total_iters = 0, total_restarts = 0, steps = 0, replacements = 0, status = ST_MAXITER;
   const int poll = cfg.poll_every > 0 ? cfg.poll_every : 8;
   auto true_resid = [&](double& out) -> int {  // |b - A x64| in FP64, r64 = b - A x64
@@ -647,7 +634,19 @@ int mixed_solve(MixedWorkspace& M, hipStream_t s, const cup3d_poisson_config& cf
     return 0;
   };
   double rnorm = 0;
-  if (true_resid(rnorm)) return -1;
+  if (d_x0) {
+    launch_getvec64(s, n, zero_row, d_rhs, d_x0, b64, x64, init, st, part, cfg.tol_rhs);
+    if (true_resid(rnorm)) return -1;
+  } else {  // r64 = b64, without the operator
+    launch_start_zero64(s, M.nb, zero_row, d_rhs, b64, r64, nullptr, x64, init, st, part,
+                        cfg.tol_rhs);
+    MCHECK(hipGetLastError());
+    MCHECK(hipMemcpyAsync(h_st, st, sizeof(SolverState), hipMemcpyDeviceToHost, s));
+    MCHECK(hipStreamSynchronize(s));
+    rnorm = std::sqrt(h_st->true_rr);
+  }
+  const double bnorm2 = h_st->bnorm2;
+  const double tol_abs = h_st->tol_abs;
   const double err_init = rnorm;
   const double tol = std::max(tol_abs, cfg.tol_rel * err_init);
   bool done = false;
@@ -683,10 +682,9 @@ int mixed_solve(MixedWorkspace& M, hipStream_t s, const cup3d_poisson_config& cf
   while (!done && steps <= cfg.max_refine) {
     const double scale = rnorm;
     const double inner_rel = std::max(cfg.inner_tol, 0.5 * tol / scale);
-    *h_st = inner_state(cfg, inner_rel);
-    MCHECK(hipMemcpyAsync(st, h_st, sizeof(SolverState), hipMemcpyHostToDevice, s));
-    k_inner_init<<<grid_vec(n), WG_THREADS, 0, s>>>(n, r64, 1.0 / scale, v, st, part);
-    k_inner_init_fin<<<1, WG_THREADS, 0, s>>>(st, part, grid_vec(n));
+    *h_st = inner_state(cfg, inner_rel);  // the loop's view until the first poll
+    k_inner_init<<<grid_vec(n), WG_THREADS, 0, s>>>(n, r64, 1.0 / scale, v, part);
+    k_inner_init_fin<<<1, WG_THREADS, 0, s>>>(*h_st, st, part, grid_vec(n));
     ++steps;
     double last = 1.0;  // recurrence residual (scaled) at the last replacement
     double progress = 1.0;  // residual at the last halving, and its iteration
@@ -789,9 +787,7 @@ int mixed_solve(MixedWorkspace& M, hipStream_t s, const cup3d_poisson_config& cf
     total_iters += h_st->iters_done;
     total_restarts += h_st->restarts;
   }
-  k_copy64<<<grid_1d(n), WG_THREADS, 0, s>>>(n, x64, d_x);
   MCHECK(hipGetLastError());
-  MCHECK(hipStreamSynchronize(s));
   if (rep) {
     rep->status = status;
     rep->iterations = total_iters;

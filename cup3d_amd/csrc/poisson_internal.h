@@ -53,7 +53,7 @@ struct alignas(64) SolverState {
   int restart_pending;  // K1 copies rhat = r
   int p_zero;           // K1 uses p = r (p = nu = 0)
   int xcur, xopt;       // rotating iterate buffers (0..2)
-  int pad[2];
+  int x_zero, opt_zero;  // the current / best iterate is 0: its buffer is not read
 };
 
 // Workspace passed to the kernels (all device pointers).
@@ -92,6 +92,7 @@ struct DevGrid {
   long long bmean_row = -1;         // cell replaced by sum h^3 x (bMean == 1)
   int bmean = 1;
   int has_iface = 0;                // any coarse-fine interface rows
+  const T* xo[3] = {};              // SPMV_FINAL: the rotating iterate buffers
   // implicit diffusion of one velocity component (FP64 only): the operator
   // gains -h^3 helm_sigma x (helm_sigma = 1 / (nu dt)) and, on the domain-
   // boundary faces whose bit f is set in dmask, the Dirichlet ghost -x

@@ -498,3 +498,41 @@ def test_capped_solve_across_block_counts(gpu, bpd, bmean):
     assert torch.equal(x, x2)
     xo, info = pyoracle.Oracle(blocks, bpd, h0, bc, bmean).bicgstab(b, tol_rel=0.0, max_iter=3)
     assert np.linalg.norm(x.cpu().numpy() - xo) <= 1e-10 * np.linalg.norm(xo)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed_fp16"])
+@pytest.mark.parametrize("bmean", [0, 1, 2, 3])
+@pytest.mark.parametrize("name", ["uniform_walls_3x2x2", "tiny_amr_periodic"])
+def test_zero_guess_equals_given_zeros(gpu, name, bmean, precision):
+    """A zero guess starts without an operator application and never reads an
+    iterate buffer before it is written; the solve is the one from a given
+    vector of zeros: the initial residual to FP64 rounding, six iterations to
+    1e-12 (FP64 rounding, little amplified by then) and in the mixed form to
+    1e-6 (FP32 iterates). What x held before does not matter."""
+    blocks, bpd, h0, bc = CASES[name]
+    n = len(blocks) * 512
+    b = dev(compatible_rhs(blocks, h0, 6))
+    out = []
+    for guess, fill in (("given", 0.0), ("zero", float("nan"))):
+        S = PoissonSolver(bpd, h0, bc, bmean=bmean, precision=precision, guess=guess, tol_rel=0.0,
+                          max_iter=6, max_refine=1).set_topology(blocks)
+        x = torch.full((n,), fill, dtype=torch.float64, device=gpu)
+        out.append((S.solve_device(b, x), x.cpu().numpy()))
+    (r0, x0), (r1, x1) = out
+    assert r0["iterations"] == r1["iterations"]
+    assert abs(r1["err_init"] - r0["err_init"]) <= 1e-13 * r0["err_init"]
+    tol = 1e-12 if precision == "fp64" else 1e-6
+    assert np.linalg.norm(x1 - x0) <= tol * np.linalg.norm(x0)
+    assert abs(r1["true_rel_resid"] - r0["true_rel_resid"]) <= tol * r0["true_rel_resid"] + 1e-14
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed_fp16"])
+def test_zero_guess_without_progress_returns_zeros(gpu, precision):
+    """A zero rhs improves on nothing: the best iterate stays the zero guess,
+    whose buffer was never written, and x comes back as zeros."""
+    blocks, bpd, h0, bc = uniform((2, 1, 1), (WALL,) * 3)
+    S = PoissonSolver(bpd, h0, bc, bmean=0, precision=precision, guess="zero",
+                      max_iter=3).set_topology(blocks)
+    x = torch.full((len(blocks) * 512,), 7.0, dtype=torch.float64, device=gpu)
+    S.solve_device(torch.zeros_like(x), x)
+    assert torch.equal(x, torch.zeros_like(x))
