@@ -199,11 +199,11 @@ __global__ __launch_bounds__(WG_THREADS) void k_precond_dst(int nb, const T* __r
     if (MODE == PREC_P) {
       // BiCGSTAB.cu:518-522
       c[iz] = pzero ? ra[iz] : fma(beta, fma(-omega, rb[iz], c[iz]), ra[iz]);
-      v.p[i] = c[iz];
+      v.pw[i] = c[iz];
       if (restart) v.rhat[i] = ra[iz];
     } else if (MODE == PREC_S) {
       c[iz] = fma(-alpha, rb[iz], ra[iz]);  // :546-549
-      v.r[i] = c[iz];
+      v.s[i] = c[iz];
     }
   }
   dst_apply<T>(Ls[w], lane, hb[b], sigma, c);

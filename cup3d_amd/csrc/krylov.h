@@ -888,7 +888,7 @@ __global__ __launch_bounds__(WG_THREADS) void k_update(long long n, KrylovVector
       load8(v.z1 + i0, z1);
       load8(v.z2 + i0, z2);
       load8(v.t + i0, t);
-      load8(v.r + i0, r);
+      load8(v.s + i0, r);
       load8(v.rhat + i0, rh);
     }
     T yr = 0;

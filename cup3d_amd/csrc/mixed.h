@@ -20,7 +20,8 @@ struct MixedWorkspace {
   void* d_vec32 = nullptr; // FP32 Krylov vectors
   void* d_res64 = nullptr; // FP64 refinement residual
   long long n = 0;
-  long long cap_n = 0;     // cells the vector buffers hold
+  long long cap_n = 0;     // cells d_res64 holds two vectors of
+  long long cap_floats = 0;  // floats d_vec32 holds
   int nb = 0;
   int timing_precision = 1;
   KrylovVectors<float> v32{};

@@ -173,7 +173,7 @@ __device__ __forceinline__ void precond_convert(int nb, int j0, int w, int l, fl
                                                 const float* __restrict__ invh,
                                                 const KrylovVectors<float>& v,
                                                 const PrecScalars& c, FillRegs<NBW, NWP>& R,
-                                                H* A0, H* A1, float* sc) {
+                                                bool write, H* A0, H* A1, float* sc) {
   typedef H H4 __attribute__((ext_vector_type(4)));
   constexpr int NPB = FillRegs<NBW, NWP>::NPB, F4 = FillRegs<NBW, NWP>::F4;
   const int jw = w * NPB;
@@ -192,8 +192,8 @@ __device__ __forceinline__ void precond_convert(int nb, int j0, int w, int l, fl
         val.z = fmaf(c.beta, fmaf(-c.omega, R.rb[u].z, R.rc[u].z), R.ra[u].z);
         val.w = fmaf(c.beta, fmaf(-c.omega, R.rb[u].w, R.rc[u].w), R.ra[u].w);
       }
-      if (b < nb) {
-        st4<NT>(v.p, i4, val);
+      if (write && b < nb) {
+        st4<NT>(v.pw, i4, val);
         if (c.restart) st4<NT>(v.rhat, i4, R.ra[u]);
       }
     } else if (MODE == PREC_S) {
@@ -201,7 +201,7 @@ __device__ __forceinline__ void precond_convert(int nb, int j0, int w, int l, fl
       val.y = fmaf(-c.alpha, R.rb[u].y, R.ra[u].y);
       val.z = fmaf(-c.alpha, R.rb[u].z, R.ra[u].z);
       val.w = fmaf(-c.alpha, R.rb[u].w, R.ra[u].w);
-      if (b < nb) st4<NT>(v.r, i4, val);
+      if (write && b < nb) st4<NT>(v.s, i4, val);
     }
     R.ra[u] = val;
     amax[u / 2] = fmaxf(amax[u / 2], fmaxf(fmaxf(fabsf(val.x), fabsf(val.y)),
@@ -234,37 +234,36 @@ __device__ __forceinline__ void precond_convert(int nb, int j0, int w, int l, fl
   }
 }
 
-// Phases 2 and 3 for GEMM wave w (of GW): output cells [64 w, 64 w + 64) of
-// all NBW blocks of the group staged in A0/A1; 16 k-steps of 32 cells, each
-// 4 (cell tiles) x NBW/16 (block tiles) x (1 or 2 passes) MFMAs, the P_inv
-// fragments of the next k-step prefetched from L2 while the current ones are
-// used; FP32 epilogue scaled by h_b^-1 and the two scales.
-template <typename H, int NBW, bool SPLIT, bool NT>
-__device__ __forceinline__ void precond_gemm(int nb, int j0, int w, int l,
-                                             const H* __restrict__ Ppk, const H* A0,
-                                             const H* A1, const float* sc,
+// P_inv fragment (it, kt) of the packed matrix: 64 lanes x 8 values at
+// ((it 16 + kt) 64 + l) 8.
+template <typename H>
+__device__ __forceinline__ const typename HalfVec<H>::type* frags(const H* Ppk, int it, int l) {
+  return reinterpret_cast<const typename HalfVec<H>::type*>(Ppk) + (size_t)it * 16 * 64 + l;
+}
+
+// Phases 2 and 3 for a GEMM wave that owns the TPW tiles of 16 output cells
+// from tile it0, for all NBW blocks of the group staged in A0/A1; 16 k-steps
+// of 32 cells, each TPW (cell tiles) x NBW/16 (block tiles) x (1 or 2 passes)
+// MFMAs; FP32 epilogue scaled by h_b^-1 and the two scales. With four tiles the
+// P_inv fragments of the next k-step are prefetched from L2 while the current
+// ones are used; with fewer all of them were loaded before phase 1 (pre).
+template <typename H, int NBW, int TPW, bool SPLIT, bool NT>
+__device__ __forceinline__ void precond_gemm(int nb, int j0, int it0, int l,
+                                             const H* __restrict__ Ppk,
+                                             const typename HalfVec<H>::type (*pre)[TPW],
+                                             const H* A0, const H* A1, const float* sc,
                                              float* __restrict__ out) {
   typedef typename HalfVec<H>::type HV;
   constexpr int JT = NBW / 16;
   static_assert(NBW % 16 == 0, "block group must fill the tiles");
   const int lr = l & 15, g = l >> 4;
-  float4_t acc[4][JT];
+  float4_t acc[TPW][JT];
 #pragma unroll
-  for (int t = 0; t < 4; ++t)
+  for (int t = 0; t < TPW; ++t)
 #pragma unroll
     for (int jt = 0; jt < JT; ++jt) acc[t][jt] = (float4_t){0.f, 0.f, 0.f, 0.f};
-  // fragment (it, kt) of the packed P_inv: 64 lanes x 8 values at ((it 16 + kt) 64 + l) 8
-  const HV* __restrict__ pb = reinterpret_cast<const HV*>(Ppk) + (size_t)(4 * w) * 16 * 64 + l;
-  HV bq[2][4];
-#pragma unroll
-  for (int t = 0; t < 4; ++t) bq[0][t] = pb[(size_t)t * 16 * 64];
-#pragma unroll 2
-  for (int kt = 0; kt < 16; ++kt) {
-    const int cur = kt & 1;
-    if (kt + 1 < 16) {
-#pragma unroll
-      for (int t = 0; t < 4; ++t) bq[cur ^ 1][t] = pb[((size_t)t * 16 + kt + 1) * 64];
-    }
+  const HV* __restrict__ pb = frags(Ppk, it0, l);
+  auto step = [&](int kt, const HV* bq) {
     HV a[JT], al[JT];
 #pragma unroll
     for (int jt = 0; jt < JT; ++jt) {
@@ -273,12 +272,29 @@ __device__ __forceinline__ void precond_gemm(int nb, int j0, int w, int l,
       if (SPLIT) al[jt] = *reinterpret_cast<const HV*>(&A1[o]);
     }
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+    for (int t = 0; t < TPW; ++t)
 #pragma unroll
       for (int jt = 0; jt < JT; ++jt) {
-        acc[t][jt] = mfma16(a[jt], bq[cur][t], acc[t][jt]);
-        if (SPLIT) acc[t][jt] = mfma16(al[jt], bq[cur][t], acc[t][jt]);
+        acc[t][jt] = mfma16(a[jt], bq[t], acc[t][jt]);
+        if (SPLIT) acc[t][jt] = mfma16(al[jt], bq[t], acc[t][jt]);
       }
+  };
+  if constexpr (TPW == 4) {
+    HV bq[2][4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) bq[0][t] = pb[(size_t)t * 16 * 64];
+#pragma unroll 2
+    for (int kt = 0; kt < 16; ++kt) {
+      const int cur = kt & 1;
+      if (kt + 1 < 16) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) bq[cur ^ 1][t] = pb[((size_t)t * 16 + kt + 1) * 64];
+      }
+      step(kt, bq[cur]);
+    }
+  } else {
+#pragma unroll
+    for (int kt = 0; kt < 16; ++kt) step(kt, pre[kt]);
   }
 #pragma unroll
   for (int jt = 0; jt < JT; ++jt)
@@ -289,15 +305,19 @@ __device__ __forceinline__ void precond_gemm(int nb, int j0, int w, int l,
       if (b < nb) {
         const float s = sc[jr];
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
-          st_stream<NT>(&out[(size_t)b * BLEN + (4 * w + t) * 16 + lr], acc[t][jt][q] * s);
+        for (int t = 0; t < TPW; ++t)
+          st_stream<NT>(&out[(size_t)b * BLEN + (it0 + t) * 16 + lr], acc[t][jt][q] * s);
       }
     }
 }
 
 // One workgroup applies M^-1 to NBW consecutive blocks: every wave fills
-// (phase 1), then every wave multiplies (phases 2 and 3).
-template <int MODE, typename H, int NBW, bool SPLIT, bool NT = false, int FIN = FIN_KERNEL>
+// (phase 1), then every wave multiplies (phases 2 and 3). With SPL > 1 the
+// group's 512 output cells are split over SPL workgroups, each of which makes
+// the group's vectors for itself (the first one writes them, to v.pw and v.s,
+// which the others do not read).
+template <int MODE, typename H, int NBW, bool SPLIT, bool NT = false, int FIN = FIN_KERNEL,
+          int SPL = 1>
 __global__ __launch_bounds__(GT) void k_precond_h(int nb, const H* __restrict__ Ppk,
                                                   float p_unscale,
                                                   const float* __restrict__ invh,
@@ -305,16 +325,25 @@ __global__ __launch_bounds__(GT) void k_precond_h(int nb, const H* __restrict__ 
                                                   const float* __restrict__ pin,
                                                   float* __restrict__ pout, SolverState* st,
                                                   FinArgs f) {
-  constexpr int NS = SPLIT ? 2 : 1;
+  typedef typename HalfVec<H>::type HV;
+  constexpr int NS = SPLIT ? 2 : 1, TPW = 4 / SPL;
   __shared__ __attribute__((aligned(16))) H As[NS][NBW * HLD];
   __shared__ float sc[NBW];
   __shared__ SolverState S;
   if (!FIN && MODE != PREC_PLAIN && st->status != ST_RUNNING) return;
-  const int j0 = (int)blockIdx.x * NBW;
+  const int j0 = (int)blockIdx.x / SPL * NBW, part = (int)blockIdx.x % SPL;
   float* __restrict__ out = MODE == PREC_PLAIN ? pout : (MODE == PREC_S ? v.z2 : v.z1);
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  const int it0 = part * (32 / SPL) + w * TPW;
   FillRegs<NBW, GW> R;
   precond_load<MODE, NBW, GW, NT>(nb, j0, w, l, v, pin, R);
+  HV pre[TPW < 4 ? 16 : 1][TPW];
+  if constexpr (TPW < 4) {
+#pragma unroll
+    for (int kt = 0; kt < 16; ++kt)
+#pragma unroll
+      for (int t = 0; t < TPW; ++t) pre[kt][t] = frags(Ppk, it0 + t, l)[kt * 64];
+  }
   const SolverState* sp = st;
   if constexpr (FIN != FIN_KERNEL) {
     float yr = 0.f;
@@ -327,16 +356,16 @@ __global__ __launch_bounds__(GT) void k_precond_h(int nb, const H* __restrict__ 
         const int b = j0 + w * FillRegs<NBW, GW>::NPB + u / 2;
         if (b < nb && (long long)b * BLEN == f.row) {
           R.rb[u].x = yr;  // the mean-constraint row of nu, which the SpMV left out
-          v.nu[f.row] = yr;
+          if (part == 0) v.nu[f.row] = yr;
         }
       }
     }
   }
   const PrecScalars c = prec_scalars<MODE>(sp);
-  precond_convert<MODE, H, NBW, SPLIT, GW, NT>(nb, j0, w, l, p_unscale, invh, v, c, R, As[0],
-                                           As[NS - 1], sc);
+  precond_convert<MODE, H, NBW, SPLIT, GW, NT>(nb, j0, w, l, p_unscale, invh, v, c, R, part == 0,
+                                               As[0], As[NS - 1], sc);
   __syncthreads();
-  precond_gemm<H, NBW, SPLIT, NT>(nb, j0, w, l, Ppk, As[0], As[NS - 1], sc, out);
+  precond_gemm<H, NBW, TPW, SPLIT, NT>(nb, j0, it0, l, Ppk, pre, As[0], As[NS - 1], sc, out);
 }
 
 // Inner-solve start: r = rhat = (float)(r64 * scale), x = 0, ||r||^2, and the
@@ -464,64 +493,89 @@ __global__ void k_cast32to64(long long n, const float* __restrict__ a, double* _
 // ---------------------------------------------------------------------------
 namespace {
 
-// Blocks per GEMM workgroup: P_inv (512 KiB in FP16) is streamed from L2 once
-// per workgroup, so 32 blocks halve that traffic against 16; 32 is also the
-// faster choice on grids too small to give every CU a workgroup (4440 blocks:
-// 14.4 us against 15.9 us for K1).
-constexpr int GEMM_NB = 32;
+// Blocks per GEMM workgroup and workgroups per group of blocks. P_inv (512 KiB
+// in FP16) is streamed from L2 once per group, so 32 blocks halve that traffic
+// against 16; but below 8192 blocks groups of 32 leave CUs idle, and a
+// workgroup's own time (its P_inv stream, its MFMAs) is what the kernel takes.
+// So the work is split as far as every workgroup still has a CU (of 256) to
+// itself: groups of 16 blocks up to 4096 blocks, their output cells over two
+// workgroups up to 2048 and over four up to 1024 (P_inv then fits the
+// registers and is loaded before phase 1). One capped solve of 32 iterations,
+// groups of 32 against this rule: 64 blocks 1451 -> 1114 us, 819 1567 -> 1271,
+// 1456 1777 -> 1485, 2856 1942 -> 1798, 4096 2149 -> 2001; a split beyond the
+// rule loses (four workgroups at 1456 blocks 1790 us, two at 2856 2173 us,
+// groups of 16 at 4440 blocks K1 15.9 us against 14.4).
+constexpr int GEMM_NB = 32, GEMM_NB_SMALL = 16, GEMM_SPLIT_MAX = 2048;
 
-template <typename H, bool SPLIT, int NBW>
+inline bool gemm_split(const MixedWorkspace& M, int nb) {
+  return !M.use_dst && nb <= GEMM_SPLIT_MAX;
+}
+
+template <typename H, bool SPLIT, int NBW, int SPL>
 void launch_precond_hw(hipStream_t s, int mode, int nb, const H* P, float unscale,
                        const float* invh, const KrylovVectors<float>& v, const float* pin,
                        float* pout, SolverState* st, int fin, const FinArgs& f) {
-  const int nwg = (nb + NBW - 1) / NBW;
+  const int nwg = (nb + NBW - 1) / NBW * SPL;
   // K1 and K3 stream their vectors nontemporally when they are large
   // (larger than any grid whose scalars are computed in the consumer)
-  const bool nt = (size_t)nb * BLEN * sizeof(float) >= STREAM_MIN_BYTES;
+  constexpr bool BIG = SPL == 1;
+  const bool nt = BIG && (size_t)nb * BLEN * sizeof(float) >= STREAM_MIN_BYTES;
   static_assert((size_t)FIN_MAX_BLOCKS * BLEN * sizeof(float) < STREAM_MIN_BYTES, "no NT with FIN");
 #define CUP3D_PREC_LAUNCH(MODE, NT, FIN)                                                     \
-  k_precond_h<MODE, H, NBW, SPLIT, NT, FIN>                                                  \
+  k_precond_h<MODE, H, NBW, SPLIT, NT, FIN, SPL>                                             \
       <<<nwg, GT, 0, s>>>(nb, P, unscale, invh, v, pin, pout, st, f)
   if (mode == PREC_P && fin) CUP3D_PREC_LAUNCH(PREC_P, false, FIN_SUMS);
-  else if (mode == PREC_P && nt) CUP3D_PREC_LAUNCH(PREC_P, true, FIN_KERNEL);
+  else if (mode == PREC_P && nt) CUP3D_PREC_LAUNCH(PREC_P, BIG, FIN_KERNEL);
   else if (mode == PREC_P) CUP3D_PREC_LAUNCH(PREC_P, false, FIN_KERNEL);
   else if (mode == PREC_S && fin == FIN_ROW) CUP3D_PREC_LAUNCH(PREC_S, false, FIN_ROW);
   else if (mode == PREC_S && fin) CUP3D_PREC_LAUNCH(PREC_S, false, FIN_SUMS);
-  else if (mode == PREC_S && nt) CUP3D_PREC_LAUNCH(PREC_S, true, FIN_KERNEL);
+  else if (mode == PREC_S && nt) CUP3D_PREC_LAUNCH(PREC_S, BIG, FIN_KERNEL);
   else if (mode == PREC_S) CUP3D_PREC_LAUNCH(PREC_S, false, FIN_KERNEL);
   else CUP3D_PREC_LAUNCH(PREC_PLAIN, false, FIN_KERNEL);
 #undef CUP3D_PREC_LAUNCH
 }
 
-template <typename H>
-void launch_precond_h(hipStream_t s, int mode, int nb, const void* Ppk, float unscale,
-                      bool split, const float* invh, const KrylovVectors<float>& v,
-                      const float* pin, float* pout, SolverState* st, int fin, const FinArgs& f) {
-  const H* P = static_cast<const H*>(Ppk);
-  if (split)
-    launch_precond_hw<H, true, GEMM_NB>(s, mode, nb, P, unscale, invh, v, pin, pout, st, fin, f);
+template <typename H, bool SPLIT>
+void launch_precond_hs(hipStream_t s, int mode, int nb, const H* P, float unscale,
+                       const float* invh, const KrylovVectors<float>& v, const float* pin,
+                       float* pout, SolverState* st, int fin, const FinArgs& f) {
+  if (nb <= GEMM_SPLIT_MAX / 2)
+    launch_precond_hw<H, SPLIT, GEMM_NB_SMALL, 4>(s, mode, nb, P, unscale, invh, v, pin, pout, st,
+                                                  fin, f);
+  else if (nb <= GEMM_SPLIT_MAX)
+    launch_precond_hw<H, SPLIT, GEMM_NB_SMALL, 2>(s, mode, nb, P, unscale, invh, v, pin, pout, st,
+                                                  fin, f);
+  else if (nb <= 4096)
+    launch_precond_hw<H, SPLIT, GEMM_NB_SMALL, 1>(s, mode, nb, P, unscale, invh, v, pin, pout, st,
+                                                  fin, f);
   else
-    launch_precond_hw<H, false, GEMM_NB>(s, mode, nb, P, unscale, invh, v, pin, pout, st, fin, f);
+    launch_precond_hw<H, SPLIT, GEMM_NB, 1>(s, mode, nb, P, unscale, invh, v, pin, pout, st, fin, f);
 }
 
-void launch_precond_mixed(const MixedWorkspace& M, hipStream_t s, int precision, int mode,
-                          const DevGrid<float>& g, const float* pin, float* pout, SolverState* st,
-                          int fin = FIN_KERNEL, const FinArgs& f = FinArgs()) {
+void launch_precond_mixed(const MixedWorkspace& M, const KrylovVectors<float>& v, hipStream_t s,
+                          int precision, int mode, const DevGrid<float>& g, const float* pin,
+                          float* pout, SolverState* st, int fin = FIN_KERNEL,
+                          const FinArgs& f = FinArgs()) {
   if (M.use_dst) {
-    KrylovVectors<float> v = M.v32;
+    KrylovVectors<float> u = v;
     if (mode == PREC_PLAIN) {
-      v.p = const_cast<float*>(pin);
-      v.z1 = pout;
+      u.p = const_cast<float*>(pin);
+      u.z1 = pout;
     }
-    launch_precond_dst32(s, mode, g.nb, g.h, v, st, fin, f);
+    launch_precond_dst32(s, mode, g.nb, g.h, u, st, fin, f);
     return;
   }
-  if (precision == CUP3D_PREC_MIXED_FP16)
-    launch_precond_h<_Float16>(s, mode, g.nb, M.d_P16, 1.0f / P16_SCALE, M.split, g.invh, M.v32,
-                               pin, pout, st, fin, f);
-  else
-    launch_precond_h<__bf16>(s, mode, g.nb, M.d_Pbf, 1.0f, M.split, g.invh, M.v32, pin, pout,
-                             st, fin, f);
+  auto launch = [&](auto tag, const void* P, float unscale) {
+    typedef decltype(tag) H;
+    if (M.split)
+      launch_precond_hs<H, true>(s, mode, g.nb, static_cast<const H*>(P), unscale, g.invh, v, pin,
+                                 pout, st, fin, f);
+    else
+      launch_precond_hs<H, false>(s, mode, g.nb, static_cast<const H*>(P), unscale, g.invh, v, pin,
+                                  pout, st, fin, f);
+  };
+  if (precision == CUP3D_PREC_MIXED_FP16) launch((_Float16)0, M.d_P16, 1.0f / P16_SCALE);
+  else launch((__bf16)0.f, M.d_Pbf, 1.0f);
 }
 
 template <int MODE>
@@ -584,14 +638,16 @@ int mixed_init_pinv(MixedWorkspace& M, const std::vector<double>& P, std::string
 
 int mixed_set_topology(MixedWorkspace& M, int nb, long long n, std::string& err) {
   // the buffers grow only: a mesh change that does not add cells keeps them
-  if (n > M.cap_n || !M.d_vec32 || !M.d_res64) {
+  const long long vecs = gemm_split(M, nb) ? 12 : 11;  // a second p
+  if (vecs * n > M.cap_floats || n > M.cap_n || !M.d_vec32 || !M.d_res64) {
     if (M.d_vec32) (void)hipFree(M.d_vec32);
     if (M.d_res64) (void)hipFree(M.d_res64);
     M.d_vec32 = M.d_res64 = nullptr;
-    M.cap_n = 0;
-    MCHECK(hipMalloc(&M.d_vec32, (size_t)11 * n * sizeof(float)));
+    M.cap_n = M.cap_floats = 0;
+    MCHECK(hipMalloc(&M.d_vec32, (size_t)vecs * n * sizeof(float)));
     MCHECK(hipMalloc(&M.d_res64, (size_t)2 * n * sizeof(double)));
     M.cap_n = n;
+    M.cap_floats = vecs * n;
   }
   M.nb = nb;
   M.n = n;
@@ -606,6 +662,8 @@ int mixed_set_topology(MixedWorkspace& M, int nb, long long n, std::string& err)
   v.z1 = base + 8 * n;
   v.z2 = base + 9 * n;
   v.b = base + 10 * n;
+  v.s = gemm_split(M, nb) ? v.b : v.r;
+  v.pw = gemm_split(M, nb) ? base + 11 * n : v.p;
   return 0;
 }
 
@@ -615,7 +673,7 @@ int mixed_solve(MixedWorkspace& M, hipStream_t s, const cup3d_poisson_config& cf
                 double* part, int origin_block, const double* d_rhs, double* d_x,
                 const double* d_x0, cup3d_solve_report* rep, std::string& err) {
   const long long n = M.n;
-  const KrylovVectors<float>& v = M.v32;
+  KrylovVectors<float> v = M.v32;  // p and pw change places when they are two
   double* x64 = d_x;
   double* b64 = v64.b;
   double* r64 = v64.r;
@@ -702,16 +760,17 @@ int mixed_solve(MixedWorkspace& M, hipStream_t s, const cup3d_poisson_config& cf
         // event pairs (2k, 2k+1) bracket the main kernel of K(k+1)
         const bool tm = M.prof && it == tm_it;
         if (tm) MCHECK(hipEventRecord(M.pev[0], s));
-        launch_precond_mixed(M, s, cfg.precision, PREC_P, g32, nullptr, nullptr, st,
+        launch_precond_mixed(M, v, s, cfg.precision, PREC_P, g32, nullptr, nullptr, st,
                              it > 0 ? fin : FIN_KERNEL, fp);
+        std::swap(v.p, v.pw);
         if (tm) MCHECK(hipEventRecord(M.pev[1], s));
         if (tm) MCHECK(hipEventRecord(M.pev[2], s));
         spmv32<SPMV_DOT1>(s, g32, v.z1, v.nu, v.rhat, st, part, !fin, tm ? M.pev[3] : nullptr);
         if (tm) MCHECK(hipEventRecord(M.pev[4], s));
-        launch_precond_mixed(M, s, cfg.precision, PREC_S, g32, nullptr, nullptr, st, fin, fs);
+        launch_precond_mixed(M, v, s, cfg.precision, PREC_S, g32, nullptr, nullptr, st, fin, fs);
         if (tm) MCHECK(hipEventRecord(M.pev[5], s));
         if (tm) MCHECK(hipEventRecord(M.pev[6], s));
-        spmv32<SPMV_DOT2>(s, g32, v.z2, v.t, v.r, st, part, !fin, tm ? M.pev[7] : nullptr);
+        spmv32<SPMV_DOT2>(s, g32, v.z2, v.t, v.s, st, part, !fin, tm ? M.pev[7] : nullptr);
         if (tm) MCHECK(hipEventRecord(M.pev[8], s));
         fp.nparts = launch_k5<float>(s, g32, v, st, part, fin, !fin || it == batch - 1,
                                      tm ? M.pev[9] : nullptr);
@@ -819,7 +878,7 @@ int mixed_apply_precond(MixedWorkspace& M, hipStream_t s, int precision, const D
   float* in = reinterpret_cast<float*>(M.d_res64);
   float* out = in + M.n;
   k_cast64to32<<<grid_1d(M.n), WG_THREADS, 0, s>>>(M.n, d_p, in);
-  launch_precond_mixed(M, s, precision, PREC_PLAIN, g32, in, out, nullptr);
+  launch_precond_mixed(M, M.v32, s, precision, PREC_PLAIN, g32, in, out, nullptr);
   k_cast32to64<<<grid_1d(M.n), WG_THREADS, 0, s>>>(M.n, out, d_z);
   MCHECK(hipGetLastError());
   return 0;
@@ -834,11 +893,11 @@ int mixed_time_kernel(MixedWorkspace& M, hipStream_t s, int which, int reps,
   auto launch = [&]() {
     switch (which) {
       case 0: spmv32<SPMV_PLAIN>(s, g32, v.z1, v.nu, nullptr, st, part); break;
-      case 1: launch_precond_mixed(M, s, precision, PREC_PLAIN, g32, v.p, v.z1, st); break;
+      case 1: launch_precond_mixed(M, M.v32, s, precision, PREC_PLAIN, g32, v.p, v.z1, st); break;
       case 2:
         launch_k5<float>(s, g32, v, st, part);
         break;
-      case 3: launch_precond_mixed(M, s, precision, PREC_P, g32, nullptr, nullptr, st); break;
+      case 3: launch_precond_mixed(M, M.v32, s, precision, PREC_P, g32, nullptr, nullptr, st); break;
       default: spmv32<SPMV_DOT1>(s, g32, v.z1, v.nu, v.rhat, st, part); break;
     }
   };

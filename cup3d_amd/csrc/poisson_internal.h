@@ -68,6 +68,9 @@ struct KrylovVectors {
   T* z1;     // M^-1 p
   T* z2;     // M^-1 s
   T* b;
+  T* s;      // where K3 leaves s: r itself, or a vector of its own when several
+             // workgroups of K3 read the same blocks of r
+  T* pw;     // where K1 leaves the new p: p itself, or the other one of a pair
 };
 
 // Grid data on the device.

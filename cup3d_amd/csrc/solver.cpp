@@ -441,6 +441,8 @@ int cup3d_poisson_set_topology(cup3d_poisson_t H, int64_t nblocks, const cup3d_b
   v.z1 = base + 8 * n;
   v.z2 = base + 9 * n;
   v.b = base + 10 * n;
+  v.s = v.r;
+  v.pw = v.p;
   // up to GUESS_MAXV (GUESS_MAXV + 1) / 2 partials per workgroup of 2048
   // cells (the warm start's Gram matrix)
   H->part_len = (size_t)((H->nb + 3) / 4 + 8) * (GUESS_MAXV * (GUESS_MAXV + 1) / 2);

@@ -346,3 +346,38 @@ def test_mixed_dst_solve_reaches_fp64_tolerance(gpu, name):
     xo, info = O.bicgstab(b, tol_abs=1e-10 * np.linalg.norm(bb), tol_rel=0.0)
     err = np.linalg.norm(x.cpu().numpy() - xo) / np.linalg.norm(xo)
     assert err < 1e-7, err
+
+
+@pytest.mark.parametrize("prec", ["mixed_fp16", "mixed_bf16"])
+@pytest.mark.parametrize("nb", [1, 17, 1024, 1025, 2048, 2049, 4096, 4097])
+def test_preconditioner_is_the_same_for_every_block_count(gpu, prec, nb):
+    """M^-1 acts block by block, and every split of the GEMM over workgroups
+    takes the products of an output cell in the same order: the first nb blocks
+    of a large grid give the same bits on a grid of nb blocks, at the block
+    counts where the split changes."""
+    big = 5000
+    p = torch.from_numpy(np.random.default_rng(3).standard_normal(big * 512)).cuda()
+
+    def apply(n):
+        S = PoissonSolver((n, 1, 1), 0.01, (2, 2, 2), bmean=0, precision=prec)
+        S.set_topology(W.uniform_blocks(n, 1, 1))
+        q = p[:n * 512].clone()
+        return S.apply_preconditioner(q, torch.zeros_like(q))
+
+    assert torch.equal(apply(nb), apply(big)[:nb * 512])
+
+
+@pytest.mark.parametrize("bmean", [0, 1])
+@pytest.mark.parametrize("bpd", [(9, 5, 3), (17, 8, 8), (13, 13, 13)])
+def test_refined_solve_across_gemm_splits(gpu, bpd, bmean):
+    """A refined FP16 solve at 135, 1088 and 2197 blocks (four, two and one
+    workgroups per group of blocks; with more than one, s and p live in vectors
+    of their own) reaches the FP64 residual asked for."""
+    h0 = 1.0 / 64
+    blocks = W.uniform_blocks(*bpd)
+    S = PoissonSolver(bpd, h0, (2, 2, 2), bmean=bmean, precision="mixed_fp16", tol_rel=0.0,
+                      tol_rhs=1e-8, max_refine=40).set_topology(blocks)
+    b = torch.from_numpy(compatible_rhs(blocks, h0, 8).reshape(-1)).cuda()
+    x = torch.zeros_like(b)
+    rep = S.solve_device(b, x)
+    assert rep["status"] == 0 and rep["true_rel_resid"] <= 1e-8
