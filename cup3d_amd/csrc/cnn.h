@@ -65,7 +65,7 @@ int cnn_set_weights(CnnState& C, const float* w, int nw, std::string& err);
 int cnn_get_weights(CnnState& C, float* w, int nw, std::string& err);
 // d_out = p_prev + s_r * net(res / (h s_r), p_prev / s_p), res = b - A p_prev.
 int cnn_predict(CnnState& C, hipStream_t s, const double* d_res, const double* d_prev,
-                double* d_out, std::string& err);
+                double* d_out, std::string& err, const double* sums = nullptr);
 // Training triple: the residual of p_prev, p_prev, and the solution p.
 int cnn_add_sample(CnnState& C, hipStream_t s, const double* d_res, const double* d_prev,
                    const double* d_p, std::string& err);

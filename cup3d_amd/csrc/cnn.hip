@@ -16,7 +16,7 @@
 // cell of the block.
 //
 // Inference (k_cnn_infer): one workgroup per block, activations in LDS as
-// FP16 channel-last [8][8][8][16] (the zero padding selected on read), the
+// FP16 channel-last cells with a shared zero ring, the
 // input as the [10][10][10] patch, each layer an implicit
 // GEMM on v_mfma_f32_16x16x32_f16 (M = 16 cells, N = 16 output channels,
 // K = 27 offsets x input channels; the 8 consecutive K of a lane are 8
@@ -95,6 +95,17 @@ __global__ __launch_bounds__(WG_THREADS) void k_cnn_rms_fin(long long n, double*
   }
 }
 
+// scal[0] = RMS(res / h_b), scal[1] = RMS(p_prev) from the sums of SPMV_NET
+__global__ __launch_bounds__(WG_THREADS) void k_cnn_scales_fin(long long n, double* scal,
+                                                               const double* part, int nparts) {
+  double tot[2];
+  grid_sum_partials<2>(part, nparts, tot);
+  if (threadIdx.x < 2) {
+    const double s = sqrt(tot[threadIdx.x] / (double)n);
+    scal[threadIdx.x] = s > 0 ? s : 1.0;
+  }
+}
+
 // scal[2] = volume-weighted mean of p - p_prev: sum h^3 (p - p_prev) / sum h^3
 __global__ __launch_bounds__(WG_THREADS) void k_cnn_dmean(long long n, const double* __restrict__ p,
                                                           const double* __restrict__ prev,
@@ -156,57 +167,112 @@ __device__ __forceinline__ int padded(int m) {  // cell 0..511 -> padded index
   return (((m >> 6) + 1) * 10 + ((m >> 3) & 7) + 1) * 10 + (m & 7) + 1;
 }
 
-// One conv layer as implicit GEMM, K-steps KT; output tile handler f(m, n,
-// value) for each of this wave's 8 M-tiles. L1: `in` is the 10^3 input patch
-// (8 halfs per cell, valid conv); otherwise `in` holds the block's 512 cells
-// (CNN_C halfs each, no halo) and reads outside the block are the zero
-// padding of the "same" conv (selected, not stored).
-template <int KT, bool L1, typename F>
-__device__ __forceinline__ void conv_layer(const _Float16* __restrict__ in,
+// Activations in LDS: cells of CNN_C halfs, rows of 8 cells behind one zero
+// cell, planes of 8 rows behind one zero row, one zero plane in front and one
+// behind. The zero cell in front of a row is also the one behind the row
+// before it (and so for rows and planes), so the "same" padding costs 820
+// cells against 1000, and three workgroups fit a CU.
+constexpr int AROW = 9, APLANE = 81, ACELLS = 9 * APLANE + 9 * AROW + AROW + 1;
+__device__ __forceinline__ constexpr int atap(int o) {  // tap o from the (-1, -1, -1) corner
+  return (o / 9) * APLANE + ((o / 3) % 3) * AROW + o % 3;
+}
+
+// Four rows (cells 16 tile + 4 g + q) of a tile's products with channel lr.
+template <typename F>
+__device__ __forceinline__ void tile_rows(const float4_t& acc, F&& f) {
+  // register q of lane l holds D[4*(l/16) + q][l % 16]
+#pragma unroll
+  for (int q = 0; q < 4; ++q) f(q, acc[q]);
+}
+
+// Layer 1 (valid) on the 10^3 input patch, 8 halfs a cell: 4 taps a k-step,
+// tap 4 kt + g in the lanes of group g. The lane's tap offsets are registers
+// made once, a tile's offset is added to one base.
+template <typename F>
+__device__ __forceinline__ void conv_first(const _Float16* __restrict__ in,
                                            const half8_t* __restrict__ wfrag, int w, int l,
                                            F&& f) {
   const int lr = l & 15, g = l >> 4;
-  half8_t bq[KT];
+  half8_t bq[CNN_KT1];
 #pragma unroll
-  for (int kt = 0; kt < KT; ++kt) bq[kt] = wfrag[kt * 64 + l];
-  half8_t zero;
+  for (int kt = 0; kt < CNN_KT1; ++kt) bq[kt] = wfrag[kt * 64 + l];
+  int po[CNN_KT1];  // halfs
 #pragma unroll
-  for (int e = 0; e < 8; ++e) zero[e] = (_Float16)0.f;
+  for (int kt = 0; kt < CNN_KT1; ++kt) {
+    const int o = 4 * kt + g;
+    po[kt] = o < 27 ? ((o / 9) * 100 + ((o / 3) % 3) * 10 + o % 3) * 8 : 0;
+  }
+  const int base = (2 * w * 100 + (lr >> 3) * 10 + (lr & 7)) * 8;
+#pragma unroll 2
   for (int t = 0; t < 8; ++t) {
-    const int tile = 8 * w + t;
-    const int m = 16 * tile + lr;  // this lane's A row (cell)
-    const int mz = m >> 6, my = (m >> 3) & 7, mx = m & 7;
+    const _Float16* p = in + base + ((t >> 2) * 100 + (t & 3) * 20) * 8;
     float4_t acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int kt = 0; kt < KT; ++kt) {
-      const int o = L1 ? 4 * kt + g : 2 * kt + (g >> 1);
-      const int c0 = L1 ? 0 : 8 * (g & 1);
-      half8_t a = zero;
-      if (o < 27) {
-        const int dz = o / 9, dy = (o / 3) % 3, dx = o % 3;
-        if (L1) {
-          const int p = ((mz + dz) * 10 + (my + dy)) * 10 + (mx + dx);
-          a = *reinterpret_cast<const half8_t*>(&in[p * 8]);
-        } else {
-          const int z = mz + dz - 1, y = my + dy - 1, x = mx + dx - 1;
-          const bool inside = (unsigned)z < 8u && (unsigned)y < 8u && (unsigned)x < 8u;
-          const int p = inside ? (z * 8 + y) * 8 + x : 0;
-          const half8_t v = *reinterpret_cast<const half8_t*>(&in[p * CNN_C + c0]);
-          a = inside ? v : zero;
-        }
+    for (int kt = 0; kt < CNN_KT1; ++kt) {
+      half8_t a = *reinterpret_cast<const half8_t*>(p + po[kt]);
+      if (kt == CNN_KT1 - 1 && g == 3) {  // there is no tap 27
+#pragma unroll
+        for (int e = 0; e < 8; ++e) a[e] = (_Float16)0.f;
       }
       acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bq[kt], acc, 0, 0, 0);
     }
-    // register q of lane l holds D[4*(l/16) + q][l % 16]
+    f(t, acc);
+  }
+}
+
+// Layers 2 and 3 (same): 2 taps a k-step, taps 2 kt and 2 kt + 1 in the lower
+// and upper lanes. The two taps of a step are 1, 7 or 61 cells apart, so three
+// base addresses and immediate offsets reach every operand.
+template <typename F>
+__device__ __forceinline__ void conv_same(const _Float16* __restrict__ in,
+                                          const half8_t* __restrict__ wfrag, int w, int l, F&& f) {
+  constexpr int KT = CNN_KT2;
+  static_assert(CNN_KT2 == CNN_KT3 && CNN_C == 16, "two taps of 16 channels a k-step");
+  const int lr = l & 15, g = l >> 4, hi = g >> 1;
+  half8_t bq[KT];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) f(16 * tile + 4 * g + q, lr, acc[q]);
+  for (int kt = 0; kt < KT; ++kt) bq[kt] = wfrag[kt * 64 + l];
+  const int base =
+      (2 * w * APLANE + (lr >> 3) * AROW + (lr & 7)) * CNN_C + 8 * (g & 1);
+  const _Float16* p1 = in + base + hi * CNN_C;
+  const _Float16* p7 = in + base + hi * 7 * CNN_C;
+  const _Float16* p61 = in + base + hi * 61 * CNN_C;
+#pragma unroll 2
+  for (int t = 0; t < 8; ++t) {
+    const int to = ((t >> 2) * APLANE + (t & 3) * 2 * AROW) * CNN_C;
+    float4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt) {
+      const int d = 2 * kt + 1 < 27 ? atap(2 * kt + 1) - atap(2 * kt) : 0;
+      const _Float16* p = d == 7 ? p7 : (d == 61 ? p61 : p1);
+      // there is no tap 27: the upper lanes read the ring's first (zero) cell
+      if (kt == KT - 1) p = hi ? in - to - atap(2 * kt) * CNN_C : p1;
+      const half8_t a = *reinterpret_cast<const half8_t*>(p + to + atap(2 * kt) * CNN_C);
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bq[kt], acc, 0, 0, 0);
+    }
+    f(t, acc);
+  }
+}
+
+// Zero the ring of an activation buffer (the 512 cells are written by a layer).
+__device__ __forceinline__ void zero_ring(_Float16* buf, int tid) {
+  half8_t zero;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) zero[e] = (_Float16)0.f;
+  for (int i = tid; i < 2 * ACELLS; i += WG_THREADS) {
+    const int c = i >> 1, r = c % APLANE;
+    if (c < APLANE || c >= 9 * APLANE || r < AROW || r % AROW == 0)
+      *reinterpret_cast<half8_t*>(&buf[i * 8]) = zero;
   }
 }
 
 // LDS of the inference: the input patch (1000 cells x 8 halfs), later the
-// second layer's activations (512 x 16), and the first layer's (512 x 16):
-// 32 KiB per workgroup, five workgroups per CU.
-constexpr int CNN_IN_HALFS = PADC * 8 > BLEN * CNN_C ? PADC * 8 : BLEN * CNN_C;
+// second layer's activations, and the first layer's: 52 KiB per workgroup,
+// three workgroups per CU. What the kernel takes is mostly the exact GELU of
+// 16 384 values a block (about 36 vector instructions each): it ran at 328 us
+// on 8192 blocks with the zero padding selected per operand (20 instructions a
+// read) and runs at about 230 us with it built into the layout.
+constexpr int CNN_IN_HALFS = PADC * 8 > ACELLS * CNN_C ? PADC * 8 : ACELLS * CNN_C;
 
 __global__ __launch_bounds__(WG_THREADS) void k_cnn_infer(int nb, const int* __restrict__ nbr,
                                                           const double* __restrict__ h,
@@ -216,11 +282,11 @@ __global__ __launch_bounds__(WG_THREADS) void k_cnn_infer(int nb, const int* __r
                                                           const _Float16* __restrict__ wpk,
                                                           const float* __restrict__ w,
                                                           double* __restrict__ out) {
-  __shared__ __attribute__((aligned(16))) _Float16 bufIn[CNN_IN_HALFS];  // input, then act2
-  __shared__ __attribute__((aligned(16))) _Float16 bufA[BLEN * CNN_C];   // act1
+  __shared__ __attribute__((aligned(16))) _Float16 bufIn[CNN_IN_HALFS];     // input, then act2
+  __shared__ __attribute__((aligned(16))) _Float16 bufA[ACELLS * CNN_C];  // act1, then the output
   const int b = xcd_remap(blockIdx.x, gridDim.x);
   if (b >= nb) return;
-  const int tid = threadIdx.x, wv = tid >> 6, l = tid & 63;
+  const int tid = threadIdx.x, wv = tid >> 6, l = tid & 63, lr = l & 15, g = l >> 4;
   const double s_r = scal[0];
   const float inv_sp = (float)(1.0 / scal[1]);
   const float inv_hs = (float)(1.0 / (h[b] * s_r));
@@ -240,6 +306,7 @@ __global__ __launch_bounds__(WG_THREADS) void k_cnn_infer(int nb, const int* __r
     rv[j] = res[gi[j]];
     pv[j] = prev[gi[j]];
   }
+  zero_ring(bufA, tid);
 #pragma unroll
   for (int j = 0; j < NP; ++j) {
     const int p = tid + j * WG_THREADS;
@@ -254,20 +321,28 @@ __global__ __launch_bounds__(WG_THREADS) void k_cnn_infer(int nb, const int* __r
   }
   __syncthreads();
   const half8_t* wf = reinterpret_cast<const half8_t*>(wpk);
-  conv_layer<CNN_KT1, true>(bufIn, wf, wv, l, [&](int m, int n, float v) {
-    bufA[m * CNN_C + n] = (_Float16)gelu(v + w[CNN_OB1 + n]);
+  // this lane's output rows in tile 0: cells (y, x) = (g / 2, 4 (g % 2) + q)
+  const int orow = ((2 * wv + 1) * APLANE + ((g >> 1) + 1) * AROW + 4 * (g & 1) + 1) * CNN_C + lr;
+  auto store = [&](_Float16* buf, float bias, int t, const float4_t& acc) {
+    _Float16* p = buf + orow + ((t >> 2) * APLANE + (t & 3) * 2 * AROW) * CNN_C;
+    tile_rows(acc, [&](int q, float v) { p[q * CNN_C] = (_Float16)gelu(v + bias); });
+  };
+  const float b1 = w[CNN_OB1 + lr], b2 = w[CNN_OB2 + lr], b3 = w[CNN_OB3];
+  conv_first(bufIn, wf, wv, l, [&](int t, const float4_t& acc) { store(bufA, b1, t, acc); });
+  __syncthreads();
+  zero_ring(bufIn, tid);
+  conv_same(bufA, wf + CNN_KT1 * 64, wv, l,
+            [&](int t, const float4_t& acc) { store(bufIn, b2, t, acc); });
+  __syncthreads();
+  float* po = reinterpret_cast<float*>(bufA);
+  conv_same(bufIn, wf + (CNN_KT1 + CNN_KT2) * 64, wv, l, [&](int t, const float4_t& acc) {
+    if (lr == 0) tile_rows(acc, [&](int q, float v) { po[128 * wv + 16 * t + 4 * g + q] = v; });
   });
   __syncthreads();
-  conv_layer<CNN_KT2, false>(bufA, wf + CNN_KT1 * 64, wv, l, [&](int m, int n, float v) {
-    bufIn[m * CNN_C + n] = (_Float16)gelu(v + w[CNN_OB2 + n]);
-  });
-  __syncthreads();
-  const float b3 = w[CNN_OB3];
   const size_t off = (size_t)b * BLEN;
-  conv_layer<CNN_KT3, false>(bufIn, wf + (CNN_KT1 + CNN_KT2) * 64, wv, l,
-                             [&](int m, int n, float v) {
-                               if (n == 0) out[off + m] = prev[off + m] + s_r * (double)(v + b3);
-                             });
+#pragma unroll
+  for (int m = tid; m < BLEN; m += WG_THREADS)
+    out[off + m] = prev[off + m] + s_r * (double)(po[m] + b3);
 }
 
 // ---------------------------------------------------------------------------
@@ -837,12 +912,13 @@ static int scales(CnnState& C, hipStream_t s, const double* res, const double* p
 }
 
 int cnn_predict(CnnState& C, hipStream_t s, const double* d_res, const double* d_prev,
-                double* d_out, std::string& err) {
+                double* d_out, std::string& err, const double* sums) {
   if (!C.have_weights) {
     err = "cnn_predict: no weights (set or train them first)";
     return -1;
   }
-  if (scales(C, s, d_res, d_prev, err)) return -1;
+  if (sums) k_cnn_scales_fin<<<1, WG_THREADS, 0, s>>>(C.n, C.d_scal, sums, (C.nb + 3) / 4);
+  else if (scales(C, s, d_res, d_prev, err)) return -1;
   k_cnn_infer<<<C.nb, WG_THREADS, 0, s>>>(C.nb, C.d_nbr, C.d_h, d_res, d_prev, C.d_scal,
                                           static_cast<const _Float16*>(C.d_wpk), C.d_w, d_out);
   CCHECK(hipGetLastError());

@@ -14,10 +14,11 @@ namespace cup3d {
 // RESID  c = a - A x, |c|^2
 // START  y = c = c2 = -h^3 sigma a - A x, its norm (Helmholtz grids; x and a are
 //        one component of an [n][3] field)
+// NET    c = a - A x, |c / h|^2, |x|^2 (bMean 0)
 // FINAL  |a - A x|^2 of the best iterate x (g.xo, the state), copied to y (may be null)
 enum SpmvMode {
   SPMV_PLAIN = 0, SPMV_INIT = 1, SPMV_DOT1 = 2, SPMV_DOT2 = 3, SPMV_RESID = 4, SPMV_START = 5,
-  SPMV_FINAL = 6
+  SPMV_FINAL = 6, SPMV_NET = 7
 };
 enum PrecMode { PREC_PLAIN = 0, PREC_P = 1, PREC_S = 2 };
 

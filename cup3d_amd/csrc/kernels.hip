@@ -59,6 +59,7 @@ void launch_spmv64(hipStream_t s, int mode, const DevGrid<double>& g, const doub
     case SPMV_DOT2: spmv_launch<double, SPMV_DOT2>(s, g, x, y, a, c, c2, st, part, fin); break;
     case SPMV_RESID: spmv_launch<double, SPMV_RESID>(s, g, x, y, a, c, c2, st, part, fin); break;
     case SPMV_START: spmv_launch<double, SPMV_START>(s, g, x, y, a, c, c2, st, part, false); break;
+    case SPMV_NET: spmv_launch<double, SPMV_NET>(s, g, x, y, a, c, c2, st, part, false); break;
     case SPMV_FINAL: spmv_launch<double, SPMV_FINAL>(s, g, x, y, a, c, c2, st, part, fin); break;
   }
 }

@@ -445,7 +445,7 @@ template <int MODE, int BM>
 struct SpmvSums {
   static constexpr int MEAN = BM == 1 || BM == 2 ? 1 : 0;
   static constexpr int DOTS =
-      MODE == SPMV_PLAIN ? 0 : (MODE == SPMV_INIT || MODE == SPMV_DOT2 ? 2 : 1);
+      MODE == SPMV_PLAIN ? 0 : (MODE == SPMV_INIT || MODE == SPMV_DOT2 || MODE == SPMV_NET ? 2 : 1);
   static constexpr int N = MEAN + DOTS;
 };
 
@@ -605,6 +605,7 @@ __global__ __launch_bounds__(WG_THREADS) void k_spmv(DevGrid<T> g, const T* __re
   // epilogue: stores and partial sums
   double v[3] = {0.0, 0.0, 0.0};  // sum h^3 x, then the dots
   if (valid) {
+    const T ih = MODE == SPMV_NET ? g.invh[b] : (T)0;
     if (NEED_SUM) v[0] = (double)h * (double)h * (double)h * msum;
     // the row's other factor, for the kernel that completes the dot (FIN_ROW)
     if (BM == 1 && (MODE == SPMV_DOT1 || MODE == SPMV_DOT2) && origin && lane == 0)
@@ -640,6 +641,11 @@ __global__ __launch_bounds__(WG_THREADS) void k_spmv(DevGrid<T> g, const T* __re
         const T rr = av[iz] - yy;
         c[i] = rr;
         v[1] += (double)rr * (double)rr;
+      } else if (MODE == SPMV_NET) {
+        const T rr = av[iz] - yy, rh = rr * ih;
+        c[i] = rr;
+        v[1] += (double)rh * (double)rh;
+        v[2] += (double)col[iz] * (double)col[iz];
       } else if (MODE == SPMV_START) {
         const T rr = -(h * h * h) * (T)g.helm_sigma * av[iz] - yy;
         y[i] = rr;
@@ -850,6 +856,8 @@ inline void spmv_launch(hipStream_t s, const DevGrid<T>& g, const T* x, T* y, co
     }
   }
   if constexpr (MODE == SPMV_START) return;  // Helmholtz grids only
+  else if constexpr (MODE == SPMV_NET)
+    spmv_launch_iface<T, MODE, 0>(s, g, x, y, a, c, c2, st, part, fin, mid);
   else
   if (g.bmean == 1) spmv_launch_iface<T, MODE, 1>(s, g, x, y, a, c, c2, st, part, fin, mid);
   else if (g.bmean == 2) spmv_launch_iface<T, MODE, 2>(s, g, x, y, a, c, c2, st, part, fin, mid);

@@ -1150,6 +1150,16 @@ int cup3d_poisson_cnn_predict(cup3d_poisson_t H, const double* d_rhs, const doub
   if (H->nb <= 0) return fail(H, "set_topology must be called first");
   if (check_vectors(H, {d_rhs, d_prev, d_out}) != 0) return -1;
   HIPCHECK(hipSetDevice(H->device));
+  // With no mean-constraint cell the residual and both scales are one pass over
+  // rhs and prev (unless out overlaps prev, which the net still reads)
+  const uintptr_t po = (uintptr_t)d_out, pp = (uintptr_t)d_prev, len = H->n * sizeof(double);
+  if (H->cfg.bmean == 0 && !(po < pp + len && pp < po + len)) {
+    launch_spmv64(H->stream, SPMV_NET, H->g64, d_prev, nullptr, d_rhs, H->v64.nu, nullptr, nullptr,
+                  H->d_part.as<double>());
+    HIPCHECK(hipGetLastError());
+    return cnn_predict(H->cnn, H->stream, H->v64.nu, d_prev, d_out, H->err,
+                       H->d_part.as<double>());
+  }
   if (increment_residual(H, d_rhs, d_prev) < 0) return -1;
   return cnn_predict(H->cnn, H->stream, H->v64.nu, H->v64.x[0], d_out, H->err);
 }
