@@ -218,12 +218,13 @@ __device__ __forceinline__ void store8(T* __restrict__ p, const T (&v)[8]) {
 
 // Start from x0 = 0: b = r = rhat = rhs without an operator application. The
 // sum is taken as the SpMV's residual mode takes it (a column of eight cells
-// per lane), so |r| has the same bits as through A x0.
+// per lane, the workgroups in the SpMV's order), so |r| has the same bits as
+// through A x0.
 [[maybe_unused]] static __global__ __launch_bounds__(WG_THREADS) void k_start_zero(
     int nb, long long zero_row, const double* __restrict__ rhs, double* __restrict__ b,
     double* __restrict__ r, double* __restrict__ rhat, double* __restrict__ x, double* part) {
   double v[1] = {0.0};
-  const int blk = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int blk = xcd_remap(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6);
   if (blk < nb) {
     const long long off = (long long)blk * BLEN + (threadIdx.x & 63);
     double q[BS];
