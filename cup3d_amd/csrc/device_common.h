@@ -29,9 +29,38 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_wave_barrier();
 }
 
+// v of the lane o away within the wavefront, o = 1, 2, 4 or 8, as a DPP move;
+// for o = 4 v must already be equal in lanes 8 apart (a rotation by 4 in a row
+// of 16 then reads the value of lane i ^ 4).
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double v) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+
+// Butterfly sum over the wavefront, lanes 32, 16, 8, 4, 2, 1 apart. Register
+// moves (v_permlane32_swap, v_permlane16_swap, DPP) instead of shuffles through
+// the LDS crossbar: the sum is the tail of every kernel with a reduction and
+// the head of those that use one (32^3 cells, 10 iterations
+// of five kernels: 387 -> 359 us with the state written to the host by the
+// finalize kernels too); the order of the additions, and so
+// the bits, are those of the shuffles.
 __device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  {
+    const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(v), __double2loint(v), false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(v), __double2hiint(v), false, false);
+    v = __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+  }
+  {
+    const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(v), __double2loint(v), false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(v), __double2hiint(v), false, false);
+    v = __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+  }
+  v += dpp_move<0x128>(v);  // row_ror:8
+  v += dpp_move<0x124>(v);  // row_ror:4
+  v += dpp_move<0x4e>(v);   // quad_perm [2, 3, 0, 1]
+  v += dpp_move<0xb1>(v);   // quad_perm [1, 0, 3, 2]
   return v;
 }
 

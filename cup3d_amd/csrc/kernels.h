@@ -40,7 +40,9 @@ inline int fin_mode(int nb, int bmean, long long row) {
 }
 // The sums of K5 lie behind those of the SpMVs, which K5 still reads.
 inline double* k5_part(double* part, int nb) { return part + 4 * (size_t)((nb + 3) / 4 + 8); }
-// Copies of the solver state (krylov.h): st[0] is the one the host reads.
+// Copies of the solver state (krylov.h): st[0] is the one that counts between
+// batches of iterations. hst, where a launch takes it: the host's pinned copy,
+// written by the finalize kernel.
 constexpr int STATE_COPIES = 3;
 
 // The state starts as `init`, with ||b|| and the absolute tolerance.
@@ -52,18 +54,19 @@ void launch_getvec64(hipStream_t s, long long n, long long zero_row, const doubl
 // scalars.
 void launch_start_zero64(hipStream_t s, int nb, long long zero_row, const double* rhs, double* b,
                          double* r, double* rhat, double* x, const SolverState& init,
-                         SolverState* st, double* part, double tol_b);
+                         SolverState* st, SolverState* hst, double* part, double tol_b);
 // The scalars of SPMV_START (nb blocks).
 void launch_start_fin(hipStream_t s, int nb, const SolverState& init, SolverState* st,
-                      const double* part, double tol_b);
+                      SolverState* hst, const double* part, double tol_b);
 // part null (SPMV_PLAIN and SPMV_RESID on a grid with bMean 0 or 3, SPMV_FINAL for
 // its copy): no sums are taken.
 void launch_spmv64(hipStream_t s, int mode, const DevGrid<double>& g, const double* x, double* y,
                    const double* a, double* c, double* c2, SolverState* st, double* part,
-                   bool fin = true);
+                   bool fin = true, SolverState* hst = nullptr);
 // K5; returns its number of partials. last: with its finalize kernel.
 int launch_update64(hipStream_t s, const DevGrid<double>& g, const KrylovVectors<double>& v,
-                    SolverState* st, double* part, int fin = FIN_KERNEL, bool last = true);
+                    SolverState* st, double* part, int fin = FIN_KERNEL, bool last = true,
+                    SolverState* hst = nullptr);
 
 // The caller around the solve (projection.hip): the rhs of the pressure
 // equation from the velocity (and an obstacle's udef / chi, both or neither

@@ -39,34 +39,34 @@ void launch_getvec64(hipStream_t s, long long n, long long zero_row, const doubl
 
 void launch_start_zero64(hipStream_t s, int nb, long long zero_row, const double* rhs, double* b,
                          double* r, double* rhat, double* x, const SolverState& init,
-                         SolverState* st, double* part, double tol_b) {
+                         SolverState* st, SolverState* hst, double* part, double tol_b) {
   k_start_zero<<<(nb + 3) / 4, WG_THREADS, 0, s>>>(nb, zero_row, rhs, b, r, rhat, x, part);
-  launch_start_fin(s, nb, init, st, part, tol_b);
+  launch_start_fin(s, nb, init, st, hst, part, tol_b);
 }
 
 void launch_start_fin(hipStream_t s, int nb, const SolverState& init, SolverState* st,
-                      const double* part, double tol_b) {
-  k_start_fin<<<1, WG_THREADS, 0, s>>>(init, st, part, (nb + 3) / 4, tol_b);
+                      SolverState* hst, const double* part, double tol_b) {
+  k_start_fin<<<1, WG_THREADS, 0, s>>>(init, st, hst, part, (nb + 3) / 4, tol_b);
 }
 
 void launch_spmv64(hipStream_t s, int mode, const DevGrid<double>& g, const double* x, double* y,
                    const double* a, double* c, double* c2, SolverState* st, double* part,
-                   bool fin) {
+                   bool fin, SolverState* hst) {
   switch (mode) {
-    case SPMV_PLAIN: spmv_launch<double, SPMV_PLAIN>(s, g, x, y, a, c, c2, st, part, fin); break;
-    case SPMV_INIT: spmv_launch<double, SPMV_INIT>(s, g, x, y, a, c, c2, st, part, fin); break;
-    case SPMV_DOT1: spmv_launch<double, SPMV_DOT1>(s, g, x, y, a, c, c2, st, part, fin); break;
-    case SPMV_DOT2: spmv_launch<double, SPMV_DOT2>(s, g, x, y, a, c, c2, st, part, fin); break;
-    case SPMV_RESID: spmv_launch<double, SPMV_RESID>(s, g, x, y, a, c, c2, st, part, fin); break;
+    case SPMV_PLAIN: spmv_launch<double, SPMV_PLAIN>(s, g, x, y, a, c, c2, st, part, fin, hst); break;
+    case SPMV_INIT: spmv_launch<double, SPMV_INIT>(s, g, x, y, a, c, c2, st, part, fin, hst); break;
+    case SPMV_DOT1: spmv_launch<double, SPMV_DOT1>(s, g, x, y, a, c, c2, st, part, fin, hst); break;
+    case SPMV_DOT2: spmv_launch<double, SPMV_DOT2>(s, g, x, y, a, c, c2, st, part, fin, hst); break;
+    case SPMV_RESID: spmv_launch<double, SPMV_RESID>(s, g, x, y, a, c, c2, st, part, fin, hst); break;
     case SPMV_START: spmv_launch<double, SPMV_START>(s, g, x, y, a, c, c2, st, part, false); break;
     case SPMV_NET: spmv_launch<double, SPMV_NET>(s, g, x, y, a, c, c2, st, part, false); break;
-    case SPMV_FINAL: spmv_launch<double, SPMV_FINAL>(s, g, x, y, a, c, c2, st, part, fin); break;
+    case SPMV_FINAL: spmv_launch<double, SPMV_FINAL>(s, g, x, y, a, c, c2, st, part, fin, hst); break;
   }
 }
 
 int launch_update64(hipStream_t s, const DevGrid<double>& g, const KrylovVectors<double>& v,
-                    SolverState* st, double* part, int fin, bool last) {
-  return launch_k5<double>(s, g, v, st, part, fin, last);
+                    SolverState* st, double* part, int fin, bool last, SolverState* hst) {
+  return launch_k5<double>(s, g, v, st, part, fin, last, hst);
 }
 
 // ---------------------------------------------------------------------------

@@ -59,11 +59,16 @@ __device__ __forceinline__ void fin_load(const SolverState* st, SolverState& S,
   grid_sum_partials<K>(part, nparts, tot);  // ends with a barrier
 }
 
-__device__ __forceinline__ void fin_store(SolverState* st, const SolverState& S) {
+// hst: the host's copy (pinned memory, null: none), complete when the kernel is;
+// a copy of 200 bytes after the kernel takes about 5 us more.
+__device__ __forceinline__ void fin_store(SolverState* st, const SolverState& S,
+                                          SolverState* hst = nullptr) {
   __syncthreads();
-  if (threadIdx.x < STATE_WORDS)
-    reinterpret_cast<unsigned*>(st)[threadIdx.x] =
-        reinterpret_cast<const unsigned*>(&S)[threadIdx.x];
+  if (threadIdx.x < STATE_WORDS) {
+    const unsigned u = reinterpret_cast<const unsigned*>(&S)[threadIdx.x];
+    reinterpret_cast<unsigned*>(st)[threadIdx.x] = u;
+    if (hst) reinterpret_cast<unsigned*>(hst)[threadIdx.x] = u;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -246,7 +251,8 @@ __device__ __forceinline__ void store8(T* __restrict__ p, const T (&v)[8]) {
 
 // The first iteration's scalars for a zero guess, |b|^2 = |r|^2 = the sum.
 [[maybe_unused]] static __global__ __launch_bounds__(WG_THREADS) void k_start_fin(
-    SolverState init, SolverState* st, const double* part, int nparts, double tol_b) {
+    SolverState init, SolverState* st, SolverState* hst, const double* part, int nparts,
+    double tol_b) {
   __shared__ SolverState S;
   double tot[1];
   grid_sum_partials<1>(part, nparts, tot);
@@ -259,7 +265,7 @@ __device__ __forceinline__ void store8(T* __restrict__ p, const T (&v)[8]) {
     S.x_zero = S.opt_zero = 1;
     begin_iteration(&S, tot[0], tot[0]);
   }
-  fin_store(st, S);
+  fin_store(st, S, hst);
 }
 
 // ---------------------------------------------------------------------------
@@ -675,8 +681,8 @@ template <typename T, int MODE, int BM>
 __global__ __launch_bounds__(WG_THREADS) void k_spmv_fin(long long row, T* __restrict__ y,
                                                          const T* __restrict__ a,
                                                          T* __restrict__ c, T* __restrict__ c2,
-                                                         SolverState* st, const double* part,
-                                                         int nparts) {
+                                                         SolverState* st, SolverState* hst,
+                                                         const double* part, int nparts) {
   using Sums = SpmvSums<MODE, BM>;
   __shared__ SolverState S;
   double sums[Sums::N], tot[3] = {0.0, 0.0, 0.0};
@@ -730,7 +736,7 @@ __global__ __launch_bounds__(WG_THREADS) void k_spmv_fin(long long row, T* __res
       S.true_rr = tot[1];
     }
   }
-  fin_store(st, S);
+  fin_store(st, S, hst);
 }
 
 // bMeanConstraint = 2 (hd_cusparseSpMV, BiCGSTAB.cu:392-411):
@@ -822,7 +828,7 @@ inline void spmv_kernel(hipStream_t s, int nwg, const DevGrid<T>& g, const T* x,
 template <typename T, int MODE, int BM, bool HELM = false>
 inline void spmv_launch_iface(hipStream_t s, const DevGrid<T>& g, const T* x, T* y, const T* a,
                               T* c, T* c2, SolverState* st, double* part, bool fin,
-                              hipEvent_t mid = nullptr) {
+                              SolverState* hst, hipEvent_t mid = nullptr) {
   int nwg = (g.nb + 3) / 4;
   bool launched = false;
   if constexpr (MODE == SPMV_DOT1 || MODE == SPMV_DOT2) {  // the per-iteration SpMVs
@@ -844,26 +850,26 @@ inline void spmv_launch_iface(hipStream_t s, const DevGrid<T>& g, const T* x, T*
     k_bmean2_apply<T, MODE><<<nwg, WG_THREADS, 0, s>>>(g, y, a, c, c2, st, part);
   }
   if constexpr (SpmvSums<MODE, BM>::N > 0)
-    k_spmv_fin<T, MODE, BM><<<1, WG_THREADS, 0, s>>>(g.bmean_row, y, a, c, c2, st, part, nwg);
+    k_spmv_fin<T, MODE, BM><<<1, WG_THREADS, 0, s>>>(g.bmean_row, y, a, c, c2, st, hst, part, nwg);
 }
 template <typename T, int MODE>
 inline void spmv_launch(hipStream_t s, const DevGrid<T>& g, const T* x, T* y, const T* a, T* c,
                         T* c2, SolverState* st, double* part, bool fin = true,
-                        hipEvent_t mid = nullptr) {
+                        SolverState* hst = nullptr, hipEvent_t mid = nullptr) {
   if constexpr (sizeof(T) == 8) {
     if (g.helm) {  // implicit diffusion: no bMean row
-      spmv_launch_iface<T, MODE, 0, true>(s, g, x, y, a, c, c2, st, part, fin, mid);
+      spmv_launch_iface<T, MODE, 0, true>(s, g, x, y, a, c, c2, st, part, fin, hst, mid);
       return;
     }
   }
   if constexpr (MODE == SPMV_START) return;  // Helmholtz grids only
   else if constexpr (MODE == SPMV_NET)
-    spmv_launch_iface<T, MODE, 0>(s, g, x, y, a, c, c2, st, part, fin, mid);
+    spmv_launch_iface<T, MODE, 0>(s, g, x, y, a, c, c2, st, part, fin, hst, mid);
   else
-  if (g.bmean == 1) spmv_launch_iface<T, MODE, 1>(s, g, x, y, a, c, c2, st, part, fin, mid);
-  else if (g.bmean == 2) spmv_launch_iface<T, MODE, 2>(s, g, x, y, a, c, c2, st, part, fin, mid);
-  else if (g.bmean == 3) spmv_launch_iface<T, MODE, 3>(s, g, x, y, a, c, c2, st, part, fin, mid);
-  else spmv_launch_iface<T, MODE, 0>(s, g, x, y, a, c, c2, st, part, fin, mid);
+  if (g.bmean == 1) spmv_launch_iface<T, MODE, 1>(s, g, x, y, a, c, c2, st, part, fin, hst, mid);
+  else if (g.bmean == 2) spmv_launch_iface<T, MODE, 2>(s, g, x, y, a, c, c2, st, part, fin, hst, mid);
+  else if (g.bmean == 3) spmv_launch_iface<T, MODE, 3>(s, g, x, y, a, c, c2, st, part, fin, hst, mid);
+  else spmv_launch_iface<T, MODE, 0>(s, g, x, y, a, c, c2, st, part, fin, hst, mid);
 }
 
 // ---------------------------------------------------------------------------
@@ -961,13 +967,13 @@ __device__ inline void update_scalars(SolverState& S, double rho, double rr) {
 
 // src: the state before K5 (st, or the consumers' last copy), dst: after it.
 static __global__ __launch_bounds__(WG_THREADS) void k_update_fin(const SolverState* src,
-                                                           SolverState* dst, const double* part,
-                                                           int nparts) {
+                                                           SolverState* dst, SolverState* hst,
+                                                           const double* part, int nparts) {
   __shared__ SolverState S;
   double tot[2];
   fin_load<2>(src, S, part, nparts, tot);
   if (threadIdx.x == 0 && S.status == ST_RUNNING) update_scalars(S, tot[0], tot[1]);
-  fin_store(dst, S);
+  fin_store(dst, S, hst);
 }
 
 // K5 and, unless the next K1 takes its sums, the finalize kernel (an event, if
@@ -975,7 +981,7 @@ static __global__ __launch_bounds__(WG_THREADS) void k_update_fin(const SolverSt
 template <typename T>
 inline int launch_k5(hipStream_t s, const DevGrid<T>& g, const KrylovVectors<T>& v,
                      SolverState* st, double* part, int fin = FIN_KERNEL, bool last = true,
-                     hipEvent_t mid = nullptr) {
+                     SolverState* hst = nullptr, hipEvent_t mid = nullptr) {
   const long long n = g.n, runs = (n + 4 * BLEN - 1) / (4 * BLEN);
   const int ch = runs >= 8192 ? 2 : 1;
   const int nwg = (int)((runs + ch - 1) / ch);
@@ -986,7 +992,7 @@ inline int launch_k5(hipStream_t s, const DevGrid<T>& g, const KrylovVectors<T>&
   else if (ch == 2) k_update<T, 2, FIN_KERNEL><<<nwg, WG_THREADS, 0, s>>>(n, v, st, f, p5);
   else k_update<T, 1, FIN_KERNEL><<<nwg, WG_THREADS, 0, s>>>(n, v, st, f, p5);
   if (mid) (void)hipEventRecord(mid, s);
-  if (last) k_update_fin<<<1, WG_THREADS, 0, s>>>(fin ? st + 2 : st, st, p5, nwg);
+  if (last) k_update_fin<<<1, WG_THREADS, 0, s>>>(fin ? st + 2 : st, st, hst, p5, nwg);
   return nwg;
 }
 

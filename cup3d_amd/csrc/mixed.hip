@@ -581,7 +581,7 @@ void launch_precond_mixed(const MixedWorkspace& M, const KrylovVectors<float>& v
 template <int MODE>
 void spmv32(hipStream_t s, const DevGrid<float>& g, const float* x, float* y, const float* a,
             SolverState* st, double* part, bool fin = true, hipEvent_t mid = nullptr) {
-  spmv_launch<float, MODE>(s, g, x, y, a, nullptr, nullptr, st, part, fin, mid);
+  spmv_launch<float, MODE>(s, g, x, y, a, nullptr, nullptr, st, part, fin, nullptr, mid);
 }
 
 int grid_1d(long long n) { return (int)std::min<long long>((n + WG_THREADS - 1) / WG_THREADS, 8192); }
@@ -685,8 +685,8 @@ int mixed_solve(MixedWorkspace& M, hipStream_t s, const cup3d_poisson_config& cf
   int total_iters = 0, total_restarts = 0, steps = 0, replacements = 0, status = ST_MAXITER;
   const int poll = cfg.poll_every > 0 ? cfg.poll_every : 8;
   auto true_resid = [&](double& out) -> int {  // |b - A x64| in FP64, r64 = b - A x64
-    launch_spmv64(s, SPMV_RESID, g64, x64, nullptr, b64, r64, nullptr, st, part);
-    MCHECK(hipMemcpyAsync(h_st, st, sizeof(SolverState), hipMemcpyDeviceToHost, s));
+    launch_spmv64(s, SPMV_RESID, g64, x64, nullptr, b64, r64, nullptr, st, part, true, h_st);
+    MCHECK(hipGetLastError());
     MCHECK(hipStreamSynchronize(s));
     out = std::sqrt(h_st->true_rr);
     return 0;
@@ -696,10 +696,9 @@ int mixed_solve(MixedWorkspace& M, hipStream_t s, const cup3d_poisson_config& cf
     launch_getvec64(s, n, zero_row, d_rhs, d_x0, b64, x64, init, st, part, cfg.tol_rhs);
     if (true_resid(rnorm)) return -1;
   } else {  // r64 = b64, without the operator
-    launch_start_zero64(s, M.nb, zero_row, d_rhs, b64, r64, nullptr, x64, init, st, part,
+    launch_start_zero64(s, M.nb, zero_row, d_rhs, b64, r64, nullptr, x64, init, st, h_st, part,
                         cfg.tol_rhs);
     MCHECK(hipGetLastError());
-    MCHECK(hipMemcpyAsync(h_st, st, sizeof(SolverState), hipMemcpyDeviceToHost, s));
     MCHECK(hipStreamSynchronize(s));
     rnorm = std::sqrt(h_st->true_rr);
   }
@@ -773,10 +772,9 @@ int mixed_solve(MixedWorkspace& M, hipStream_t s, const cup3d_poisson_config& cf
         spmv32<SPMV_DOT2>(s, g32, v.z2, v.t, v.s, st, part, !fin, tm ? M.pev[7] : nullptr);
         if (tm) MCHECK(hipEventRecord(M.pev[8], s));
         fp.nparts = launch_k5<float>(s, g32, v, st, part, fin, !fin || it == batch - 1,
-                                     tm ? M.pev[9] : nullptr);
+                                     it == batch - 1 ? h_st : nullptr, tm ? M.pev[9] : nullptr);
       }
       MCHECK(hipGetLastError());
-      MCHECK(hipMemcpyAsync(h_st, st, sizeof(SolverState), hipMemcpyDeviceToHost, s));
       MCHECK(hipStreamSynchronize(s));
       if (M.prof && h_st->iter - iter0 > tm_it) {
         for (int k = 0; k < 5; ++k) {
@@ -841,8 +839,6 @@ int mixed_solve(MixedWorkspace& M, hipStream_t s, const cup3d_poisson_config& cf
       }
       break;
     }
-    MCHECK(hipMemcpyAsync(h_st, st, sizeof(SolverState), hipMemcpyDeviceToHost, s));
-    MCHECK(hipStreamSynchronize(s));
     total_iters += h_st->iters_done;
     total_restarts += h_st->restarts;
   }

@@ -226,11 +226,11 @@ int run_bicgstab64(cup3d_poisson* H, const DevGrid<double>& g, const KrylovVecto
       launch_spmv64(s, SPMV_DOT1, g, v.z1, v.nu, v.rhat, nullptr, nullptr, st, part, !fin);
       launch_precond_fp64(H, g, PREC_S, v, fin, fs);
       launch_spmv64(s, SPMV_DOT2, g, v.z2, v.t, v.r, nullptr, nullptr, st, part, !fin);
-      fp.nparts = launch_update64(s, g, v, st, part, fin, !fin || k == batch - 1);
+      fp.nparts = launch_update64(s, g, v, st, part, fin, !fin || k == batch - 1,
+                                  k == batch - 1 ? H->h_state : nullptr);
     }
     launched += batch;
     HIPCHECK(hipGetLastError());
-    HIPCHECK(hipMemcpyAsync(H->h_state, st, sizeof(SolverState), hipMemcpyDeviceToHost, s));
     HIPCHECK(hipStreamSynchronize(s));
     if (H->h_state->status != ST_RUNNING) break;
     if (launched > (long long)H->h_state->max_iter + 4LL * poll)
@@ -492,7 +492,8 @@ static void start64(cup3d_poisson_t H, const DevGrid<double>& g, const KrylovVec
   SolverState* st = H->d_state.as<SolverState>();
   double* part = H->d_part.as<double>();
   if (!d_x0) {
-    launch_start_zero64(s, H->nb, zero_row, d_rhs, v.b, v.r, v.rhat, nullptr, init, st, part, tol_b);
+    launch_start_zero64(s, H->nb, zero_row, d_rhs, v.b, v.r, v.rhat, nullptr, init, st, nullptr, part,
+                        tol_b);
     return;
   }
   launch_getvec64(s, H->n, zero_row, d_rhs, d_x0, v.b, v.x[0], init, st, part, tol_b);
@@ -500,7 +501,7 @@ static void start64(cup3d_poisson_t H, const DevGrid<double>& g, const KrylovVec
 }
 
 // The best iterate into d_out (null: left in its buffer) and its true residual
-// ||b - A x|| in FP64, in one pass; the state follows into h (pinned).
+// ||b - A x|| in FP64, in one pass; the state goes to h (pinned) too.
 static int finish64(cup3d_poisson_t H, DevGrid<double> g, const KrylovVectors<double>& v,
                     double* d_out, SolverState* h) {
   for (int k = 0; k < 3; ++k) g.xo[k] = v.x[k];
@@ -509,13 +510,12 @@ static int finish64(cup3d_poisson_t H, DevGrid<double> g, const KrylovVectors<do
     launch_spmv64(H->stream, SPMV_FINAL, g, nullptr, d_out ? d_out : v.p, v.b, nullptr, nullptr, st,
                   nullptr);
     launch_spmv64(H->stream, SPMV_RESID, g, d_out ? d_out : v.p, nullptr, v.b, v.nu, nullptr, st,
-                  H->d_part.as<double>());
+                  H->d_part.as<double>(), true, h);
   } else {
     launch_spmv64(H->stream, SPMV_FINAL, g, nullptr, d_out, v.b, nullptr, nullptr, st,
-                  H->d_part.as<double>());
+                  H->d_part.as<double>(), true, h);
   }
   HIPCHECK(hipGetLastError());
-  HIPCHECK(hipMemcpyAsync(h, st, sizeof(SolverState), hipMemcpyDeviceToHost, H->stream));
   return 0;
 }
 
@@ -544,9 +544,8 @@ static double increment_residual(cup3d_poisson_t H, const double* d_rhs, const d
   launch_getvec64(s, H->n, zero_row, d_rhs, d_prev, H->v64.b, H->v64.x[0], make_state(H->cfg), st,
                   part, 0.0);
   launch_spmv64(s, SPMV_RESID, H->g64, H->v64.x[0], nullptr, H->v64.b, H->v64.nu, nullptr, st,
-                part);
-  if (hipMemcpyAsync(H->h_state, st, sizeof(SolverState), hipMemcpyDeviceToHost, s) != hipSuccess ||
-      hipStreamSynchronize(s) != hipSuccess)
+                part, true, H->h_state);
+  if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s) != hipSuccess)
     return fail(H, "increment residual failed");
   return std::sqrt(H->h_state->true_rr);
 }
@@ -1075,7 +1074,7 @@ int cup3d_diffusion_step_device(cup3d_poisson_t H, double nu, double dt, double 
       if (pool[k] != sol[0] && pool[k] != sol[1]) v.x[m++] = pool[k];
     HIPCHECK(hipEventRecord(ev[2 * c], s));
     launch_spmv64(s, SPMV_START, grid[c], d_vel + c, v.b, d_vel_old + c, v.r, v.rhat, st, part);
-    launch_start_fin(s, H->nb, init, st, part, 0.0);
+    launch_start_fin(s, H->nb, init, st, nullptr, part, 0.0);
     if (run_bicgstab64(H, grid[c], v, first_batch) != 0) return -1;
     const SolverState& S = *H->h_state;
     first_batch = std::max(1, S.iters_done);

@@ -381,3 +381,21 @@ def test_refined_solve_across_gemm_splits(gpu, bpd, bmean):
     x = torch.zeros_like(b)
     rep = S.solve_device(b, x)
     assert rep["status"] == 0 and rep["true_rel_resid"] <= 1e-8
+
+
+@pytest.mark.parametrize("bpd", [(5, 3, 2), (24, 20, 20)])
+def test_zero_guess_has_the_bits_of_given_zeros(gpu, bpd):
+    """The zero-guess start sums |r|^2 in the order of the residual A x0 takes,
+    so the FP32 solves from a zero guess and from given zeros are the same to
+    the bit (30 blocks and 9600, whose sums span many workgroups)."""
+    h0 = 1.0 / 64
+    blocks = W.uniform_blocks(*bpd)
+    b = torch.from_numpy(np.random.default_rng(4).standard_normal(len(blocks) * 512)).cuda()
+    out = []
+    for guess in ("given", "zero"):
+        S = PoissonSolver(bpd, h0, (2, 2, 2), bmean=0, precision="mixed_fp16", guess=guess,
+                          tol_rel=0.0, max_iter=4, max_refine=1).set_topology(blocks)
+        x = torch.zeros_like(b)
+        out.append((S.solve_device(b, x)["err_init"], x))
+    assert out[0][0] == out[1][0]
+    assert torch.equal(out[0][1], out[1][1])
