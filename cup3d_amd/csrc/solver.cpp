@@ -79,6 +79,7 @@ struct DevBuf {
 }  // namespace
 
 constexpr int HOST_STATES = 4;
+constexpr int COPY_THREADS = 16;
 
 // Device topology tables of one generation (topology_gpu.hip).
 struct DevTopo {
@@ -122,11 +123,13 @@ struct cup3d_poisson {
   // learned warm start
   CnnState cnn;
 
-  // staging of the host entry point: pinned rhs + x and their device copies,
-  // allocated by the first host solve on a topology and kept
-  double* h_stage = nullptr;  // 2 n doubles, pinned
+  // staging of the host entry point: device copies of rhs and x, and a pinned
+  // ring of two chunks per copying thread with an event each, allocated by the
+  // first host solve that needs them and kept
   DevBuf d_stage;             // 2 n doubles
-  long long stage_n = 0;
+  double* h_ring = nullptr;   // pinned
+  size_t ring_chunks = 0;
+  hipEvent_t ring_ev[2 * COPY_THREADS] = {};
 
   // warm start: the guesses handed in by the last cfg.extrapolate solves on
   // this topology (the caller's pressures of the previous steps), most
@@ -240,26 +243,108 @@ int run_bicgstab64(cup3d_poisson* H, const DevGrid<double>& g, const KrylovVecto
   return 0;
 }
 
-// Runs fn(b0, b1) over [0, nb) split into contiguous ranges on up to 16 host
-// threads (one for small grids): the gather and scatter of the host solve
-// are memory-bound copies that one core cannot feed at the host's bandwidth.
-template <typename F>
-void parallel_blocks(int nb, F&& fn) {
+// Host blocks <-> device vector of the host entry point. Contiguous ranges of
+// blocks on up to 16 host threads (one for small grids: one core cannot feed
+// PCIe), each copying chunk by chunk through its two slots of the pinned ring,
+// so that the copies of one chunk and the transfer of another overlap. On the
+// handle's stream; ends with every block copied (to the device: with every
+// transfer enqueued). A capped FP64 solve of 4440 blocks from and to host
+// arrays, zero guess: 2.34 ms, against 2.79 ms with whole vectors staged
+// between the copies and x uploaded too.
+constexpr int RING_BLOCKS = 256;  // 1 MiB
+
+int copy_range(cup3d_poisson* H, bool up, int t, int b0, int b1, double* dev,
+               double* const* blocks, double* contig) {
+  hipError_t e = hipSetDevice(H->device);
+  double* slot[2];
+  hipEvent_t ev[2];
+  for (int k = 0; k < 2; ++k) {
+    slot[k] = H->h_ring + (size_t)(2 * t + k) * RING_BLOCKS * BLEN;
+    ev[k] = H->ring_ev[2 * t + k];
+  }
+  const int chunks = (b1 - b0 + RING_BLOCKS - 1) / RING_BLOCKS;
+  auto range = [&](int c, int& c0, int& m) {
+    c0 = b0 + c * RING_BLOCKS;
+    m = std::min(RING_BLOCKS, b1 - c0);
+  };
+  auto host = [&](int b) { return blocks ? blocks[b] : contig + (size_t)b * BLEN; };
+  auto move = [&](int c, bool fill) {  // between the slot of chunk c and the host blocks
+    int c0, m;
+    range(c, c0, m);
+    double* p = slot[c & 1];
+    if (!blocks) {
+      std::memcpy(fill ? p : host(c0), fill ? host(c0) : p, (size_t)m * BLEN * sizeof(double));
+      return;
+    }
+    for (int b = 0; b < m; ++b)
+      std::memcpy(fill ? p + (size_t)b * BLEN : host(c0 + b),
+                  fill ? host(c0 + b) : p + (size_t)b * BLEN, BLEN * sizeof(double));
+  };
+  auto transfer = [&](int c) {
+    int c0, m;
+    range(c, c0, m);
+    const size_t bytes = (size_t)m * BLEN * sizeof(double);
+    double* d = dev + (size_t)c0 * BLEN;
+    e = up ? hipMemcpyAsync(d, slot[c & 1], bytes, hipMemcpyHostToDevice, H->stream)
+           : hipMemcpyAsync(slot[c & 1], d, bytes, hipMemcpyDeviceToHost, H->stream);
+    if (e == hipSuccess) e = hipEventRecord(ev[c & 1], H->stream);
+  };
+  if (up) {
+    for (int c = 0; c < chunks && e == hipSuccess; ++c) {
+      e = hipEventSynchronize(ev[c & 1]);  // the slot's last transfer (none yet: returns at once)
+      if (e == hipSuccess) {
+        move(c, true);
+        transfer(c);
+      }
+    }
+  } else {
+    for (int c = 0; c < std::min(2, chunks) && e == hipSuccess; ++c) transfer(c);
+    for (int c = 0; c < chunks && e == hipSuccess; ++c) {
+      e = hipEventSynchronize(ev[c & 1]);
+      if (e != hipSuccess) break;
+      move(c, false);
+      if (c + 2 < chunks) transfer(c + 2);
+    }
+  }
+  return (int)e;
+}
+
+int copy_blocks(cup3d_poisson* H, bool up, double* dev, double* const* blocks, double* contig) {
   const unsigned hw = std::max(1u, std::thread::hardware_concurrency());
-  const int nt = (int)std::min<unsigned>(std::min(hw, 16u), (unsigned)std::max(1, nb / 512));
-  if (nt <= 1) {
-    fn(0, nb);
-    return;
+  const int nb = H->nb;
+  const int nt = (int)std::min<unsigned>(std::min(hw, (unsigned)COPY_THREADS),
+                                        (unsigned)std::max(1, nb / 512));
+  if (H->ring_chunks < (size_t)2 * nt) {
+    if (H->h_ring) (void)hipHostFree(H->h_ring);
+    H->h_ring = nullptr;
+    H->ring_chunks = 0;
+    HIPCHECK(hipHostMalloc((void**)&H->h_ring,
+                           (size_t)2 * nt * RING_BLOCKS * BLEN * sizeof(double),
+                           hipHostMallocDefault));
+    H->ring_chunks = 2 * nt;
   }
-  std::vector<std::thread> pool;
-  pool.reserve(nt - 1);
+  for (int k = 0; k < 2 * nt; ++k)
+    if (!H->ring_ev[k])
+      HIPCHECK(hipEventCreateWithFlags(&H->ring_ev[k], hipEventDisableTiming));
   const int chunk = (nb + nt - 1) / nt;
-  for (int t = 1; t < nt; ++t) {
+  int err[COPY_THREADS] = {};
+  auto part = [&](int t) {
     const int b0 = t * chunk, b1 = std::min(nb, b0 + chunk);
-    if (b0 < b1) pool.emplace_back([&fn, b0, b1] { fn(b0, b1); });
+    if (b0 < b1) err[t] = copy_range(H, up, t, b0, b1, dev, blocks, contig);
+  };
+  std::thread pool[COPY_THREADS - 1];
+  int started = 1;
+  try {
+    for (; started < nt; ++started) pool[started - 1] = std::thread(part, started);
+  } catch (const std::exception&) {  // no more threads: the rest is done here
   }
-  fn(0, std::min(nb, chunk));
-  for (std::thread& th : pool) th.join();
+  part(0);
+  for (int t = started; t < nt; ++t) part(t);
+  for (int t = 1; t < started; ++t) pool[t - 1].join();
+  for (int t = 0; t < nt; ++t)
+    if (err[t] != hipSuccess)
+      return fail(H, std::string("host copy failed: ") + hipGetErrorString((hipError_t)err[t]));
+  return 0;
 }
 
 }  // namespace
@@ -832,44 +917,19 @@ int cup3d_poisson_solve(cup3d_poisson_t H, const double* const* rhs_blocks,
   if (H->nb <= 0) return fail(H, "set_topology must be called before solve");
   if ((!rhs_blocks && !rhs_contig) || (!x_blocks && !x_contig)) return fail(H, "null vector");
   HIPCHECK(hipSetDevice(H->device));
-  const size_t n = (size_t)H->n, bytes = n * sizeof(double);
-  if (H->stage_n != H->n) {
-    if (H->h_stage) (void)hipHostFree(H->h_stage);
-    H->h_stage = nullptr;
-    H->stage_n = 0;
-    H->d_stage.release();
-    HIPCHECK(hipHostMalloc((void**)&H->h_stage, 2 * bytes, hipHostMallocDefault));
-    if (H->d_stage.alloc(2 * bytes) != hipSuccess) return fail(H, "hipMalloc(staging) failed");
-    H->stage_n = H->n;
-  }
-  double *hb = H->h_stage, *hx = H->h_stage + n;
+  const size_t n = (size_t)H->n;
+  if (H->d_stage.reserve(2 * n * sizeof(double)) != hipSuccess)
+    return fail(H, "hipMalloc(staging) failed");
   double *db = H->d_stage.as<double>(), *dx = db + n;
-  // getVec gather (PoissonSolverExp.cpp:389-417)
-  parallel_blocks(H->nb, [&](int b0, int b1) {
-    for (int b = b0; b < b1; ++b) {
-      std::memcpy(hb + (size_t)b * BLEN,
-                  rhs_blocks ? rhs_blocks[b] : rhs_contig + (size_t)b * BLEN, BLEN * sizeof(double));
-      std::memcpy(hx + (size_t)b * BLEN, x_blocks ? x_blocks[b] : x_contig + (size_t)b * BLEN,
-                  BLEN * sizeof(double));
-    }
-  });
-  int st = -1;
-  if (hipMemcpy(db, hb, bytes, hipMemcpyHostToDevice) == hipSuccess &&
-      hipMemcpy(dx, hx, bytes, hipMemcpyHostToDevice) == hipSuccess) {
-    st = cup3d_poisson_solve_device(H, db, dx, rep);
-    if (st >= 0 && hipMemcpy(hx, dx, bytes, hipMemcpyDeviceToHost) == hipSuccess) {
-      // scatter into the pressure blocks (.cpp:452-472)
-      parallel_blocks(H->nb, [&](int b0, int b1) {
-        for (int b = b0; b < b1; ++b)
-          std::memcpy(x_blocks ? x_blocks[b] : x_contig + (size_t)b * BLEN, hx + (size_t)b * BLEN,
-                      BLEN * sizeof(double));
-      });
-    } else if (st >= 0) {
-      st = fail(H, "hipMemcpy D2H failed");
-    }
-  } else {
-    st = fail(H, "hipMemcpy H2D failed");
-  }
+  // getVec gather (PoissonSolverExp.cpp:389-417); with a zero guess x is not read
+  if (copy_blocks(H, true, db, const_cast<double* const*>(rhs_blocks),
+                  const_cast<double*>(rhs_contig)) != 0)
+    return -1;
+  if (H->cfg.guess != CUP3D_GUESS_ZERO && copy_blocks(H, true, dx, x_blocks, x_contig) != 0)
+    return -1;
+  const int st = cup3d_poisson_solve_device(H, db, dx, rep);
+  // scatter into the pressure blocks (.cpp:452-472)
+  if (st >= 0 && copy_blocks(H, false, dx, x_blocks, x_contig) != 0) return -1;
   return st;
 }
 
@@ -1353,7 +1413,9 @@ void cup3d_poisson_destroy(cup3d_poisson_t H) {
   cnn_free(H->cnn);
   mixed_free(H->mixed);
   if (H->h_state) (void)hipHostFree(H->h_state);
-  if (H->h_stage) (void)hipHostFree(H->h_stage);
+  if (H->h_ring) (void)hipHostFree(H->h_ring);
+  for (hipEvent_t e : H->ring_ev)
+    if (e) (void)hipEventDestroy(e);
   if (H->ev0) (void)hipEventDestroy(H->ev0);
   if (H->ev1) (void)hipEventDestroy(H->ev1);
   for (hipEvent_t e : H->evc)

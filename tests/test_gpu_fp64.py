@@ -536,3 +536,27 @@ def test_zero_guess_without_progress_returns_zeros(gpu, precision):
     x = torch.full((len(blocks) * 512,), 7.0, dtype=torch.float64, device=gpu)
     S.solve_device(torch.zeros_like(x), x)
     assert torch.equal(x, torch.zeros_like(x))
+
+
+@pytest.mark.parametrize("nb", [1, 255, 257, 1025, 5000])
+@pytest.mark.parametrize("guess", ["given", "zero"])
+def test_host_solve_across_chunks(gpu, nb, guess):
+    """The host entry point at block counts around its chunk (256 blocks), its
+    threads (one per 512 blocks) and its ring of two chunks per thread: the
+    device-resident solve, bitwise, through contiguous arrays and through block
+    pointers, twice on one handle."""
+    blocks, bpd, h0, bc = uniform((nb, 1, 1), (WALL,) * 3, 0.01)
+    S = PoissonSolver(bpd, h0, bc, bmean=0, guess=guess, tol_rel=0.0, max_iter=2)
+    S.set_topology(blocks)
+    rng = np.random.default_rng(7)
+    b, x0 = rng.standard_normal(nb * 512), rng.standard_normal(nb * 512)
+    x = dev(x0)
+    S.solve_device(dev(b), x)
+    want = x.cpu().numpy()
+    for _ in range(2):
+        h = x0.copy()
+        S.solve_host(b, h)
+        assert np.array_equal(h, want)
+        hb = [c.copy() for c in x0.reshape(nb, 512)]
+        S.solve_blocks(list(b.reshape(nb, 512)), hb)
+        assert np.array_equal(np.concatenate(hb), want)
