@@ -84,6 +84,7 @@ constexpr int COPY_THREADS = 16;
 // Device topology tables of one generation (topology_gpu.hip).
 struct DevTopo {
   DevBuf blocks, nbr, fkind, fnb, bpar, h, invh, h3, hf, invhf, meta, keys, vals, info;
+  size_t clean = 0;  // slots of the hash table that are clear, with the info words (0: dirty)
 };
 
 struct cup3d_poisson {
@@ -128,6 +129,8 @@ struct cup3d_poisson {
   // first host solve that needs them and kept
   DevBuf d_stage;             // 2 n doubles
   double* h_ring = nullptr;   // pinned
+  int* h_pin = nullptr;       // pinned: block list and info words of a topology build
+  size_t pin_bytes = 0;
   size_t ring_chunks = 0;
   hipEvent_t ring_ev[2 * COPY_THREADS] = {};
 
@@ -403,6 +406,10 @@ int cup3d_poisson_create(const cup3d_poisson_config* cfg, cup3d_poisson_t* out) 
     g_create_error = "hipMalloc(state) failed";
     return -1;
   }
+  if (hipMemset(H->d_state.p, 0, STATE_COPIES * sizeof(SolverState)) != hipSuccess) {
+    g_create_error = "hipMemset(state) failed";
+    return -1;
+  }
   *out = H.release();
   return 0;
 }
@@ -412,17 +419,27 @@ int cup3d_poisson_set_topology(cup3d_poisson_t H, int64_t nblocks, const cup3d_b
   if (nblocks <= 0 || !blocks) return fail(H, "empty block list");
   if (nblocks > (1LL << 22)) return fail(H, "too many blocks (limit 4194304)");
   HIPCHECK(hipSetDevice(H->device));
-  std::vector<int> bl(nblocks * 4);
-  for (int64_t b = 0; b < nblocks; ++b) {
-    bl[4 * b] = blocks[b].level;
-    for (int d = 0; d < 3; ++d) bl[4 * b + 1 + d] = blocks[b].index[d];
+  static_assert(sizeof(cup3d_block_desc) == 4 * sizeof(int), "a block is four words");
+  // pinned: the block list on its way to the device, then the info words
+  const size_t list_bytes = (size_t)nblocks * sizeof(cup3d_block_desc);
+  if (H->pin_bytes < list_bytes + TOPO_INFO_WORDS * sizeof(int)) {
+    if (H->h_pin) (void)hipHostFree(H->h_pin);
+    H->h_pin = nullptr;
+    H->pin_bytes = 0;
+    HIPCHECK(hipHostMalloc((void**)&H->h_pin, list_bytes + TOPO_INFO_WORDS * sizeof(int),
+                           hipHostMallocDefault));
+    H->pin_bytes = list_bytes + TOPO_INFO_WORDS * sizeof(int);
   }
+  std::memcpy(H->h_pin, blocks, list_bytes);
+  std::vector<int> bl(H->h_pin, H->h_pin + 4 * nblocks);
   // build the tables on the device into the other generation: a rejected
   // block list leaves the handle as it was
   const size_t nb = (size_t)nblocks;
   size_t cap = 1024;
   while (cap < 2 * nb) cap <<= 1;
   DevTopo& D = H->tp[1 - H->tcur];
+  DevTopo& E = H->tp[H->tcur];
+  const size_t held = D.keys.bytes + D.vals.bytes + D.info.bytes;
   if (D.blocks.reserve(nb * 4 * sizeof(int)) || D.nbr.reserve(nb * 6 * sizeof(int)) ||
       D.fkind.reserve(nb * 6) || D.fnb.reserve(nb * 24 * sizeof(int)) || D.bpar.reserve(nb) ||
       D.h.reserve(nb * sizeof(double)) || D.invh.reserve(nb * sizeof(double)) ||
@@ -431,8 +448,9 @@ int cup3d_poisson_set_topology(cup3d_poisson_t H, int64_t nblocks, const cup3d_b
       D.keys.reserve(cap * sizeof(unsigned long long)) ||
       D.vals.reserve(cap * sizeof(int)) || D.info.reserve(TOPO_INFO_WORDS * sizeof(int)))
     return fail(H, "hipMalloc(topology tables) failed");
+  if (D.keys.bytes + D.vals.bytes + D.info.bytes != held) D.clean = 0;  // grown: new memory
   hipStream_t s = H->stream;
-  HIPCHECK(hipMemcpyAsync(D.blocks.p, bl.data(), nb * 4 * sizeof(int), hipMemcpyHostToDevice, s));
+  HIPCHECK(hipMemcpyAsync(D.blocks.p, H->h_pin, list_bytes, hipMemcpyHostToDevice, s));
   TopoParams tpar;
   tpar.nb = (int)nb;
   for (int d = 0; d < 3; ++d) {
@@ -446,11 +464,19 @@ int cup3d_poisson_set_topology(cup3d_poisson_t H, int64_t nblocks, const cup3d_b
                      D.bpar.as<int8_t>(), D.h.as<double>(),  D.invh.as<double>(),
                      D.h3.as<double>(), D.hf.as<float>(),  D.invhf.as<float>(),
                      D.meta.as<int>()};
-  launch_topology_build(s, tpar, ttab, tout, D.info.as<int>());
+  const bool clear = D.clean < cap;
+  // the current generation's table has served its build: leave it clear for the next one
+  const size_t ecap = E.keys.p ? std::min(E.keys.bytes / sizeof(unsigned long long),
+                                          E.vals.bytes / sizeof(int)) : 0;
+  const TopoTable etab{E.keys.as<unsigned long long>(), E.vals.as<int>(),
+                       (unsigned long long)ecap - 1};
+  D.clean = E.clean = 0;
+  launch_topology_build(s, tpar, ttab, tout, D.info.as<int>(), clear, etab, E.info.as<int>());
   HIPCHECK(hipGetLastError());
-  int info[TOPO_INFO_WORDS];
-  HIPCHECK(hipMemcpyAsync(info, D.info.p, sizeof(info), hipMemcpyDeviceToHost, s));
+  int* info = H->h_pin + 4 * nb;
+  HIPCHECK(hipMemcpyAsync(info, D.info.p, TOPO_INFO_WORDS * sizeof(int), hipMemcpyDeviceToHost, s));
   HIPCHECK(hipStreamSynchronize(s));
+  E.clean = ecap;
   // the first offending block in list order, with the message of the
   // sequential checks (level/index, domain, index width, duplicate)
   const int NONE = 0x7fffffff;
@@ -546,11 +572,9 @@ int cup3d_poisson_set_topology(cup3d_poisson_t H, int64_t nblocks, const cup3d_b
   if (!H->d_gdots.p &&
       H->d_gdots.alloc(GUESS_MAXV * (GUESS_MAXV + 1) / 2 * sizeof(double)) != hipSuccess)
     return fail(H, "hipMalloc(guess dots) failed");
-  HIPCHECK(hipMemset(H->d_state.p, 0, STATE_COPIES * sizeof(SolverState)));
   if (mixed_set_topology(H->mixed, H->nb, H->n, H->err) != 0) return -1;
   if (cnn_set_topology(H->cnn, H->nb, C.nbr.as<int>(), C.h.as<double>(), H->err) != 0)
     return -1;
-  HIPCHECK(hipDeviceSynchronize());
   commit.ok = true;
   return 0;
 }
@@ -903,10 +927,10 @@ int cup3d_poisson_remove_mean(cup3d_poisson_t H, double* d_x, double* mean) {
   launch_remove_mean(H->stream, H->n, d_x, H->tp[H->tcur].h3.as<double>(), inv_vol,
                      H->d_part.as<double>(), H->d_gdots.as<double>());
   HIPCHECK(hipGetLastError());
-  double wsum = 0.0;
-  HIPCHECK(hipMemcpyAsync(&wsum, H->d_gdots.p, sizeof(double), hipMemcpyDeviceToHost, H->stream));
+  double* wsum = &H->h_state->mean_sum;  // pinned
+  HIPCHECK(hipMemcpyAsync(wsum, H->d_gdots.p, sizeof(double), hipMemcpyDeviceToHost, H->stream));
   HIPCHECK(hipStreamSynchronize(H->stream));
-  if (mean) *mean = wsum * inv_vol;  // the value the kernel subtracted
+  if (mean) *mean = *wsum * inv_vol;  // the value the kernel subtracted
   return 0;
 }
 
@@ -1414,6 +1438,7 @@ void cup3d_poisson_destroy(cup3d_poisson_t H) {
   mixed_free(H->mixed);
   if (H->h_state) (void)hipHostFree(H->h_state);
   if (H->h_ring) (void)hipHostFree(H->h_ring);
+  if (H->h_pin) (void)hipHostFree(H->h_pin);
   for (hipEvent_t e : H->ring_ev)
     if (e) (void)hipEventDestroy(e);
   if (H->ev0) (void)hipEventDestroy(H->ev0);

@@ -1,5 +1,5 @@
 // Device topology build (topology_gpu.hip): parameters, hash table and
-// output tables of the three build kernels.
+// output tables of the build kernels.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -55,7 +55,10 @@ __host__ __device__ inline int TopoInfoInit(unsigned long long i) {
   return i == TI_ORIGIN ? -1 : (i >= TI_N_COARSE ? 0 : 0x7fffffff);
 }
 
+// clear: t and info have to be cleared first. other, other_info: a table and
+// info words to leave cleared for the next build (keys null: none).
 void launch_topology_build(hipStream_t s, const TopoParams& p, const TopoTable& t,
-                           const TopoOut& o, int* info);
+                           const TopoOut& o, int* info, bool clear, const TopoTable& other,
+                           int* other_info);
 
 }  // namespace cup3d

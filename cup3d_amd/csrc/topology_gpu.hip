@@ -8,19 +8,25 @@
 // the periodic wrap of .cpp:361), which reruns after every mesh change
 // (Simulation.cpp:385).
 //
-//   k_topo_init    clear the hash table and the info words (a fill kernel,
-//                  no memset)
+//   k_topo_init    clear the hash table and the info words (a fill kernel, no
+//                  memset), where the build before did not
 //   k_topo_insert  one thread per block: validate level and index, insert
 //                  key(level, i, j, k) -> the smallest block id holding it
 //                  (open addressing, linear probing, 64-bit CAS)
-//   k_topo_blocks  one thread per block: duplicate test, h, 1/h, h^3 (FP64
-//                  and FP32), index parities, the origin block
-//   k_topo_faces   one thread per block face: same-level neighbour (with the
-//                  periodic wrap), else the coarser block, else the four finer
-//                  blocks by quadrant; a face with none of them violates the
-//                  2:1 balance
+//   k_topo_tables  eight threads per block: one per face: same-level neighbour
+//                  (with the periodic wrap), else the coarser block, else the
+//                  four finer blocks by quadrant; a face with none of them
+//                  violates the 2:1 balance; one for the duplicate test, h,
+//                  1/h, h^3 (FP64 and FP32), index parities, the origin block.
+//                  It also clears the other generation's hash table and info
+//                  words, which nothing reads any more and the next build uses
 // Errors are reported as the smallest offending block (or block face) id, so
 // the message names the same block a sequential pass would stop at.
+//
+// Bound by launches and the round trips of the hash probes: a mesh change of
+// 4440 blocks with one operator application takes 72 us (97 us with a clearing
+// kernel, separate kernels per block and per face, one counter update per face
+// and pageable copies).
 
 #include <hip/hip_runtime.h>
 
@@ -117,12 +123,9 @@ __global__ __launch_bounds__(WG_THREADS) void k_topo_insert(TopoParams p, TopoTa
   atomicMin(&info[TI_FULL], b);  // unreachable: the table holds >= 2 nb slots
 }
 
-__global__ __launch_bounds__(WG_THREADS) void k_topo_blocks(TopoParams p, TopoTable t,
-                                                            TopoOut o, int* info) {
-  const int b = blockIdx.x * WG_THREADS + threadIdx.x;
-  if (b >= p.nb) return;
-  const int4 B = reinterpret_cast<const int4*>(p.blocks)[b];
-  if (!block_ok(p, B)) return;  // reported by k_topo_insert
+// Block b's own entries.
+__device__ void topo_block(const TopoParams& p, const TopoTable& t, const TopoOut& o, int* info,
+                           int b, int4 B) {
   if (tfind(t, B.x, B.y, B.z, B.w) != b) atomicMin(&info[TI_DUPLICATE], b);
   // h0 / 2^l is exact (a power-of-two scaling), as is its FP32 rounding of
   // the same FP64 value
@@ -133,19 +136,16 @@ __global__ __launch_bounds__(WG_THREADS) void k_topo_blocks(TopoParams p, TopoTa
   o.h3[b] = h * h * h;
   o.hf[b] = (float)h;
   o.invhf[b] = (float)ih;
-  o.bpar[b] = (int8_t)((B.y & 1) | ((B.z & 1) << 1) | ((B.w & 1) << 2));
-  o.meta[(size_t)b * 32 + 30] = o.bpar[b];
+  const int8_t par = (int8_t)((B.y & 1) | ((B.z & 1) << 1) | ((B.w & 1) << 2));
+  o.bpar[b] = par;
+  o.meta[(size_t)b * 32 + 30] = par;
   o.meta[(size_t)b * 32 + 31] = 0;
   if (B.y == 0 && B.z == 0 && B.w == 0) atomicMax(&info[TI_ORIGIN], b);
 }
 
-__global__ __launch_bounds__(WG_THREADS) void k_topo_faces(TopoParams p, TopoTable t,
-                                                           TopoOut o, int* info) {
-  const int gid = blockIdx.x * WG_THREADS + threadIdx.x;
-  if (gid >= p.nb * 6) return;
-  const int b = gid / 6, f = gid - 6 * b;
-  const int4 B = reinterpret_cast<const int4*>(p.blocks)[b];
-  if (!block_ok(p, B)) return;  // reported by k_topo_insert
+// Face f of block b; returns its kind.
+__device__ int topo_face(const TopoParams& p, const TopoTable& t, const TopoOut& o, int* info,
+                         int b, int f, int4 B) {
   const int l = B.x;
   const int d = f >> 1, s = (f & 1) ? 1 : -1;
   const int n = p.bpd[d] << l;
@@ -163,7 +163,6 @@ __global__ __launch_bounds__(WG_THREADS) void k_topo_faces(TopoParams p, TopoTab
       if (c >= 0) {
         kind = FACE_COARSE;
         part[0] = c;
-        atomicAdd(&info[TI_N_COARSE], 1);
       } else {
         const int t1 = d == 0 ? 1 : (d == 1 ? 2 : 0), t2 = d == 0 ? 2 : (d == 1 ? 0 : 1);
         bool ok = true;
@@ -177,33 +176,64 @@ __global__ __launch_bounds__(WG_THREADS) void k_topo_faces(TopoParams p, TopoTab
         }
         if (ok) {
           kind = FACE_FINE;
-          atomicAdd(&info[TI_N_FINE], 1);
         } else {
-          atomicMin(&info[TI_BALANCE], gid);
+          atomicMin(&info[TI_BALANCE], b * 6 + f);
           for (int q = 0; q < 4; ++q) part[q] = -1;
         }
       }
     }
   }
+  const size_t gid = (size_t)b * 6 + f;
   o.kind[gid] = (int8_t)kind;
   o.nbr[gid] = nbr;
   reinterpret_cast<int4*>(o.fnb)[gid] = make_int4(part[0], part[1], part[2], part[3]);
   reinterpret_cast<int4*>(o.meta + (size_t)b * 32)[f] = make_int4(part[0], part[1], part[2], part[3]);
   o.meta[(size_t)b * 32 + 24 + f] = kind;
+  return kind;
+}
+
+__global__ __launch_bounds__(WG_THREADS) void k_topo_tables(TopoParams p, TopoTable t, TopoOut o,
+                                                            int* info, TopoTable other,
+                                                            int* other_info) {
+  const long long gid = (long long)blockIdx.x * WG_THREADS + threadIdx.x;
+  const int b = (int)(gid >> 3), f = (int)(gid & 7);
+  int kind = FACE_NONE;
+  if (b < p.nb) {
+    const int4 B = reinterpret_cast<const int4*>(p.blocks)[b];
+    if (block_ok(p, B)) {  // else reported by k_topo_insert
+      if (f < 6) kind = topo_face(p, t, o, info, b, f, B);
+      else if (f == 6) topo_block(p, t, o, info, b, B);
+    }
+  }
+  // one counter update per wavefront
+  const unsigned long long nc = __ballot(kind == FACE_COARSE), nf = __ballot(kind == FACE_FINE);
+  if ((threadIdx.x & 63) == 0) {
+    if (nc) atomicAdd(&info[TI_N_COARSE], __popcll(nc));
+    if (nf) atomicAdd(&info[TI_N_FINE], __popcll(nf));
+  }
+  if (other.keys) {
+    for (unsigned long long i = gid; i <= other.mask; i += (unsigned long long)gridDim.x * WG_THREADS) {
+      other.keys[i] = KEY_EMPTY;
+      other.vals[i] = 0x7fffffff;
+    }
+    if (gid < TOPO_INFO_WORDS) other_info[gid] = TopoInfoInit(gid);
+  }
 }
 
 }  // namespace
 
 void launch_topology_build(hipStream_t s, const TopoParams& p, const TopoTable& t,
-                           const TopoOut& o, int* info) {
-  const unsigned long long cap = t.mask + 1;
-  const int ninit = (int)((cap + WG_THREADS - 1) / WG_THREADS);
-  k_topo_init<<<ninit, WG_THREADS, 0, s>>>(t, info);
+                           const TopoOut& o, int* info, bool clear, const TopoTable& other,
+                           int* other_info) {
+  if (clear) {
+    const unsigned long long cap = t.mask + 1;
+    const int ninit = (int)((cap + WG_THREADS - 1) / WG_THREADS);
+    k_topo_init<<<ninit, WG_THREADS, 0, s>>>(t, info);
+  }
   const int nwb = (p.nb + WG_THREADS - 1) / WG_THREADS;
   k_topo_insert<<<nwb, WG_THREADS, 0, s>>>(p, t, info);
-  k_topo_blocks<<<nwb, WG_THREADS, 0, s>>>(p, t, o, info);
-  const int nwf = (p.nb * 6 + WG_THREADS - 1) / WG_THREADS;
-  k_topo_faces<<<nwf, WG_THREADS, 0, s>>>(p, t, o, info);
+  const int nwt = (int)(((long long)p.nb * 8 + WG_THREADS - 1) / WG_THREADS);
+  k_topo_tables<<<nwt, WG_THREADS, 0, s>>>(p, t, o, info, other, other_info);
 }
 
 }  // namespace cup3d

@@ -162,7 +162,7 @@ class PoissonSolver:
         blocks = np.ascontiguousarray(blocks, np.int32).reshape(-1, 4)
         # cup3d_block_desc is {level, index[3]}: four int32, the row layout
         assert ctypes.sizeof(BlockDesc) == 16
-        arr = (BlockDesc * len(blocks)).from_buffer_copy(blocks.tobytes())
+        arr = ctypes.cast(blocks.ctypes.data, ctypes.POINTER(BlockDesc))
         if self.L.cup3d_poisson_set_topology(self.h, len(blocks), arr) != 0:
             raise self._err("set_topology")
         self.nb = len(blocks)

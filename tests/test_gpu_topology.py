@@ -89,3 +89,32 @@ def test_mesh_change_sequence(gpu):
         r0, r1 = S.solve_device(b, x), S1.solve_device(b, x1)
         assert r0["iterations"] == r1["iterations"] == 12
         assert torch.equal(x, x1), len(blocks)
+
+
+def test_sequence_of_mesh_changes(gpu):
+    """Tables after every kind of change on one handle (each build uses the hash
+    table the one before left clear): larger, smaller, a rejected list, the same
+    list again and a much larger one, each equal to the build of a fresh
+    handle."""
+    bpd, bc = (4, 4, 4), (W.BC_WALL,) * 3
+    h0 = 1.0 / 32
+    amr = W.amr_sphere_blocks(bpd, h0, 2, (0.3, 0.15), (0.5, 0.5, 0.5), 0.2)
+    small = W.amr_sphere_blocks(bpd, h0, 1, (0.2,), (0.5, 0.5, 0.5), 0.2)
+    uni = W.uniform_blocks(*bpd)
+    fine = W.uniform_blocks(16, 16, 16)
+    fine[:, 0] = 2
+    S = PoissonSolver(bpd, h0, bc, bmean=0)
+    for blocks in (uni, amr, small, None, small, amr, fine, uni):
+        if blocks is None:
+            bad = amr.copy()
+            bad[-1] = bad[0]
+            with pytest.raises(RuntimeError, match="duplicate"):
+                S.set_topology(bad)
+            continue
+        S.set_topology(blocks)
+        fresh = PoissonSolver(bpd, h0, bc, bmean=0).set_topology(blocks)
+        x = torch.from_numpy(np.random.default_rng(len(blocks)).standard_normal(
+            len(blocks) * 512)).to(gpu)
+        assert S.coarse_fine_faces() == fresh.coarse_fine_faces()
+        assert torch.equal(S.apply_operator(x, torch.zeros_like(x)),
+                           fresh.apply_operator(x, torch.zeros_like(x)))
