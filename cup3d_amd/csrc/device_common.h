@@ -86,13 +86,18 @@ __device__ __forceinline__ void wg_sum(double (&v)[K], double (*red)[4]) {
 // sums (plain stores; the kernel boundary makes them visible to the
 // finalize kernel that follows on the same stream).
 template <int K>
-__device__ __forceinline__ void grid_store_partial(double (&v)[K], double* __restrict__ part) {
+__device__ __forceinline__ void store_partial(double (&v)[K], double* __restrict__ part,
+                                              size_t slot) {
   __shared__ double red[K][4];
   wg_sum<K>(v, red);
   if (threadIdx.x == 0) {
 #pragma unroll
-    for (int k = 0; k < K; ++k) part[(size_t)blockIdx.x * K + k] = v[k];
+    for (int k = 0; k < K; ++k) part[slot * K + k] = v[k];
   }
+}
+template <int K>
+__device__ __forceinline__ void grid_store_partial(double (&v)[K], double* __restrict__ part) {
+  store_partial<K>(v, part, blockIdx.x);
 }
 
 // Consumer side (one workgroup): sums the partials of `nparts` producer

@@ -9,11 +9,13 @@
 
 namespace cup3d {
 
-// PLAIN  y = A x                       INIT   y = A x, c = c2 = a - y, |y|^2, |c|^2
-// DOT1   y = A x, (a, y)               DOT2   y = A x, (a, y), (y, y)
+// PLAIN  y = A x                       INIT   c = c2 = a - A x, |A x|^2, |c|^2
+//                                             (y: room for bMean 2)
+// DOT1   y = A x, (a, y), a from c     DOT2   y = A x, (a, y), (y, y)
+//        after a restart (c may be null)
 // RESID  c = a - A x, |c|^2
-// START  y = c = c2 = -h^3 sigma a - A x, its norm (Helmholtz grids; x and a are
-//        one component of an [n][3] field)
+// START  -h^3 sigma a - A x into g.xo[0 .. 2] and its norms, for the three
+//        components of the [n][3] fields x and a (Helmholtz grids)
 // NET    c = a - A x, |c / h|^2, |x|^2 (bMean 0)
 // FINAL  |a - A x|^2 of the best iterate x (g.xo, the state), copied to y (may be null)
 enum SpmvMode {
@@ -40,6 +42,9 @@ inline int fin_mode(int nb, int bmean, long long row) {
 }
 // The sums of K5 lie behind those of the SpMVs, which K5 still reads.
 inline double* k5_part(double* part, int nb) { return part + 4 * (size_t)((nb + 3) / 4 + 8); }
+// Behind both, those of SPMV_START: (nb + 3) / 4 per component, kept until each
+// component's solve.
+inline double* start_part(double* part, int nb) { return part + 8 * (size_t)((nb + 3) / 4 + 8); }
 // Copies of the solver state (krylov.h): st[0] is the one that counts between
 // batches of iterations. hst, where a launch takes it: the host's pinned copy,
 // written by the finalize kernel.
@@ -49,13 +54,12 @@ constexpr int STATE_COPIES = 3;
 void launch_getvec64(hipStream_t s, long long n, long long zero_row, const double* rhs,
                      const double* x0, double* b, double* x, const SolverState& init,
                      SolverState* st, double* part, double tol_b);
-// The same and the initial residual for x0 = 0: b = r = rhat = rhs (zero in the
-// bMean cell; rhat may be null), x = 0 unless null, and the first iteration's
-// scalars.
+// The same and the initial residual for x0 = 0: b = rhs (zero in the bMean
+// cell), r = b and x = 0 unless null, and the first iteration's scalars.
 void launch_start_zero64(hipStream_t s, int nb, long long zero_row, const double* rhs, double* b,
-                         double* r, double* rhat, double* x, const SolverState& init,
+                         double* r, double* x, const SolverState& init,
                          SolverState* st, SolverState* hst, double* part, double tol_b);
-// The scalars of SPMV_START (nb blocks).
+// The scalars of one component of SPMV_START (nb blocks, its partial sums).
 void launch_start_fin(hipStream_t s, int nb, const SolverState& init, SolverState* st,
                       SolverState* hst, const double* part, double tol_b);
 // part null (SPMV_PLAIN and SPMV_RESID on a grid with bMean 0 or 3, SPMV_FINAL for

@@ -38,9 +38,9 @@ void launch_getvec64(hipStream_t s, long long n, long long zero_row, const doubl
 }
 
 void launch_start_zero64(hipStream_t s, int nb, long long zero_row, const double* rhs, double* b,
-                         double* r, double* rhat, double* x, const SolverState& init,
+                         double* r, double* x, const SolverState& init,
                          SolverState* st, SolverState* hst, double* part, double tol_b) {
-  k_start_zero<<<(nb + 3) / 4, WG_THREADS, 0, s>>>(nb, zero_row, rhs, b, r, rhat, x, part);
+  k_start_zero<<<(nb + 3) / 4, WG_THREADS, 0, s>>>(nb, zero_row, rhs, b, r, x, part);
   launch_start_fin(s, nb, init, st, hst, part, tol_b);
 }
 

@@ -32,6 +32,7 @@ __device__ inline void begin_iteration(SolverState* st, double rho, double rr) {
       return;
     }
     st->restart_pending = 1;  // rhat = r (done by K1)
+    st->rhat_own = 1;
     st->p_zero = 1;           // p = nu = 0
     st->rho_curr = rr;        // ||rhat||^2 after rhat = r
     st->rhrh = rr;
@@ -221,13 +222,14 @@ __device__ __forceinline__ void store8(T* __restrict__ p, const T (&v)[8]) {
   fin_store(st, S);
 }
 
-// Start from x0 = 0: b = r = rhat = rhs without an operator application. The
-// sum is taken as the SpMV's residual mode takes it (a column of eight cells
-// per lane, the workgroups in the SpMV's order), so |r| has the same bits as
-// through A x0.
+// Start from x0 = 0: b = rhs, the residual, without an operator application
+// (the first iteration reads b for r and rhat, see run_bicgstab64; r and x are
+// written where they are given). The sum is taken as the SpMV's residual mode
+// takes it (a column of eight cells per lane, the workgroups in the SpMV's
+// order), so |r| has the same bits as through A x0.
 [[maybe_unused]] static __global__ __launch_bounds__(WG_THREADS) void k_start_zero(
     int nb, long long zero_row, const double* __restrict__ rhs, double* __restrict__ b,
-    double* __restrict__ r, double* __restrict__ rhat, double* __restrict__ x, double* part) {
+    double* __restrict__ r, double* __restrict__ x, double* part) {
   double v[1] = {0.0};
   const int blk = xcd_remap(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6);
   if (blk < nb) {
@@ -240,8 +242,7 @@ __device__ __forceinline__ void store8(T* __restrict__ p, const T (&v)[8]) {
       const long long i = off + iz * 64;
       if (i == zero_row) q[iz] = 0.0;
       b[i] = q[iz];
-      r[i] = q[iz];
-      if (rhat) rhat[i] = q[iz];
+      if (r) r[i] = q[iz];
       if (x) x[i] = 0.0;
       v[0] += q[iz] * q[iz];
     }
@@ -456,6 +457,12 @@ struct SpmvSums {
   static constexpr int N = MEAN + DOTS;
 };
 
+// SPMV_DOT1's operand: a, or after a restart c (unless null).
+template <typename T>
+__device__ __forceinline__ const T* dot_operand(const T* a, const T* c, const SolverState* st) {
+  return c && st->rhat_own ? c : a;
+}
+
 template <typename T, int MODE, int BM, bool IFACE, bool HELM = false, bool NT = false>
 __global__ __launch_bounds__(WG_THREADS) void k_spmv(DevGrid<T> g, const T* __restrict__ xin,
                                                      T* __restrict__ y, const T* a, T* c, T* c2,
@@ -477,10 +484,21 @@ __global__ __launch_bounds__(WG_THREADS) void k_spmv(DevGrid<T> g, const T* __re
   if ((MODE == SPMV_DOT1 || MODE == SPMV_DOT2) && st->status != ST_RUNNING) return;
   // FINAL: the best iterate; while that is still 0, its buffer holds nothing
   const T* __restrict__ x = MODE == SPMV_FINAL ? g.xo[st->xopt] : xin;
+  if (MODE == SPMV_DOT1) a = dot_operand(a, c, st);
   const bool zero = MODE == SPMV_FINAL && st->opt_zero;
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int ix = lane & 7, iy = lane >> 3;
-  const int b = xcd_remap(blockIdx.x, gridDim.x) * 4 + w;
+  // START: the three components of four blocks are neighbours on one XCD, whose
+  // L2 then serves the interleaved velocities to the second and third
+  const int pos = xcd_remap(blockIdx.x, gridDim.x);
+  const int comp = MODE == SPMV_START ? pos % 3 : 0;
+  if (MODE == SPMV_START) {
+    x = xin + comp;
+    a += comp;
+    y = g.xo[comp];
+  }
+  const int chunk = MODE == SPMV_START ? pos / 3 : pos;
+  const int b = chunk * 4 + w;
   const bool valid = b < g.nb;
   const size_t off = (size_t)b * BLEN;
   T col[BS], av[BS], hx[BS], hy[BS], zlo = 0, zhi = 0;
@@ -570,7 +588,7 @@ __global__ __launch_bounds__(WG_THREADS) void k_spmv(DevGrid<T> g, const T* __re
       int dm = 0;
 #pragma unroll
       for (int f = 0; f < 6; ++f) dm |= (g.fkind[6 * b + f] == FACE_NONE ? 1 : 0) << f;
-      dm &= g.dmask;
+      dm &= MODE == SPMV_START ? g.dmask >> (6 * comp) : g.dmask;
       const T shift = -(h * h * h) * (T)g.helm_sigma;
       const int nxy = (ix == 0 ? (dm & 1) : 0) + (ix == BS - 1 ? ((dm >> 1) & 1) : 0) +
                       (iy == 0 ? ((dm >> 2) & 1) : 0) + (iy == BS - 1 ? ((dm >> 3) & 1) : 0);
@@ -631,8 +649,8 @@ __global__ __launch_bounds__(WG_THREADS) void k_spmv(DevGrid<T> g, const T* __re
       if (MODE == SPMV_PLAIN) {
         st_stream<NT>(&y[i], yy);
       } else if (MODE == SPMV_INIT) {
-        st_stream<NT>(&y[i], yy);
         const T rr = av[iz] - yy;
+        if (BM == 2) y[i] = yy;  // for k_bmean2_apply
         c[i] = rr;
         c2[i] = rr;
         v[1] += (double)yy * (double)yy;
@@ -656,8 +674,6 @@ __global__ __launch_bounds__(WG_THREADS) void k_spmv(DevGrid<T> g, const T* __re
       } else if (MODE == SPMV_START) {
         const T rr = -(h * h * h) * (T)g.helm_sigma * av[iz] - yy;
         y[i] = rr;
-        c[i] = rr;
-        c2[i] = rr;
         v[1] += (double)rr * (double)rr;
       } else if (MODE == SPMV_FINAL) {
         const T rr = zero ? av[iz] : av[iz] - yy;
@@ -671,7 +687,10 @@ __global__ __launch_bounds__(WG_THREADS) void k_spmv(DevGrid<T> g, const T* __re
     double p[Sums::N];
 #pragma unroll
     for (int k = 0; k < Sums::N; ++k) p[k] = v[k + 1 - Sums::MEAN];
-    grid_store_partial<Sums::N>(p, part);
+    if constexpr (MODE == SPMV_START)  // per component, in the order of blocks
+      store_partial<1>(p, part, (size_t)comp * (gridDim.x / 3) + chunk);
+    else
+      grid_store_partial<Sums::N>(p, part);
   }
 }
 
@@ -697,7 +716,6 @@ __global__ __launch_bounds__(WG_THREADS) void k_spmv_fin(long long row, T* __res
       if (MODE == SPMV_PLAIN) {
         y[row] = yr;
       } else if (MODE == SPMV_INIT) {
-        y[row] = yr;
         const T rr = a[row] - yr;
         c[row] = rr;
         c2[row] = rr;
@@ -705,7 +723,7 @@ __global__ __launch_bounds__(WG_THREADS) void k_spmv_fin(long long row, T* __res
         tot[2] += (double)rr * (double)rr;
       } else if (MODE == SPMV_DOT1) {
         y[row] = yr;
-        tot[1] += (double)a[row] * (double)yr;
+        tot[1] += (double)dot_operand(a, c, st)[row] * (double)yr;
       } else if (MODE == SPMV_DOT2) {
         y[row] = yr;
         tot[1] += (double)a[row] * (double)yr;
@@ -787,6 +805,7 @@ __global__ __launch_bounds__(WG_THREADS) void k_bmean2_apply(DevGrid<T> g, T* __
 #pragma unroll
       for (int e = 0; e < 8; ++e) yv[e] += corr;
       store8(y + i, yv);
+      if (MODE == SPMV_DOT1) a = dot_operand(a, c, st);
       if (MODE != SPMV_PLAIN) load8(a + i, av);
       if (MODE == SPMV_INIT) {
         T rr[8];
@@ -829,7 +848,7 @@ template <typename T, int MODE, int BM, bool HELM = false>
 inline void spmv_launch_iface(hipStream_t s, const DevGrid<T>& g, const T* x, T* y, const T* a,
                               T* c, T* c2, SolverState* st, double* part, bool fin,
                               SolverState* hst, hipEvent_t mid = nullptr) {
-  int nwg = (g.nb + 3) / 4;
+  int nwg = (g.nb + 3) / 4 * (MODE == SPMV_START ? 3 : 1);
   bool launched = false;
   if constexpr (MODE == SPMV_DOT1 || MODE == SPMV_DOT2) {  // the per-iteration SpMVs
     if ((size_t)g.n * sizeof(T) >= STREAM_MIN_BYTES) {
@@ -904,7 +923,7 @@ __global__ __launch_bounds__(WG_THREADS) void k_update(long long n, KrylovVector
       load8(v.z2 + i0, z2);
       load8(v.t + i0, t);
       load8(v.s + i0, r);
-      load8(v.rhat + i0, rh);
+      load8((st->rhat_own ? v.rhat : v.rhat0) + i0, rh);
     }
     T yr = 0;
     const SolverState* sp = st;

@@ -662,6 +662,7 @@ int mixed_set_topology(MixedWorkspace& M, int nb, long long n, std::string& err)
   v.z1 = base + 8 * n;
   v.z2 = base + 9 * n;
   v.b = base + 10 * n;
+  v.rhat0 = v.rhat;
   v.s = gemm_split(M, nb) ? v.b : v.r;
   v.pw = gemm_split(M, nb) ? base + 11 * n : v.p;
   return 0;
@@ -696,7 +697,7 @@ int mixed_solve(MixedWorkspace& M, hipStream_t s, const cup3d_poisson_config& cf
     launch_getvec64(s, n, zero_row, d_rhs, d_x0, b64, x64, init, st, part, cfg.tol_rhs);
     if (true_resid(rnorm)) return -1;
   } else {  // r64 = b64, without the operator
-    launch_start_zero64(s, M.nb, zero_row, d_rhs, b64, r64, nullptr, x64, init, st, h_st, part,
+    launch_start_zero64(s, M.nb, zero_row, d_rhs, b64, r64, x64, init, st, h_st, part,
                         cfg.tol_rhs);
     MCHECK(hipGetLastError());
     MCHECK(hipStreamSynchronize(s));

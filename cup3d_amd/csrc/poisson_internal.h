@@ -54,6 +54,7 @@ struct alignas(64) SolverState {
   int p_zero;           // K1 uses p = r (p = nu = 0)
   int xcur, xopt;       // rotating iterate buffers (0..2)
   int x_zero, opt_zero;  // the current / best iterate is 0: its buffer is not read
+  int rhat_own;          // rhat is in v.rhat (a restart put it there), else in v.rhat0
 };
 
 // Workspace passed to the kernels (all device pointers).
@@ -71,6 +72,7 @@ struct KrylovVectors {
   T* s;      // where K3 leaves s: r itself, or a vector of its own when several
              // workgroups of K3 read the same blocks of r
   T* pw;     // where K1 leaves the new p: p itself, or the other one of a pair
+  const T* rhat0;  // rhat until a restart: rhat itself, or b after a zero guess
 };
 
 // Grid data on the device.
@@ -95,13 +97,14 @@ struct DevGrid {
   long long bmean_row = -1;         // cell replaced by sum h^3 x (bMean == 1)
   int bmean = 1;
   int has_iface = 0;                // any coarse-fine interface rows
-  const T* xo[3] = {};              // SPMV_FINAL: the rotating iterate buffers
+  // SPMV_FINAL: the rotating iterate buffers; SPMV_START: the three outputs
+  T* xo[3] = {};
   // implicit diffusion of one velocity component (FP64 only): the operator
   // gains -h^3 helm_sigma x (helm_sigma = 1 / (nu dt)) and, on the domain-
   // boundary faces whose bit f is set in dmask, the Dirichlet ghost -x
   // (h (-x - x) per face) instead of the zero-flux ghost x
   int helm = 0;
-  int dmask = 0;
+  int dmask = 0;  // (SPMV_START: six bits per velocity component)
   double helm_sigma = 0.0;
 };
 

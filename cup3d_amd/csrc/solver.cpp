@@ -204,8 +204,9 @@ void launch_precond_fp64(cup3d_poisson* H, const DevGrid<double>& g, int mode,
 }
 
 // Run the FP64 classical BiCGSTAB on the device from a started state: v.b, the
-// initial residual in v.r and v.rhat, the first iteration's scalars. Leaves
-// the final state in H->h_state.
+// initial residual in v.r and v.rhat, or (from a zero guess: v.rhat0 = v.b) in
+// v.b alone, the first iteration's scalars. Leaves the final state in
+// H->h_state.
 // With a Helmholtz grid (g.helm, implicit diffusion) the preconditioner is
 // the block inverse of each block's level.
 int run_bicgstab64(cup3d_poisson* H, const DevGrid<double>& g, const KrylovVectors<double>& v,
@@ -228,9 +229,11 @@ int run_bicgstab64(cup3d_poisson* H, const DevGrid<double>& g, const KrylovVecto
     const int left = (int)std::max(1LL, H->cfg.max_iter - launched);
     batch = std::min(batch, left);
     for (int k = 0; k < batch; ++k) {
-      launch_precond_fp64(H, g, PREC_P, v, k > 0 ? fin : FIN_KERNEL, fp);
-      launch_spmv64(s, SPMV_DOT1, g, v.z1, v.nu, v.rhat, nullptr, nullptr, st, part, !fin);
-      launch_precond_fp64(H, g, PREC_S, v, fin, fs);
+      KrylovVectors<double> u = v;  // K1 and K3 of the first iteration read r = b
+      if (launched + k == 0 && v.rhat0 == v.b) u.r = v.b;
+      launch_precond_fp64(H, g, PREC_P, u, k > 0 ? fin : FIN_KERNEL, fp);
+      launch_spmv64(s, SPMV_DOT1, g, v.z1, v.nu, v.rhat0, v.rhat, nullptr, st, part, !fin);
+      launch_precond_fp64(H, g, PREC_S, u, fin, fs);
       launch_spmv64(s, SPMV_DOT2, g, v.z2, v.t, v.r, nullptr, nullptr, st, part, !fin);
       fp.nparts = launch_update64(s, g, v, st, part, fin, !fin || k == batch - 1,
                                   k == batch - 1 ? H->h_state : nullptr);
@@ -554,6 +557,7 @@ int cup3d_poisson_set_topology(cup3d_poisson_t H, int64_t nblocks, const cup3d_b
   v.b = base + 10 * n;
   v.s = v.r;
   v.pw = v.p;
+  v.rhat0 = v.rhat;
   // up to GUESS_MAXV (GUESS_MAXV + 1) / 2 partials per workgroup of 2048
   // cells (the warm start's Gram matrix)
   H->part_len = (size_t)((H->nb + 3) / 4 + 8) * (GUESS_MAXV * (GUESS_MAXV + 1) / 2);
@@ -593,16 +597,17 @@ static void report64(const SolverState& S, cup3d_solve_report* rep) {
 }
 
 // The initial residual r = b - A x0 in v.r and v.rhat (BiCGSTAB.cu:435-467); a
-// zero guess (d_x0 null) takes no operator application.
-static void start64(cup3d_poisson_t H, const DevGrid<double>& g, const KrylovVectors<double>& v,
+// zero guess (d_x0 null) takes no operator application and leaves it in v.b.
+static void start64(cup3d_poisson_t H, const DevGrid<double>& g, KrylovVectors<double>& v,
                     long long zero_row, const double* d_rhs, const double* d_x0,
                     const SolverState& init, double tol_b) {
   hipStream_t s = H->stream;
   SolverState* st = H->d_state.as<SolverState>();
   double* part = H->d_part.as<double>();
   if (!d_x0) {
-    launch_start_zero64(s, H->nb, zero_row, d_rhs, v.b, v.r, v.rhat, nullptr, init, st, nullptr, part,
+    launch_start_zero64(s, H->nb, zero_row, d_rhs, v.b, nullptr, nullptr, init, st, nullptr, part,
                         tol_b);
+    v.rhat0 = v.b;
     return;
   }
   launch_getvec64(s, H->n, zero_row, d_rhs, d_x0, v.b, v.x[0], init, st, part, tol_b);
@@ -633,9 +638,10 @@ static int solve_fp64(cup3d_poisson_t H, const double* d_rhs, double* d_x, const
   const long long zero_row = (H->cfg.bmean == 1 || H->cfg.bmean == 3) && H->topo.origin_block >= 0
                                  ? (long long)H->topo.origin_block * BLEN
                                  : -1;
-  start64(H, H->g64, H->v64, zero_row, d_rhs, d_x0, make_state(H->cfg), H->cfg.tol_rhs);
-  if (run_bicgstab64(H, H->g64, H->v64) != 0) return -1;
-  if (finish64(H, H->g64, H->v64, d_x, H->h_state) != 0) return -1;
+  KrylovVectors<double> v = H->v64;
+  start64(H, H->g64, v, zero_row, d_rhs, d_x0, make_state(H->cfg), H->cfg.tol_rhs);
+  if (run_bicgstab64(H, H->g64, v) != 0) return -1;
+  if (finish64(H, H->g64, v, d_x, H->h_state) != 0) return -1;
   HIPCHECK(hipStreamSynchronize(H->stream));
   if (rep) report64(*H->h_state, rep);
   return H->h_state->status;
@@ -1103,9 +1109,10 @@ int cup3d_diffusion_solve_device(cup3d_poisson_t H, int comp, double nu, double 
   HIPCHECK(hipSetDevice(H->device));
   hipStream_t s = H->stream;
   HIPCHECK(hipEventRecord(H->ev0, s));
-  start64(H, g, H->v64, -1, d_rhs, d_x, diffusion_state(H, tol_abs, tol_rel), 0.0);
-  if (run_bicgstab64(H, g, H->v64) != 0) return -1;
-  if (finish64(H, g, H->v64, d_x, H->h_state) != 0) return -1;
+  KrylovVectors<double> v = H->v64;
+  start64(H, g, v, -1, d_rhs, d_x, diffusion_state(H, tol_abs, tol_rel), 0.0);
+  if (run_bicgstab64(H, g, v) != 0) return -1;
+  if (finish64(H, g, v, d_x, H->h_state) != 0) return -1;
   HIPCHECK(hipEventRecord(H->ev1, s));
   HIPCHECK(hipEventSynchronize(H->ev1));
   float ms = 0;
@@ -1119,15 +1126,19 @@ int cup3d_diffusion_solve_device(cup3d_poisson_t H, int comp, double nu, double 
   return H->h_state->status;
 }
 
-// Three solves, one after the other, between one pass that makes each
-// component's rhs and one that adds the three solutions. rhs = h^3 (-(h lap
+// Three solves, one after the other, between one pass that makes the three
+// rhs and one that adds the three solutions. rhs = h^3 (-(h lap
 // u*)/h^3 + (u* - u^n)/(dt nu)) (KernelDiffusionRHS and
 // AdvectionDiffusionImplicit.cpp:376-400) = a - A u* with the Helmholtz
 // operator A = h lap - h^3 sigma and a = -h^3 sigma u^n; x0 = 0 (the reference
-// zeroes sim.pres before each solve, :398), so the residual starts as the rhs.
+// zeroes sim.pres before each solve, :398), so the residual starts as the rhs,
+// which is not copied (the velocities are interleaved: a pass per component
+// reads all of them; on 4.19 M cells three passes of 54-60 us with three copies
+// of the rhs each, against 84 us for the one; 300 MB, 60 us at copy rate).
 // The Laplacian of component c reads component c only, so the velocity is
 // updated once, at the end: the solutions stay in their iterate buffers (three
-// per solve out of five, two of them borrowed from the mixed form's scratch).
+// per solve out of five, two of them, and two of the rhs, borrowed from the
+// mixed form's scratch).
 // The host waits for the polls and at the end; a component's first poll comes
 // after as many iterations as the one before it took.
 int cup3d_diffusion_step_device(cup3d_poisson_t H, double nu, double dt, double tol_abs,
@@ -1148,17 +1159,28 @@ int cup3d_diffusion_step_device(cup3d_poisson_t H, double nu, double dt, double 
   SolverState* st = H->d_state.as<SolverState>();
   double* part = H->d_part.as<double>();
   double* const spare = static_cast<double*>(H->mixed.d_res64);
+  double* const spare2 = static_cast<double*>(H->mixed.d_vec32);  // 5.5 n doubles
+  DevGrid<double> gs = grid[0];
+  gs.dmask = grid[0].dmask | grid[1].dmask << 6 | grid[2].dmask << 12;
+  gs.xo[0] = H->v64.b;
+  gs.xo[1] = spare2;
+  gs.xo[2] = spare2 + H->n;
   double* pool[5] = {H->v64.x[0], H->v64.x[1], H->v64.x[2], spare, spare + H->n};
   const SolverState init = diffusion_state(H, tol_abs, tol_rel);
   const double* sol[3] = {};
   int worst = 0, first_batch = 1;
+  HIPCHECK(hipEventRecord(ev[0], s));
+  launch_spmv64(s, SPMV_START, gs, d_vel, nullptr, d_vel_old, nullptr, nullptr, st,
+                start_part(part, H->nb));
   for (int c = 0; c < 3; ++c) {
     KrylovVectors<double> v = H->v64;
+    v.b = gs.xo[c];
+    v.rhat0 = v.b;
     for (int k = 0, m = 0; k < 5 && m < 3; ++k)
       if (pool[k] != sol[0] && pool[k] != sol[1]) v.x[m++] = pool[k];
-    HIPCHECK(hipEventRecord(ev[2 * c], s));
-    launch_spmv64(s, SPMV_START, grid[c], d_vel + c, v.b, d_vel_old + c, v.r, v.rhat, st, part);
-    launch_start_fin(s, H->nb, init, st, nullptr, part, 0.0);
+    if (c > 0) HIPCHECK(hipEventRecord(ev[2 * c], s));
+    launch_start_fin(s, H->nb, init, st, nullptr,
+                     start_part(part, H->nb) + (size_t)c * ((H->nb + 3) / 4), 0.0);
     if (run_bicgstab64(H, grid[c], v, first_batch) != 0) return -1;
     const SolverState& S = *H->h_state;
     first_batch = std::max(1, S.iters_done);

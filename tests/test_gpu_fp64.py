@@ -526,6 +526,29 @@ def test_zero_guess_equals_given_zeros(gpu, name, bmean, precision):
     assert abs(r1["true_rel_resid"] - r0["true_rel_resid"]) <= tol * r0["true_rel_resid"] + 1e-14
 
 
+@pytest.mark.parametrize("bmean", [0, 1, 2, 3])
+@pytest.mark.parametrize("name", ["uniform_walls_3x2x2", "tiny_amr_periodic"])
+def test_zero_guess_restarts(gpu, name, bmean):
+    """From a zero guess the shadow residual is b itself until a restart replaces
+    it. At 100 iterations without a tolerance rounding has forced a restart (in
+    the oracle too); the products after it take the new one: the same bits as
+    from given zeros, where both residuals start as copies (bMean 2 sums the
+    start in another order: its residual only)."""
+    blocks, bpd, h0, bc = CASES[name]
+    b = dev(compatible_rhs(blocks, h0, 6))
+    out = []
+    for guess in ("given", "zero"):
+        S = PoissonSolver(bpd, h0, bc, bmean=bmean, guess=guess, tol_rel=0.0, tol_abs=0.0,
+                          max_iter=100, max_restarts=100).set_topology(blocks)
+        x = torch.zeros(len(blocks) * 512, dtype=torch.float64, device=gpu)
+        out.append((S.solve_device(b, x), x))
+    (r0, x0), (r1, x1) = out
+    assert r0["restarts"] >= 1 and r1["restarts"] >= 1
+    assert r1["true_rel_resid"] <= 1e-9
+    if bmean != 2:
+        assert r0["restarts"] == r1["restarts"] and torch.equal(x0, x1)
+
+
 @pytest.mark.parametrize("precision", ["fp64", "mixed_fp16"])
 def test_zero_guess_without_progress_returns_zeros(gpu, precision):
     """A zero rhs improves on nothing: the best iterate stays the zero guess,
