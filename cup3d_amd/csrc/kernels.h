@@ -31,6 +31,11 @@ struct FinArgs {
   const double* part = nullptr;
   int nparts = 0;
   long long row = -1;
+  // K1: where the host follows the iterations (both pinned, null: nowhere). The
+  // word takes 2 * iterations done, + 1 when that ended the solve; the state is
+  // there before such a word.
+  unsigned long long* prog = nullptr;
+  SolverState* hst = nullptr;
 };
 constexpr int FIN_MAX_BLOCKS = 8192;
 
@@ -70,7 +75,7 @@ void launch_spmv64(hipStream_t s, int mode, const DevGrid<double>& g, const doub
 // K5; returns its number of partials. last: with its finalize kernel.
 int launch_update64(hipStream_t s, const DevGrid<double>& g, const KrylovVectors<double>& v,
                     SolverState* st, double* part, int fin = FIN_KERNEL, bool last = true,
-                    SolverState* hst = nullptr);
+                    SolverState* hst = nullptr, unsigned long long* prog = nullptr);
 
 // The caller around the solve (projection.hip): the rhs of the pressure
 // equation from the velocity (and an obstacle's udef / chi, both or neither

@@ -65,8 +65,9 @@ void launch_spmv64(hipStream_t s, int mode, const DevGrid<double>& g, const doub
 }
 
 int launch_update64(hipStream_t s, const DevGrid<double>& g, const KrylovVectors<double>& v,
-                    SolverState* st, double* part, int fin, bool last, SolverState* hst) {
-  return launch_k5<double>(s, g, v, st, part, fin, last, hst);
+                    SolverState* st, double* part, int fin, bool last, SolverState* hst,
+                    unsigned long long* prog) {
+  return launch_k5<double>(s, g, v, st, part, fin, last, hst, nullptr, prog);
 }
 
 // ---------------------------------------------------------------------------

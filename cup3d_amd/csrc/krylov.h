@@ -72,6 +72,23 @@ __device__ __forceinline__ void fin_store(SolverState* st, const SolverState& S,
   }
 }
 
+// The end of an iteration for the host (one workgroup, every thread of it): the
+// state first, when the solve ended, then the word it watches (FinArgs).
+__device__ __forceinline__ void report_progress(const SolverState& S, SolverState* hst,
+                                                unsigned long long* prog) {
+  const bool stop = S.status != ST_RUNNING;
+  if (stop) {
+    if (threadIdx.x < STATE_WORDS)
+      reinterpret_cast<unsigned*>(hst)[threadIdx.x] =
+          reinterpret_cast<const unsigned*>(&S)[threadIdx.x];
+    __threadfence_system();
+    __syncthreads();
+  }
+  if (threadIdx.x == 0)
+    __hip_atomic_store(prog, 2ull * S.iters_done + stop, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // ---------------------------------------------------------------------------
 // Scalars in the consumer (FIN_SUMS, FIN_ROW): on grids of up to
 // FIN_MAX_BLOCKS blocks the kernel that needs a sum adds the producer's
@@ -146,14 +163,20 @@ __device__ __forceinline__ void consumer_state(SolverState* st, const FinArgs& f
     tot[1] += aux * (double)yr;
     if (USE == USE_X) tot[K - 1] += (double)yr * (double)yr;
   }
-  if (tid == 0 && S.status == ST_RUNNING) {
-    if (USE == USE_P) update_scalars(S, tot[0], tot[K - 1]);
-    else if (USE == USE_S) set_alpha(S, tot[K - 1]);
-    else set_omega(S, tot[K - 2], tot[K - 1]);
+  __shared__ bool ran;
+  if (tid == 0) {
+    ran = S.status == ST_RUNNING;
+    if (ran) {
+      if (USE == USE_P) update_scalars(S, tot[0], tot[K - 1]);
+      else if (USE == USE_S) set_alpha(S, tot[K - 1]);
+      else set_omega(S, tot[K - 2], tot[K - 1]);
+    }
   }
   __syncthreads();
-  if (blockIdx.x == 0 && tid < STATE_WORDS)
+  if (blockIdx.x != 0) return;
+  if (tid < STATE_WORDS)
     reinterpret_cast<unsigned*>(dst)[tid] = reinterpret_cast<const unsigned*>(&S)[tid];
+  if (USE == USE_P && f.prog && ran) report_progress(S, f.hst, f.prog);
 }
 
 // Contiguous 8-element vector access (16-byte loads/stores).
@@ -985,14 +1008,21 @@ __device__ inline void update_scalars(SolverState& S, double rho, double rr) {
 }
 
 // src: the state before K5 (st, or the consumers' last copy), dst: after it.
+// With prog the host follows the word, and hst is written when the solve ends.
 static __global__ __launch_bounds__(WG_THREADS) void k_update_fin(const SolverState* src,
                                                            SolverState* dst, SolverState* hst,
+                                                           unsigned long long* prog,
                                                            const double* part, int nparts) {
   __shared__ SolverState S;
+  __shared__ bool ran;
   double tot[2];
   fin_load<2>(src, S, part, nparts, tot);
-  if (threadIdx.x == 0 && S.status == ST_RUNNING) update_scalars(S, tot[0], tot[1]);
-  fin_store(dst, S, hst);
+  if (threadIdx.x == 0) {
+    ran = S.status == ST_RUNNING;
+    if (ran) update_scalars(S, tot[0], tot[1]);
+  }
+  fin_store(dst, S, prog ? nullptr : hst);
+  if (prog && ran) report_progress(S, hst, prog);
 }
 
 // K5 and, unless the next K1 takes its sums, the finalize kernel (an event, if
@@ -1000,7 +1030,8 @@ static __global__ __launch_bounds__(WG_THREADS) void k_update_fin(const SolverSt
 template <typename T>
 inline int launch_k5(hipStream_t s, const DevGrid<T>& g, const KrylovVectors<T>& v,
                      SolverState* st, double* part, int fin = FIN_KERNEL, bool last = true,
-                     SolverState* hst = nullptr, hipEvent_t mid = nullptr) {
+                     SolverState* hst = nullptr, hipEvent_t mid = nullptr,
+                     unsigned long long* prog = nullptr) {
   const long long n = g.n, runs = (n + 4 * BLEN - 1) / (4 * BLEN);
   const int ch = runs >= 8192 ? 2 : 1;
   const int nwg = (int)((runs + ch - 1) / ch);
@@ -1011,7 +1042,7 @@ inline int launch_k5(hipStream_t s, const DevGrid<T>& g, const KrylovVectors<T>&
   else if (ch == 2) k_update<T, 2, FIN_KERNEL><<<nwg, WG_THREADS, 0, s>>>(n, v, st, f, p5);
   else k_update<T, 1, FIN_KERNEL><<<nwg, WG_THREADS, 0, s>>>(n, v, st, f, p5);
   if (mid) (void)hipEventRecord(mid, s);
-  if (last) k_update_fin<<<1, WG_THREADS, 0, s>>>(fin ? st + 2 : st, st, hst, p5, nwg);
+  if (last) k_update_fin<<<1, WG_THREADS, 0, s>>>(fin ? st + 2 : st, st, hst, prog, p5, nwg);
   return nwg;
 }
 

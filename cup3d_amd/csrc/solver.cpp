@@ -78,7 +78,7 @@ struct DevBuf {
 
 }  // namespace
 
-constexpr int HOST_STATES = 4;
+constexpr int HOST_STATES = 5;
 constexpr int COPY_THREADS = 16;
 
 // Device topology tables of one generation (topology_gpu.hip).
@@ -116,7 +116,8 @@ struct cup3d_poisson {
   DevBuf d_vec64;  // 11 vectors of n doubles
   KrylovVectors<double> v64{};
   DevBuf d_state, d_part;
-  SolverState* h_state = nullptr;  // pinned: [0] polls, [1 .. 3] results per component
+  SolverState* h_state = nullptr;  // pinned: [0] a solve's state, [1 .. 3] results per component,
+                                   // [4] the progress word (run_bicgstab64)
   size_t part_len = 0;
 
   // mixed precision workspace
@@ -209,42 +210,75 @@ void launch_precond_fp64(cup3d_poisson* H, const DevGrid<double>& g, int mode,
 // H->h_state.
 // With a Helmholtz grid (g.helm, implicit diffusion) the preconditioner is
 // the block inverse of each block's level.
+// The host stays LEAD iterations ahead of the ones the device reports as done
+// (report_progress), so the GPU never waits for it, and when the solve ends
+// no more than the rest of the next iteration is in the stream, whose kernels
+// find the state stopped. Waiting after batches of 1, 2, 4, ... iterations took
+// a finalize kernel, a synchronisation and an idle GPU each: ten iterations on
+// 64 blocks 363 us, 307-320 us this way, eight on 8192 blocks 1241 and 1219 us.
+// But the K1 that finds a solve at its end has read its vectors, and the
+// kernels after it begin theirs: 42 us on 8192 blocks, three times a diffusion
+// step (1750 us against 1585 us), whose solves take a few iterations each. So
+// those first wait with nothing launched ahead, after `check` iterations (1, or
+// how many the component before took) and after 3; 0: never.
+// No more than the iterations the cap leaves are launched.
+constexpr int LEAD = 2;  // the sums of an iteration are known in the next one's K1
+
 int run_bicgstab64(cup3d_poisson* H, const DevGrid<double>& g, const KrylovVectors<double>& v,
-                   int first_batch = 1) {
+                   int check = 0) {
   hipStream_t s = H->stream;
   SolverState* st = H->d_state.as<SolverState>();
   double* part = H->d_part.as<double>();
-  const int poll = H->cfg.poll_every > 0 ? H->cfg.poll_every : 8;
-  // Batches of 1 (or first_batch), 2, 4, ... iterations up to `poll` between status polls: a
-  // short solve (the implicit-diffusion solves take a few iterations) is not
-  // held up by the host enqueueing the rest of a full batch, whose kernels
-  // would only find the state converged; a long solve polls a few more times.
-  // No more than the iterations the cap leaves are launched.
+  // after the states in pinned memory; no kernel that writes it is in the stream
+  unsigned long long* prog = reinterpret_cast<unsigned long long*>(H->h_state + HOST_STATES - 1);
   const int fin = fin_mode(g.nb, g.bmean, g.bmean_row);
-  const FinArgs fs{part, (g.nb + 3) / 4, g.bmean_row};  // K2's sums, for K3
-  FinArgs fp{k5_part(part, g.nb), 0, -1};               // K5's, for the next K1
-  int batch = std::min(first_batch, poll);
-  long long launched = 0;
-  while (true) {
-    const int left = (int)std::max(1LL, H->cfg.max_iter - launched);
-    batch = std::min(batch, left);
-    for (int k = 0; k < batch; ++k) {
+  const FinArgs fs{part, (g.nb + 3) / 4, g.bmean_row};                // K2's sums, for K3
+  FinArgs fp{k5_part(part, g.nb), 0, -1, prog, H->h_state};           // K5's, for the next K1
+  const long long cap = std::max(1, H->cfg.max_iter);
+  __atomic_store_n(prog, 0ull, __ATOMIC_RELEASE);
+  unsigned long long seen = 0;
+  int first_fin = FIN_KERNEL;  // the state is complete before the first K1 and after a wait
+  long long stop = check > 0 ? std::min<long long>(check, cap) : cap;  // the next wait
+  for (long long launched = 0; !(seen & 1);) {
+    const long long done = (long long)(seen >> 1);
+    if (done == stop) {
+      first_fin = FIN_KERNEL;
+      check = stop < 3 ? 3 : 0;
+      stop = check > 0 ? std::min<long long>(check, cap) : cap;
+    }
+    for (; launched < (check > 0 ? stop : std::min(stop, done + LEAD)); ++launched) {
       KrylovVectors<double> u = v;  // K1 and K3 of the first iteration read r = b
-      if (launched + k == 0 && v.rhat0 == v.b) u.r = v.b;
-      launch_precond_fp64(H, g, PREC_P, u, k > 0 ? fin : FIN_KERNEL, fp);
+      if (launched == 0 && v.rhat0 == v.b) u.r = v.b;
+      launch_precond_fp64(H, g, PREC_P, u, first_fin, fp);
+      first_fin = fin;
       launch_spmv64(s, SPMV_DOT1, g, v.z1, v.nu, v.rhat0, v.rhat, nullptr, st, part, !fin);
       launch_precond_fp64(H, g, PREC_S, u, fin, fs);
       launch_spmv64(s, SPMV_DOT2, g, v.z2, v.t, v.r, nullptr, nullptr, st, part, !fin);
-      fp.nparts = launch_update64(s, g, v, st, part, fin, !fin || k == batch - 1,
-                                  k == batch - 1 ? H->h_state : nullptr);
+      fp.nparts = launch_update64(s, g, v, st, part, fin, !fin || launched + 1 == stop, H->h_state,
+                                  prog);
     }
-    launched += batch;
     HIPCHECK(hipGetLastError());
-    HIPCHECK(hipStreamSynchronize(s));
-    if (H->h_state->status != ST_RUNNING) break;
-    if (launched > (long long)H->h_state->max_iter + 4LL * poll)
-      return fail(H, "device state machine did not stop");
-    batch = std::min(2 * batch, poll);
+    const unsigned long long before = seen;
+    for (int spin = 1; (seen = __atomic_load_n(prog, __ATOMIC_ACQUIRE)) == before; ++spin) {
+      if (spin < 1024) {
+        __builtin_ia32_pause();
+        continue;
+      }
+      // a long iteration, or nothing left that could report: the solve had
+      // stopped before its first iteration, or the device failed
+      spin = 0;
+      const hipError_t q = hipStreamQuery(s);
+      if (q == hipErrorNotReady) {
+        std::this_thread::yield();
+        continue;
+      }
+      HIPCHECK(q);
+      if (__atomic_load_n(prog, __ATOMIC_ACQUIRE) != before) continue;
+      HIPCHECK(hipMemcpyAsync(H->h_state, st, sizeof(SolverState), hipMemcpyDeviceToHost, s));
+      HIPCHECK(hipStreamSynchronize(s));
+      if (H->h_state->status == ST_RUNNING) return fail(H, "device state machine did not stop");
+      return 0;
+    }
   }
   return 0;
 }
@@ -1111,7 +1145,7 @@ int cup3d_diffusion_solve_device(cup3d_poisson_t H, int comp, double nu, double 
   HIPCHECK(hipEventRecord(H->ev0, s));
   KrylovVectors<double> v = H->v64;
   start64(H, g, v, -1, d_rhs, d_x, diffusion_state(H, tol_abs, tol_rel), 0.0);
-  if (run_bicgstab64(H, g, v) != 0) return -1;
+  if (run_bicgstab64(H, g, v, 1) != 0) return -1;
   if (finish64(H, g, v, d_x, H->h_state) != 0) return -1;
   HIPCHECK(hipEventRecord(H->ev1, s));
   HIPCHECK(hipEventSynchronize(H->ev1));
@@ -1139,8 +1173,8 @@ int cup3d_diffusion_solve_device(cup3d_poisson_t H, int comp, double nu, double 
 // updated once, at the end: the solutions stay in their iterate buffers (three
 // per solve out of five, two of them, and two of the rhs, borrowed from the
 // mixed form's scratch).
-// The host waits for the polls and at the end; a component's first poll comes
-// after as many iterations as the one before it took.
+// The host waits for a component's iterations, first after as many as the one
+// before it took, and at the end.
 int cup3d_diffusion_step_device(cup3d_poisson_t H, double nu, double dt, double tol_abs,
                                 double tol_rel, const double* d_vel_old, double* d_vel,
                                 cup3d_solve_report* reps) {
@@ -1168,7 +1202,7 @@ int cup3d_diffusion_step_device(cup3d_poisson_t H, double nu, double dt, double 
   double* pool[5] = {H->v64.x[0], H->v64.x[1], H->v64.x[2], spare, spare + H->n};
   const SolverState init = diffusion_state(H, tol_abs, tol_rel);
   const double* sol[3] = {};
-  int worst = 0, first_batch = 1;
+  int worst = 0, check = 1;
   HIPCHECK(hipEventRecord(ev[0], s));
   launch_spmv64(s, SPMV_START, gs, d_vel, nullptr, d_vel_old, nullptr, nullptr, st,
                 start_part(part, H->nb));
@@ -1181,9 +1215,9 @@ int cup3d_diffusion_step_device(cup3d_poisson_t H, double nu, double dt, double 
     if (c > 0) HIPCHECK(hipEventRecord(ev[2 * c], s));
     launch_start_fin(s, H->nb, init, st, nullptr,
                      start_part(part, H->nb) + (size_t)c * ((H->nb + 3) / 4), 0.0);
-    if (run_bicgstab64(H, grid[c], v, first_batch) != 0) return -1;
+    if (run_bicgstab64(H, grid[c], v, check) != 0) return -1;
     const SolverState& S = *H->h_state;
-    first_batch = std::max(1, S.iters_done);
+    check = std::max(1, S.iters_done);
     sol[c] = S.opt_zero ? nullptr : v.x[S.xopt];
     worst = std::max(worst, S.status);
     if (finish64(H, grid[c], v, nullptr, H->h_state + 1 + c) != 0) return -1;

@@ -115,7 +115,8 @@ typedef struct {
      FP64 residual) */
   double inner_tol;
   int max_refine;
-  int poll_every;    /* iterations between host polls of the device status (0 = default) */
+  int poll_every;    /* mixed forms: iterations between host polls of the device status
+                      * (0 = default); the FP64 form follows every iteration */
   int gemm_passes;   /* mixed only: 0 (or 2, 3) = input split into hi + lo, two MFMA
                         passes, linear to FP32 precision; 1 = one FP16/BF16 pass */
   int extrapolate;   /* 0 = off (the reference contract); K = 1..8 = also extrapolate

@@ -549,6 +549,30 @@ def test_zero_guess_restarts(gpu, name, bmean):
         assert r0["restarts"] == r1["restarts"] and torch.equal(x0, x1)
 
 
+@pytest.mark.parametrize("bmean", [0, 1, 2])
+@pytest.mark.parametrize("poll_every", [0, 1])
+def test_iteration_caps(gpu, bmean, poll_every):
+    """Caps around the iterations that the host launches ahead of the device, with
+    the scalars in the consumers (bMean 0 and 1) and in finalize kernels (2), one
+    solve after the other on a handle's device: the capped iteration of the oracle
+    (1e-10; few iterations amplify rounding little), and a rhs of zeros between."""
+    blocks, bpd, h0, bc = CASES["uniform_walls_3x2x2"]
+    b = compatible_rhs(blocks, h0, 3)
+    O = pyoracle.Oracle(blocks, bpd, h0, bc, bmean)
+    x = torch.zeros(O.n, dtype=torch.float64, device=gpu)
+    for cap in (1, 2, 3, 4, 7):
+        S = PoissonSolver(bpd, h0, bc, bmean=bmean, tol_rel=0.0, guess="zero", max_iter=cap,
+                          poll_every=poll_every).set_topology(blocks)
+        for _ in range(2):
+            x.fill_(float("nan"))
+            rep = S.solve_device(dev(b), x)
+            assert rep["status"] == 1 and rep["iterations"] == cap
+            xo, info = O.bicgstab(b, tol_rel=0.0, max_iter=cap)
+            assert np.linalg.norm(x.cpu().numpy() - xo) <= 1e-10 * np.linalg.norm(xo)
+            S.solve_device(torch.zeros_like(x), x)
+            assert torch.equal(x, torch.zeros_like(x))
+
+
 @pytest.mark.parametrize("precision", ["fp64", "mixed_fp16"])
 def test_zero_guess_without_progress_returns_zeros(gpu, precision):
     """A zero rhs improves on nothing: the best iterate stays the zero guess,
