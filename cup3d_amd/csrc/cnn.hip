@@ -41,7 +41,16 @@ namespace cup3d {
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ float gelu(float x) { return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f)); }
+// GELU of two values as FP16, x in the lower half: the last product is rounded
+// once, from its exact value, and lands in its half of the word.
+__device__ __forceinline__ unsigned gelu_pair(float x, float y) {
+  const float hx = 0.5f * x, ex = 1.0f + erff(x * 0.70710678118654752f);
+  const float hy = 0.5f * y, ey = 1.0f + erff(y * 0.70710678118654752f);
+  unsigned r;
+  asm("v_fma_mixlo_f16 %0, %1, %2, 0 op_sel_hi:[0,0,0]" : "=v"(r) : "v"(hx), "v"(ex));
+  asm("v_fma_mixhi_f16 %0, %1, %2, 0 op_sel_hi:[0,0,0]" : "+v"(r) : "v"(hy), "v"(ey));
+  return r;
+}
 
 // Index into a field of the cell that padded position (pz, py, px) in 0..9
 // of block b takes its value from (the halo rule above).
@@ -172,18 +181,20 @@ __device__ __forceinline__ int padded(int m) {  // cell 0..511 -> padded index
 // behind. The zero cell in front of a row is also the one behind the row
 // before it (and so for rows and planes), so the "same" padding costs 820
 // cells against 1000, and three workgroups fit a CU.
+// The two 16-byte halves of a cell (channels 0-7 and 8-15) change places in the
+// padded rows 4 to 7. A tile is the rows y and y + 4 of a plane: the sixteen
+// cells that lanes 0-15 read are then in sixteen different 16-byte slots of the
+// 64 banks (in the input patch too, whose rows are 40 cells apart), and a read
+// takes 6 cycles; with the rows y and y + 1, or the halves in place, 9.4.
 constexpr int AROW = 9, APLANE = 81, ACELLS = 9 * APLANE + 9 * AROW + AROW + 1;
 __device__ __forceinline__ constexpr int atap(int o) {  // tap o from the (-1, -1, -1) corner
   return (o / 9) * APLANE + ((o / 3) % 3) * AROW + o % 3;
 }
 
-// Four rows (cells 16 tile + 4 g + q) of a tile's products with channel lr.
-template <typename F>
-__device__ __forceinline__ void tile_rows(const float4_t& acc, F&& f) {
-  // register q of lane l holds D[4*(l/16) + q][l % 16]
-#pragma unroll
-  for (int q = 0; q < 4; ++q) f(q, acc[q]);
-}
+// A wavefront owns two planes, eight tiles: tile 4 p + j is the rows j and j + 4
+// of plane p. Products are taken with the weights as the first operand, so that
+// register q of lane l holds channel 4 (l / 16) + q of cell l % 16 of the tile:
+// four channels of a cell are one 8-byte store.
 
 // Layer 1 (valid) on the 10^3 input patch, 8 halfs a cell: 4 taps a k-step,
 // tap 4 kt + g in the lanes of group g. The lane's tap offsets are registers
@@ -202,10 +213,10 @@ __device__ __forceinline__ void conv_first(const _Float16* __restrict__ in,
     const int o = 4 * kt + g;
     po[kt] = o < 27 ? ((o / 9) * 100 + ((o / 3) % 3) * 10 + o % 3) * 8 : 0;
   }
-  const int base = (2 * w * 100 + (lr >> 3) * 10 + (lr & 7)) * 8;
-#pragma unroll 2
+  const int base = (2 * w * 100 + (lr >> 3) * 40 + (lr & 7)) * 8;
+#pragma unroll
   for (int t = 0; t < 8; ++t) {
-    const _Float16* p = in + base + ((t >> 2) * 100 + (t & 3) * 20) * 8;
+    const _Float16* p = in + base + ((t >> 2) * 100 + (t & 3) * 10) * 8;
     float4_t acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int kt = 0; kt < CNN_KT1; ++kt) {
@@ -214,64 +225,112 @@ __device__ __forceinline__ void conv_first(const _Float16* __restrict__ in,
 #pragma unroll
         for (int e = 0; e < 8; ++e) a[e] = (_Float16)0.f;
       }
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bq[kt], acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(bq[kt], a, acc, 0, 0, 0);
     }
     f(t, acc);
   }
 }
 
 // Layers 2 and 3 (same): 2 taps a k-step, taps 2 kt and 2 kt + 1 in the lower
-// and upper lanes. The two taps of a step are 1, 7 or 61 cells apart, so three
-// base addresses and immediate offsets reach every operand.
+// and upper lanes, 1, 7 or 61 cells apart. The operand of padded rows r and
+// r + 4 of a padded plane from column dx serves every output tile that meets it
+// with a tap pair of the same distance (rows r - dy, plane z - dz): it is read
+// once for all of them, 78 reads for the 112 products. Planes, rows and columns
+// are walked in ascending order, so a tile's k-steps come in ascending order.
+// Every address is one of seven bases and an immediate offset.
 template <typename F>
 __device__ __forceinline__ void conv_same(const _Float16* __restrict__ in,
                                           const half8_t* __restrict__ wfrag, int w, int l, F&& f) {
   constexpr int KT = CNN_KT2;
   static_assert(CNN_KT2 == CNN_KT3 && CNN_C == 16, "two taps of 16 channels a k-step");
-  const int lr = l & 15, g = l >> 4, hi = g >> 1;
+  const int lr = l & 15, g = l >> 4, hi = g >> 1, rr = lr >> 3;
   half8_t bq[KT];
 #pragma unroll
   for (int kt = 0; kt < KT; ++kt) bq[kt] = wfrag[kt * 64 + l];
-  const int base =
-      (2 * w * APLANE + (lr >> 3) * AROW + (lr & 7)) * CNN_C + 8 * (g & 1);
-  const _Float16* p1 = in + base + hi * CNN_C;
-  const _Float16* p7 = in + base + hi * 7 * CNN_C;
-  const _Float16* p61 = in + base + hi * 61 * CNN_C;
-#pragma unroll 2
-  for (int t = 0; t < 8; ++t) {
-    const int to = ((t >> 2) * APLANE + (t & 3) * 2 * AROW) * CNN_C;
-    float4_t acc = {0.f, 0.f, 0.f, 0.f};
+  // a base per distance and place of the halves (lower lanes' row, upper lanes'
+  // row at or past 4: fl, fu)
+  const int c0 = (2 * w * APLANE + rr * 4 * AROW + (lr & 7)) * CNN_C, s = (g & 1) ^ rr;
+  auto base = [&](int d, int fl, int fu) {
+    return in + c0 + hi * d * CNN_C + 8 * (s ^ (hi ? fu : fl));
+  };
+  const _Float16* const p1[2] = {base(1, 0, 0), base(1, 1, 1)};
+  const _Float16* const p7[3] = {base(7, 0, 0), base(7, 0, 1), base(7, 1, 1)};
+  const _Float16* const p61[2] = {base(61, 0, 0), base(61, 1, 0)};
+  float4_t acc[2][4];
 #pragma unroll
-    for (int kt = 0; kt < KT; ++kt) {
-      const int d = 2 * kt + 1 < 27 ? atap(2 * kt + 1) - atap(2 * kt) : 0;
-      const _Float16* p = d == 7 ? p7 : (d == 61 ? p61 : p1);
-      // there is no tap 27: the upper lanes read the ring's first (zero) cell
-      if (kt == KT - 1) p = hi ? in - to - atap(2 * kt) * CNN_C : p1;
-      const half8_t a = *reinterpret_cast<const half8_t*>(p + to + atap(2 * kt) * CNN_C);
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bq[kt], acc, 0, 0, 0);
+  for (int p = 0; p < 2; ++p)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[p][j] = (float4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int z = 0; z < 4; ++z) {
+#pragma unroll
+    for (int r = 0; r < 6; ++r)
+#pragma unroll
+      for (int dx = 0; dx < 3; ++dx) {
+        const int at = (z * APLANE + r * AROW + dx) * CNN_C;
+        // one operand per distance: 1 (dx 0 and 1), 7, 61, or the last tap alone
+#pragma unroll
+        for (int cls = 0; cls < 4; ++cls) {
+          bool used = false;
+          half8_t a;
+#pragma unroll
+          for (int dz = 0; dz < 3; ++dz)
+#pragma unroll
+            for (int dy = 0; dy < 3; ++dy) {
+              const int o = 9 * dz + 3 * dy + dx, p = z - dz, j = r - dy;
+              const int c = dx < 2 ? 0 : (o == 26 ? 3 : (o == 8 ? 2 : 1));
+              if (o % 2 || c != cls || p < 0 || p > 1 || j < 0 || j > 3) continue;
+              if (!used) {
+                const _Float16* q = cls == 0   ? p1[r >= 4]
+                                    : cls == 1 ? p7[(r >= 3) + (r >= 4)]
+                                    : cls == 2 ? p61[r >= 4]
+                                               : p1[r >= 4];
+                // there is no tap 27: the upper lanes read the ring's first (zero) cell
+                if (cls == 3) q = hi ? in - at : q;
+                a = *reinterpret_cast<const half8_t*>(q + at);
+                used = true;
+              }
+              acc[p][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bq[o / 2], a, acc[p][j], 0, 0, 0);
+            }
+        }
+      }
+    if (z >= 2) {  // the last plane that output plane z - 2 reads
+#pragma unroll
+      for (int j = 0; j < 4; ++j) f(4 * (z - 2) + j, acc[z - 2][j]);
     }
-    f(t, acc);
   }
 }
 
-// Zero the ring of an activation buffer (the 512 cells are written by a layer).
+// Zero the ring of an activation buffer (the 512 cells are written by a layer):
+// the planes in front and behind, then each plane's first row and the first
+// cell of its other rows.
+constexpr int ARING = ACELLS - BLEN;
 __device__ __forceinline__ void zero_ring(_Float16* buf, int tid) {
   half8_t zero;
 #pragma unroll
   for (int e = 0; e < 8; ++e) zero[e] = (_Float16)0.f;
-  for (int i = tid; i < 2 * ACELLS; i += WG_THREADS) {
-    const int c = i >> 1, r = c % APLANE;
-    if (c < APLANE || c >= 9 * APLANE || r < AROW || r % AROW == 0)
-      *reinterpret_cast<half8_t*>(&buf[i * 8]) = zero;
+  constexpr int ENDS = ARING - BS * (AROW + BS);
+#pragma unroll
+  for (int i = tid; i < ARING; i += WG_THREADS) {
+    const int k = i - ENDS, z = k / (AROW + BS), m = k - z * (AROW + BS);
+    const int c = i < APLANE ? i
+                  : i < ENDS ? 9 * APLANE + i - APLANE
+                             : (z + 1) * APLANE + (m < AROW ? m : (m - BS) * AROW);
+    half8_t* p = reinterpret_cast<half8_t*>(&buf[c * CNN_C]);
+    p[0] = zero;
+    p[1] = zero;
   }
 }
 
 // LDS of the inference: the input patch (1000 cells x 8 halfs), later the
 // second layer's activations, and the first layer's: 52 KiB per workgroup,
-// three workgroups per CU. What the kernel takes is mostly the exact GELU of
-// 16 384 values a block (about 36 vector instructions each): it ran at 328 us
-// on 8192 blocks with the zero padding selected per operand (20 instructions a
-// read) and runs at about 230 us with it built into the layout.
+// three workgroups per CU. The vector ALUs bound it, mostly by the exact GELU of
+// 16 384 values a block (about 36 instructions each, 120 us of 8192 blocks); the
+// LDS reads and the products (60 us) run beside them. 328 us on 8192 blocks with
+// the zero padding selected per operand (20 instructions a read), 230 us with it
+// built into the layout, 185 us with conflict-free reads shared by the tiles,
+// four channels a store and the halo positions by face (a predict of 8192 blocks
+// 264 -> 221 us).
 constexpr int CNN_IN_HALFS = PADC * 8 > ACELLS * CNN_C ? PADC * 8 : ACELLS * CNN_C;
 
 __global__ __launch_bounds__(WG_THREADS) void k_cnn_infer(int nb, const int* __restrict__ nbr,
@@ -292,13 +351,51 @@ __global__ __launch_bounds__(WG_THREADS) void k_cnn_infer(int nb, const int* __r
   const float inv_hs = (float)(1.0 / (h[b] * s_r));
   // input: 8-channel cells (2 real); the indices of a thread's (up to 4)
   // positions first, then all 8 loads, so the gather costs two memory round
-  // trips, not one per position
-  constexpr int NP = (PADC + WG_THREADS - 1) / WG_THREADS;
+  // trips, not one per position. Positions: two cells of the block, then the
+  // halo, a face per wavefront (so its axis is a scalar), edges and corners.
+  constexpr int NP = 4, HALO = PADC - BLEN;
+  static_assert(WG_THREADS == 256 && HALO <= 2 * WG_THREADS, "two cells and two halo positions");
   size_t gi[NP];
+  int pi[NP];
 #pragma unroll
-  for (int j = 0; j < NP; ++j) {
-    const int p = tid + j * WG_THREADS;
-    gi[j] = p < PADC ? halo_index(nbr, b, p / 100, (p / 10) % 10, p % 10) : (size_t)b * BLEN;
+  for (int j = 0; j < 2; ++j) {
+    const int m = tid + j * WG_THREADS;
+    gi[j] = (size_t)b * BLEN + m;
+    pi[j] = padded(m);
+  }
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int i = tid + j * WG_THREADS;
+    const int face = __builtin_amdgcn_readfirstlane(i >> 6);
+    int src = b, c, p;
+    if (face < 6) {
+      const int d = face >> 1, side = face & 1, u = l & 7, v = l >> 3;
+      const int sd = d == 0 ? 1 : (d == 1 ? 8 : 64), pd = d == 0 ? 1 : (d == 1 ? 10 : 100);
+      const int s1 = d == 0 ? 8 : 1, s2 = d == 2 ? 8 : 64;
+      const int p1 = d == 0 ? 10 : 1, p2 = d == 2 ? 10 : 100;
+      const int nbf = nbr[b * 6 + face];
+      if (nbf >= 0) src = nbf;
+      c = ((side != 0) == (nbf < 0) ? 7 : 0) * sd + u * s1 + v * s2;
+      p = (side ? 9 : 0) * pd + (u + 1) * p1 + (v + 1) * p2;
+    } else {  // the nearest cell: 12 edges of 8, then 8 corners
+      const int e = i - 384, ed = e >> 3, t = e & 7;
+      int q[3];  // padded position
+      if (e < 96) {
+        const int d = ed >> 2, lo = ed & 1 ? 9 : 0, hi = ed & 2 ? 9 : 0;
+        q[0] = d == 0 ? t + 1 : lo;
+        q[1] = d == 1 ? t + 1 : (d == 0 ? lo : hi);
+        q[2] = d == 2 ? t + 1 : hi;
+      } else {
+        q[0] = e & 1 ? 9 : 0;
+        q[1] = e & 2 ? 9 : 0;
+        q[2] = e & 4 ? 9 : 0;
+      }
+      auto near = [](int x) { return min(max(x - 1, 0), 7); };
+      c = near(q[0]) + 8 * near(q[1]) + 64 * near(q[2]);
+      p = i < HALO ? q[0] + 10 * q[1] + 100 * q[2] : -1;
+    }
+    gi[2 + j] = (size_t)src * BLEN + c;
+    pi[2 + j] = p;
   }
   double rv[NP], pv[NP];
 #pragma unroll
@@ -309,25 +406,36 @@ __global__ __launch_bounds__(WG_THREADS) void k_cnn_infer(int nb, const int* __r
   zero_ring(bufA, tid);
 #pragma unroll
   for (int j = 0; j < NP; ++j) {
-    const int p = tid + j * WG_THREADS;
-    if (p < PADC) {
+    if (pi[j] >= 0) {
       half8_t v;
 #pragma unroll
       for (int e = 0; e < 8; ++e) v[e] = (_Float16)0.f;
       v[0] = (_Float16)((float)rv[j] * inv_hs);
       v[1] = (_Float16)((float)pv[j] * inv_sp);
-      *reinterpret_cast<half8_t*>(&bufIn[p * 8]) = v;
+      *reinterpret_cast<half8_t*>(&bufIn[pi[j] * 8]) = v;
     }
   }
   __syncthreads();
   const half8_t* wf = reinterpret_cast<const half8_t*>(wpk);
-  // this lane's output rows in tile 0: cells (y, x) = (g / 2, 4 (g % 2) + q)
-  const int orow = ((2 * wv + 1) * APLANE + ((g >> 1) + 1) * AROW + 4 * (g & 1) + 1) * CNN_C + lr;
-  auto store = [&](_Float16* buf, float bias, int t, const float4_t& acc) {
-    _Float16* p = buf + orow + ((t >> 2) * APLANE + (t & 3) * 2 * AROW) * CNN_C;
-    tile_rows(acc, [&](int q, float v) { p[q * CNN_C] = (_Float16)gelu(v + bias); });
+  // this lane's cell in tile 0, its four channels 4 g .. 4 g + 3 (rows j = 3 and 7
+  // are the padded rows 4 and 8, where the halves' places change)
+  const int rr = lr >> 3;
+  const int ocell = ((2 * wv + 1) * APLANE + (4 * rr + 1) * AROW + (lr & 7) + 1) * CNN_C + 4 * (g & 1);
+  const int oh[2] = {ocell + 8 * ((g >> 1) ^ rr), ocell + 8 * ((g >> 1) ^ rr ^ 1)};
+  auto store = [&](_Float16* buf, const float (&bias)[4], int t, const float4_t& acc) {
+    typedef unsigned uint2_t __attribute__((ext_vector_type(2)));
+    const uint2_t v = {gelu_pair(acc[0] + bias[0], acc[1] + bias[1]),
+                       gelu_pair(acc[2] + bias[2], acc[3] + bias[3])};
+    *reinterpret_cast<uint2_t*>(
+        &buf[oh[(t & 3) == 3] + ((t >> 2) * APLANE + (t & 3) * AROW) * CNN_C]) = v;
   };
-  const float b1 = w[CNN_OB1 + lr], b2 = w[CNN_OB2 + lr], b3 = w[CNN_OB3];
+  float b1[4], b2[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    b1[q] = w[CNN_OB1 + 4 * g + q];
+    b2[q] = w[CNN_OB2 + 4 * g + q];
+  }
+  const float b3 = w[CNN_OB3];
   conv_first(bufIn, wf, wv, l, [&](int t, const float4_t& acc) { store(bufA, b1, t, acc); });
   __syncthreads();
   zero_ring(bufIn, tid);
@@ -335,8 +443,9 @@ __global__ __launch_bounds__(WG_THREADS) void k_cnn_infer(int nb, const int* __r
             [&](int t, const float4_t& acc) { store(bufIn, b2, t, acc); });
   __syncthreads();
   float* po = reinterpret_cast<float*>(bufA);
+  const int ocol = 128 * wv + 32 * rr + (lr & 7);
   conv_same(bufIn, wf + (CNN_KT1 + CNN_KT2) * 64, wv, l, [&](int t, const float4_t& acc) {
-    if (lr == 0) tile_rows(acc, [&](int q, float v) { po[128 * wv + 16 * t + 4 * g + q] = v; });
+    if (g == 0) po[ocol + 64 * (t >> 2) + 8 * (t & 3)] = acc[0];
   });
   __syncthreads();
   const size_t off = (size_t)b * BLEN;

@@ -162,3 +162,28 @@ def test_predict_in_place_equals_out_of_place(gpu, name, bmean):
     S.cnn_predict(rhs, prev, out)
     S.cnn_predict(rhs, inplace, inplace)
     assert torch.linalg.norm(out - inplace) <= 1e-6 * torch.linalg.norm(out - prev)
+
+
+@pytest.mark.parametrize("bpd,bc", [((1, 1, 1), 2), ((1, 1, 1), 1), ((2, 1, 3), 1), ((3, 3, 3), 0)])
+def test_predict_of_rough_fields_cell_by_cell(gpu, bpd, bc):
+    """White-noise inputs on the smallest grids (a block that is its own
+    neighbour, walls on all sides), the largest error of any cell: a halo cell
+    or a zero of the padding taken from the wrong place moves cells next to it
+    by one of 27 taps, about 0.2 of a typical increment. FP16 inputs, weights
+    and two layers of activations each round by 2^-12 RMS of a term, so a cell
+    of three layers is off by about 1e-3, and the worst of 14 000 by 5e-3."""
+    blocks = W.uniform_blocks(*bpd)
+    S = PoissonSolver(bpd, 0.125, (bc,) * 3, bmean=0).set_topology(blocks)
+    w = C.init_weights(9)
+    S.cnn_set_weights(w.astype(np.float32))
+    rng = np.random.default_rng(11)
+    shape = (len(blocks), 8, 8, 8)
+    prev = rng.standard_normal(shape)
+    rhs = 0.125 ** 3 * rng.standard_normal(shape)
+    out = torch.zeros(prev.size, dtype=torch.float64, device=gpu)
+    S.cnn_predict(dev(rhs), dev(prev), out)
+    res = residual(blocks, bpd, 0.125, (bc,) * 3, rhs, prev)
+    ref = C.predict(w, res, prev, np.full(len(blocks), 0.125), nbr_table(blocks, bpd, (bc,) * 3))
+    err = np.abs(out.cpu().numpy().reshape(shape) - ref).max()
+    inc = np.sqrt(np.mean((ref - prev) ** 2))
+    assert err <= 0.02 * inc, (err, inc)
