@@ -24,4 +24,14 @@ void launch_precond_dst32(hipStream_t s, int mode, int nb, const float* h,
 // vel[:, c] += x[c] (null: 0) for the three components of an [n][3] field.
 void launch_diffusion_add(hipStream_t s, long long n, const double* const x[3], double* vel);
 
+
+// K1 and K2 (PREC_P: v.nu and v.p to v.pw and y) or K3 and K4 (PREC_S: v.r and
+// v.nu to v.s and y) in one kernel, on grids for which fused_blocks() holds; the
+// outputs overlap none of the inputs. part: g.nb sums of up to three values and one
+// word, other than f.part. PREC_S takes its scalars from the sums (fin is not
+// FIN_KERNEL).
+void launch_precond_spmv64(hipStream_t s, int mode, const DevGrid<double>& g,
+                           const KrylovVectors<double>& v, double* y, SolverState* st, int fin,
+                           const FinArgs& f, double* part);
+
 }  // namespace cup3d

@@ -212,6 +212,165 @@ __global__ __launch_bounds__(WG_THREADS) void k_precond_dst(int nb, const T* __r
   for (int iz = 0; iz < BS; ++iz) out[off + iz * 64] = c[iz];
 }
 
+// K1 and K2, or K3 and K4, in one kernel: the block inverse and the operator on
+// its result, for single-level grids of up to FUSE_MAX_BLOCKS blocks. Such
+// kernels are bound by their launches and by chains of memory latencies, not by
+// the work, so a workgroup of seven wavefronts makes the vectors of its block and
+// of the six neighbours for itself (each wavefront one block, seven times the
+// arithmetic) and needs no other workgroup's result: three launches an iteration
+// instead of five. On 64 blocks K1 and K2 took 6.7 + 4.7 us and take 8.1, K3 and K4
+// 5.5 + 4.3 us and take 7.1; a solve of ten iterations 320 -> 275 us.
+// Wavefront 0 has the workgroup's own block and writes it; the neighbours'
+// wavefronts leave the layer of cells that touches it in LDS. The product is
+// split over four wavefronts, two z planes each. What a neighbour's workgroup
+// reads is not written in the same kernel: p, nu and s leave for vectors other
+// than those they are made from (v.pw, y of PREC_P, v.s), and so do the sums.
+//   PREC_P  p, z1, y = nu = A z1; sums (rhat, nu)
+//   PREC_S  s, z2, y = t = A z2;  sums (t, s), (t, t)
+// BM1: the mean-constraint row as k_spmv leaves it (its sum first, its other
+// factor behind the sums). HELM: as in k_spmv.
+constexpr int FUSE_T = 7 * 64;
+
+template <int MODE, int FIN, bool BM1, bool HELM>
+__global__ __launch_bounds__(FUSE_T) void k_precond_spmv(DevGrid<double> g,
+                                                         KrylovVectors<double> v,
+                                                         double* __restrict__ y, SolverState* st,
+                                                         FinArgs f, double* __restrict__ part) {
+  constexpr int N = (BM1 ? 1 : 0) + (MODE == PREC_P ? 1 : 2);
+  __shared__ double Ls[7][DL_WAVE];
+  __shared__ double xs[BLEN], fc[6][64], sv[MODE == PREC_S ? BLEN : 1], red[N][4];
+  __shared__ SolverState S;
+  if (!FIN && st->status != ST_RUNNING) return;
+  const int b = xcd_remap(blockIdx.x, gridDim.x);
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int ix = lane & 7, iy = lane >> 3;
+  const int bw = w == 0 ? b : g.nbr[b * 6 + w - 1];  // -1: no block there
+  const size_t off = (size_t)(bw < 0 ? 0 : bw) * BLEN + lane, own = (size_t)b * BLEN + lane;
+  double c[BS], ra[BS], rb[BS];
+  const bool fresh = !FIN && MODE == PREC_P && st->p_zero;
+  if (bw >= 0) {
+#pragma unroll
+    for (int iz = 0; iz < BS; ++iz) {
+      const size_t i = off + iz * 64;
+      ra[iz] = v.r[i];
+      if (!fresh) rb[iz] = v.nu[i];
+      if (MODE == PREC_P && !fresh) c[iz] = v.p[i];
+    }
+  }
+  const SolverState* sp = st;
+  if constexpr (FIN != FIN_KERNEL) {
+    double yr = 0;
+    consumer_state<MODE == PREC_P ? USE_P : USE_S, FIN, double>(st, f, S, yr);
+    if (S.status != ST_RUNNING) return;
+    sp = &S;
+    if (FIN == FIN_ROW && MODE == PREC_S && bw >= 0 && (long long)off == f.row) {
+      rb[0] = yr;  // the mean-constraint row of nu, which the product left out
+      if (w == 0) v.nu[off] = yr;
+    }
+  }
+  const int pzero = MODE == PREC_P ? sp->p_zero : 0;
+  const int restart = MODE == PREC_P ? sp->restart_pending : 0;
+  // rhat in the cells of this wavefront's two planes (r itself after a restart)
+  double a[2] = {};
+  if (MODE == PREC_P && w < 4) {
+    const double* rhat = restart ? v.r : (sp->rhat_own ? v.rhat : v.rhat0);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) a[k] = rhat[own + (2 * w + k) * 64];
+  }
+  if (bw >= 0) {
+    const double beta = MODE == PREC_P ? sp->beta : 0.0, omega = MODE == PREC_P ? sp->omega : 0.0;
+    const double alpha = MODE == PREC_S ? sp->alpha : 0.0;
+#pragma unroll
+    for (int iz = 0; iz < BS; ++iz) {
+      const size_t i = off + iz * 64;
+      if (MODE == PREC_P) {
+        c[iz] = pzero ? ra[iz] : fma(beta, fma(-omega, rb[iz], c[iz]), ra[iz]);
+        if (w == 0) v.pw[i] = c[iz];
+        if (w == 0 && restart) v.rhat[i] = ra[iz];
+      } else {
+        c[iz] = fma(-alpha, rb[iz], ra[iz]);
+        if (w == 0) {
+          v.s[i] = c[iz];
+          sv[iz * 64 + lane] = c[iz];
+        }
+      }
+    }
+    dst_apply<double>(Ls[w], lane, g.h[bw], HELM ? g.helm_sigma : 0.0, c);
+    if (w == 0) {
+      double* __restrict__ out = MODE == PREC_S ? v.z2 : v.z1;
+#pragma unroll
+      for (int iz = 0; iz < BS; ++iz) {
+        out[off + iz * 64] = c[iz];
+        xs[iz * 64 + lane] = c[iz];
+      }
+    } else if (w < 3) {  // the neighbour's last (first) layer in x
+      if (ix == (w == 1 ? 7 : 0)) {
+#pragma unroll
+        for (int iz = 0; iz < BS; ++iz) fc[w - 1][iz * 8 + iy] = c[iz];
+      }
+    } else if (w < 5) {
+      if (iy == (w == 3 ? 7 : 0)) {
+#pragma unroll
+        for (int iz = 0; iz < BS; ++iz) fc[w - 1][iz * 8 + ix] = c[iz];
+      }
+    } else {
+      fc[w - 1][lane] = w == 5 ? c[7] : c[0];
+    }
+  }
+  __syncthreads();
+  if (w < 4) {
+    const double h = g.h[b];
+    int none = 0;  // faces without a neighbour: the ghost is the cell itself
+#pragma unroll
+    for (int q = 0; q < 6; ++q) none |= (g.nbr[b * 6 + q] < 0 ? 1 : 0) << q;
+    const bool origin = g.bmean_row == (long long)b * BLEN;
+    double sum[3] = {0.0, 0.0, 0.0};  // sum of x, then the dots
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const int iz = 2 * w + k, li = iz * 64 + lane;
+      const double c0 = xs[li];
+      auto side = [&](bool inside, int step, int face, int cell) {
+        if (inside) return xs[li + step];
+        return (none >> face) & 1 ? c0 : fc[face][cell];
+      };
+      const double xm = side(ix > 0, -1, 0, iz * 8 + iy), xp = side(ix < 7, 1, 1, iz * 8 + iy);
+      const double ym = side(iy > 0, -8, 2, iz * 8 + ix), yp = side(iy < 7, 8, 3, iz * 8 + ix);
+      const double zm = side(iz > 0, -64, 4, lane), zp = side(iz < 7, 64, 5, lane);
+      double yy = h * ((((xm + xp) + (ym + yp)) + (zm + zp)) - 6.0 * c0);
+      if (HELM) {
+        const int dm = none & g.dmask;
+        const int nd = (ix == 0 ? (dm & 1) : 0) + (ix == 7 ? ((dm >> 1) & 1) : 0) +
+                       (iy == 0 ? ((dm >> 2) & 1) : 0) + (iy == 7 ? ((dm >> 3) & 1) : 0) +
+                       (iz == 0 ? ((dm >> 4) & 1) : 0) + (iz == 7 ? ((dm >> 5) & 1) : 0);
+        yy += (-(h * h * h) * g.helm_sigma - (double)(2 * nd) * h) * c0;
+      }
+      if (MODE == PREC_S) a[k] = sv[li];
+      sum[0] += c0;
+      if (origin && li == 0) {
+        if (BM1) {  // the row is the sum over the grid, which the consumer adds
+          part[(size_t)N * gridDim.x] = a[k];
+          continue;
+        }
+        if (g.bmean == 3) yy = h * c0;  // row h I
+      }
+      y[own + iz * 64] = yy;
+      sum[1] += a[k] * yy;
+      sum[2] += yy * yy;
+    }
+    sum[0] *= h * h * h;
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+      const double t = wave_sum(sum[q + (BM1 ? 0 : 1)]);
+      if (lane == 0) red[q][w] = t;
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < N) {
+    const double* r = red[threadIdx.x];
+    part[(size_t)b * N + threadIdx.x] = ((r[0] + r[1]) + r[2]) + r[3];
+  }
+}
+
 template <typename T, int MODE, int FIN>
 void launch_precond_dst_m(hipStream_t s, int nb, const T* h, T sigma,
                           const KrylovVectors<T>& v, SolverState* st, const FinArgs& f) {
@@ -267,6 +426,30 @@ void launch_precond_dst32(hipStream_t s, int mode, int nb, const float* h,
                           const KrylovVectors<float>& v, SolverState* st, int fin,
                           const FinArgs& f) {
   launch_precond_dst_t<float>(s, mode, nb, h, 0.0f, v, st, fin, f);
+}
+
+template <int MODE, int FIN>
+static void launch_fused_m(hipStream_t s, const DevGrid<double>& g, const KrylovVectors<double>& v,
+                           double* y, SolverState* st, const FinArgs& f, double* part) {
+  if (g.helm)
+    k_precond_spmv<MODE, FIN, false, true><<<g.nb, FUSE_T, 0, s>>>(g, v, y, st, f, part);
+  else if (g.bmean == 1 && g.bmean_row >= 0)
+    k_precond_spmv<MODE, FIN, true, false><<<g.nb, FUSE_T, 0, s>>>(g, v, y, st, f, part);
+  else
+    k_precond_spmv<MODE, FIN, false, false><<<g.nb, FUSE_T, 0, s>>>(g, v, y, st, f, part);
+}
+
+void launch_precond_spmv64(hipStream_t s, int mode, const DevGrid<double>& g,
+                           const KrylovVectors<double>& v, double* y, SolverState* st, int fin,
+                           const FinArgs& f, double* part) {
+  if (mode == PREC_P && fin) launch_fused_m<PREC_P, FIN_SUMS>(s, g, v, y, st, f, part);
+  else if (mode == PREC_P) launch_fused_m<PREC_P, FIN_KERNEL>(s, g, v, y, st, f, part);
+  else if (fin == FIN_ROW)
+    k_precond_spmv<PREC_S, FIN_ROW, true, false><<<g.nb, FUSE_T, 0, s>>>(g, v, y, st, f, part);
+  else if (g.helm)
+    k_precond_spmv<PREC_S, FIN_SUMS, false, true><<<g.nb, FUSE_T, 0, s>>>(g, v, y, st, f, part);
+  else
+    k_precond_spmv<PREC_S, FIN_SUMS, false, false><<<g.nb, FUSE_T, 0, s>>>(g, v, y, st, f, part);
 }
 
 void launch_diffusion_add(hipStream_t s, long long n, const double* const x[3], double* vel) {

@@ -47,6 +47,21 @@ inline int fin_mode(int nb, int bmean, long long row) {
 }
 // The sums of K5 lie behind those of the SpMVs, which K5 still reads.
 inline double* k5_part(double* part, int nb) { return part + 4 * (size_t)((nb + 3) / 4 + 8); }
+// Grids whose FP64 iterations take three kernels instead of five
+// (launch_precond_spmv64): one level, and a workgroup a CU at most. Ten iterations
+// with five kernels and with three: 64 blocks 320 -> 275 us, 128 327 -> 285, 256
+// 331 -> 304; past one workgroup a CU the seven-fold work tells, 384 blocks 343 ->
+// 365 us, 1024 397 -> 510.
+constexpr int FUSE_MAX_BLOCKS = 256;
+constexpr int FUSE_VECTORS = 3;  // second vectors of p and nu, one for s
+inline bool fused_blocks(int nb, bool has_iface, int fin) {
+  return nb <= FUSE_MAX_BLOCKS && !has_iface && fin != FIN_KERNEL;
+}
+// Their sums, of the first product (which 0) and the second: up to three values
+// a block and one word, behind all others.
+inline double* fused_part(double* part, int nb, int which) {
+  return part + 16 * (size_t)((nb + 3) / 4 + 8) + which * (size_t)(3 * nb + 8);
+}
 // Behind both, those of SPMV_START: (nb + 3) / 4 per component, kept until each
 // component's solve.
 inline double* start_part(double* part, int nb) { return part + 8 * (size_t)((nb + 3) / 4 + 8); }
@@ -72,10 +87,12 @@ void launch_start_fin(hipStream_t s, int nb, const SolverState& init, SolverStat
 void launch_spmv64(hipStream_t s, int mode, const DevGrid<double>& g, const double* x, double* y,
                    const double* a, double* c, double* c2, SolverState* st, double* part,
                    bool fin = true, SolverState* hst = nullptr);
-// K5; returns its number of partials. last: with its finalize kernel.
+// K5; returns its number of partials. last: with its finalize kernel. sums: where
+// those of K4 are (null: at part, a value per four blocks).
 int launch_update64(hipStream_t s, const DevGrid<double>& g, const KrylovVectors<double>& v,
                     SolverState* st, double* part, int fin = FIN_KERNEL, bool last = true,
-                    SolverState* hst = nullptr, unsigned long long* prog = nullptr);
+                    SolverState* hst = nullptr, unsigned long long* prog = nullptr,
+                    const FinArgs* sums = nullptr);
 
 // The caller around the solve (projection.hip): the rhs of the pressure
 // equation from the velocity (and an obstacle's udef / chi, both or neither

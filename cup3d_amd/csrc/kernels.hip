@@ -16,7 +16,8 @@
 //   K4 k_spmv<DOT2>   t = A z2; omega = (t, s) / ((t, t) + eps)
 //   K5 k_update       x' = x + alpha z1 + omega z2; r = s - omega t;
 //                     rho' = (rhat, r), |r|; x_opt / convergence / restart
-// M^-1 = blockdiag(h_b^-1 P_inv), applied by sine transforms (diffusion.hip).
+// M^-1 = blockdiag(h_b^-1 P_inv), applied by sine transforms (diffusion.hip). On
+// small single-level grids K1 and K2, and K3 and K4, are one kernel each.
 
 #include <hip/hip_runtime.h>
 
@@ -66,8 +67,8 @@ void launch_spmv64(hipStream_t s, int mode, const DevGrid<double>& g, const doub
 
 int launch_update64(hipStream_t s, const DevGrid<double>& g, const KrylovVectors<double>& v,
                     SolverState* st, double* part, int fin, bool last, SolverState* hst,
-                    unsigned long long* prog) {
-  return launch_k5<double>(s, g, v, st, part, fin, last, hst, nullptr, prog);
+                    unsigned long long* prog, const FinArgs* sums) {
+  return launch_k5<double>(s, g, v, st, part, fin, last, hst, nullptr, prog, sums);
 }
 
 // ---------------------------------------------------------------------------

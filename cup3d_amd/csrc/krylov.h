@@ -1031,11 +1031,11 @@ template <typename T>
 inline int launch_k5(hipStream_t s, const DevGrid<T>& g, const KrylovVectors<T>& v,
                      SolverState* st, double* part, int fin = FIN_KERNEL, bool last = true,
                      SolverState* hst = nullptr, hipEvent_t mid = nullptr,
-                     unsigned long long* prog = nullptr) {
+                     unsigned long long* prog = nullptr, const FinArgs* sums = nullptr) {
   const long long n = g.n, runs = (n + 4 * BLEN - 1) / (4 * BLEN);
   const int ch = runs >= 8192 ? 2 : 1;
   const int nwg = (int)((runs + ch - 1) / ch);
-  const FinArgs f{part, (g.nb + 3) / 4, g.bmean_row};
+  const FinArgs f = sums ? *sums : FinArgs{part, (g.nb + 3) / 4, g.bmean_row};
   double* p5 = k5_part(part, g.nb);
   if (fin == FIN_SUMS) k_update<T, 1, FIN_SUMS><<<nwg, WG_THREADS, 0, s>>>(n, v, st, f, p5);
   else if (fin == FIN_ROW) k_update<T, 1, FIN_ROW><<<nwg, WG_THREADS, 0, s>>>(n, v, st, f, p5);

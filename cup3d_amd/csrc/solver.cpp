@@ -113,8 +113,9 @@ struct cup3d_poisson {
   std::vector<double> P;
 
   // FP64 Krylov workspace
-  DevBuf d_vec64;  // 11 vectors of n doubles
+  DevBuf d_vec64;  // 11 vectors of n doubles, small grids FUSE_VECTORS more
   KrylovVectors<double> v64{};
+  double* fused = nullptr;  // those
   DevBuf d_state, d_part;
   SolverState* h_state = nullptr;  // pinned: [0] a solve's state, [1 .. 3] results per component,
                                    // [4] the progress word (run_bicgstab64)
@@ -232,7 +233,11 @@ int run_bicgstab64(cup3d_poisson* H, const DevGrid<double>& g, const KrylovVecto
   // after the states in pinned memory; no kernel that writes it is in the stream
   unsigned long long* prog = reinterpret_cast<unsigned long long*>(H->h_state + HOST_STATES - 1);
   const int fin = fin_mode(g.nb, g.bmean, g.bmean_row);
-  const FinArgs fs{part, (g.nb + 3) / 4, g.bmean_row};                // K2's sums, for K3
+  const bool fused = fused_blocks(g.nb, g.has_iface != 0, fin);
+  double *const fs_part = fused_part(part, g.nb, 0), *const ft_part = fused_part(part, g.nb, 1);
+  const FinArgs fs = fused ? FinArgs{fs_part, g.nb, g.bmean_row}
+                           : FinArgs{part, (g.nb + 3) / 4, g.bmean_row};  // K2's sums, for K3
+  const FinArgs ft{ft_part, g.nb, g.bmean_row};  // K4's, for K5 (fused)
   FinArgs fp{k5_part(part, g.nb), 0, -1, prog, H->h_state};           // K5's, for the next K1
   const long long cap = std::max(1, H->cfg.max_iter);
   __atomic_store_n(prog, 0ull, __ATOMIC_RELEASE);
@@ -249,6 +254,22 @@ int run_bicgstab64(cup3d_poisson* H, const DevGrid<double>& g, const KrylovVecto
     for (; launched < (check > 0 ? stop : std::min(stop, done + LEAD)); ++launched) {
       KrylovVectors<double> u = v;  // K1 and K3 of the first iteration read r = b
       if (launched == 0 && v.rhat0 == v.b) u.r = v.b;
+      if (fused) {
+        double *const ps[2] = {v.p, H->fused}, *const nus[2] = {v.nu, H->fused + g.n};
+        const int in = launched & 1, out = 1 - in;
+        u.p = ps[in];
+        u.pw = ps[out];
+        u.nu = nus[in];
+        launch_precond_spmv64(s, PREC_P, g, u, nus[out], st, first_fin, fp, fs_part);
+        first_fin = fin;
+        u.nu = nus[out];
+        u.s = H->fused + 2 * g.n;
+        launch_precond_spmv64(s, PREC_S, g, u, v.t, st, fin, fs, ft_part);
+        u.r = v.r;
+        fp.nparts = launch_update64(s, g, u, st, part, fin, launched + 1 == stop, H->h_state, prog,
+                                    &ft);
+        continue;
+      }
       launch_precond_fp64(H, g, PREC_P, u, first_fin, fp);
       first_fin = fin;
       launch_spmv64(s, SPMV_DOT1, g, v.z1, v.nu, v.rhat0, v.rhat, nullptr, st, part, !fin);
@@ -577,7 +598,8 @@ int cup3d_poisson_set_topology(cup3d_poisson_t H, int64_t nblocks, const cup3d_b
   fill(H->g32, C.hf.p, C.invhf.p);
   // FP64 Krylov vectors: x[3], r, rhat, p, nu, t, z1, z2, b
   const size_t n = (size_t)H->n;
-  if (H->d_vec64.reserve(11 * n * sizeof(double)) != hipSuccess) return fail(H, "hipMalloc(vectors) failed");
+  const size_t nvec = 11 + (H->nb <= FUSE_MAX_BLOCKS ? FUSE_VECTORS : 0);
+  if (H->d_vec64.reserve(nvec * n * sizeof(double)) != hipSuccess) return fail(H, "hipMalloc(vectors) failed");
   double* base = H->d_vec64.as<double>();
   KrylovVectors<double>& v = H->v64;
   for (int k = 0; k < 3; ++k) v.x[k] = base + k * n;
@@ -589,6 +611,7 @@ int cup3d_poisson_set_topology(cup3d_poisson_t H, int64_t nblocks, const cup3d_b
   v.z1 = base + 8 * n;
   v.z2 = base + 9 * n;
   v.b = base + 10 * n;
+  H->fused = base + 11 * n;
   v.s = v.r;
   v.pw = v.p;
   v.rhat0 = v.rhat;

@@ -14,7 +14,7 @@ import torch
 
 from cup3d_amd import workloads as W
 from cup3d_amd.poisson import PoissonSolver, solver_for
-from helpers import (PER, WALL, compatible_rhs, fft_solution_periodic, grid_cases,
+from helpers import (FREE, PER, WALL, compatible_rhs, fft_solution_periodic, grid_cases,
                      index_encoded_case, random_field, school4_small, tiny_amr, uniform)
 
 pytestmark = pytest.mark.gpu
@@ -498,6 +498,39 @@ def test_capped_solve_across_block_counts(gpu, bpd, bmean):
     assert torch.equal(x, x2)
     xo, info = pyoracle.Oracle(blocks, bpd, h0, bc, bmean).bicgstab(b, tol_rel=0.0, max_iter=3)
     assert np.linalg.norm(x.cpu().numpy() - xo) <= 1e-10 * np.linalg.norm(xo)
+
+
+@pytest.mark.parametrize("bmean", [0, 1, 3])
+@pytest.mark.parametrize("bpd,level,bc", [
+    ((1, 1, 1), 0, (PER,) * 3), ((2, 1, 3), 0, (PER, WALL, FREE)), ((2, 2, 2), 1, (PER,) * 3),
+    ((8, 8, 4), 0, (WALL, PER, FREE)), ((257, 1, 1), 0, (PER, WALL, WALL))])
+def test_capped_solve_of_small_single_level_grids(gpu, bpd, level, bc, bmean):
+    """Up to 256 blocks of one level the block inverse and the operator on it are
+    one kernel, which makes the neighbours' vectors for itself: a block that is
+    its own neighbour on all sides, mixed boundaries, a grid of refined blocks
+    only, the largest such grid and the smallest that is not one. Five iterations
+    (p and nu change places in each) against the oracle's iterate to 1e-10, from
+    a zero guess, and given zeros end in the same bits (with bMean 1, whose row
+    the start from given zeros adds to |r| last, within 1e-12)."""
+    n = [b << level for b in bpd]
+    blocks = W.uniform_blocks(*n)
+    blocks[:, 0] = level
+    h0 = 1.0 / (8 * max(bpd))
+    b = compatible_rhs(blocks, h0, 8)
+    out = []
+    for guess in ("zero", "given"):
+        S = PoissonSolver(bpd, h0, bc, level_max=level, bmean=bmean, guess=guess, tol_rel=0.0,
+                          max_iter=5).set_topology(blocks)
+        out.append(torch.zeros(len(b), dtype=torch.float64, device=gpu))
+        rep = S.solve_device(dev(b), out[-1])
+        assert rep["iterations"] == 5 and rep["status"] == 1
+    O = pyoracle.Oracle(blocks, bpd, h0, bc, bmean, level_max=level)
+    xo, _ = O.bicgstab(b, tol_rel=0.0, max_iter=5)
+    assert np.linalg.norm(out[0].cpu().numpy() - xo) <= 1e-10 * np.linalg.norm(xo)
+    if bmean == 1:
+        assert torch.linalg.norm(out[0] - out[1]) <= 1e-12 * torch.linalg.norm(out[0])
+    else:
+        assert torch.equal(out[0], out[1])
 
 
 @pytest.mark.parametrize("precision", ["fp64", "mixed_fp16"])
