@@ -108,6 +108,8 @@ void launch_remove_mean(hipStream_t s, long long n, double* x, const double* h3,
                         double* part, double* wsum);
 // b = a over n4 float4 (the copy-rate probe of the diagnostics).
 void launch_stream_copy(hipStream_t s, long long n4, const void* a, void* b);
+// b = a over n4 16-byte words, one of them pinned host memory.
+void launch_host_copy(hipStream_t s, long long n4, const void* a, void* b);
 
 // Warm start from several guesses (device vectors of n doubles).
 constexpr int HIST_MAX = 8;                // differences of previous pressures

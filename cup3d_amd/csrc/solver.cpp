@@ -79,7 +79,7 @@ struct DevBuf {
 }  // namespace
 
 constexpr int HOST_STATES = 5;
-constexpr int COPY_THREADS = 16;
+constexpr int COPY_THREADS = 8;
 
 // Device topology tables of one generation (topology_gpu.hip).
 struct DevTopo {
@@ -305,13 +305,18 @@ int run_bicgstab64(cup3d_poisson* H, const DevGrid<double>& g, const KrylovVecto
 }
 
 // Host blocks <-> device vector of the host entry point. Contiguous ranges of
-// blocks on up to 16 host threads (one for small grids: one core cannot feed
+// blocks on up to 8 host threads (one for small grids: one core cannot feed
 // PCIe), each copying chunk by chunk through its two slots of the pinned ring,
 // so that the copies of one chunk and the transfer of another overlap. On the
 // handle's stream; ends with every block copied (to the device: with every
-// transfer enqueued). A capped FP64 solve of 4440 blocks from and to host
-// arrays, zero guess: 2.34 ms, against 2.79 ms with whole vectors staged
-// between the copies and x uploaded too.
+// transfer enqueued). The transfers are copy kernels on the pinned memory: the
+// copy engine takes 16 us more for each, a third of its time at 1 MiB. 4440
+// blocks by 8 threads and the engine 720 us to the device and 730 us back, by
+// kernels 560 and 530 us, and by 4 threads (a thread is 15 us to start) 515 and
+// 490 us, against 330 us for either way in one transfer. A capped FP64 solve of
+// 4440 blocks from and to host arrays, zero guess:
+// 2.30 ms with the engine and 8 threads, 1.85 ms now; 16 384 blocks, two iterations,
+// 5.1 and 4.0 ms.
 constexpr int RING_BLOCKS = 256;  // 1 MiB
 
 int copy_range(cup3d_poisson* H, bool up, int t, int b0, int b1, double* dev,
@@ -346,8 +351,8 @@ int copy_range(cup3d_poisson* H, bool up, int t, int b0, int b1, double* dev,
     range(c, c0, m);
     const size_t bytes = (size_t)m * BLEN * sizeof(double);
     double* d = dev + (size_t)c0 * BLEN;
-    e = up ? hipMemcpyAsync(d, slot[c & 1], bytes, hipMemcpyHostToDevice, H->stream)
-           : hipMemcpyAsync(slot[c & 1], d, bytes, hipMemcpyDeviceToHost, H->stream);
+    launch_host_copy(H->stream, bytes / 16, up ? slot[c & 1] : d, up ? d : slot[c & 1]);
+    e = hipGetLastError();
     if (e == hipSuccess) e = hipEventRecord(ev[c & 1], H->stream);
   };
   if (up) {
@@ -373,8 +378,8 @@ int copy_range(cup3d_poisson* H, bool up, int t, int b0, int b1, double* dev,
 int copy_blocks(cup3d_poisson* H, bool up, double* dev, double* const* blocks, double* contig) {
   const unsigned hw = std::max(1u, std::thread::hardware_concurrency());
   const int nb = H->nb;
-  const int nt = (int)std::min<unsigned>(std::min(hw, (unsigned)COPY_THREADS),
-                                        (unsigned)std::max(1, nb / 512));
+  const int nt = (int)std::min<unsigned>(
+      hw, (unsigned)(nb < 16384 ? std::min(4, std::max(1, nb / 512)) : COPY_THREADS));
   if (H->ring_chunks < (size_t)2 * nt) {
     if (H->h_ring) (void)hipHostFree(H->h_ring);
     H->h_ring = nullptr;
