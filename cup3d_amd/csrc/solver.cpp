@@ -83,7 +83,7 @@ constexpr int COPY_THREADS = 8;
 
 // Device topology tables of one generation (topology_gpu.hip).
 struct DevTopo {
-  DevBuf blocks, nbr, fkind, fnb, bpar, h, invh, h3, hf, invhf, meta, keys, vals, info;
+  DevBuf blocks, nbr, fkind, fnb, bpar, h, invh, h3, hf, invhf, meta, keys, vals, info, count;
   size_t clean = 0;  // slots of the hash table that are clear, with the info words (0: dirty)
 };
 
@@ -494,7 +494,6 @@ int cup3d_poisson_set_topology(cup3d_poisson_t H, int64_t nblocks, const cup3d_b
     H->pin_bytes = list_bytes + TOPO_INFO_WORDS * sizeof(int);
   }
   std::memcpy(H->h_pin, blocks, list_bytes);
-  std::vector<int> bl(H->h_pin, H->h_pin + 4 * nblocks);
   // build the tables on the device into the other generation: a rejected
   // block list leaves the handle as it was
   const size_t nb = (size_t)nblocks;
@@ -509,11 +508,11 @@ int cup3d_poisson_set_topology(cup3d_poisson_t H, int64_t nblocks, const cup3d_b
       D.h3.reserve(nb * sizeof(double)) || D.hf.reserve(nb * sizeof(float)) ||
       D.invhf.reserve(nb * sizeof(float)) || D.meta.reserve(nb * 32 * sizeof(int)) ||
       D.keys.reserve(cap * sizeof(unsigned long long)) ||
-      D.vals.reserve(cap * sizeof(int)) || D.info.reserve(TOPO_INFO_WORDS * sizeof(int)))
+      D.vals.reserve(cap * sizeof(int)) || D.info.reserve(TOPO_INFO_WORDS * sizeof(int)) ||
+      D.count.reserve(topo_waves(nb) * sizeof(int2)))
     return fail(H, "hipMalloc(topology tables) failed");
   if (D.keys.bytes + D.vals.bytes + D.info.bytes != held) D.clean = 0;  // grown: new memory
   hipStream_t s = H->stream;
-  HIPCHECK(hipMemcpyAsync(D.blocks.p, H->h_pin, list_bytes, hipMemcpyHostToDevice, s));
   TopoParams tpar;
   tpar.nb = (int)nb;
   for (int d = 0; d < 3; ++d) {
@@ -521,12 +520,13 @@ int cup3d_poisson_set_topology(cup3d_poisson_t H, int64_t nblocks, const cup3d_b
     tpar.bc[d] = H->cfg.bc[d];
   }
   tpar.h0 = H->cfg.h0;
+  tpar.list = H->h_pin;
   tpar.blocks = D.blocks.as<int>();
   const TopoTable ttab{D.keys.as<unsigned long long>(), D.vals.as<int>(), (unsigned long long)cap - 1};
   const TopoOut tout{D.nbr.as<int>(),  D.fkind.as<int8_t>(), D.fnb.as<int>(),
                      D.bpar.as<int8_t>(), D.h.as<double>(),  D.invh.as<double>(),
                      D.h3.as<double>(), D.hf.as<float>(),  D.invhf.as<float>(),
-                     D.meta.as<int>()};
+                     D.meta.as<int>(), D.count.as<int2>()};
   const bool clear = D.clean < cap;
   // the current generation's table has served its build: leave it clear for the next one
   const size_t ecap = E.keys.p ? std::min(E.keys.bytes / sizeof(unsigned long long),
@@ -534,10 +534,10 @@ int cup3d_poisson_set_topology(cup3d_poisson_t H, int64_t nblocks, const cup3d_b
   const TopoTable etab{E.keys.as<unsigned long long>(), E.vals.as<int>(),
                        (unsigned long long)ecap - 1};
   D.clean = E.clean = 0;
-  launch_topology_build(s, tpar, ttab, tout, D.info.as<int>(), clear, etab, E.info.as<int>());
-  HIPCHECK(hipGetLastError());
   int* info = H->h_pin + 4 * nb;
-  HIPCHECK(hipMemcpyAsync(info, D.info.p, TOPO_INFO_WORDS * sizeof(int), hipMemcpyDeviceToHost, s));
+  launch_topology_build(s, tpar, ttab, tout, D.info.as<int>(), clear, etab, E.info.as<int>(), info);
+  HIPCHECK(hipGetLastError());
+  std::vector<int> bl(H->h_pin, H->h_pin + 4 * nblocks);  // while the kernels run
   HIPCHECK(hipStreamSynchronize(s));
   E.clean = ecap;
   // the first offending block in list order, with the message of the

@@ -13,7 +13,8 @@ struct TopoParams {
   int bpd[3];        // base blocks per direction, each < 2^16
   int bc[3];         // 0 freespace, 1 periodic, 2 wall
   double h0;
-  const int* blocks;  // [nb][4] (level, ix, iy, iz), 16-byte aligned
+  const int* list;   // [nb][4] (level, ix, iy, iz), 16-byte aligned, pinned host memory
+  int* blocks;       // the same on the device, written by the build
 };
 
 // Open-addressing table: key(level, i, j, k) -> smallest block id with it.
@@ -34,7 +35,10 @@ struct TopoOut {
   float* hf;
   float* invhf;
   int* meta;      // [nb][32]: fnb (24), kind (6), bpar, 0 (the SpMV's one load per lane)
+  int2* count;    // [topo_waves(nb)] coarse and fine faces per wavefront of k_topo_tables
 };
+// eight threads a block, in workgroups of four wavefronts
+constexpr size_t topo_waves(size_t nb) { return (nb * 8 + 255) / 256 * 4; }
 
 // Info words written by the build. The error words hold the smallest
 // offending block id (TI_BALANCE: block * 6 + face), INT_MAX when none.
@@ -46,8 +50,8 @@ enum TopoInfo : int {
   TI_BALANCE = 4,    // a face with no same-level, coarser or four finer blocks
   TI_FULL = 5,       // hash table full (cannot happen at capacity >= 2 nb)
   TI_ORIGIN = 6,     // largest block id at index (0, 0, 0), or -1
-  TI_N_COARSE = 7,   // faces with a coarser neighbour
-  TI_N_FINE = 8,     // faces with finer neighbours
+  TI_N_COARSE = 7,   // faces with a coarser neighbour (in the host's words only)
+  TI_N_FINE = 8,     // faces with finer neighbours (the same)
   TOPO_INFO_WORDS = 9
 };
 
@@ -56,9 +60,10 @@ __host__ __device__ inline int TopoInfoInit(unsigned long long i) {
 }
 
 // clear: t and info have to be cleared first. other, other_info: a table and
-// info words to leave cleared for the next build (keys null: none).
+// info words to leave cleared for the next build (keys null: none). host_info:
+// pinned, takes the info words.
 void launch_topology_build(hipStream_t s, const TopoParams& p, const TopoTable& t,
                            const TopoOut& o, int* info, bool clear, const TopoTable& other,
-                           int* other_info);
+                           int* other_info, int* host_info);
 
 }  // namespace cup3d

@@ -1,7 +1,7 @@
 // Topology build on the device: the per-face tables the SpMV, the caller
 // kernels and the learned warm start read (same-level neighbours, face
 // kinds, coarse/fine partners, index parities, per-block h, 1/h, h^3), built
-// from the block list (level, index[3]) in three kernels instead of a serial
+// from the block list (level, index[3]) in a few kernels instead of a serial
 // host pass. It replaces the face classification of the reference's
 // PoissonSolverExp::getMat (source/poisson/PoissonSolverExp.cpp:221-373: the
 // per-face same-level / coarser / finer tests of makeFlux, .cpp:157-219, and
@@ -10,7 +10,8 @@
 //
 //   k_topo_init    clear the hash table and the info words (a fill kernel, no
 //                  memset), where the build before did not
-//   k_topo_insert  one thread per block: validate level and index, insert
+//   k_topo_insert  one thread per block: read it from the caller's list (pinned
+//                  host memory) and keep it, validate level and index, insert
 //                  key(level, i, j, k) -> the smallest block id holding it
 //                  (open addressing, linear probing, 64-bit CAS)
 //   k_topo_tables  eight threads per block: one per face: same-level neighbour
@@ -20,13 +21,18 @@
 //                  1/h, h^3 (FP64 and FP32), index parities, the origin block.
 //                  It also clears the other generation's hash table and info
 //                  words, which nothing reads any more and the next build uses
+//   k_topo_report  the info words, with the face counts added up, to the host
+//                  (pinned memory)
 // Errors are reported as the smallest offending block (or block face) id, so
 // the message names the same block a sequential pass would stop at.
 //
-// Bound by launches and the round trips of the hash probes: a mesh change of
-// 4440 blocks with one operator application takes 72 us (97 us with a clearing
-// kernel, separate kernels per block and per face, one counter update per face
-// and pageable copies).
+// Bound by launches and the round trips of the hash probes, of which a face's
+// first six are in flight together. A mesh change of 4440 blocks with one operator
+// application takes 63 us: 97 us with a clearing kernel, separate kernels per block
+// and per face and pageable copies, 70 us with the list and the info words moved by
+// the copy engine, the probes one after the other and a counter update per
+// wavefront (whose 7400 updates of two words were most of the 116 us the tables of
+// 59 012 blocks took; now 31 us).
 
 #include <hip/hip_runtime.h>
 
@@ -56,15 +62,32 @@ __device__ __forceinline__ unsigned long long mix64(unsigned long long x) {
   return x;
 }
 
-__device__ int tfind(const TopoTable& t, int l, int i, int j, int k) {
-  if (l < 0 || l > LEVEL_MAX || i < 0 || j < 0 || k < 0 || i >= (1 << INDEX_BITS) ||
-      j >= (1 << INDEX_BITS) || k >= (1 << INDEX_BITS))
-    return -1;
-  const unsigned long long key = tkey(l, i, j, k);
-  unsigned long long slot = mix64(key) & t.mask;
-  for (unsigned long long probe = 0; probe <= t.mask; ++probe) {
+// A lookup in two parts, so that the first probes of several are in flight
+// together (key and value of a slot with them): tprobe() starts one, tresolve()
+// returns the block, or -1.
+struct Probe {
+  unsigned long long key, slot, k0;
+  int v0;
+  bool ok;
+};
+__device__ __forceinline__ Probe tprobe(const TopoTable& t, int l, int i, int j, int k) {
+  Probe q;
+  q.ok = l >= 0 && l <= LEVEL_MAX && i >= 0 && j >= 0 && k >= 0 && i < (1 << INDEX_BITS) &&
+         j < (1 << INDEX_BITS) && k < (1 << INDEX_BITS);
+  q.key = tkey(l, i, j, k);
+  q.slot = q.ok ? mix64(q.key) & t.mask : 0;
+  q.k0 = t.keys[q.slot];
+  q.v0 = t.vals[q.slot];
+  return q;
+}
+__device__ __forceinline__ int tresolve(const TopoTable& t, const Probe& q) {
+  if (!q.ok || q.k0 == KEY_EMPTY) return -1;
+  if (q.k0 == q.key) return q.v0;
+  unsigned long long slot = (q.slot + 1) & t.mask;
+  for (unsigned long long probe = 0; probe < t.mask; ++probe) {
     const unsigned long long s = t.keys[slot];
-    if (s == key) return t.vals[slot];
+    const int v = t.vals[slot];
+    if (s == q.key) return v;
     if (s == KEY_EMPTY) return -1;
     slot = (slot + 1) & t.mask;
   }
@@ -93,7 +116,8 @@ __global__ __launch_bounds__(WG_THREADS) void k_topo_insert(TopoParams p, TopoTa
                                                             int* info) {
   const int b = blockIdx.x * WG_THREADS + threadIdx.x;
   if (b >= p.nb) return;
-  const int4 B = reinterpret_cast<const int4*>(p.blocks)[b];
+  const int4 B = reinterpret_cast<const int4*>(p.list)[b];
+  reinterpret_cast<int4*>(p.blocks)[b] = B;
   const int l = B.x, I[3] = {B.y, B.z, B.w};
   if (l < 0 || l > LEVEL_MAX || I[0] < 0 || I[1] < 0 || I[2] < 0) {
     atomicMin(&info[TI_INVALID], b);
@@ -126,7 +150,7 @@ __global__ __launch_bounds__(WG_THREADS) void k_topo_insert(TopoParams p, TopoTa
 // Block b's own entries.
 __device__ void topo_block(const TopoParams& p, const TopoTable& t, const TopoOut& o, int* info,
                            int b, int4 B) {
-  if (tfind(t, B.x, B.y, B.z, B.w) != b) atomicMin(&info[TI_DUPLICATE], b);
+  if (tresolve(t, tprobe(t, B.x, B.y, B.z, B.w)) != b) atomicMin(&info[TI_DUPLICATE], b);
   // h0 / 2^l is exact (a power-of-two scaling), as is its FP32 rounding of
   // the same FP64 value
   const double h = p.h0 / (double)(1 << B.x);
@@ -154,30 +178,41 @@ __device__ int topo_face(const TopoParams& p, const TopoTable& t, const TopoOut&
   const bool boundary = (s < 0) ? I[d] == 0 : I[d] == n - 1;
   if (!(boundary && p.bc[d] != 1)) {  // a wall or freespace face has no flux
     I[d] = ((I[d] + s) % n + n) % n;
-    const int same = tfind(t, l, I[0], I[1], I[2]);
+    // the block of every case at once: the same level, the coarser one, and the
+    // four children adjacent to this face
+    const int t1 = d == 0 ? 1 : (d == 1 ? 2 : 0), t2 = d == 0 ? 2 : (d == 1 ? 0 : 1);
+    const Probe ps = tprobe(t, l, I[0], I[1], I[2]);
+    const Probe pc = tprobe(t, l - 1, I[0] >> 1, I[1] >> 1, I[2] >> 1);
+    Probe pf[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      int C[3] = {2 * I[0], 2 * I[1], 2 * I[2]};
+      C[d] += (s < 0) ? 1 : 0;
+      C[t1] += q & 1;
+      C[t2] += (q >> 1) & 1;
+      pf[q] = tprobe(t, l + 1, C[0], C[1], C[2]);
+    }
+    const int same = tresolve(t, ps);
     if (same >= 0) {
       kind = FACE_SAME;
       nbr = same;
     } else {
-      const int c = tfind(t, l - 1, I[0] >> 1, I[1] >> 1, I[2] >> 1);
+      const int c = tresolve(t, pc);
       if (c >= 0) {
         kind = FACE_COARSE;
         part[0] = c;
       } else {
-        const int t1 = d == 0 ? 1 : (d == 1 ? 2 : 0), t2 = d == 0 ? 2 : (d == 1 ? 0 : 1);
         bool ok = true;
-        for (int q = 0; q < 4; ++q) {  // the children adjacent to this face
-          int C[3] = {2 * I[0], 2 * I[1], 2 * I[2]};
-          C[d] += (s < 0) ? 1 : 0;
-          C[t1] += q & 1;
-          C[t2] += (q >> 1) & 1;
-          part[q] = tfind(t, l + 1, C[0], C[1], C[2]);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          part[q] = tresolve(t, pf[q]);
           ok = ok && part[q] >= 0;
         }
         if (ok) {
           kind = FACE_FINE;
         } else {
           atomicMin(&info[TI_BALANCE], b * 6 + f);
+#pragma unroll
           for (int q = 0; q < 4; ++q) part[q] = -1;
         }
       }
@@ -205,12 +240,9 @@ __global__ __launch_bounds__(WG_THREADS) void k_topo_tables(TopoParams p, TopoTa
       else if (f == 6) topo_block(p, t, o, info, b, B);
     }
   }
-  // one counter update per wavefront
+  // a count per wavefront, added by k_topo_report
   const unsigned long long nc = __ballot(kind == FACE_COARSE), nf = __ballot(kind == FACE_FINE);
-  if ((threadIdx.x & 63) == 0) {
-    if (nc) atomicAdd(&info[TI_N_COARSE], __popcll(nc));
-    if (nf) atomicAdd(&info[TI_N_FINE], __popcll(nf));
-  }
+  if ((threadIdx.x & 63) == 0) o.count[gid >> 6] = make_int2(__popcll(nc), __popcll(nf));
   if (other.keys) {
     for (unsigned long long i = gid; i <= other.mask; i += (unsigned long long)gridDim.x * WG_THREADS) {
       other.keys[i] = KEY_EMPTY;
@@ -220,11 +252,29 @@ __global__ __launch_bounds__(WG_THREADS) void k_topo_tables(TopoParams p, TopoTa
   }
 }
 
+__global__ __launch_bounds__(WG_THREADS) void k_topo_report(const int* info, const int2* count,
+                                                            int waves, int* host) {
+  __shared__ int sum[2];
+  if (threadIdx.x < 2) sum[threadIdx.x] = 0;
+  __syncthreads();
+  int nc = 0, nf = 0;
+  for (int i = threadIdx.x; i < waves; i += WG_THREADS) {
+    nc += count[i].x;
+    nf += count[i].y;
+  }
+  atomicAdd(&sum[0], nc);
+  atomicAdd(&sum[1], nf);
+  __syncthreads();
+  const int i = threadIdx.x;
+  if (i < TOPO_INFO_WORDS)
+    host[i] = i == TI_N_COARSE ? sum[0] : (i == TI_N_FINE ? sum[1] : info[i]);
+}
+
 }  // namespace
 
 void launch_topology_build(hipStream_t s, const TopoParams& p, const TopoTable& t,
                            const TopoOut& o, int* info, bool clear, const TopoTable& other,
-                           int* other_info) {
+                           int* other_info, int* host_info) {
   if (clear) {
     const unsigned long long cap = t.mask + 1;
     const int ninit = (int)((cap + WG_THREADS - 1) / WG_THREADS);
@@ -234,6 +284,7 @@ void launch_topology_build(hipStream_t s, const TopoParams& p, const TopoTable& 
   k_topo_insert<<<nwb, WG_THREADS, 0, s>>>(p, t, info);
   const int nwt = (int)(((long long)p.nb * 8 + WG_THREADS - 1) / WG_THREADS);
   k_topo_tables<<<nwt, WG_THREADS, 0, s>>>(p, t, o, info, other, other_info);
+  k_topo_report<<<1, WG_THREADS, 0, s>>>(info, o.count, nwt * (WG_THREADS / 64), host_info);
 }
 
 }  // namespace cup3d
