@@ -103,9 +103,9 @@ void launch_grad_p_update(hipStream_t s, const DevGrid<double>& g, const double*
                           double* vel);
 
 // x -= the volume-weighted mean of x (h3 per block, inv_vol = 1 / sum 512 h^3);
-// the weighted sum is left in wsum[0].
+// the weighted sum is left in host[0] (pinned); wsum: a word of scratch.
 void launch_remove_mean(hipStream_t s, long long n, double* x, const double* h3, double inv_vol,
-                        double* part, double* wsum);
+                        double* part, double* wsum, double* host);
 // b = a over n4 float4 (the copy-rate probe of the diagnostics).
 void launch_stream_copy(hipStream_t s, long long n4, const void* a, void* b);
 // b = a over n4 16-byte words, one of them pinned host memory.

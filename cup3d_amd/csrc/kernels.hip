@@ -205,28 +205,50 @@ __global__ __launch_bounds__(WG_THREADS) void k_wsum(long long n, const double* 
 }
 
 __global__ __launch_bounds__(WG_THREADS) void k_wsum_fin(const double* part, int nparts,
-                                                         double* out) {
+                                                         double* out, double* host) {
   double tot[1];
   grid_sum_partials<1>(part, nparts, tot);
-  if (threadIdx.x == 0) out[0] = tot[0];
+  if (threadIdx.x == 0) out[0] = host[0] = tot[0];
 }
 
+// x -= mean. SUMS: every workgroup adds the partials itself, in the finalize
+// kernel's order, and the first one gives the sum to the host.
+template <bool SUMS>
 __global__ __launch_bounds__(WG_THREADS) void k_sub_mean(long long n, double* __restrict__ x,
-                                                         const double* __restrict__ wsum,
-                                                         double inv_vol) {
-  const double m = wsum[0] * inv_vol;
-  for (long long i = (long long)blockIdx.x * WG_THREADS + threadIdx.x; i < n;
+                                                         const double* __restrict__ part,
+                                                         int nparts, double inv_vol,
+                                                         double* __restrict__ host) {
+  typedef double double2_t __attribute__((ext_vector_type(2)));
+  double tot[1];
+  if (SUMS) {
+    grid_sum_partials<1>(part, nparts, tot);
+    if (blockIdx.x == 0 && threadIdx.x == 0) host[0] = tot[0];
+  } else {
+    tot[0] = part[0];
+  }
+  const double m = tot[0] * inv_vol;
+  double2_t* __restrict__ x2 = reinterpret_cast<double2_t*>(x);
+  for (long long i = (long long)blockIdx.x * WG_THREADS + threadIdx.x; i < n / 2;
        i += (long long)gridDim.x * WG_THREADS)
-    x[i] -= m;
+    x2[i] -= (double2_t){m, m};
 }
 
+// On grids of up to FIN_MAX_BLOCKS blocks (2048 partials) the sum's finalize
+// kernel, 3 us and a launch, is left out; adding all partials in every workgroup
+// costs as much at 16 384 blocks (45 us either way) and 118 against 107 us at
+// 51 200. A call on 64 blocks 21.4 -> 17.7 us, on 8192 35.5 -> 33.7 us (with the
+// sum written to the host by a kernel, not copied).
 void launch_remove_mean(hipStream_t s, long long n, double* x, const double* h3, double inv_vol,
-                        double* part, double* wsum) {
+                        double* part, double* wsum, double* host) {
   const int nwg = (int)((n + 4 * BLEN - 1) / (4 * BLEN));
+  const int nsub = (int)std::min<long long>((n / 2 + WG_THREADS - 1) / WG_THREADS, 8192);
   k_wsum<<<nwg, WG_THREADS, 0, s>>>(n, x, h3, part);
-  k_wsum_fin<<<1, WG_THREADS, 0, s>>>(part, nwg, wsum);
-  const int nsub = (int)std::min<long long>((n + WG_THREADS - 1) / WG_THREADS, 8192);
-  k_sub_mean<<<nsub, WG_THREADS, 0, s>>>(n, x, wsum, inv_vol);
+  if (n <= (long long)FIN_MAX_BLOCKS * BLEN) {
+    k_sub_mean<true><<<std::min(nsub, 1024), WG_THREADS, 0, s>>>(n, x, part, nwg, inv_vol, host);
+  } else {
+    k_wsum_fin<<<1, WG_THREADS, 0, s>>>(part, nwg, wsum, host);
+    k_sub_mean<false><<<nsub, WG_THREADS, 0, s>>>(n, x, wsum, 1, inv_vol, host);
+  }
 }
 
 

@@ -992,11 +992,10 @@ int cup3d_poisson_remove_mean(cup3d_poisson_t H, double* d_x, double* mean) {
     }
   }
   const double inv_vol = 1.0 / H->volume;
-  launch_remove_mean(H->stream, H->n, d_x, H->tp[H->tcur].h3.as<double>(), inv_vol,
-                     H->d_part.as<double>(), H->d_gdots.as<double>());
-  HIPCHECK(hipGetLastError());
   double* wsum = &H->h_state->mean_sum;  // pinned
-  HIPCHECK(hipMemcpyAsync(wsum, H->d_gdots.p, sizeof(double), hipMemcpyDeviceToHost, H->stream));
+  launch_remove_mean(H->stream, H->n, d_x, H->tp[H->tcur].h3.as<double>(), inv_vol,
+                     H->d_part.as<double>(), H->d_gdots.as<double>(), wsum);
+  HIPCHECK(hipGetLastError());
   HIPCHECK(hipStreamSynchronize(H->stream));
   if (mean) *mean = *wsum * inv_vol;  // the value the kernel subtracted
   return 0;
