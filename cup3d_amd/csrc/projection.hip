@@ -28,7 +28,7 @@
 // in, 3 out). With one thread per cell (strided 8-byte loads, the interface
 // code in every thread, its index arrays in scratch memory) the rhs took
 // 1036 us and the update 827 us on the 30.2 M-cell grid (966 MB and 1.69 GB
-// of vectors); now they take 241 us (4.0 TB/s) and 318 us (5.3 TB/s).
+// of vectors); now they take 231 us (4.2 TB/s) and 318 us (5.3 TB/s).
 
 #include <hip/hip_runtime.h>
 
@@ -159,23 +159,24 @@ __device__ __forceinline__ void load_block(const double* __restrict__ F, size_t 
   for (int k = 0; k < V2; ++k) r[k] = p[k * 64 + lane];
 }
 
+// A block is a workgroup of its own: its 12.5 KiB of LDS come free with it, not
+// with the slowest of four (3-level AMR grid of 4440 blocks, with an obstacle: a
+// call 50 -> 47 us). On the school grid's 59 012 blocks the reads bound it, 0.98 GB
+// for 0.73 GB of velocity, the rest neighbours' faces no longer in the L2: 231 us
+// (5.3 TB/s) either way. Storing the result past the caches takes 7 us less there,
+// but the increment form, which reads it next, as much more.
 // KernelPressureRHS: out = fac (uE - uW + vN - vS + wB - wF) - chi fac (the
 // same of udef) + the finer faces' flux corrections, fac = h^2 / (2 dt).
 template <bool IFACE, bool OBST>
-__global__ __launch_bounds__(WG_THREADS) void k_pressure_rhs(DevGrid<double> g,
-                                                             const double* __restrict__ vel,
-                                                             const double* __restrict__ udef,
-                                                             const double* __restrict__ chi,
-                                                             double dt,
-                                                             double* __restrict__ out) {
-  __shared__ double Ls[WG_THREADS / 64][VLEN];
-  __shared__ double pls[IFACE ? WG_THREADS / 64 : 1][IFACE ? 64 : 1];
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int b = xcd_remap(blockIdx.x, gridDim.x) * (WG_THREADS / 64) + w;
-  if (b >= g.nb) return;  // no workgroup barrier below: only this wavefront's slice
+__global__ __launch_bounds__(64) void k_pressure_rhs(DevGrid<double> g,
+                                                     const double* __restrict__ vel,
+                                                     const double* __restrict__ udef,
+                                                     const double* __restrict__ chi, double dt,
+                                                     double* __restrict__ out) {
+  __shared__ double L[VLEN], pl[IFACE ? 64 : 1];
+  const int lane = threadIdx.x, b = xcd_remap(blockIdx.x, gridDim.x);
   const int ix = lane & 7, iy = lane >> 3;
   const size_t off = (size_t)b * BLEN;
-  double* L = Ls[w];
   int meta = 0;
   if (IFACE) meta = g.bmeta[(size_t)b * 32 + (lane & 31)];
   const int* nb6 = g.nbr + b * 6;
@@ -249,10 +250,10 @@ __global__ __launch_bounds__(WG_THREADS) void k_pressure_rhs(DevGrid<double> g,
           c_fine = -fac_f;
         }
         const double term = iface_term<3>(
-            F, OBST && field ? chi : nullptr, [&](int cell) { return L[3 * cell + d]; }, pls[w], f,
+            F, OBST && field ? chi : nullptr, [&](int cell) { return L[3 * cell + d]; }, pl, f,
             fk, d, par, lane, __builtin_amdgcn_readlane(meta, 4 * f), __shfl(meta, 4 * f + fq, 64),
             c_own, c_fine);
-        scatter_face(pls[w], f, lane, term, acc);
+        scatter_face(pl, f, lane, term, acc);
       }
     }
   }
@@ -363,15 +364,14 @@ __global__ __launch_bounds__(WG_THREADS) void k_grad_p_update(DevGrid<double> g,
 
 void launch_pressure_rhs(hipStream_t s, const DevGrid<double>& g, const double* vel,
                          const double* udef, const double* chi, double dt, double* out) {
-  const int nwg = (g.nb + WG_THREADS / 64 - 1) / (WG_THREADS / 64);
   if (g.has_iface && udef)
-    k_pressure_rhs<true, true><<<nwg, WG_THREADS, 0, s>>>(g, vel, udef, chi, dt, out);
+    k_pressure_rhs<true, true><<<g.nb, 64, 0, s>>>(g, vel, udef, chi, dt, out);
   else if (g.has_iface)
-    k_pressure_rhs<true, false><<<nwg, WG_THREADS, 0, s>>>(g, vel, udef, chi, dt, out);
+    k_pressure_rhs<true, false><<<g.nb, 64, 0, s>>>(g, vel, udef, chi, dt, out);
   else if (udef)
-    k_pressure_rhs<false, true><<<nwg, WG_THREADS, 0, s>>>(g, vel, udef, chi, dt, out);
+    k_pressure_rhs<false, true><<<g.nb, 64, 0, s>>>(g, vel, udef, chi, dt, out);
   else
-    k_pressure_rhs<false, false><<<nwg, WG_THREADS, 0, s>>>(g, vel, udef, chi, dt, out);
+    k_pressure_rhs<false, false><<<g.nb, 64, 0, s>>>(g, vel, udef, chi, dt, out);
 }
 
 void launch_grad_p_update(hipStream_t s, const DevGrid<double>& g, const double* p, double dt,
