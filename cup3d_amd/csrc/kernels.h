@@ -74,11 +74,13 @@ constexpr int STATE_COPIES = 3;
 void launch_getvec64(hipStream_t s, long long n, long long zero_row, const double* rhs,
                      const double* x0, double* b, double* x, const SolverState& init,
                      SolverState* st, double* part, double tol_b);
-// The same and the initial residual for x0 = 0: b = rhs (zero in the bMean
-// cell), r = b and x = 0 unless null, and the first iteration's scalars.
-void launch_start_zero64(hipStream_t s, int nb, long long zero_row, const double* rhs, double* b,
-                         double* r, double* x, const SolverState& init,
-                         SolverState* st, SolverState* hst, double* part, double tol_b);
+// The same and the first iteration's scalars for x0 = 0, where b is the initial
+// residual. Returns b: rhs itself, or its copy in `b` where the bMean row is zeroed
+// or the rhs overlaps x, which takes the solution (30.2 M cells: 48 us to sum it
+// against 158 us with copies to b and r and a cleared x).
+const double* launch_start_zero64(hipStream_t s, int nb, long long zero_row, const double* rhs,
+                                  const double* x, double* b, const SolverState& init,
+                                  SolverState* st, SolverState* hst, double* part, double tol_b);
 // The scalars of one component of SPMV_START (nb blocks, its partial sums).
 void launch_start_fin(hipStream_t s, int nb, const SolverState& init, SolverState* st,
                       SolverState* hst, const double* part, double tol_b);

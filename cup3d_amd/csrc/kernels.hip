@@ -38,11 +38,14 @@ void launch_getvec64(hipStream_t s, long long n, long long zero_row, const doubl
   k_getvec_fin<<<1, WG_THREADS, 0, s>>>(init, st, part, nwg, tol_b);
 }
 
-void launch_start_zero64(hipStream_t s, int nb, long long zero_row, const double* rhs, double* b,
-                         double* r, double* x, const SolverState& init,
-                         SolverState* st, SolverState* hst, double* part, double tol_b) {
-  k_start_zero<<<(nb + 3) / 4, WG_THREADS, 0, s>>>(nb, zero_row, rhs, b, r, x, part);
+const double* launch_start_zero64(hipStream_t s, int nb, long long zero_row, const double* rhs,
+                                  const double* x, double* b, const SolverState& init,
+                                  SolverState* st, SolverState* hst, double* part, double tol_b) {
+  const uintptr_t n = (uintptr_t)nb * BLEN * sizeof(double), r0 = (uintptr_t)rhs, x0 = (uintptr_t)x;
+  const bool copy = zero_row >= 0 || (r0 < x0 + n && x0 < r0 + n);
+  k_start_zero<<<(nb + 3) / 4, WG_THREADS, 0, s>>>(nb, zero_row, rhs, copy ? b : nullptr, part);
   launch_start_fin(s, nb, init, st, hst, part, tol_b);
+  return copy ? b : rhs;
 }
 
 void launch_start_fin(hipStream_t s, int nb, const SolverState& init, SolverState* st,

@@ -246,13 +246,13 @@ __device__ __forceinline__ void store8(T* __restrict__ p, const T (&v)[8]) {
 }
 
 // Start from x0 = 0: b = rhs, the residual, without an operator application
-// (the first iteration reads b for r and rhat, see run_bicgstab64; r and x are
-// written where they are given). The sum is taken as the SpMV's residual mode
+// (the first iteration reads b for r and rhat, see run_bicgstab64). b null: not
+// written, the caller reads rhs itself (zero_row < 0). The sum is taken as the SpMV's residual mode
 // takes it (a column of eight cells per lane, the workgroups in the SpMV's
 // order), so |r| has the same bits as through A x0.
 [[maybe_unused]] static __global__ __launch_bounds__(WG_THREADS) void k_start_zero(
     int nb, long long zero_row, const double* __restrict__ rhs, double* __restrict__ b,
-    double* __restrict__ r, double* __restrict__ x, double* part) {
+    double* part) {
   double v[1] = {0.0};
   const int blk = xcd_remap(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6);
   if (blk < nb) {
@@ -264,9 +264,7 @@ __device__ __forceinline__ void store8(T* __restrict__ p, const T (&v)[8]) {
     for (int iz = 0; iz < BS; ++iz) {
       const long long i = off + iz * 64;
       if (i == zero_row) q[iz] = 0.0;
-      b[i] = q[iz];
-      if (r) r[i] = q[iz];
-      if (x) x[i] = 0.0;
+      if (b) b[i] = q[iz];
       v[0] += q[iz] * q[iz];
     }
   }

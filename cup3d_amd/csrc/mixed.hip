@@ -368,8 +368,9 @@ __global__ __launch_bounds__(GT) void k_precond_h(int nb, const H* __restrict__ 
   precond_gemm<H, NBW, TPW, SPLIT, NT>(nb, j0, it0, l, Ppk, pre, As[0], As[NS - 1], sc, out);
 }
 
-// Inner-solve start: r = rhat = (float)(r64 * scale), x = 0, ||r||^2, and the
-// iteration-0 scalars (BiCGSTAB.cu:435-471 with x0 = 0).
+// Inner-solve start: rhat = (float)(r64 * scale), which the first iteration reads
+// for r too, x = 0, ||r||^2, and the iteration-0 scalars (BiCGSTAB.cu:435-471 with
+// x0 = 0).
 __global__ __launch_bounds__(WG_THREADS) void k_inner_init(long long n, const double* __restrict__ r64,
                                                            double scale, KrylovVectors<float> v,
                                                            double* part) {
@@ -384,7 +385,6 @@ __global__ __launch_bounds__(WG_THREADS) void k_inner_init(long long n, const do
       r[e] = (float)(rd[e] * scale);
       s[0] += (double)r[e] * (double)r[e];
     }
-    store8(v.r + i0, r);
     store8(v.rhat + i0, r);
   }
   grid_store_partial<1>(s, part);
@@ -410,16 +410,23 @@ __global__ __launch_bounds__(WG_THREADS) void k_inner_init_fin(SolverState init,
 
 // Fold the FP32 increment into the FP64 iterate: x64 += scale * x32[k], with
 // k = xcur (cur = 1: the recurrence continues from this iterate, its increment
-// then 0, see k_replace_fin) or xopt (cur = 0: the process ends here).
+// then 0, see k_replace_fin) or xopt (cur = 0: the process ends here). fresh: x64
+// is 0 and holds nothing yet.
 __global__ __launch_bounds__(WG_THREADS) void k_fold(long long n, double* __restrict__ x64,
                                                      KrylovVectors<float> v,
                                                      const SolverState* st, double scale,
-                                                     int cur) {
-  if (cur ? st->x_zero : st->opt_zero) return;
+                                                     int cur, bool fresh) {
+  const bool none = cur ? st->x_zero : st->opt_zero;
+  if (none && !fresh) return;
   const float* __restrict__ d = v.x[cur ? st->xcur : st->xopt];
   for (long long i = (long long)blockIdx.x * WG_THREADS + threadIdx.x; i < n;
        i += (long long)gridDim.x * WG_THREADS)
-    x64[i] = fma(scale, (double)d[i], x64[i]);
+    x64[i] = fma(scale, none ? 0.0 : (double)d[i], fresh ? 0.0 : x64[i]);
+}
+__global__ __launch_bounds__(WG_THREADS) void k_zero64(long long n, double* __restrict__ x) {
+  for (long long i = (long long)blockIdx.x * WG_THREADS + threadIdx.x; i < n;
+       i += (long long)gridDim.x * WG_THREADS)
+    x[i] = 0.0;
 }
 
 // Residual replacement: r32 = r64 * inv_scale (the true FP64 residual of
@@ -676,7 +683,7 @@ int mixed_solve(MixedWorkspace& M, hipStream_t s, const cup3d_poisson_config& cf
   const long long n = M.n;
   KrylovVectors<float> v = M.v32;  // p and pw change places when they are two
   double* x64 = d_x;
-  double* b64 = v64.b;
+  const double* b64 = v64.b;
   double* r64 = v64.r;
   // getVec + ||b|| (FP64); the iterate is d_x itself
   SolverState init = inner_state(cfg, 0.0);
@@ -693,12 +700,15 @@ int mixed_solve(MixedWorkspace& M, hipStream_t s, const cup3d_poisson_config& cf
     return 0;
   };
   double rnorm = 0;
-  if (d_x0) {
-    launch_getvec64(s, n, zero_row, d_rhs, d_x0, b64, x64, init, st, part, cfg.tol_rhs);
+  const bool zero = !d_x0;
+  bool fresh = zero;          // x64 is 0 and not written yet
+  const double* start = r64;  // the first inner solve's residual
+  if (!zero) {
+    launch_getvec64(s, n, zero_row, d_rhs, d_x0, v64.b, x64, init, st, part, cfg.tol_rhs);
     if (true_resid(rnorm)) return -1;
-  } else {  // r64 = b64, without the operator
-    launch_start_zero64(s, M.nb, zero_row, d_rhs, b64, r64, x64, init, st, h_st, part,
-                        cfg.tol_rhs);
+  } else {  // r = b, without the operator
+    b64 = start = launch_start_zero64(s, M.nb, zero_row, d_rhs, x64, v64.b, init, st, h_st, part,
+                                      cfg.tol_rhs);
     MCHECK(hipGetLastError());
     MCHECK(hipStreamSynchronize(s));
     rnorm = std::sqrt(h_st->true_rr);
@@ -741,7 +751,9 @@ int mixed_solve(MixedWorkspace& M, hipStream_t s, const cup3d_poisson_config& cf
     const double scale = rnorm;
     const double inner_rel = std::max(cfg.inner_tol, 0.5 * tol / scale);
     *h_st = inner_state(cfg, inner_rel);  // the loop's view until the first poll
-    k_inner_init<<<grid_vec(n), WG_THREADS, 0, s>>>(n, r64, 1.0 / scale, v, part);
+    k_inner_init<<<grid_vec(n), WG_THREADS, 0, s>>>(n, start, 1.0 / scale, v, part);
+    start = r64;
+    bool first = true;
     k_inner_init_fin<<<1, WG_THREADS, 0, s>>>(*h_st, st, part, grid_vec(n));
     ++steps;
     double last = 1.0;  // recurrence residual (scaled) at the last replacement
@@ -760,6 +772,8 @@ int mixed_solve(MixedWorkspace& M, hipStream_t s, const cup3d_poisson_config& cf
         // event pairs (2k, 2k+1) bracket the main kernel of K(k+1)
         const bool tm = M.prof && it == tm_it;
         if (tm) MCHECK(hipEventRecord(M.pev[0], s));
+        float* const r = v.r;
+        if (first) v.r = v.rhat;  // K1 and K3 of the first iteration
         launch_precond_mixed(M, v, s, cfg.precision, PREC_P, g32, nullptr, nullptr, st,
                              it > 0 ? fin : FIN_KERNEL, fp);
         std::swap(v.p, v.pw);
@@ -768,6 +782,8 @@ int mixed_solve(MixedWorkspace& M, hipStream_t s, const cup3d_poisson_config& cf
         spmv32<SPMV_DOT1>(s, g32, v.z1, v.nu, v.rhat, st, part, !fin, tm ? M.pev[3] : nullptr);
         if (tm) MCHECK(hipEventRecord(M.pev[4], s));
         launch_precond_mixed(M, v, s, cfg.precision, PREC_S, g32, nullptr, nullptr, st, fin, fs);
+        v.r = r;
+        first = false;
         if (tm) MCHECK(hipEventRecord(M.pev[5], s));
         if (tm) MCHECK(hipEventRecord(M.pev[6], s));
         spmv32<SPMV_DOT2>(s, g32, v.z2, v.t, v.s, st, part, !fin, tm ? M.pev[7] : nullptr);
@@ -805,7 +821,8 @@ int mixed_solve(MixedWorkspace& M, hipStream_t s, const cup3d_poisson_config& cf
         break;
       }
       if ((ist == ST_RUNNING || ist == ST_CONVERGED) && REPLACE_DROP > 0) {
-        k_fold<<<grid_1d(n), WG_THREADS, 0, s>>>(n, x64, v, st, scale, 1);
+        k_fold<<<grid_1d(n), WG_THREADS, 0, s>>>(n, x64, v, st, scale, 1, fresh);
+        fresh = false;
         if (true_resid(rnorm)) return -1;
         ++replacements;
         if (!std::isfinite(rnorm)) {
@@ -827,7 +844,8 @@ int mixed_solve(MixedWorkspace& M, hipStream_t s, const cup3d_poisson_config& cf
       }
       // breakdown or iteration cap (or a stop without replacements): keep the
       // best iterate, restart
-      k_fold<<<grid_1d(n), WG_THREADS, 0, s>>>(n, x64, v, st, scale, 0);
+      k_fold<<<grid_1d(n), WG_THREADS, 0, s>>>(n, x64, v, st, scale, 0, fresh);
+      fresh = false;
       if (true_resid(rnorm)) return -1;
       if (!std::isfinite(rnorm)) {
         status = ST_NONFINITE;
@@ -843,6 +861,7 @@ int mixed_solve(MixedWorkspace& M, hipStream_t s, const cup3d_poisson_config& cf
     total_iters += h_st->iters_done;
     total_restarts += h_st->restarts;
   }
+  if (fresh) k_zero64<<<grid_1d(n), WG_THREADS, 0, s>>>(n, x64);  // no increment was made
   MCHECK(hipGetLastError());
   if (rep) {
     rep->status = status;

@@ -659,16 +659,17 @@ static void report64(const SolverState& S, cup3d_solve_report* rep) {
 }
 
 // The initial residual r = b - A x0 in v.r and v.rhat (BiCGSTAB.cu:435-467); a
-// zero guess (d_x0 null) takes no operator application and leaves it in v.b.
+// zero guess (d_x0 null) takes no operator application and leaves it in v.b, which
+// is only read (the rhs itself unless it overlaps d_x).
 static void start64(cup3d_poisson_t H, const DevGrid<double>& g, KrylovVectors<double>& v,
-                    long long zero_row, const double* d_rhs, const double* d_x0,
+                    long long zero_row, const double* d_rhs, const double* d_x, const double* d_x0,
                     const SolverState& init, double tol_b) {
   hipStream_t s = H->stream;
   SolverState* st = H->d_state.as<SolverState>();
   double* part = H->d_part.as<double>();
   if (!d_x0) {
-    launch_start_zero64(s, H->nb, zero_row, d_rhs, v.b, nullptr, nullptr, init, st, nullptr, part,
-                        tol_b);
+    v.b = const_cast<double*>(launch_start_zero64(s, H->nb, zero_row, d_rhs, d_x, v.b, init, st,
+                                                  nullptr, part, tol_b));
     v.rhat0 = v.b;
     return;
   }
@@ -701,7 +702,7 @@ static int solve_fp64(cup3d_poisson_t H, const double* d_rhs, double* d_x, const
                                  ? (long long)H->topo.origin_block * BLEN
                                  : -1;
   KrylovVectors<double> v = H->v64;
-  start64(H, H->g64, v, zero_row, d_rhs, d_x0, make_state(H->cfg), H->cfg.tol_rhs);
+  start64(H, H->g64, v, zero_row, d_rhs, d_x, d_x0, make_state(H->cfg), H->cfg.tol_rhs);
   if (run_bicgstab64(H, H->g64, v) != 0) return -1;
   if (finish64(H, H->g64, v, d_x, H->h_state) != 0) return -1;
   HIPCHECK(hipStreamSynchronize(H->stream));
@@ -1171,7 +1172,7 @@ int cup3d_diffusion_solve_device(cup3d_poisson_t H, int comp, double nu, double 
   hipStream_t s = H->stream;
   HIPCHECK(hipEventRecord(H->ev0, s));
   KrylovVectors<double> v = H->v64;
-  start64(H, g, v, -1, d_rhs, d_x, diffusion_state(H, tol_abs, tol_rel), 0.0);
+  start64(H, g, v, -1, d_rhs, d_x, d_x, diffusion_state(H, tol_abs, tol_rel), 0.0);
   if (run_bicgstab64(H, g, v, 1) != 0) return -1;
   if (finish64(H, g, v, d_x, H->h_state) != 0) return -1;
   HIPCHECK(hipEventRecord(H->ev1, s));

@@ -559,6 +559,29 @@ def test_zero_guess_equals_given_zeros(gpu, name, bmean, precision):
     assert abs(r1["true_rel_resid"] - r0["true_rel_resid"]) <= tol * r0["true_rel_resid"] + 1e-14
 
 
+@pytest.mark.parametrize("precision", ["fp64", "mixed_fp16"])
+@pytest.mark.parametrize("bmean", [0, 1, 2])
+@pytest.mark.parametrize("shift", [-512, 0, 512])
+def test_zero_guess_over_its_rhs(gpu, precision, bmean, shift):
+    """From a zero guess the rhs is read where it is unless x overlaps it: solving
+    onto the rhs, or a block before or behind it, gives the bits of a solve into
+    a vector of its own, which leaves the rhs as it was."""
+    blocks, bpd, h0, bc = CASES["amr3_walls"]
+    n = len(blocks) * 512
+    b = dev(compatible_rhs(blocks, h0, 9))
+    S = PoissonSolver(bpd, h0, bc, bmean=bmean, precision=precision, guess="zero", tol_rel=1e-6,
+                      level_max=2).set_topology(blocks)
+    x, rhs = torch.full_like(b, float("nan")), b.clone()
+    r0 = S.solve_device(rhs, x)
+    assert torch.equal(rhs, b)
+    buf = torch.zeros(n + 1024, dtype=torch.float64, device=gpu)
+    over, rhs = buf[512 + shift:512 + shift + n], buf[512:512 + n]
+    rhs.copy_(b)
+    r1 = S.solve_device(rhs, over)
+    assert r0["iterations"] == r1["iterations"] and r0["status"] == r1["status"]
+    assert torch.equal(x, over)
+
+
 @pytest.mark.parametrize("bmean", [0, 1, 2, 3])
 @pytest.mark.parametrize("name", ["uniform_walls_3x2x2", "tiny_amr_periodic"])
 def test_zero_guess_restarts(gpu, name, bmean):
