@@ -40,11 +40,12 @@ struct MixedWorkspace {
 
 int mixed_init_pinv(MixedWorkspace& M, const std::vector<double>& P, std::string& err);
 int mixed_set_topology(MixedWorkspace& M, int nb, long long n, std::string& err);
+// Ends with a wait for `end`, recorded behind the last of its work.
 int mixed_solve(MixedWorkspace& M, hipStream_t s, const cup3d_poisson_config& cfg,
                 const DevGrid<double>& g64, const DevGrid<float>& g32,
                 const KrylovVectors<double>& v64, SolverState* st, SolverState* h_st,
                 double* part, int origin_block, const double* d_rhs, double* d_x,
-                const double* d_x0, cup3d_solve_report* rep, std::string& err);
+                const double* d_x0, hipEvent_t end, cup3d_solve_report* rep, std::string& err);
 // y = A x with the FP32 operator of the inner solve (x, y FP64 device vectors).
 int mixed_apply_operator32(MixedWorkspace& M, hipStream_t s, const DevGrid<float>& g32,
                            SolverState* st, double* part, const double* d_x, double* d_y,

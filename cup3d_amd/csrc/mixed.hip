@@ -679,7 +679,7 @@ int mixed_solve(MixedWorkspace& M, hipStream_t s, const cup3d_poisson_config& cf
                 const DevGrid<double>& g64, const DevGrid<float>& g32,
                 const KrylovVectors<double>& v64, SolverState* st, SolverState* h_st,
                 double* part, int origin_block, const double* d_rhs, double* d_x,
-                const double* d_x0, cup3d_solve_report* rep, std::string& err) {
+                const double* d_x0, hipEvent_t end, cup3d_solve_report* rep, std::string& err) {
   const long long n = M.n;
   KrylovVectors<float> v = M.v32;  // p and pw change places when they are two
   double* x64 = d_x;
@@ -692,10 +692,13 @@ int mixed_solve(MixedWorkspace& M, hipStream_t s, const cup3d_poisson_config& cf
       (cfg.bmean == 1 || cfg.bmean == 3) && origin_block >= 0 ? (long long)origin_block * BLEN : -1;
   int total_iters = 0, total_restarts = 0, steps = 0, replacements = 0, status = ST_MAXITER;
   const int poll = cfg.poll_every > 0 ? cfg.poll_every : 8;
+  bool ended = false;  // `end` is behind everything in the stream, and was waited for
   auto true_resid = [&](double& out) -> int {  // |b - A x64| in FP64, r64 = b - A x64
     launch_spmv64(s, SPMV_RESID, g64, x64, nullptr, b64, r64, nullptr, st, part, true, h_st);
     MCHECK(hipGetLastError());
-    MCHECK(hipStreamSynchronize(s));
+    MCHECK(hipEventRecord(end, s));
+    MCHECK(hipEventSynchronize(end));
+    ended = true;
     out = std::sqrt(h_st->true_rr);
     return 0;
   };
@@ -751,6 +754,7 @@ int mixed_solve(MixedWorkspace& M, hipStream_t s, const cup3d_poisson_config& cf
     const double scale = rnorm;
     const double inner_rel = std::max(cfg.inner_tol, 0.5 * tol / scale);
     *h_st = inner_state(cfg, inner_rel);  // the loop's view until the first poll
+    ended = false;
     k_inner_init<<<grid_vec(n), WG_THREADS, 0, s>>>(n, start, 1.0 / scale, v, part);
     start = r64;
     bool first = true;
@@ -835,6 +839,7 @@ int mixed_solve(MixedWorkspace& M, hipStream_t s, const cup3d_poisson_config& cf
           done = true;
           break;
         }
+        ended = false;
         k_replace<<<grid_vec(n), WG_THREADS, 0, s>>>(n, r64, 1.0 / scale, v, part);
         k_replace_fin<<<1, WG_THREADS, 0, s>>>(st, part, grid_vec(n));
         last = rnorm / scale;
@@ -863,6 +868,10 @@ int mixed_solve(MixedWorkspace& M, hipStream_t s, const cup3d_poisson_config& cf
   }
   if (fresh) k_zero64<<<grid_1d(n), WG_THREADS, 0, s>>>(n, x64);  // no increment was made
   MCHECK(hipGetLastError());
+  if (fresh || !ended) {
+    MCHECK(hipEventRecord(end, s));
+    MCHECK(hipEventSynchronize(end));
+  }
   if (rep) {
     rep->status = status;
     rep->iterations = total_iters;
