@@ -64,6 +64,26 @@ __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
+// Maximum over the wavefront, the same way.
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float wave_max(float v) {
+  {
+    const auto u = __builtin_amdgcn_permlane32_swap(__float_as_int(v), __float_as_int(v), false, false);
+    v = fmaxf(__int_as_float(u[0]), __int_as_float(u[1]));
+  }
+  {
+    const auto u = __builtin_amdgcn_permlane16_swap(__float_as_int(v), __float_as_int(v), false, false);
+    v = fmaxf(__int_as_float(u[0]), __int_as_float(u[1]));
+  }
+  v = fmaxf(v, dpp_move<0x128>(v));
+  v = fmaxf(v, dpp_move<0x124>(v));
+  v = fmaxf(v, dpp_move<0x4e>(v));
+  return fmaxf(v, dpp_move<0xb1>(v));
+}
+
 // Sum K values over the 256-thread workgroup in a fixed order; the result is
 // valid in thread 0 only.
 template <int K>

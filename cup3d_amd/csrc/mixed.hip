@@ -138,15 +138,17 @@ struct FillRegs {
   static constexpr int F4 = 2 * NPB;     // float4 per lane per vector (a block is 2 x 64 float4)
   static_assert(NBW % NWP == 0, "block group must fill the waves");
   float4 ra[F4], rb[F4], rc[F4];
+  float ih[NPB];  // h^-1 of the blocks
 };
 
 template <int MODE, int NBW, int NWP, bool NT>
 __device__ __forceinline__ void precond_load(int nb, int j0, int w, int l,
                                              const KrylovVectors<float>& v,
                                              const float* __restrict__ pin,
+                                             const float* __restrict__ invh,
                                              FillRegs<NBW, NWP>& R) {
-  constexpr int F4 = FillRegs<NBW, NWP>::F4;
-  const int jw = w * FillRegs<NBW, NWP>::NPB;
+  constexpr int F4 = FillRegs<NBW, NWP>::F4, NPB = FillRegs<NBW, NWP>::NPB;
+  const int jw = w * NPB;
 #pragma unroll
   for (int u = 0; u < F4; ++u) {
     const int b = j0 + jw + u / 2;
@@ -165,6 +167,15 @@ __device__ __forceinline__ void precond_load(int nb, int j0, int w, int l,
     } else {
       R.ra[u] = R.rb[u] = R.rc[u] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
+  }
+  // behind the vectors: where it is used, every wavefront of the workgroup waits
+  // for it before the products (819 blocks, 32 iterations, with the maximum by
+  // register moves: 1101 -> 1077 us, 8192 blocks 2990 -> 2950 us). Vectors that
+  // come past the caches (NT) keep two workgroups of a CU apart, and it costs K1
+  // 2 % there (59 012 blocks 131.5 -> 134 us).
+  if (!NT) {
+#pragma unroll
+    for (int jj = 0; jj < NPB; ++jj) R.ih[jj] = invh[min(j0 + jw + jj, nb - 1)];
   }
 }
 
@@ -208,9 +219,7 @@ __device__ __forceinline__ void precond_convert(int nb, int j0, int w, int l, fl
                                            fmaxf(fabsf(val.z), fabsf(val.w))));
   }
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1)
-#pragma unroll
-    for (int jj = 0; jj < NPB; ++jj) amax[jj] = fmaxf(amax[jj], __shfl_xor(amax[jj], o, 64));
+  for (int jj = 0; jj < NPB; ++jj) amax[jj] = wave_max(amax[jj]);
 #pragma unroll
   for (int u = 0; u < F4; ++u) {
     const int jj = u / 2;
@@ -229,7 +238,7 @@ __device__ __forceinline__ void precond_convert(int nb, int j0, int w, int l, fl
     if (SPLIT) *reinterpret_cast<H4*>(&A1[o]) = lo;
     if ((u & 1) == 0 && l == 0) {
       const int b = j0 + jw + jj;
-      sc[jw + jj] = b < nb ? invh[b] * p_unscale / s : 0.f;
+      sc[jw + jj] = b < nb ? (NT ? invh[b] : R.ih[jj]) * p_unscale / s : 0.f;
     }
   }
 }
@@ -336,7 +345,7 @@ __global__ __launch_bounds__(GT) void k_precond_h(int nb, const H* __restrict__ 
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
   const int it0 = part * (32 / SPL) + w * TPW;
   FillRegs<NBW, GW> R;
-  precond_load<MODE, NBW, GW, NT>(nb, j0, w, l, v, pin, R);
+  precond_load<MODE, NBW, GW, NT>(nb, j0, w, l, v, pin, invh, R);
   HV pre[TPW < 4 ? 16 : 1][TPW];
   if constexpr (TPW < 4) {
 #pragma unroll
