@@ -18,6 +18,7 @@
 #include <cstring>
 #include <initializer_list>
 #include <memory>
+#include <new>
 #include <string>
 #include <thread>
 #include <vector>
@@ -537,7 +538,13 @@ int cup3d_poisson_set_topology(cup3d_poisson_t H, int64_t nblocks, const cup3d_b
   int* info = H->h_pin + 4 * nb;
   launch_topology_build(s, tpar, ttab, tout, D.info.as<int>(), clear, etab, E.info.as<int>(), info);
   HIPCHECK(hipGetLastError());
-  std::vector<int> bl(H->h_pin, H->h_pin + 4 * nblocks);  // while the kernels run
+  std::vector<int> bl;
+  try {
+    bl.assign(H->h_pin, H->h_pin + 4 * nblocks);  // while the kernels run
+  } catch (const std::bad_alloc&) {
+    (void)hipStreamSynchronize(s);  // they read the pinned list
+    return fail(H, "out of host memory");
+  }
   HIPCHECK(hipStreamSynchronize(s));
   E.clean = ecap;
   // the first offending block in list order, with the message of the
