@@ -780,7 +780,8 @@ int mixed_solve(MixedWorkspace& M, hipStream_t s, const cup3d_poisson_config& cf
       const int tm_it = poll / 2;
       const int iter0 = h_st->iter;
       // no more than the iterations the cap leaves
-      const int batch = std::min(poll, std::max(1, cfg.max_iter - h_st->iters_done));
+      const int done0 = h_st->iters_done;
+      const int batch = std::min(poll, std::max(1, cfg.max_iter - done0));
       for (int it = 0; it < batch; ++it) {
         // event pairs (2k, 2k+1) bracket the main kernel of K(k+1)
         const bool tm = M.prof && it == tm_it;
@@ -806,6 +807,8 @@ int mixed_solve(MixedWorkspace& M, hipStream_t s, const cup3d_poisson_config& cf
       }
       MCHECK(hipGetLastError());
       MCHECK(hipStreamSynchronize(s));
+      // the iterations behind a stop left p where it was, and the process may go on
+      if ((batch - (h_st->iters_done - done0)) & 1) std::swap(v.p, v.pw);
       if (M.prof && h_st->iter - iter0 > tm_it) {
         for (int k = 0; k < 5; ++k) {
           float ms = 0.f;

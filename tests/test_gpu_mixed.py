@@ -399,3 +399,31 @@ def test_zero_guess_has_the_bits_of_given_zeros(gpu, bpd):
         out.append((S.solve_device(b, x)["err_init"], x))
     assert out[0][0] == out[1][0]
     assert torch.equal(out[0][1], out[1][1])
+
+
+@pytest.mark.parametrize("prec,bmean", [("mixed_fp16", 0), ("mixed_bf16", 1)])
+@pytest.mark.parametrize("bpd", [(9, 5, 3), (17, 8, 8), (13, 13, 13)])
+@pytest.mark.parametrize("poll", [2, 8, 9])
+def test_inner_process_resumes_with_its_own_vectors(gpu, poll, bpd, prec, bmean):
+    """With inner_tol above the fall that a replacement waits for (0.1), every
+    FP64 correction follows a stop of the inner process, mostly with iterations
+    launched behind it that find it stopped, and the process then goes on. How
+    many of those there are must not matter: polling after every iteration, when
+    there are none, takes the same iterations to the same bits (135, 1088 and
+    2197 blocks: p in two vectors on the first two). Two inner processes of 48
+    iterations, below the 50 after which polls look for a stall."""
+    h0 = 1.0 / 64
+    blocks = W.uniform_blocks(*bpd)
+    b = torch.from_numpy(compatible_rhs(blocks, h0, 8)).cuda()
+    out = []
+    for every in (1, poll):
+        S = PoissonSolver(bpd, h0, (2, 2, 2), bmean=bmean, precision=prec, guess="zero",
+                          tol_rel=0.0, inner_tol=0.2, max_iter=48, max_refine=1,
+                          poll_every=every).set_topology(blocks)
+        x = torch.zeros_like(b)
+        out.append((S.solve_device(b, x), x))
+    (r0, x0), (r1, x1) = out
+    assert r0["status"] == r1["status"] == 1
+    assert r0["iterations"] == r1["iterations"] == 96
+    assert r0["refinements"] == r1["refinements"] >= 5
+    assert torch.equal(x0, x1)
