@@ -70,7 +70,8 @@ inline double* start_part(double* part, int nb) { return part + 8 * (size_t)((nb
 // written by the finalize kernel.
 constexpr int STATE_COPIES = 3;
 
-// The state starts as `init`, with ||b|| and the absolute tolerance.
+// The state starts as `init`, with ||b|| and the absolute tolerance. x may be x0, and
+// the rhs may overlap either.
 void launch_getvec64(hipStream_t s, long long n, long long zero_row, const double* rhs,
                      const double* x0, double* b, double* x, const SolverState& init,
                      SolverState* st, double* part, double tol_b);

@@ -34,7 +34,12 @@ void launch_getvec64(hipStream_t s, long long n, long long zero_row, const doubl
                      const double* x0, double* b, double* x, const SolverState& init,
                      SolverState* st, double* part, double tol_b) {
   const int nwg = (int)((n + 4 * BLEN - 1) / (4 * BLEN));
-  k_getvec<<<nwg, WG_THREADS, 0, s>>>(n, zero_row, rhs, x0, b, x, part);
+  // in place, and the rhs shares a part of x: the zeroed cell is another cell of the
+  // rhs, which another workgroup reads, so it is zeroed behind the copy
+  const uintptr_t r0 = (uintptr_t)rhs, xa = (uintptr_t)x, len = (uintptr_t)n * sizeof(double);
+  const bool later = x == x0 && rhs != x && r0 < xa + len && xa < r0 + len;
+  k_getvec<<<nwg, WG_THREADS, 0, s>>>(n, zero_row, rhs, x0, b, later ? nullptr : x, part);
+  if (later) launch_zero_cell(s, x, zero_row);
   k_getvec_fin<<<1, WG_THREADS, 0, s>>>(init, st, part, nwg, tol_b);
 }
 

@@ -206,8 +206,8 @@ __device__ __forceinline__ void store8(T* __restrict__ p, const T (&v)[8]) {
 
 // ---------------------------------------------------------------------------
 // getVec (PoissonSolverExp.cpp:375-418): b = rhs, x = x0 (may be the same
-// vector), both zeroed at the bMean cell for bMeanConstraint 1 and 3; also
-// ||b||^2.
+// vector, null: not written), both zeroed at the bMean cell for bMeanConstraint 1
+// and 3; also ||b||^2.
 // ---------------------------------------------------------------------------
 [[maybe_unused]] static __global__ __launch_bounds__(WG_THREADS) void k_getvec(
     long long n, long long zero_row, const double* __restrict__ rhs, const double* x0,
@@ -217,7 +217,7 @@ __device__ __forceinline__ void store8(T* __restrict__ p, const T (&v)[8]) {
   if (i0 < n) {
     double bv[8], xv[8];
     load8(rhs + i0, bv);
-    const bool copy = x != x0 || (zero_row >= i0 && zero_row < i0 + 8);
+    const bool copy = x && (x != x0 || (zero_row >= i0 && zero_row < i0 + 8));
     if (x0 && copy) load8(x0 + i0, xv);
 #pragma unroll
     for (int e = 0; e < 8; ++e) {

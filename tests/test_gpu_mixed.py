@@ -427,3 +427,24 @@ def test_inner_process_resumes_with_its_own_vectors(gpu, poll, bpd, prec, bmean)
     assert r0["iterations"] == r1["iterations"] == 96
     assert r0["refinements"] == r1["refinements"] >= 5
     assert torch.equal(x0, x1)
+
+
+@pytest.mark.parametrize("bmean", [0, 1, 3])
+@pytest.mark.parametrize("shift", [-4000, -1, 0, 1, 4000])
+def test_given_guess_that_overlaps_the_rhs(gpu, shift, bmean):
+    """The mixed form iterates in the caller's x and zeroes the mean-constraint
+    cell there; where the rhs shares a part of x that cell is another cell of the
+    rhs, read by another workgroup. x lies `shift` blocks behind the rhs: the
+    bits of a solve with vectors of their own."""
+    blocks = W.uniform_blocks(16, 16, 16)
+    n = len(blocks) * 512
+    buf = torch.from_numpy(np.random.default_rng(12).standard_normal(n + 512 * abs(shift))).cuda()
+    S = PoissonSolver((16, 16, 16), 1.0 / 128, (2, 2, 2), bmean=bmean, precision="mixed_fp16",
+                      tol_rel=0.0, max_iter=4, max_refine=1).set_topology(blocks)
+    at = max(0, -shift) * 512
+    rhs, x = buf[at:at + n], buf[at + shift * 512:at + shift * 512 + n]
+    b, want = rhs.clone(), x.clone()
+    r0 = S.solve_device(b, want)
+    r1 = S.solve_device(rhs, x)
+    assert r0["err_init"] == r1["err_init"] and r0["rhs_norm"] == r1["rhs_norm"]
+    assert torch.equal(x, want)
