@@ -53,8 +53,10 @@ struct DevBuf {
   }
   hipError_t alloc(size_t b) {
     release();
-    bytes = b;
-    return hipMalloc(&p, b ? b : 1);
+    const hipError_t e = hipMalloc(&p, b ? b : 1);
+    if (e == hipSuccess) bytes = b;
+    else p = nullptr;
+    return e;
   }
   // at least b bytes; keeps the allocation when it is large enough (the
   // contents are not preserved either way)
@@ -502,7 +504,10 @@ int cup3d_poisson_set_topology(cup3d_poisson_t H, int64_t nblocks, const cup3d_b
   while (cap < 2 * nb) cap <<= 1;
   DevTopo& D = H->tp[1 - H->tcur];
   DevTopo& E = H->tp[H->tcur];
-  const size_t held = D.keys.bytes + D.vals.bytes + D.info.bytes;
+  // new memory is not clear, also where a later allocation fails
+  if (D.keys.bytes < cap * sizeof(unsigned long long) || D.vals.bytes < cap * sizeof(int) ||
+      D.info.bytes < TOPO_INFO_WORDS * sizeof(int))
+    D.clean = 0;
   if (D.blocks.reserve(nb * 4 * sizeof(int)) || D.nbr.reserve(nb * 6 * sizeof(int)) ||
       D.fkind.reserve(nb * 6) || D.fnb.reserve(nb * 24 * sizeof(int)) || D.bpar.reserve(nb) ||
       D.h.reserve(nb * sizeof(double)) || D.invh.reserve(nb * sizeof(double)) ||
@@ -512,7 +517,6 @@ int cup3d_poisson_set_topology(cup3d_poisson_t H, int64_t nblocks, const cup3d_b
       D.vals.reserve(cap * sizeof(int)) || D.info.reserve(TOPO_INFO_WORDS * sizeof(int)) ||
       D.count.reserve(topo_waves(nb) * sizeof(int2)))
     return fail(H, "hipMalloc(topology tables) failed");
-  if (D.keys.bytes + D.vals.bytes + D.info.bytes != held) D.clean = 0;  // grown: new memory
   hipStream_t s = H->stream;
   TopoParams tpar;
   tpar.nb = (int)nb;

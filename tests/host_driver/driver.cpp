@@ -1,0 +1,187 @@
+// The host side of the solver (cup3d_amd/csrc/solver.cpp, as it is) over a
+// stand-in HIP runtime: device memory is host memory full of garbage, every
+// allocation is counted and any one of them can be made to fail, and the kernel
+// launches that a test looks at check their arguments instead. Calls that no
+// test reaches stay unresolved. One scenario a run, named by argv[1]; exit
+// status 0 when it holds.
+#include "../../cup3d_amd/csrc/solver.cpp"
+
+#include <cstdio>
+#include <cstdlib>
+#include <set>
+
+namespace {
+
+int g_allocs = 0;        // device and pinned allocations so far
+int g_pinned = 0;        // pinned ones
+int g_fail_at = -1;      // number of the allocation that fails (-1: none)
+std::set<void*> g_live;  // what is allocated
+
+hipError_t take(void** p, size_t bytes) {
+  *p = nullptr;
+  if (g_allocs++ == g_fail_at) return hipErrorOutOfMemory;
+  *p = std::malloc(bytes ? bytes : 1);
+  std::memset(*p, 0x5a, bytes);
+  g_live.insert(*p);
+  return hipSuccess;
+}
+hipError_t give(void* p) {
+  if (!p) return hipSuccess;
+  if (!g_live.erase(p)) {
+    std::printf("free of memory that is not allocated\n");
+    std::exit(1);
+  }
+  std::free(p);
+  return hipSuccess;
+}
+
+void check(bool ok, const char* what) {
+  if (ok) return;
+  std::printf("%s\n", what);
+  std::exit(1);
+}
+
+}  // namespace
+
+extern "C" {
+hipError_t hipMalloc(void** p, size_t n) { return take(p, n); }
+hipError_t hipFree(void* p) { return give(p); }
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+  ++g_pinned;
+  return take(p, n);
+}
+hipError_t hipHostFree(void* p) { return give(p); }
+hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) {
+  std::memcpy(d, s, n);
+  return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
+  std::memcpy(d, s, n);
+  return hipSuccess;
+}
+hipError_t hipMemset(void* d, int v, size_t n) {
+  std::memset(d, v, n);
+  return hipSuccess;
+}
+hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t) { return hipMemset(d, v, n); }
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipGetDeviceCount(int* n) {
+  *n = 1;
+  return hipSuccess;
+}
+hipError_t hipGetLastError() { return hipSuccess; }
+const char* hipGetErrorString(hipError_t) { return "stand-in error"; }
+hipError_t hipStreamCreate(hipStream_t* s) {
+  *s = nullptr;
+  return hipSuccess;
+}
+hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t* e) {
+  *e = nullptr;
+  return hipSuccess;
+}
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) {
+  *ms = 1.f;
+  return hipSuccess;
+}
+}
+
+namespace cup3d {
+
+int mixed_init_pinv(MixedWorkspace&, const std::vector<double>&, std::string&) { return 0; }
+int mixed_set_topology(MixedWorkspace&, int, long long, std::string&) { return 0; }
+void mixed_free(MixedWorkspace&) {}
+int cnn_init(CnnState&, std::string&) { return 0; }
+int cnn_set_topology(CnnState&, int, const int*, const double*, std::string&) { return 0; }
+void cnn_free(CnnState&) {}
+
+// A build wants its hash table and info words clear (it clears them when it is
+// told to) and leaves them used, the others clear.
+void launch_topology_build(hipStream_t, const TopoParams& p, const TopoTable& t, const TopoOut& o,
+                           int* info, bool clear, const TopoTable& other, int* other_info,
+                           int* host_info) {
+  auto wipe = [](const TopoTable& q, int* words) {
+    for (unsigned long long i = 0; i <= q.mask; ++i) {
+      q.keys[i] = ~0ull;
+      q.vals[i] = 0x7fffffff;
+    }
+    for (int i = 0; i < TOPO_INFO_WORDS; ++i) words[i] = TopoInfoInit(i);
+  };
+  if (clear) wipe(t, info);
+  bool clean = true;
+  for (unsigned long long i = 0; i <= t.mask; ++i)
+    clean = clean && t.keys[i] == ~0ull && t.vals[i] == 0x7fffffff;
+  for (int i = 0; i < TOPO_INFO_WORDS; ++i) clean = clean && info[i] == TopoInfoInit(i);
+  check(clean, "a topology build found its hash table or info words used");
+  for (unsigned long long i = 0; i <= t.mask; ++i) t.keys[i] = i;
+  for (int i = 0; i < TOPO_INFO_WORDS; ++i) info[i] = i;
+  std::memcpy(p.blocks, p.list, (size_t)p.nb * 4 * sizeof(int));
+  std::memset(o.meta, 0, (size_t)p.nb * 32 * sizeof(int));
+  for (size_t i = 0; i < topo_waves(p.nb); ++i) o.count[i] = int2{0, 0};
+  if (other.keys) wipe(other, other_info);
+  for (int i = 0; i < TOPO_INFO_WORDS; ++i) host_info[i] = TopoInfoInit(i);
+}
+
+}  // namespace cup3d
+
+namespace {
+
+cup3d_poisson_t make() {
+  cup3d_poisson_config c;
+  std::memset(&c, 0, sizeof(c));
+  for (int d = 0; d < 3; ++d) {
+    c.bpd[d] = 1 << 10;
+    c.bc[d] = CUP3D_BC_WALL;
+  }
+  c.h0 = 1.0 / 24;
+  c.max_iter = 10;
+  c.max_restarts = 100;
+  cup3d_poisson_t H = nullptr;
+  check(cup3d_poisson_create(&c, &H) == 0, "create failed");
+  return H;
+}
+
+std::vector<cup3d_block_desc> row(int n) {
+  std::vector<cup3d_block_desc> b(n);
+  for (int i = 0; i < n; ++i) b[i] = {0, {i % 1024, i / 1024, 0}};
+  return b;
+}
+
+int topology(cup3d_poisson_t H, int n) {
+  const std::vector<cup3d_block_desc> b = row(n);
+  return cup3d_poisson_set_topology(H, n, b.data());
+}
+
+// Small lists, a larger one whose k-th allocation fails, and small ones again,
+// for every k: each build that runs starts from a clear table.
+void failed_allocations() {
+  for (int k = 0;; ++k) {
+    cup3d_poisson_t H = make();
+    for (int i = 0; i < 3; ++i) check(topology(H, 100) == 0, "a small list failed");
+    g_fail_at = g_allocs + k;
+    const bool failed = topology(H, 5000) != 0;
+    g_fail_at = -1;
+    for (int n : {100, 120, 100, 5000, 100, 6000})
+      check(topology(H, n) == 0 && H->nb == n, "a list failed after a failed allocation");
+    cup3d_poisson_destroy(H);
+    if (!failed) {  // every allocation had its turn
+      check(k >= 10, "too few allocations were made to fail");
+      return;
+    }
+  }
+}
+
+}  // namespace
+
+int main(int argc, char** argv) {
+  const std::string what = argc > 1 ? argv[1] : "";
+  if (what == "failed_allocations") failed_allocations();
+  else check(false, "no such scenario");
+  check(g_live.empty(), "memory was left allocated");
+  std::printf("ok\n");
+  return 0;
+}
