@@ -100,11 +100,10 @@ struct cup3d_poisson {
 
   // topology: the tables live on the device (built there by the topology
   // kernels, two generations so that a rejected block list leaves the
-  // current one in place); the host keeps the block list, the volume, the
-  // origin block and the face counts
+  // current one in place); the host keeps the volume, the origin block and the
+  // face counts
   HostTopology topo;
-  std::vector<int> blocks;  // nb x 4
-  double volume = 0.0;      // sum of 512 h_b^3 in block order (0: not summed yet)
+  double volume = 0.0;  // sum of 512 h_b^3 in block order
   int nb = 0;
   long long n = 0;
   DevTopo tp[2];
@@ -542,13 +541,13 @@ int cup3d_poisson_set_topology(cup3d_poisson_t H, int64_t nblocks, const cup3d_b
   int* info = H->h_pin + 4 * nb;
   launch_topology_build(s, tpar, ttab, tout, D.info.as<int>(), clear, etab, E.info.as<int>(), info);
   HIPCHECK(hipGetLastError());
-  std::vector<int> bl;
-  try {
-    bl.assign(H->h_pin, H->h_pin + 4 * nblocks);  // while the kernels run
-  } catch (const std::bad_alloc&) {
-    (void)hipStreamSynchronize(s);  // they read the pinned list
-    return fail(H, "out of host memory");
+  // while the kernels run; a level out of range is found by them
+  double vol[16], volume = 0.0;
+  for (int l = 0; l < 16; ++l) {
+    const double h = H->cfg.h0 / double(1 << l);
+    vol[l] = 512.0 * (h * h * h);
   }
+  for (size_t b = 0; b < nb; ++b) volume += vol[blocks[b].level & 15];
   HIPCHECK(hipStreamSynchronize(s));
   E.clean = ecap;
   // the first offending block in list order, with the message of the
@@ -576,9 +575,8 @@ int cup3d_poisson_set_topology(cup3d_poisson_t H, int64_t nblocks, const cup3d_b
   Tn.n_fine_faces = info[TI_N_FINE];
   if (H->cfg.bmean == 1 && Tn.origin_block >= 0) Tn.bmean_row = (long long)Tn.origin_block * BLEN;
   H->tcur = 1 - H->tcur;
-  H->blocks.swap(bl);
   H->topo = std::move(Tn);
-  H->volume = 0.0;
+  H->volume = volume;
   // from here on a failure (device allocation) leaves the handle without a
   // topology: solves are refused until set_topology succeeds
   struct Commit {
@@ -996,12 +994,6 @@ int cup3d_poisson_remove_mean(cup3d_poisson_t H, double* d_x, double* mean) {
   if (H->nb <= 0) return fail(H, "set_topology must be called first");
   if (check_vectors(H, {d_x}) != 0) return -1;
   HIPCHECK(hipSetDevice(H->device));
-  if (H->volume == 0.0) {
-    for (int b = 0; b < H->nb; ++b) {
-      const double h = H->cfg.h0 / double(1 << H->blocks[4 * b]);
-      H->volume += 512.0 * (h * h * h);
-    }
-  }
   const double inv_vol = 1.0 / H->volume;
   double* wsum = &H->h_state->mean_sum;  // pinned
   launch_remove_mean(H->stream, H->n, d_x, H->tp[H->tcur].h3.as<double>(), inv_vol,

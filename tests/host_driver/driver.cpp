@@ -16,6 +16,8 @@ int g_allocs = 0;        // device and pinned allocations so far
 int g_pinned = 0;        // pinned ones
 int g_fail_at = -1;      // number of the allocation that fails (-1: none)
 std::set<void*> g_live;  // what is allocated
+bool g_reject = false;   // the next topology build finds a duplicate block
+double g_inv_vol = 0.0;  // of the last mean removal
 
 hipError_t take(void** p, size_t bytes) {
   *p = nullptr;
@@ -124,6 +126,12 @@ void launch_topology_build(hipStream_t, const TopoParams& p, const TopoTable& t,
   for (size_t i = 0; i < topo_waves(p.nb); ++i) o.count[i] = int2{0, 0};
   if (other.keys) wipe(other, other_info);
   for (int i = 0; i < TOPO_INFO_WORDS; ++i) host_info[i] = TopoInfoInit(i);
+  if (g_reject) host_info[TI_DUPLICATE] = 1;
+}
+
+void launch_remove_mean(hipStream_t, long long, double*, const double*, double inv_vol, double*,
+                        double*, double*) {
+  g_inv_vol = inv_vol;
 }
 
 }  // namespace cup3d
@@ -147,7 +155,7 @@ cup3d_poisson_t make() {
 
 std::vector<cup3d_block_desc> row(int n) {
   std::vector<cup3d_block_desc> b(n);
-  for (int i = 0; i < n; ++i) b[i] = {0, {i % 1024, i / 1024, 0}};
+  for (int i = 0; i < n; ++i) b[i] = {i % 3, {i % 1024, i / 1024, 0}};
   return b;
 }
 
@@ -175,11 +183,34 @@ void failed_allocations() {
   }
 }
 
+// The volume is summed by the mesh change, in the order of its blocks, and a
+// mean removal divides by it; a rejected list leaves it.
+void volume() {
+  cup3d_poisson_t H = make();
+  alignas(16) double x[2] = {};
+  for (int n : {7, 1000, 5}) {
+    const std::vector<cup3d_block_desc> b = row(n);
+    double want = 0.0;
+    for (const cup3d_block_desc& d : b) {
+      const double h = 1.0 / 24 / double(1 << d.level);
+      want += 512.0 * (h * h * h);
+    }
+    check(topology(H, n) == 0 && H->volume == want, "volume of a new mesh");
+    g_reject = true;
+    check(topology(H, 13) != 0, "a duplicate block was accepted");
+    g_reject = false;
+    check(cup3d_poisson_remove_mean(H, x, nullptr) == 0 && g_inv_vol == 1.0 / want,
+          "volume of a mean removal");
+  }
+  cup3d_poisson_destroy(H);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "failed_allocations") failed_allocations();
+  else if (what == "volume") volume();
   else check(false, "no such scenario");
   check(g_live.empty(), "memory was left allocated");
   std::printf("ok\n");
