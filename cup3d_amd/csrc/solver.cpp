@@ -82,11 +82,17 @@ struct DevBuf {
 }  // namespace
 
 constexpr int HOST_STATES = 5;
+// Blocks of a topology's list on their way to the device at a time (1 MiB of
+// pinned memory, allocated with the handle). A pinned allocation takes 0.3-0.5 ms, as
+// much as the kernels of many mesh changes, so none follows the size of the mesh:
+// one as long as the list made every mesh larger than all before it 20 % slower
+// than a pageable copy.
+constexpr int LIST_BLOCKS = 1 << 16;
 constexpr int COPY_THREADS = 8;
 
 // Device topology tables of one generation (topology_gpu.hip).
 struct DevTopo {
-  DevBuf blocks, nbr, fkind, fnb, bpar, h, invh, h3, hf, invhf, meta, keys, vals, info, count;
+  DevBuf blocks, nbr, fkind, fnb, bpar, h, invh, h3, hf, invhf, meta, keys, vals, info;
   size_t clean = 0;  // slots of the hash table that are clear, with the info words (0: dirty)
 };
 
@@ -120,7 +126,8 @@ struct cup3d_poisson {
   double* fused = nullptr;  // those
   DevBuf d_state, d_part;
   SolverState* h_state = nullptr;  // pinned: [0] a solve's state, [1 .. 3] results per component,
-                                   // [4] the progress word (run_bicgstab64)
+                                   // [4] the progress word (run_bicgstab64), then h_list
+  int* h_list = nullptr;           // info words of a topology build, the list (LIST_BLOCKS)
   size_t part_len = 0;
 
   // mixed precision workspace
@@ -133,8 +140,6 @@ struct cup3d_poisson {
   // first host solve that needs them and kept
   DevBuf d_stage;             // 2 n doubles
   double* h_ring = nullptr;   // pinned
-  int* h_pin = nullptr;       // pinned: block list and info words of a topology build
-  size_t pin_bytes = 0;
   size_t ring_chunks = 0;
   hipEvent_t ring_ev[2 * COPY_THREADS] = {};
 
@@ -455,11 +460,14 @@ int cup3d_poisson_create(const cup3d_poisson_config* cfg, cup3d_poisson_t* out) 
   H->device = c.device;
   if (hipSetDevice(c.device) != hipSuccess || hipStreamCreate(&H->stream) != hipSuccess ||
       hipEventCreate(&H->ev0) != hipSuccess || hipEventCreate(&H->ev1) != hipSuccess ||
-      hipHostMalloc((void**)&H->h_state, HOST_STATES * sizeof(SolverState),
+      hipHostMalloc((void**)&H->h_state,
+                    HOST_STATES * sizeof(SolverState) +
+                        (TOPO_INFO_PAD + 4 * (size_t)LIST_BLOCKS) * sizeof(int),
                     hipHostMallocDefault) != hipSuccess) {
     g_create_error = "HIP stream/event/pinned allocation failed";
     return -1;
   }
+  H->h_list = reinterpret_cast<int*>(H->h_state + HOST_STATES);
   // block-Jacobi inverse (PoissonSolverExp ctor): the dense matrix of the
   // half-precision GEMM
   build_pinv_dst(H->P);
@@ -485,17 +493,6 @@ int cup3d_poisson_set_topology(cup3d_poisson_t H, int64_t nblocks, const cup3d_b
   if (nblocks > (1LL << 22)) return fail(H, "too many blocks (limit 4194304)");
   HIPCHECK(hipSetDevice(H->device));
   static_assert(sizeof(cup3d_block_desc) == 4 * sizeof(int), "a block is four words");
-  // pinned: the block list on its way to the device, then the info words
-  const size_t list_bytes = (size_t)nblocks * sizeof(cup3d_block_desc);
-  if (H->pin_bytes < list_bytes + TOPO_INFO_WORDS * sizeof(int)) {
-    if (H->h_pin) (void)hipHostFree(H->h_pin);
-    H->h_pin = nullptr;
-    H->pin_bytes = 0;
-    HIPCHECK(hipHostMalloc((void**)&H->h_pin, list_bytes + TOPO_INFO_WORDS * sizeof(int),
-                           hipHostMallocDefault));
-    H->pin_bytes = list_bytes + TOPO_INFO_WORDS * sizeof(int);
-  }
-  std::memcpy(H->h_pin, blocks, list_bytes);
   // build the tables on the device into the other generation: a rejected
   // block list leaves the handle as it was
   const size_t nb = (size_t)nblocks;
@@ -511,10 +508,10 @@ int cup3d_poisson_set_topology(cup3d_poisson_t H, int64_t nblocks, const cup3d_b
       D.fkind.reserve(nb * 6) || D.fnb.reserve(nb * 24 * sizeof(int)) || D.bpar.reserve(nb) ||
       D.h.reserve(nb * sizeof(double)) || D.invh.reserve(nb * sizeof(double)) ||
       D.h3.reserve(nb * sizeof(double)) || D.hf.reserve(nb * sizeof(float)) ||
-      D.invhf.reserve(nb * sizeof(float)) || D.meta.reserve(nb * 32 * sizeof(int)) ||
+      D.invhf.reserve(nb * sizeof(float)) ||
+      D.meta.reserve(nb * 32 * sizeof(int) + topo_waves(nb) * sizeof(int2)) ||  // and the counts
       D.keys.reserve(cap * sizeof(unsigned long long)) ||
-      D.vals.reserve(cap * sizeof(int)) || D.info.reserve(TOPO_INFO_WORDS * sizeof(int)) ||
-      D.count.reserve(topo_waves(nb) * sizeof(int2)))
+      D.vals.reserve(cap * sizeof(int)) || D.info.reserve(TOPO_INFO_WORDS * sizeof(int)))
     return fail(H, "hipMalloc(topology tables) failed");
   hipStream_t s = H->stream;
   TopoParams tpar;
@@ -524,13 +521,13 @@ int cup3d_poisson_set_topology(cup3d_poisson_t H, int64_t nblocks, const cup3d_b
     tpar.bc[d] = H->cfg.bc[d];
   }
   tpar.h0 = H->cfg.h0;
-  tpar.list = H->h_pin;
   tpar.blocks = D.blocks.as<int>();
   const TopoTable ttab{D.keys.as<unsigned long long>(), D.vals.as<int>(), (unsigned long long)cap - 1};
   const TopoOut tout{D.nbr.as<int>(),  D.fkind.as<int8_t>(), D.fnb.as<int>(),
                      D.bpar.as<int8_t>(), D.h.as<double>(),  D.invh.as<double>(),
                      D.h3.as<double>(), D.hf.as<float>(),  D.invhf.as<float>(),
-                     D.meta.as<int>(), D.count.as<int2>()};
+                     D.meta.as<int>(),
+                     reinterpret_cast<int2*>(D.meta.as<int>() + nb * 32)};
   const bool clear = D.clean < cap;
   // the current generation's table has served its build: leave it clear for the next one
   const size_t ecap = E.keys.p ? std::min(E.keys.bytes / sizeof(unsigned long long),
@@ -538,8 +535,15 @@ int cup3d_poisson_set_topology(cup3d_poisson_t H, int64_t nblocks, const cup3d_b
   const TopoTable etab{E.keys.as<unsigned long long>(), E.vals.as<int>(),
                        (unsigned long long)ecap - 1};
   D.clean = E.clean = 0;
-  int* info = H->h_pin + 4 * nb;
-  launch_topology_build(s, tpar, ttab, tout, D.info.as<int>(), clear, etab, E.info.as<int>(), info);
+  int *info = H->h_list, *list = info + TOPO_INFO_PAD;
+  for (size_t b = 0; b < nb; b += LIST_BLOCKS) {
+    if (b > 0) HIPCHECK(hipStreamSynchronize(s));  // the kernel has read the range before
+    const size_t m = std::min(nb - b, (size_t)LIST_BLOCKS);
+    std::memcpy(list, blocks + b, m * sizeof(cup3d_block_desc));
+    launch_topology_insert(s, tpar, ttab, D.info.as<int>(), clear && b == 0, (int)b, (int)m, list);
+    HIPCHECK(hipGetLastError());
+  }
+  launch_topology_tables(s, tpar, ttab, tout, D.info.as<int>(), etab, E.info.as<int>(), info);
   HIPCHECK(hipGetLastError());
   // while the kernels run; a level out of range is found by them
   double vol[16], volume = 0.0;
@@ -1524,7 +1528,6 @@ void cup3d_poisson_destroy(cup3d_poisson_t H) {
   mixed_free(H->mixed);
   if (H->h_state) (void)hipHostFree(H->h_state);
   if (H->h_ring) (void)hipHostFree(H->h_ring);
-  if (H->h_pin) (void)hipHostFree(H->h_pin);
   for (hipEvent_t e : H->ring_ev)
     if (e) (void)hipEventDestroy(e);
   if (H->ev0) (void)hipEventDestroy(H->ev0);

@@ -13,8 +13,7 @@ struct TopoParams {
   int bpd[3];        // base blocks per direction, each < 2^16
   int bc[3];         // 0 freespace, 1 periodic, 2 wall
   double h0;
-  const int* list;   // [nb][4] (level, ix, iy, iz), 16-byte aligned, pinned host memory
-  int* blocks;       // the same on the device, written by the build
+  int* blocks;       // [nb][4] (level, ix, iy, iz) on the device, written by the build
 };
 
 // Open-addressing table: key(level, i, j, k) -> smallest block id with it.
@@ -54,16 +53,21 @@ enum TopoInfo : int {
   TI_N_FINE = 8,     // faces with finer neighbours (the same)
   TOPO_INFO_WORDS = 9
 };
+constexpr int TOPO_INFO_PAD = 16;  // room for them in front of 16-byte words
 
 __host__ __device__ inline int TopoInfoInit(unsigned long long i) {
   return i == TI_ORIGIN ? -1 : (i >= TI_N_COARSE ? 0 : 0x7fffffff);
 }
 
-// clear: t and info have to be cleared first. other, other_info: a table and
-// info words to leave cleared for the next build (keys null: none). host_info:
-// pinned, takes the info words.
-void launch_topology_build(hipStream_t s, const TopoParams& p, const TopoTable& t,
-                           const TopoOut& o, int* info, bool clear, const TopoTable& other,
-                           int* other_info, int* host_info);
+// The build, in two parts. First the blocks, range by range: count of them from
+// block `first`, list[count][4] (16-byte aligned, pinned host memory); clear: t and
+// info have to be cleared before. Then the tables. other, other_info: a hash
+// table and info words to leave cleared for the next build (keys null: none).
+// host_info: pinned, takes the info words.
+void launch_topology_insert(hipStream_t s, const TopoParams& p, const TopoTable& t, int* info,
+                            bool clear, int first, int count, const int* list);
+void launch_topology_tables(hipStream_t s, const TopoParams& p, const TopoTable& t,
+                            const TopoOut& o, int* info, const TopoTable& other, int* other_info,
+                            int* host_info);
 
 }  // namespace cup3d

@@ -112,11 +112,12 @@ __global__ __launch_bounds__(WG_THREADS) void k_topo_init(TopoTable t, int* info
   if (i < TOPO_INFO_WORDS) info[i] = TopoInfoInit(i);
 }
 
-__global__ __launch_bounds__(WG_THREADS) void k_topo_insert(TopoParams p, TopoTable t,
-                                                            int* info) {
-  const int b = blockIdx.x * WG_THREADS + threadIdx.x;
-  if (b >= p.nb) return;
-  const int4 B = reinterpret_cast<const int4*>(p.list)[b];
+__global__ __launch_bounds__(WG_THREADS) void k_topo_insert(TopoParams p, TopoTable t, int* info,
+                                                            int first, int count,
+                                                            const int* __restrict__ list) {
+  const int i = blockIdx.x * WG_THREADS + threadIdx.x, b = first + i;
+  if (i >= count) return;
+  const int4 B = reinterpret_cast<const int4*>(list)[i];
   reinterpret_cast<int4*>(p.blocks)[b] = B;
   const int l = B.x, I[3] = {B.y, B.z, B.w};
   if (l < 0 || l > LEVEL_MAX || I[0] < 0 || I[1] < 0 || I[2] < 0) {
@@ -272,16 +273,20 @@ __global__ __launch_bounds__(WG_THREADS) void k_topo_report(const int* info, con
 
 }  // namespace
 
-void launch_topology_build(hipStream_t s, const TopoParams& p, const TopoTable& t,
-                           const TopoOut& o, int* info, bool clear, const TopoTable& other,
-                           int* other_info, int* host_info) {
+void launch_topology_insert(hipStream_t s, const TopoParams& p, const TopoTable& t, int* info,
+                            bool clear, int first, int count, const int* list) {
   if (clear) {
     const unsigned long long cap = t.mask + 1;
     const int ninit = (int)((cap + WG_THREADS - 1) / WG_THREADS);
     k_topo_init<<<ninit, WG_THREADS, 0, s>>>(t, info);
   }
-  const int nwb = (p.nb + WG_THREADS - 1) / WG_THREADS;
-  k_topo_insert<<<nwb, WG_THREADS, 0, s>>>(p, t, info);
+  const int nwb = (count + WG_THREADS - 1) / WG_THREADS;
+  k_topo_insert<<<nwb, WG_THREADS, 0, s>>>(p, t, info, first, count, list);
+}
+
+void launch_topology_tables(hipStream_t s, const TopoParams& p, const TopoTable& t,
+                            const TopoOut& o, int* info, const TopoTable& other, int* other_info,
+                            int* host_info) {
   const int nwt = (int)(((long long)p.nb * 8 + WG_THREADS - 1) / WG_THREADS);
   k_topo_tables<<<nwt, WG_THREADS, 0, s>>>(p, t, o, info, other, other_info);
   k_topo_report<<<1, WG_THREADS, 0, s>>>(info, o.count, nwt * (WG_THREADS / 64), host_info);

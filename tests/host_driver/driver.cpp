@@ -23,7 +23,7 @@ hipError_t take(void** p, size_t bytes) {
   *p = nullptr;
   if (g_allocs++ == g_fail_at) return hipErrorOutOfMemory;
   *p = std::malloc(bytes ? bytes : 1);
-  std::memset(*p, 0x5a, bytes);
+  std::memset(*p, 0x5a, std::min(bytes, (size_t)1 << 24));
   g_live.insert(*p);
   return hipSuccess;
 }
@@ -103,27 +103,34 @@ void cnn_free(CnnState&) {}
 
 // A build wants its hash table and info words clear (it clears them when it is
 // told to) and leaves them used, the others clear.
-void launch_topology_build(hipStream_t, const TopoParams& p, const TopoTable& t, const TopoOut& o,
-                           int* info, bool clear, const TopoTable& other, int* other_info,
-                           int* host_info) {
-  auto wipe = [](const TopoTable& q, int* words) {
-    for (unsigned long long i = 0; i <= q.mask; ++i) {
-      q.keys[i] = ~0ull;
-      q.vals[i] = 0x7fffffff;
-    }
-    for (int i = 0; i < TOPO_INFO_WORDS; ++i) words[i] = TopoInfoInit(i);
-  };
+void wipe(const TopoTable& t, int* info) {
+  for (unsigned long long i = 0; i <= t.mask; ++i) {
+    t.keys[i] = ~0ull;
+    t.vals[i] = 0x7fffffff;
+  }
+  for (int i = 0; i < TOPO_INFO_WORDS; ++i) info[i] = TopoInfoInit(i);
+}
+
+void launch_topology_insert(hipStream_t, const TopoParams& p, const TopoTable& t, int* info,
+                            bool clear, int first, int count, const int* list) {
   if (clear) wipe(t, info);
   bool clean = true;
   for (unsigned long long i = 0; i <= t.mask; ++i)
     clean = clean && t.keys[i] == ~0ull && t.vals[i] == 0x7fffffff;
   for (int i = 0; i < TOPO_INFO_WORDS; ++i) clean = clean && info[i] == TopoInfoInit(i);
-  check(clean, "a topology build found its hash table or info words used");
+  check(clean || first > 0, "a topology build found its hash table or info words used");
+  std::memcpy(p.blocks + 4 * (size_t)first, list, (size_t)count * 4 * sizeof(int));
+  t.keys[0] = 0;
+}
+
+void launch_topology_tables(hipStream_t, const TopoParams& p, const TopoTable& t,
+                            const TopoOut& o, int* info, const TopoTable& other, int* other_info,
+                            int* host_info) {
   for (unsigned long long i = 0; i <= t.mask; ++i) t.keys[i] = i;
   for (int i = 0; i < TOPO_INFO_WORDS; ++i) info[i] = i;
-  std::memcpy(p.blocks, p.list, (size_t)p.nb * 4 * sizeof(int));
   std::memset(o.meta, 0, (size_t)p.nb * 32 * sizeof(int));
-  for (size_t i = 0; i < topo_waves(p.nb); ++i) o.count[i] = int2{0, 0};
+  for (size_t i = 0; i < topo_waves(p.nb); ++i) o.count[i] = int2{1, 1};
+  for (size_t i = 0; i < (size_t)p.nb * 32; ++i) check(o.meta[i] == 0, "overlapping tables");
   if (other.keys) wipe(other, other_info);
   for (int i = 0; i < TOPO_INFO_WORDS; ++i) host_info[i] = TopoInfoInit(i);
   if (g_reject) host_info[TI_DUPLICATE] = 1;
@@ -155,7 +162,7 @@ cup3d_poisson_t make() {
 
 std::vector<cup3d_block_desc> row(int n) {
   std::vector<cup3d_block_desc> b(n);
-  for (int i = 0; i < n; ++i) b[i] = {i % 3, {i % 1024, i / 1024, 0}};
+  for (int i = 0; i < n; ++i) b[i] = {i % 3, {i % 1024, i / 1024, n}};
   return b;
 }
 
@@ -205,12 +212,28 @@ void volume() {
   cup3d_poisson_destroy(H);
 }
 
+// Meshes each larger than all before: no pinned allocation, and the whole list
+// reaches the device, also one longer than the pinned memory it goes through.
+void growing_meshes() {
+  cup3d_poisson_t H = make();
+  const int pinned = g_pinned;
+  for (int n : {1, 100, 5000, 65535, 65536, 65537, 140000}) {
+    const std::vector<cup3d_block_desc> b = row(n);
+    check(topology(H, n) == 0, "a larger mesh failed");
+    check(!std::memcmp(H->tp[H->tcur].blocks.p, b.data(), n * sizeof(b[0])),
+          "the block list on the device");
+  }
+  check(g_pinned == pinned, "a mesh change allocated pinned memory");
+  cup3d_poisson_destroy(H);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "failed_allocations") failed_allocations();
   else if (what == "volume") volume();
+  else if (what == "growing_meshes") growing_meshes();
   else check(false, "no such scenario");
   check(g_live.empty(), "memory was left allocated");
   std::printf("ok\n");
