@@ -1483,6 +1483,7 @@ int cup3d_debug_time_diffusion_kernel(cup3d_poisson_t H, int which, double nu, d
   hipStream_t s = H->stream;
   SolverState init = make_state(H->cfg);
   init.beta = 0.0;  // K1 recomputes p = r on every repetition
+  init.p_zero = 0;  // from all its vectors
   init.iter = 1;
   *H->h_state = init;
   SolverState* st = H->d_state.as<SolverState>();

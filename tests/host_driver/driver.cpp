@@ -18,6 +18,7 @@ int g_fail_at = -1;      // number of the allocation that fails (-1: none)
 std::set<void*> g_live;  // what is allocated
 bool g_reject = false;   // the next topology build finds a duplicate block
 double g_inv_vol = 0.0;  // of the last mean removal
+int g_short_k1 = 0;      // K1 launches that would not read p and nu
 
 hipError_t take(void** p, size_t bytes) {
   *p = nullptr;
@@ -136,6 +137,13 @@ void launch_topology_tables(hipStream_t, const TopoParams& p, const TopoTable& t
   if (g_reject) host_info[TI_DUPLICATE] = 1;
 }
 
+void launch_spmv64(hipStream_t, int, const DevGrid<double>&, const double*, double*, const double*,
+                   double*, double*, SolverState*, double*, bool, SolverState*) {}
+void launch_precond_dst(hipStream_t, int mode, int, const double*, double,
+                        const KrylovVectors<double>&, SolverState* st, int, const FinArgs&) {
+  if (mode == PREC_P) g_short_k1 += st->p_zero;
+}
+
 void launch_remove_mean(hipStream_t, long long, double*, const double*, double inv_vol, double*,
                         double*, double*) {
   g_inv_vol = inv_vol;
@@ -227,6 +235,21 @@ void growing_meshes() {
   cup3d_poisson_destroy(H);
 }
 
+// The timed K1 of the implicit diffusion moves the five vectors that its reported
+// bytes count: the state it starts from has a p.
+void timed_diffusion_kernels() {
+  cup3d_poisson_t H = make();
+  check(topology(H, 10) == 0, "topology");
+  for (int which = 0; which < 3; ++which) {
+    double ms = 0, bytes = 0, flops = 0;
+    check(cup3d_debug_time_diffusion_kernel(H, which, 1e-3, 1e-2, 3, &ms, &bytes, &flops) == 0,
+          "timing failed");
+    check(bytes == (which == 1 ? 5.0 : 2.0) * 8 * 512 * 10, "bytes of a timed kernel");
+  }
+  check(g_short_k1 == 0, "the timed K1 reads three vectors and is reported with five");
+  cup3d_poisson_destroy(H);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -234,6 +257,7 @@ int main(int argc, char** argv) {
   if (what == "failed_allocations") failed_allocations();
   else if (what == "volume") volume();
   else if (what == "growing_meshes") growing_meshes();
+  else if (what == "timed_diffusion_kernels") timed_diffusion_kernels();
   else check(false, "no such scenario");
   check(g_live.empty(), "memory was left allocated");
   std::printf("ok\n");

@@ -22,7 +22,8 @@ def driver(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["failed_allocations", "volume", "growing_meshes"])
+@pytest.mark.parametrize("scenario", ["failed_allocations", "volume", "growing_meshes",
+                                      "timed_diffusion_kernels"])
 def test_scenario(driver, scenario):
     r = subprocess.run([str(driver), scenario], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0 and r.stdout == "ok\n", (r.returncode, r.stdout, r.stderr)
