@@ -117,9 +117,6 @@ struct cup3d_poisson {
   DevGrid<double> g64;
   DevGrid<float> g32;
 
-  // preconditioner
-  std::vector<double> P;
-
   // FP64 Krylov workspace
   DevBuf d_vec64;  // 11 vectors of n doubles, small grids FUSE_VECTORS more
   KrylovVectors<double> v64{};
@@ -470,8 +467,9 @@ int cup3d_poisson_create(const cup3d_poisson_config* cfg, cup3d_poisson_t* out) 
   H->h_list = reinterpret_cast<int*>(H->h_state + HOST_STATES);
   // block-Jacobi inverse (PoissonSolverExp ctor): the dense matrix of the
   // half-precision GEMM
-  build_pinv_dst(H->P);
-  if (mixed_init_pinv(H->mixed, H->P, H->err) != 0 || cnn_init(H->cnn, H->err) != 0) {
+  std::vector<double> P;
+  build_pinv_dst(P);
+  if (mixed_init_pinv(H->mixed, P, H->err) != 0 || cnn_init(H->cnn, H->err) != 0) {
     g_create_error = H->err;
     return -1;
   }
