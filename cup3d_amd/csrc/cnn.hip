@@ -326,11 +326,11 @@ __device__ __forceinline__ void zero_ring(_Float16* buf, int tid) {
 // second layer's activations, and the first layer's: 52 KiB per workgroup,
 // three workgroups per CU. The vector ALUs bound it, mostly by the exact GELU of
 // 16 384 values a block (about 36 instructions each, 120 us of 8192 blocks); the
-// LDS reads and the products (60 us) run beside them. 328 us on 8192 blocks with
-// the zero padding selected per operand (20 instructions a read), 230 us with it
-// built into the layout, 185 us with conflict-free reads shared by the tiles,
-// four channels a store and the halo positions by face (a predict of 8192 blocks
-// 264 -> 221 us).
+// LDS reads and the products (60 us) run beside them. A predict of 8192 blocks, of
+// which this kernel is all but 35 us (210 us under the profiler): 396 us with the
+// zero padding selected per operand (20 instructions a read), 264 us with it built
+// into the layout, 221 us with conflict-free reads shared by the tiles, four
+// channels a store and the halo positions by face.
 constexpr int CNN_IN_HALFS = PADC * 8 > ACELLS * CNN_C ? PADC * 8 : ACELLS * CNN_C;
 
 __global__ __launch_bounds__(WG_THREADS) void k_cnn_infer(int nb, const int* __restrict__ nbr,

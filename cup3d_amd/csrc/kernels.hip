@@ -5,10 +5,13 @@
 // j = blockID*512 + iz*64 + iy*8 + ix of PoissonSolverAMR.cpp:76).
 //
 // One classical BiCGSTAB iteration (BiCGSTAB.cu:474-608) runs as five fused
-// kernels; every reduction is a deterministic two-pass sum (per-workgroup
-// partials, then the last workgroup adds them in workgroup order) and the
-// scalar recurrences run on the device, so the host only polls a status word
-// every few iterations:
+// kernels. Every reduction is a deterministic two-pass sum: per-workgroup
+// partials, then these in workgroup order, by every workgroup of the kernel that
+// uses the sum on grids of up to FIN_MAX_BLOCKS blocks, by a finalize kernel of
+// one workgroup beyond (and at the ends of batches). The scalar recurrences run
+// with them, on the device. The host of an FP64 solve follows a progress word
+// that each iteration writes, two iterations ahead of it; that of a mixed solve
+// waits every few iterations:
 //   K1 k_precond_dst<P> p = r + beta (p - omega nu)  [p = r after a restart,
 //                     rhat = r]; z1 = M^-1 p
 //   K2 k_spmv<DOT1>   nu = A z1; alpha = rho / ((rhat, nu) + eps)
