@@ -10,8 +10,9 @@
 //
 //   k_topo_init    clear the hash table and the info words (a fill kernel, no
 //                  memset), where the build before did not
-//   k_topo_insert  one thread per block: read it from the caller's list (pinned
-//                  host memory) and keep it, validate level and index, insert
+//   k_topo_insert  one thread per block: read it from the copy of the caller's
+//                  list in pinned host memory (a launch per 65 536 blocks, which
+//                  that memory holds) and keep it, validate level and index, insert
 //                  key(level, i, j, k) -> the smallest block id holding it
 //                  (open addressing, linear probing, 64-bit CAS)
 //   k_topo_tables  eight threads per block: one per face: same-level neighbour
